@@ -470,7 +470,6 @@ __global__ void a_reduce(int E, double Emod, int bilinear, const double *grad, c
 
 }  // namespace
 
-hipError_t launch_reaction_f32(wfx_ctx *c, const float *fi32, double *dev_out, hipStream_t s);
 std::vector<std::pair<void *, size_t>> fused_state_buffers(wfx_ctx *c);
 
 }  // namespace wfx
@@ -652,16 +651,14 @@ static int adjoint_forward(wfx_ctx *c, int nsteps, bool want_hist, hipStream_t s
   for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, false, st));
   LAUNCH(launch_fused_pack<T>(c, st));
   if (A->cfl) LAUNCH(launch_cfl_begin<T>(c, st, true));
-  T *v, *ud, *pa, *fi;
-  node_arrays<T>(c, &v, &ud, &pa, &fi);
+  const ReactRecord rec(c, want_hist ? A->hist : nullptr, nsteps, sizeof(T));
   for (int k = 0; k < nsteps; ++k) {
     if (k % A->every == 0) LAUNCH(save_ck<T>(c, k / A->every, st));
-    LAUNCH(fused_step<T>(c, k + 1 < nsteps, k, k + 1 == nsteps, nullptr, st));
-    if (want_hist && c->ngroups > 0) {
-      double *h = A->hist + (size_t)k * A->ng;
-      if constexpr (std::is_same<T, double>::value) LAUNCH(launch_reaction(c, 2, h, st));
-      else LAUNCH(launch_reaction_f32(c, c->fi32, h, st));
-    }
+    c->fused_rz = rec.row(k);
+    const hipError_t e = fused_step<T>(c, k + 1 < nsteps, k, k + 1 == nsteps, nullptr, st);
+    c->fused_rz = nullptr;
+    LAUNCH(e);
+    if (rec.full(k)) LAUNCH(launch_reaction_rows<T>(c, rec, k, st));
   }
   LAUNCH(launch_fused_unpack<T>(c, st));
   LAUNCH(launch_fused_phase<T>(c, 5, 0, st, -1));
@@ -788,6 +785,10 @@ int wfx_adjoint_forward(wfx_ctx *c, int nsteps, int checkpoint_every, double *re
   if (rc) return rc;
   rc = adj_alloc(c, nsteps, checkpoint_every);
   if (rc) return rc;
+  if (reaction_hist) {
+    rc = ensure_react_ring(c);
+    if (rc) return rc;
+  }
   hipStream_t st = as_stream(s);
   Adjoint *A = c->adj;
   A->cfl = c->prm.cfl > 0.0;

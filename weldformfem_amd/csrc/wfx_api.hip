@@ -70,6 +70,10 @@ static void free_all(wfx_ctx *c) {
   c->e32 = DevElem<float>();
   for (int d = 0; d < 3; ++d) { c->bc_nod[d] = nullptr; c->bc_val[d] = nullptr; c->bc_count[d] = 0; }
   c->react = nullptr;
+  c->react_bits = nullptr;
+  c->react_base = c->react_rank = nullptr;
+  c->react_ring = nullptr;
+  c->react_n = c->react_rows = 0;
   c->bc_slot = c->bc_mask = nullptr;
   c->bc_tab = nullptr;
   c->v32 = c->pa32 = c->ud32 = c->fi32 = nullptr;
@@ -1098,6 +1102,28 @@ int wfx_set_reaction_groups(wfx_ctx *c, const int *nodes, int count, const int *
   c->react = p;
   c->react_off = q;
   c->ngroups = ngroups;
+  // the record of a run keeps one value per distinct node: ranks in node order
+  std::vector<unsigned long long> bits((size_t)(c->N + 63) / 64, 0);
+  for (int k = 0; k < count; ++k) bits[nodes[k] >> 6] |= 1ull << (nodes[k] & 63);
+  std::vector<int> base(bits.size()), rank(count);
+  int nr = 0;
+  for (size_t w = 0; w < bits.size(); ++w) {
+    base[w] = nr;
+    nr += __builtin_popcountll(bits[w]);
+  }
+  for (int k = 0; k < count; ++k)
+    rank[k] = base[nodes[k] >> 6] + __builtin_popcountll(bits[nodes[k] >> 6] & ((1ull << (nodes[k] & 63)) - 1));
+  dfree(c, c->react_bits); dfree(c, c->react_base); dfree(c, c->react_rank);
+  char *ring = (char *)c->react_ring;
+  dfree(c, ring);
+  c->react_ring = nullptr;
+  WFX_CHECK_HIP(dalloc(c, &c->react_bits, bits.size()));
+  WFX_CHECK_HIP(dalloc(c, &c->react_base, base.size()));
+  WFX_CHECK_HIP(dalloc(c, &c->react_rank, rank.size()));
+  WFX_CHECK_HIP(hipMemcpy(c->react_bits, bits.data(), bits.size() * sizeof(bits[0]), hipMemcpyHostToDevice));
+  WFX_CHECK_HIP(hipMemcpy(c->react_base, base.data(), base.size() * sizeof(int), hipMemcpyHostToDevice));
+  if (count) WFX_CHECK_HIP(hipMemcpy(c->react_rank, rank.data(), rank.size() * sizeof(int), hipMemcpyHostToDevice));
+  c->react_n = nr;
   c->hist_cap = 0;  // history layout changed
   return WFX_OK;
 }
@@ -1240,8 +1266,6 @@ int wfx_impose_bca(wfx_ctx *c, int dim, wfx_stream s) {
   return WFX_OK;
 }
 
-// One SolveChungHulbert loop body (Solver_explicit.C:524-978, CPU order).
-// When hist is given, the reaction force after assembly goes to *hist.
 // per-step CFL time step (Solver_explicit.C:576-600) from the current
 // positions and velocities; the per-step kernels take dt by value, so it
 // comes back to the host
@@ -1285,7 +1309,9 @@ static int check_run_status(wfx_ctx *c, hipStream_t st) {
   return WFX_ERR_NONFINITE;
 }
 
-static int step_api(wfx_ctx *c, hipStream_t st, double *hist) {
+// One SolveChungHulbert loop body (Solver_explicit.C:524-978, CPU order);
+// with react_row the reaction nodes' forces after assembly are recorded there.
+static int step_api(wfx_ctx *c, hipStream_t st, double *react_row) {
   // external face areas every 10 steps, at the step's start (Solver_explicit.C:446-451)
   if (c->contact.on && c->contact.step_count % 10 == 0) LAUNCH(contact_face_areas(c, st));
   LAUNCH(launch_update_prediction(c, st));
@@ -1307,7 +1333,7 @@ static int step_api(wfx_ctx *c, hipStream_t st, double *hist) {
   LAUNCH(BY_PRECISION(c, launch_hourglass, c, st));
   if (c->contact.on) LAUNCH(contact_forces(c, st));  // CalcContactForces (Solver_explicit.C:769-770)
   LAUNCH(BY_PRECISION(c, launch_assembly, c, st));
-  if (hist && c->ngroups) LAUNCH(launch_reaction(c, 2, hist, st));
+  if (react_row) LAUNCH(launch_reaction_gather(c, react_row, st));
   LAUNCH(launch_calc_accel(c, st));
   for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, true, st));
   LAUNCH(launch_correction_accvel(c, st));
@@ -1353,6 +1379,24 @@ static int ensure_hist(wfx_ctx *c, int nsteps, double **out) {
   return WFX_OK;
 }
 
+}  // extern "C"
+
+// Rows of the reaction record: 512 steps, fewer when those would take more
+// than 64 MiB (the 40,401-node face of the 200x200x100 block: 207), at least
+// one; the sums run once per filled ring, so a longer ring gains nothing.
+int wfx::ensure_react_ring(wfx_ctx *c) {
+  if (c->ngroups == 0 || c->react_ring) return WFX_OK;
+  const size_t row = (size_t)std::max(c->react_n, 1) * sizeof(double);
+  const size_t rows = std::min<size_t>(512, std::max<size_t>(1, ((size_t)64 << 20) / row));
+  char *p = nullptr;
+  WFX_CHECK_HIP(dalloc(c, &p, row * rows));
+  c->react_ring = p;
+  c->react_rows = (int)rows;
+  return WFX_OK;
+}
+
+extern "C" {
+
 int wfx_step_api(wfx_ctx *c, wfx_stream s) {
   REQUIRE_MESH(c);
   REQUIRE(c->initialized, WFX_ERR_STATE, "call wfx_init first");
@@ -1367,13 +1411,16 @@ int wfx_run(wfx_ctx *c, int nsteps, double *reaction_hist, wfx_stream s) {
   double *dh = nullptr;
   if (reaction_hist && nsteps > 0) {
     int rc = ensure_hist(c, nsteps, &dh);
+    if (!rc) rc = ensure_react_ring(c);
     if (rc) return rc;
   }
   const int ng = c->ngroups > 0 ? c->ngroups : 1;
   c->dt_hist_h.clear();
+  const ReactRecord rec(c, dh, nsteps, sizeof(double));
   for (int k = 0; k < nsteps; ++k) {
-    int rc = step_api(c, st, dh ? dh + (long)k * ng : nullptr);
+    int rc = step_api(c, st, (double *)rec.row(k));
     if (rc) return rc;
+    if (rec.full(k)) LAUNCH(launch_reaction_rows<double>(c, rec, k, st));
   }
   if (dh) {
     WFX_CHECK_HIP(hipMemcpyAsync(reaction_hist, dh, (size_t)nsteps * ng * sizeof(double), hipMemcpyDeviceToHost, st));
@@ -1393,6 +1440,7 @@ int wfx_step_fused(wfx_ctx *c, int nsteps, double *reaction_hist, wfx_stream s) 
   double *dh = nullptr;
   if (reaction_hist) {
     int rc = ensure_hist(c, nsteps, &dh);
+    if (!rc) rc = ensure_react_ring(c);
     if (rc) return rc;
   }
   int rc = ensure_dt_hist(c, nsteps);
@@ -1648,6 +1696,7 @@ int wfx_graph_capture(wfx_ctx *c, int nsteps, int with_reaction, wfx_stream s) {
   double *dh = nullptr;
   if (with_reaction) {
     int rc = ensure_hist(c, nsteps, &dh);
+    if (!rc) rc = ensure_react_ring(c);
     if (rc) return rc;
   }
   {

@@ -40,6 +40,7 @@
 #include "wfx_cluster.hpp"
 #include "wfx_contact.hpp"
 #include "wfx_kernels.hpp"
+#include "wfx_launch.hpp"
 
 namespace wfx {
 namespace {
@@ -1223,7 +1224,26 @@ struct NodeParams {
   double *vmax_part;  //   and the per-block largest predicted speed
   const double *qcont;  // contact heat conduction per node (thermal with contact), or null
   double cp_T;
+  // reaction record (rz null: none): one bit per reaction node, the rank of
+  // each word's first one, and the step's row of z forces (the nodal type)
+  const unsigned long long *rbits;
+  const int *rbase;
+  void *rz;
 };
+
+// The step's z force of a reaction node into its row.  A wavefront's 64 nodes
+// share one word of bits, so the test costs one scalar load; storing every
+// node's force instead (and reading the reaction nodes' back) cost 24 B per
+// node and step.
+template <typename T>
+__device__ __forceinline__ void record_reaction(const NodeParams &np, int i, double fz) {
+  if (!np.rz) return;
+  const int w = __builtin_amdgcn_readfirstlane(i >> 6);
+  const unsigned long long b = np.rbits[w];
+  const int l = i & 63;
+  if ((b >> l) & 1ull)
+    static_cast<T *>(np.rz)[np.rbase[w] + __popcll(b & ((1ull << l) - 1ull))] = (T)fz;
+}
 
 // the step-length terms of NodeParams for step length dt (same expressions
 // as node_params on the host)
@@ -1318,6 +1338,7 @@ __device__ __forceinline__ double node_update(
   for (int d = 0; d < 3; ++d)
     if (!isfinite(f[d])) { f[d] = 0.0; ++bad; }
   if (bad) atomicAdd(status, bad);
+  record_reaction<T>(np, i, f[2]);
   const int slot = s.slot;
   const int mask = slot >= 0 ? bc_mask[slot] : 0;
   const double m = s.m;
@@ -1545,9 +1566,6 @@ hipError_t launch_rigid_update(wfx_ctx *c, bool device_dt, hipStream_t s) {
 
 }  // namespace
 
-hipError_t launch_reaction(wfx_ctx *c, int dim, double *dev_out, hipStream_t s);
-hipError_t launch_reaction_f32(wfx_ctx *c, const float *fi32, double *dev_out, hipStream_t s);
-
 template <typename T>
 hipError_t launch_vsum0(wfx_ctx *c, hipStream_t s) {
   if (c->f2_lanes) {
@@ -1585,6 +1603,9 @@ inline NodeParams node_params(wfx_ctx *c, int predict) {
   np.vmax_part = nullptr;
   np.qcont = (c->thermal.on && c->contact.on) ? c->contact.q_cont : nullptr;
   np.cp_T = c->thermal.cp_T;
+  np.rbits = c->react_bits;
+  np.rbase = c->react_base;
+  np.rz = c->fused_rz;
   return np;
 }
 
@@ -1803,7 +1824,7 @@ hipError_t launch_fused_unpack(wfx_ctx *c, hipStream_t s) {
 
 template <typename T>
 hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t s, hipEvent_t *ev) {
-  constexpr bool mixed = !std::is_same<T, double>::value;
+  const ReactRecord rec(c, hist, nsteps, sizeof(T));
   {
     hipError_t e = launch_fused_pack<T>(c, s);
     if (e != hipSuccess) return e;
@@ -1817,9 +1838,8 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
       hipError_t e = launch_ext_face_areas(c, s);  // every 10 steps, at the step's start
       if (e != hipSuccess) return e;
     }
-    // the internal force is observed after the run and by the reaction
-    // history, the element outputs after the run
-    c->fused_write_fi = (k + 1 == nsteps || hist) ? 1 : 0;
+    // the internal force and the element outputs are observed after the run
+    c->fused_write_fi = (k + 1 == nsteps) ? 1 : 0;
     c->fused_write_out = (k + 1 == nsteps) ? 1 : 0;
     // the increment is predicted again from v' and prev_a after the first
     // step, unless each step has its own length
@@ -1832,7 +1852,9 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
         hipError_t e = hipEventRecord(ev[4 * k + ph - 1], s);
         if (e != hipSuccess) return e;
       }
+      c->fused_rz = ph == 4 ? rec.row(k) : nullptr;
       hipError_t e = launch_fused_phase<T>(c, ph, k + 1 < nsteps, s, k);
+      c->fused_rz = nullptr;
       if (e != hipSuccess) {
         c->fused_write_fi = c->fused_write_out = c->fused_read_ud = c->fused_write_ud = 1;
         c->fused_run_first = c->fused_run_last = 1;
@@ -1845,9 +1867,8 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
       hipError_t e = hipEventRecord(ev[4 * nsteps], s);
       if (e != hipSuccess) return e;
     }
-    if (hist) {
-      hipError_t e = mixed ? launch_reaction_f32(c, c->fi32, hist + (long)k * c->ngroups, s)
-                           : launch_reaction(c, 2, hist + (long)k * c->ngroups, s);
+    if (rec.full(k)) {
+      hipError_t e = launch_reaction_rows<T>(c, rec, k, s);
       if (e != hipSuccess) return e;
     }
   }

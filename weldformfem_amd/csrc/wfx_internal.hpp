@@ -190,6 +190,14 @@ struct wfx_ctx {
   int *react_off = nullptr;         // group g = react[react_off[g] .. react_off[g+1])
   std::vector<int> react_off_h;
   int ngroups = 0;
+  // reaction record of a run: the distinct reaction nodes as one bit per node
+  // (64 to a word) with each word's first rank, each list entry's rank, and
+  // the rows of the z forces [react_rows][react_n] the node passes fill
+  unsigned long long *react_bits = nullptr;
+  int *react_base = nullptr, *react_rank = nullptr;
+  int react_n = 0, react_rows = 0;
+  void *react_ring = nullptr;
+  void *fused_rz = nullptr;  // the row the next fused node pass fills (set inside runs)
   // per-node Dirichlet data for the fused node pass: slot or -1, bit mask of
   // constrained directions and the three prescribed values per slot
   int *bc_slot = nullptr, *bc_mask = nullptr;

@@ -75,10 +75,22 @@ hipError_t launch_reaction(wfx_ctx *c, int dim, double *dev_out, hipStream_t s) 
   return hipGetLastError();
 }
 
-hipError_t launch_reaction_f32(wfx_ctx *c, const float *fi32, double *dev_out, hipStream_t s) {
-  if (c->ngroups == 0) return hipSuccess;
-  hipLaunchKernelGGL((k_reaction<float>), dim3(c->ngroups), dim3(kBlock), 0, s, c->react_off, c->react,
-                     fi32 + 2L * c->N, dev_out);
+template <typename T>
+hipError_t launch_reaction_rows(wfx_ctx *c, const ReactRecord &r, int k, hipStream_t s) {
+  const int k0 = r.first(k);
+  hipLaunchKernelGGL((k_reaction_rows<T>), dim3(c->ngroups, k + 1 - k0), dim3(kBlock), 0, s, c->react_off,
+                     c->react_rank, static_cast<const T *>(c->react_ring), c->react_n,
+                     r.hist + (long)k0 * c->ngroups);
+  return hipGetLastError();
+}
+template hipError_t launch_reaction_rows<double>(wfx_ctx *, const ReactRecord &, int, hipStream_t);
+template hipError_t launch_reaction_rows<float>(wfx_ctx *, const ReactRecord &, int, hipStream_t);
+
+hipError_t launch_reaction_gather(wfx_ctx *c, double *row, hipStream_t s) {
+  const int count = (int)c->react_h.size();
+  if (count == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_reaction_gather, dim3(nblocks(count)), dim3(kBlock), 0, s, count, c->react, c->react_rank,
+                     c->nd.fi + 2L * c->N, row);
   return hipGetLastError();
 }
 

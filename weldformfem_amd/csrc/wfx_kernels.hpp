@@ -1132,6 +1132,36 @@ __global__ __launch_bounds__(kBlock) void k_reaction(const int *__restrict__ gof
   if (threadIdx.x == 0) out[g] = r;
 }
 
+// The same sums for a run of steps at once: row s of `ring` holds the force
+// component of the distinct reaction nodes at step s (by rank), written by
+// the node passes; one work-group per (group, step) adds them in
+// k_reaction's order, so the history equals the per-step sums bit for bit.
+// One launch per step left the chip to one work-group per group for as long
+// as it took (the 40,401-node face of the 200x200x100 block: 102 us of a
+// 760 us step); here the steps run side by side.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_reaction_rows(const int *__restrict__ goff,
+                                                          const int *__restrict__ rank,
+                                                          const T *__restrict__ ring, int nr,
+                                                          double *__restrict__ out) {
+  __shared__ double sh[kBlock];
+  const int g = blockIdx.x, k0 = goff[g], k1 = goff[g + 1];
+  const T *row = ring + (long)blockIdx.y * nr;
+  double s = 0.0;
+  for (int k = k0 + threadIdx.x; k < k1; k += blockDim.x) s += (double)row[rank[k]];
+  const double r = block_sum(s, sh);
+  if (threadIdx.x == 0) out[(long)blockIdx.y * gridDim.x + g] = r;
+}
+
+// a row of that record from the assembled forces (per-step path)
+__global__ __launch_bounds__(kBlock) void k_reaction_gather(int count, const int *__restrict__ nodes,
+                                                            const int *__restrict__ rank,
+                                                            const double *__restrict__ fcomp,
+                                                            double *__restrict__ row) {
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k < count) row[rank[k]] = fcomp[nodes[k]];  // a node listed twice writes the same value twice
+}
+
 // calcMinEdgeLength (Domain_d.C:2224-2260): per-block minimum, then one block
 __global__ __launch_bounds__(kBlock) void k_min_edge(int E, int N, int n, const int *__restrict__ elnod,
                                                      const double *__restrict__ x,

@@ -42,6 +42,32 @@ WFX_DECLARE_SPECIALISATIONS(float)
 // step and after the last, for per-phase durations of a run
 template <typename T>
 hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t s, hipEvent_t *ev);
+
+// The reaction record of a run of nsteps steps into hist (null, or no
+// reaction group: nothing is recorded): the node pass of step k fills row(k),
+// and where full(k) holds launch_reaction_rows sums the rows filled since
+// the last time.
+struct ReactRecord {
+  const wfx_ctx *c;
+  double *hist;
+  int nsteps;
+  size_t es;  // bytes of a recorded value
+  ReactRecord(const wfx_ctx *c_, double *hist_, int nsteps_, size_t es_)
+      : c(c_), hist(c_->ngroups > 0 && c_->react_ring ? hist_ : nullptr), nsteps(nsteps_), es(es_) {}
+  void *row(int k) const {
+    return hist ? static_cast<char *>(c->react_ring) + (size_t)(k % c->react_rows) * c->react_n * es : nullptr;
+  }
+  bool full(int k) const { return hist && (k + 1 == nsteps || (k + 1) % c->react_rows == 0); }
+  int first(int k) const { return k / c->react_rows * c->react_rows; }  // the step of the ring's first row
+};
+template <typename T> hipError_t launch_reaction_rows(wfx_ctx *c, const ReactRecord &r, int k, hipStream_t s);
+extern template hipError_t launch_reaction_rows<double>(wfx_ctx *, const ReactRecord &, int, hipStream_t);
+extern template hipError_t launch_reaction_rows<float>(wfx_ctx *, const ReactRecord &, int, hipStream_t);
+// row k of the record from nd.fi (per-step path)
+hipError_t launch_reaction_gather(wfx_ctx *c, double *row, hipStream_t s);
+// the context's ring of recorded rows, allocated once per set of reaction nodes
+int ensure_react_ring(wfx_ctx *c);
+
 template <typename T> hipError_t launch_vsum0(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_fused_phase(wfx_ctx *c, int phase, int predict, hipStream_t s, int step);
 template <typename T> hipError_t launch_cfl_step(wfx_ctx *c, int step, hipStream_t s);
@@ -78,7 +104,6 @@ hipError_t launch_correction_pos(wfx_ctx *c, hipStream_t s);
 hipError_t launch_reaction(wfx_ctx *c, int dim, double *dev_out, hipStream_t s);
 hipError_t launch_min_edge(wfx_ctx *c, double *partial, double *dev_out, hipStream_t s);
 int min_edge_partial_count(wfx_ctx *c);
-hipError_t launch_reaction_f32(wfx_ctx *c, const float *fi32, double *dev_out, hipStream_t s);
 
 // rigid-surface contact, per-step API (wfx_k64.hip)
 hipError_t contact_face_areas(wfx_ctx *c, hipStream_t s);
