@@ -25,6 +25,7 @@ UNITS = [
     ("wfx_api.hip", ["-ffp-contract=off"]),
     ("wfx_adjoint.hip", ["-ffp-contract=off"]),
     ("wfx_frames.hip", []),
+    ("wfx_fields.hip", []),
 ]
 
 

@@ -166,7 +166,7 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
   A(c->nd.voln0_sum, N) A(c->nd.anp_ratio, N) A(c->nd.T, N)
   A(c->ms.elnod, n * E) A(c->ms.nodel, n * E) A(c->ms.nodel_loc, n * E) A(c->ms.nodel_offset, N)
   A(c->ms.nodel_count, N) A(c->ms.nodel_pk, n * E) A(c->ms.nodel_pad, 8 * N) A(c->bc_slot, N)
-  A(c->scalars, 64) A(c->status, 16)
+  A(c->scalars, 64) A(c->status, 16) A(c->ms.o2s, E)
   c->ms.ncl = plan.clusters();
   c->ms.nslot = plan.slots();
   // more than 12 elements per node on average (tetrahedra: about 23): the
@@ -213,6 +213,7 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     for (size_t a = 0; a < n; ++a) es[a * E + k] = c->elnod_h[(size_t)c->el_s2o[k] * n + a];
   std::vector<int> nodel_s(n * E);
   for (size_t k = 0; k < n * E; ++k) nodel_s[k] = c->el_o2s[c->nodel_h[k]];
+  WFX_CHECK_HIP(hipMemcpy(c->ms.o2s, c->el_o2s.data(), E * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->nd.x, xs.data(), 3 * N * sizeof(double), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.elnod, es.data(), n * E * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel, nodel_s.data(), n * E * sizeof(int), hipMemcpyHostToDevice));
@@ -487,6 +488,7 @@ int wfx_create(wfx_ctx **out, int precision) {
 int wfx_destroy(wfx_ctx *c) {
   if (!c) return WFX_OK;
   free_all(c);
+  staging_free(c);
   delete c;
   return WFX_OK;
 }
@@ -1870,6 +1872,11 @@ static bool fused_intermediate(const char *name) {
   return false;
 }
 
+static FieldMove field_move(const wfx_ctx *c, const FieldDesc &f) {
+  return FieldMove{f.dev, f.cnt, f.rows, f.kind == 1, f.elem && c->precision == WFX_FP32_MIXED,
+                   f.per_elem ? c->ms.o2s : nullptr};
+}
+
 int wfx_get_field(wfx_ctx *c, const char *name, void *host, long count) {
   REQUIRE_MESH(c);
   FieldDesc f;
@@ -1879,10 +1886,10 @@ int wfx_get_field(wfx_ctx *c, const char *name, void *host, long count) {
           std::string(name) + " is a per-step intermediate not kept by wfx_step_fused; "
           "call the per-step entry point that produces it first");
   WFX_CHECK_HIP(hipDeviceSynchronize());
-  const long cnt = f.cnt;
-  // device column of host item i (element fields are stored in cluster order)
-  auto col = [&](long i) { return f.per_elem ? (long)c->el_o2s[i] : i; };
   if (f.is_int) {
+    const long cnt = f.cnt;
+    // device column of host item i (element fields are stored in cluster order)
+    auto col = [&](long i) { return f.per_elem ? (long)c->el_o2s[i] : i; };
     std::vector<int> tmp(cnt * f.rows);
     WFX_CHECK_HIP(hipMemcpy(tmp.data(), f.dev, tmp.size() * sizeof(int), hipMemcpyDeviceToHost));
     int *h = (int *)host;
@@ -1893,21 +1900,7 @@ int wfx_get_field(wfx_ctx *c, const char *name, void *host, long count) {
       }
     return WFX_OK;
   }
-  int drows = f.kind == 1 ? 3 : f.rows;
-  std::vector<double> tmp((size_t)drows * cnt);
-  int rc = download_real(c, tmp.data(), f.dev, tmp.size(), f.elem);
-  if (rc) return rc;
-  double *h = (double *)host;
-  if (f.kind == 1) {
-    for (long i = 0; i < cnt; ++i) {
-      h[i * 6 + 0] = h[i * 6 + 1] = h[i * 6 + 2] = 0.0;
-      for (int r = 0; r < 3; ++r) h[i * 6 + 3 + r] = tmp[(long)r * cnt + col(i)];
-    }
-  } else {
-    for (long i = 0; i < cnt; ++i)
-      for (int r = 0; r < f.rows; ++r) h[i * f.rows + r] = tmp[(long)r * cnt + col(i)];
-  }
-  return WFX_OK;
+  return field_to_host(c, field_move(c, f), (double *)host);
 }
 
 int wfx_set_field(wfx_ctx *c, const char *name, const void *host, long count) {
@@ -1917,24 +1910,9 @@ int wfx_set_field(wfx_ctx *c, const char *name, const void *host, long count) {
   REQUIRE(host && count == f.cnt * f.rows, WFX_ERR_ARG, std::string("size mismatch for field ") + name);
   REQUIRE(!f.is_int, WFX_ERR_ARG, "connectivity and CSR are set through the mesh calls");
   WFX_CHECK_HIP(hipDeviceSynchronize());
-  const long cnt = f.cnt;
   const double *h = (const double *)host;
-  int drows = f.kind == 1 ? 3 : f.rows;
-  std::vector<double> tmp((size_t)drows * cnt);
-  auto col = [&](long i) { return f.per_elem ? (long)c->el_o2s[i] : i; };
-  if (f.kind == 1) {
-    for (long i = 0; i < cnt; ++i)
-      for (int r = 0; r < 3; ++r) tmp[(long)r * cnt + col(i)] = h[i * 6 + 3 + r];
-  } else {
-    for (long i = 0; i < cnt; ++i)
-      for (int r = 0; r < f.rows; ++r) tmp[(long)r * cnt + col(i)] = h[i * f.rows + r];
-  }
-  if (!std::strcmp(name, "fe")) {
-    c->has_fe = 0;
-    for (double v : tmp)
-      if (v != 0.0) { c->has_fe = 1; break; }
-  }
-  int rc = upload_real(c, f.dev, tmp.data(), tmp.size(), f.elem);
+  if (!std::strcmp(name, "fe")) c->has_fe = std::any_of(h, h + count, [](double v) { return v != 0.0; });
+  int rc = field_from_host(c, field_move(c, f), h);
   if (rc == WFX_OK && (!std::strcmp(name, "rho") || !std::strcmp(name, "vol0"))) rc = scan_elements(c);
   return rc;
 }

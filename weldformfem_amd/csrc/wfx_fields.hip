@@ -1,0 +1,266 @@
+// Field transfer between the host's layout ([items][components], the
+// reference's element order, double) and the device's ([components][items],
+// stored element order, double or float).
+//
+// The kernels read and write pinned host memory directly, so that the
+// transposition, the element permutation and the float conversion happen on
+// the device, in the same pass that crosses the host link.  Before, the host
+// did them in one thread over a pageable copy: the stress of the 4M-element
+// block (192 MB) took 92 ms to read, now 12; a nodal vector of one element 27
+// us, now 19.  What bounds it: the host link (57 GB/s pinned) and, for the
+// fresh pages of a new array, the host's page faults, which is why several
+// threads copy from the pinned ring to the caller's memory.
+#include <algorithm>
+#include <atomic>
+#include <condition_variable>
+#include <cstring>
+#include <exception>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "../../include/wfx.h"
+#include "wfx_internal.hpp"
+#include "wfx_launch.hpp"
+
+namespace wfx {
+
+// The pinned ring: kSlots chunks of kChunkBytes.  Measured on the stress of
+// the 4M-element block (192 MB), read into the same array again / a new one /
+// set: 1 MiB chunks 9.7 / 15.8 / 4.7 ms, 2 MiB 7.3 / 14.6 / 4.1, 4 MiB 5.7 /
+// 11.9 / 4.0 (the link alone: 3.4); 12 or 16 threads instead of 8 gain nothing
+// at 4 MiB.  Transfers of one chunk use a buffer of their own.
+constexpr size_t kChunkBytes = (size_t)4 << 20;
+constexpr int kSlots = 16, kCopyThreads = 8;
+
+struct Staging {
+  char *small = nullptr;  // one chunk
+  char *ring = nullptr;   // kSlots chunks, allocated by the first transfer that needs them
+  hipEvent_t ev[kSlots] = {};
+};
+
+void staging_free(wfx_ctx *c) {
+  if (!c->stage) return;
+  for (hipEvent_t e : c->stage->ev)
+    if (e) (void)hipEventDestroy(e);
+  if (c->stage->small) (void)hipHostFree(c->stage->small);
+  if (c->stage->ring) (void)hipHostFree(c->stage->ring);
+  delete c->stage;
+  c->stage = nullptr;
+}
+
+static int staging_ready(wfx_ctx *c, bool ring) {
+  if (!c->stage) c->stage = new Staging();
+  Staging &s = *c->stage;
+  if (!ring && !s.small) WFX_CHECK_HIP(hipHostMalloc((void **)&s.small, kChunkBytes, hipHostMallocPortable));
+  if (ring && !s.ring) {
+    for (hipEvent_t &e : s.ev)
+      if (!e) WFX_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    WFX_CHECK_HIP(hipHostMalloc((void **)&s.ring, kChunkBytes * kSlots, hipHostMallocPortable));
+  }
+  return WFX_OK;
+}
+
+namespace {
+
+constexpr int kB = 256;
+
+// device row of host component r, or -1 (the spin's zero diagonal: host
+// columns 0..2 of 6, device rows 0..2 for columns 3..5)
+template <bool SPIN>
+__device__ __forceinline__ int device_row(int r) {
+  return SPIN ? r - 3 : r;
+}
+
+// host values [k0, k0 + n) of the flat [items][rows] array, one per thread:
+// consecutive threads write consecutive host addresses (full link packets);
+// the scattered device reads stay in L2, which outruns the link by far
+template <typename T, bool SPIN>
+__global__ __launch_bounds__(kB) void k_field_out(long k0, long n, int rows, long cnt, const int *__restrict__ perm,
+                                                  const T *__restrict__ dev, double *__restrict__ host) {
+  const long t = (long)blockIdx.x * kB + threadIdx.x;
+  if (t >= n) return;
+  const long k = k0 + t, i = k / rows;
+  const int r = device_row<SPIN>((int)(k - i * rows));
+  double v = 0.0;
+  if (r >= 0) v = (double)dev[(long)r * cnt + (perm ? (long)perm[i] : i)];
+  host[t] = v;
+}
+template <typename T, bool SPIN>
+__global__ __launch_bounds__(kB) void k_field_in(long k0, long n, int rows, long cnt, const int *__restrict__ perm,
+                                                 const double *__restrict__ host, T *__restrict__ dev) {
+  const long t = (long)blockIdx.x * kB + threadIdx.x;
+  if (t >= n) return;
+  const long k = k0 + t, i = k / rows;
+  const int r = device_row<SPIN>((int)(k - i * rows));
+  if (r >= 0) dev[(long)r * cnt + (perm ? (long)perm[i] : i)] = (T)host[t];
+}
+
+template <bool OUT>
+hipError_t launch_chunk(const FieldMove &f, long k0, long n, double *pinned) {
+  const dim3 grid((unsigned)((n + kB - 1) / kB)), block(kB);
+  auto go = [&](auto *dev, auto spin) {
+    using T = std::remove_pointer_t<decltype(dev)>;
+    constexpr bool S = decltype(spin)::value;
+    if constexpr (OUT)
+      hipLaunchKernelGGL((k_field_out<T, S>), grid, block, 0, nullptr, k0, n, f.rows, f.cnt, f.perm,
+                         (const T *)dev, pinned);
+    else
+      hipLaunchKernelGGL((k_field_in<T, S>), grid, block, 0, nullptr, k0, n, f.rows, f.cnt, f.perm,
+                         (const double *)pinned, dev);
+  };
+  if (f.f32) {
+    if (f.spin) go((float *)f.dev, std::true_type());
+    else go((float *)f.dev, std::false_type());
+  } else {
+    if (f.spin) go((double *)f.dev, std::true_type());
+    else go((double *)f.dev, std::false_type());
+  }
+  return hipGetLastError();
+}
+
+// Threads that copy chunks between the ring and the caller's array: chunk c
+// is handed out once ready exceeds c, and done[c] is set when its copy ended.
+// Host memory only; every GPU call stays in the calling thread.
+class Copiers {
+ public:
+  Copiers(long chunks, int threads, void (*copy)(void *, long), void *arg)
+      : done_(chunks, 0), chunks_(chunks), copy_(copy), arg_(arg) {
+    try {
+      for (int t = 0; t < threads; ++t) th_.emplace_back([this] { work(); });
+    } catch (const std::exception &) {  // fewer threads (or none: the caller copies)
+    }
+  }
+  ~Copiers() {
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      stop_ = true;
+    }
+    cv_.notify_all();
+    for (auto &t : th_) t.join();
+  }
+  void hand_out(long upto) {  // chunks below upto may be copied
+    if (th_.empty()) {
+      for (; ready_ < upto; ++ready_) {
+        copy_(arg_, ready_);
+        done_[ready_] = 1;
+      }
+      return;
+    }
+    {
+      std::lock_guard<std::mutex> l(mu_);
+      ready_ = upto;
+    }
+    cv_.notify_all();
+  }
+  void wait(long c) {  // until chunk c (handed out before) is copied
+    std::unique_lock<std::mutex> l(mu_);
+    cv_done_.wait(l, [&] { return done_[c] != 0; });
+  }
+
+ private:
+  void work() {
+    for (;;) {
+      long c;
+      {
+        std::unique_lock<std::mutex> l(mu_);
+        cv_.wait(l, [&] { return stop_ || next_ < ready_; });
+        if (next_ >= ready_) return;  // stopping, nothing handed out is left
+        c = next_++;
+      }
+      copy_(arg_, c);
+      {
+        std::lock_guard<std::mutex> l(mu_);
+        done_[c] = 1;
+      }
+      cv_done_.notify_one();
+    }
+  }
+  std::vector<char> done_;
+  long chunks_, ready_ = 0, next_ = 0;
+  void (*copy_)(void *, long);
+  void *arg_;
+  bool stop_ = false;
+  std::mutex mu_;
+  std::condition_variable cv_, cv_done_;
+  std::vector<std::thread> th_;
+};
+
+struct CopyJob {
+  char *ring, *user;
+  long total;  // bytes
+  bool out;
+  static void run(void *p, long c) {
+    const CopyJob &j = *static_cast<CopyJob *>(p);
+    char *a = j.ring + (size_t)(c % kSlots) * kChunkBytes, *b = j.user + (size_t)c * kChunkBytes;
+    const size_t n = std::min<size_t>(kChunkBytes, (size_t)j.total - (size_t)c * kChunkBytes);
+    if (j.out) std::memcpy(b, a, n);
+    else std::memcpy(a, b, n);
+  }
+};
+
+// The caller has synchronised the device.  Returns when the transfer is over.
+template <bool OUT>
+int move_field(wfx_ctx *c, const FieldMove &f, double *user) {
+  const long values = f.cnt * f.rows, per = (long)(kChunkBytes / sizeof(double));
+  if (values == 0) return WFX_OK;
+  const long chunks = (values + per - 1) / per;
+  int rc = staging_ready(c, chunks > 1);
+  if (rc) return rc;
+  Staging &s = *c->stage;
+  if (chunks == 1) {
+    double *pin = (double *)s.small;
+    if (!OUT) std::memcpy(pin, user, values * sizeof(double));
+    WFX_CHECK_HIP(launch_chunk<OUT>(f, 0, values, pin));
+    WFX_CHECK_HIP(hipStreamSynchronize(nullptr));
+    if (OUT) std::memcpy(user, pin, values * sizeof(double));
+    return WFX_OK;
+  }
+  auto slot = [&](long k) { return (double *)(s.ring + (size_t)(k % kSlots) * kChunkBytes); };
+  auto launch = [&](long k) {
+    hipError_t e = launch_chunk<OUT>(f, k * per, std::min(per, values - k * per), slot(k));
+    return e == hipSuccess ? hipEventRecord(s.ev[k % kSlots], nullptr) : e;
+  };
+  CopyJob job{s.ring, (char *)user, values * (long)sizeof(double), OUT};
+  hipError_t err = hipSuccess;
+  {
+    Copiers cp(chunks, (int)std::min<long>(kCopyThreads, chunks), CopyJob::run, &job);
+    if (OUT) {
+      long sent = 0;
+      for (long k = 0; k < chunks && err == hipSuccess; ++k) {
+        for (; sent < chunks && sent < k + kSlots && err == hipSuccess; ++sent) {
+          if (sent >= kSlots) cp.wait(sent - kSlots);  // handed out: sent - kSlots < k
+          err = launch(sent);
+        }
+        if (err == hipSuccess) err = hipEventSynchronize(s.ev[k % kSlots]);
+        if (err == hipSuccess) cp.hand_out(k + 1);
+      }
+    } else {
+      cp.hand_out(std::min<long>(kSlots, chunks));
+      for (long k = 0; k < chunks && err == hipSuccess; ++k) {
+        cp.wait(k);
+        err = launch(k);
+        // the slot of chunk k takes chunk k + kSlots once the kernel has read
+        // it; freed half a ring late, so that the copies stay ahead
+        const long f0 = k - kSlots / 2;
+        if (err == hipSuccess && f0 >= 0 && f0 + kSlots < chunks) {
+          err = hipEventSynchronize(s.ev[f0 % kSlots]);
+          if (err == hipSuccess) cp.hand_out(f0 + kSlots + 1);
+        }
+      }
+    }
+  }  // the copies handed out end here
+  const hipError_t end = hipStreamSynchronize(nullptr);  // no kernel uses the ring any more
+  WFX_CHECK_HIP(err);
+  WFX_CHECK_HIP(end);
+  return WFX_OK;
+}
+
+}  // namespace
+
+int field_to_host(wfx_ctx *c, const FieldMove &f, double *host) { return move_field<true>(c, f, host); }
+int field_from_host(wfx_ctx *c, const FieldMove &f, const double *host) {
+  return move_field<false>(c, f, const_cast<double *>(host));
+}
+
+}  // namespace wfx

@@ -115,6 +115,20 @@ hipError_t contact_rigid_update(wfx_ctx *c, double dt, hipStream_t s);
 // and around the adjoint's recomputation)
 std::vector<std::pair<void *, size_t>> fused_state_buffers(wfx_ctx *c);
 void adjoint_free(wfx_ctx *c);
+
+// A real field's transfer: host [cnt][rows] double, device [rows][cnt]
+// (spin: 3 device rows for host columns 3..5 of 6, the others zero), float
+// when f32; perm maps a host item to its device column (null: the same).
+// The device must be idle; both return when the transfer is over.
+struct FieldMove {
+  void *dev;
+  long cnt;
+  int rows, spin, f32;
+  const int *perm;
+};
+int field_to_host(wfx_ctx *c, const FieldMove &f, double *host);
+int field_from_host(wfx_ctx *c, const FieldMove &f, const double *host);
+void staging_free(wfx_ctx *c);
 void frames_free(wfx_ctx *c);
 void frames_join(wfx_ctx *c);
 
