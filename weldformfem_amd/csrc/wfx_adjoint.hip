@@ -164,16 +164,15 @@ struct NodeAdj {
 // vv = v' + gamma dt ac, ud = ud + beta dt^2 ac and the prediction
 // ud' = dt (vv + (0.5 - beta) dt ac), v'' = vv + (1 - gamma) dt ac, with ac the
 // corrected acceleration (1/(1-alpha)) (a - alpha pa)
-__global__ void a_node1(int N, int E, NodeAdj P, const double *rec, const double *fe, const int *bc_slot,
-                        const int *bc_mask, const int *rgroup, const double *hbar_k, double *xb, double *vb,
+__global__ void a_node1(int N, int E, NodeAdj P, const double *rec, const double *fe, const int *bc_word,
+                        const int *rgroup, const double *hbar_k, double *xb, double *vb,
                         double *udb, double *pab, double *fib, double *mb, double *dtb) {
   int i = (int)tid();
   if (i >= N) return;
   const long Ns = N;
   const double *fi = rec + 6 * Ns, m = rec[9 * Ns + i];
   const double *vrec = rec + 3 * Ns, *parec = rec + 11 * Ns + 7L * E;
-  const int slot = bc_slot[i];
-  const int mask = slot >= 0 ? bc_mask[slot] : 0;
+  const int mask = bc_word[i] & 7;
   const double dt = P.dt, ia = 1.0 / (1.0 - P.alpha);
   double mbar = 0.0, dtbar = 0.0;
   for (int d = 0; d < 3; ++d) {
@@ -739,7 +738,7 @@ static int adjoint_backward(wfx_ctx *c, hipStream_t st) {
       const double *rec = A->slot + (size_t)(k - k0) * A->slot_stride;
       if (A->cfl) NP.dt = K.dt = A->dts_h[k];
       double *dtb_n = A->cfl ? A->dtb : nullptr, *dtb_e = A->cfl ? A->dtb + N : nullptr;
-      hipLaunchKernelGGL(a_node1, dim3(nb(N)), dim3(kB), 0, st, N, E, NP, rec, c->nd.fe, c->bc_slot, c->bc_mask,
+      hipLaunchKernelGGL(a_node1, dim3(nb(N)), dim3(kB), 0, st, N, E, NP, rec, c->nd.fe, c->bc_word,
                          A->rgroup, A->hbar + (size_t)k * A->ng, A->xb, A->vb, A->udb, A->pab, A->fib, A->mb,
                          dtb_n);
       if (n == 8)

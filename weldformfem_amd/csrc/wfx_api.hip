@@ -74,11 +74,14 @@ static void free_all(wfx_ctx *c) {
   c->react_base = c->react_rank = nullptr;
   c->react_ring = nullptr;
   c->react_n = c->react_rows = 0;
-  c->bc_slot = c->bc_mask = nullptr;
+  c->bc_word = nullptr;
   c->bc_tab = nullptr;
   c->v32 = c->pa32 = c->ud32 = c->fi32 = nullptr;
   c->x_start = nullptr;
   c->x_lo = nullptr;
+  c->pair = 0;
+  c->x_b = nullptr;
+  c->v_b = c->pa_b = c->ud_b = nullptr;
   c->temp_e = c->temp_buf = nullptr;
   c->contact = wfx::Contact();
   c->has_fe = 0;
@@ -149,6 +152,76 @@ static int scratch_address(double **out) {
   return WFX_OK;
 }
 
+// The plan's slot entries as the element pass reads them: groups of four LDS
+// byte offsets, so that the pass extracts an address with one instruction and
+// adds without a test per entry.
+struct EntryTables {
+  std::vector<int4> desc;
+  std::vector<uint16_t> goff;
+  std::vector<uint2> ent;
+};
+static EntryTables entry_tables(const wfx_ctx *c, const ClusterPlan &plan) {
+  EntryTables t;
+  const int C = plan.clusters(), n = c->n;
+  const unsigned es = c->precision == WFX_FP64 ? 8 : 4, zero = (unsigned)(n * kCluster) * es;
+  t.desc.resize(C);
+  t.goff.resize(plan.slots() + C);
+  t.ent.reserve((size_t)c->E * n / 3);
+  for (int k = 0; k < C; ++k) {
+    const int e0 = plan.eoff[k], s0 = plan.sbase[k], ne = plan.eoff[k + 1] - e0, m = plan.sbase[k + 1] - s0;
+    const size_t g0 = t.ent.size();
+    t.desc[k] = make_int4(e0, s0, ne | m << 16, (int)g0);
+    const uint16_t *lo = plan.loff.data() + s0 + k, *en = plan.ent.data() + (size_t)e0 * n;
+    for (int j = 0; j < m; ++j) {
+      t.goff[s0 + k + j] = (uint16_t)(t.ent.size() - g0);
+      for (int q = lo[j]; q < lo[j + 1]; q += 4) {
+        unsigned v[4];
+        for (int h = 0; h < 4; ++h) {
+          const int e = q + h < lo[j + 1] ? en[q + h] : -1;
+          v[h] = e < 0 ? zero : (unsigned)((e & 7) * kCluster + (e >> 3)) * es;
+        }
+        t.ent.push_back(make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16));
+      }
+    }
+    t.goff[s0 + k + m] = (uint16_t)(t.ent.size() - g0);
+  }
+  t.ent.resize(t.ent.size() + 8, make_uint2(0, 0));  // a slot's first six groups are read whatever their number
+  return t;
+}
+
+// Tables of the paired passes; pw 0: the mesh takes the separate ones.
+// The line: 256 clusters, one work-group on each of the 256 CUs.  Below it the
+// launches and dependent loads count and the repeated node updates (1.7 times,
+// hexahedra) are free; above it they are not.  Measured in graph replay, us per
+// step, paired / separate: FP64 hexahedra 1 element 10.2 / 11.2, 20^3 13.4 /
+// 15.2, 30^3 (106 clusters) 15.5 / 16.9, 50^3 (489) 34.4 / 30.6; tetrahedra 8
+// cells 11.2 / 12.8, 27 cells (363) 17.8 / 17.9.  Launched one by one the
+// separate passes never take less than the 17 us their four launches cost.
+constexpr int kPairMaxClusters = 256;
+constexpr int kPairMaxElems = 32;  // elements of a node
+struct PairTables {
+  int pw = 0;
+  std::vector<int4> rec;
+  std::vector<int> ent;
+};
+static PairTables pair_tables(const wfx_ctx *c, const ClusterPlan &plan) {
+  PairTables t;
+  const int most = c->nodel_count_h.empty() ? 0 : *std::max_element(c->nodel_count_h.begin(), c->nodel_count_h.end());
+  if (plan.clusters() > kPairMaxClusters || most > kPairMaxElems) return t;
+  // a node of no element has no slot: only the separate node pass reaches it
+  if (*std::min_element(c->nodel_count_h.begin(), c->nodel_count_h.end()) == 0) return t;
+  t.pw = (most + 7) / 8 * 8;
+  const long S = plan.slots();
+  t.rec.resize(S);
+  t.ent.resize((size_t)S * t.pw);
+  for (long s = 0; s < S; ++s) {
+    const int i = plan.snode[s], o = plan.nsl_off[i], cnt = c->nodel_count_h[i], co = c->nodel_offset_h[i];
+    t.rec[s] = make_int4(i, o, plan.nsl_off[i + 1] - o, (int)((unsigned)cnt | (plan.nsl[o] == s ? 0x80000000u : 0u)));
+    for (int k = 0; k < t.pw; ++k) t.ent[(size_t)s * t.pw + k] = c->el_o2s[c->nodel_h[co + std::min(k, cnt - 1)]];
+  }
+  return t;
+}
+
 // Allocates every device buffer for the mesh held on the host and uploads
 // coordinates, connectivity and CSR.
 static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
@@ -163,9 +236,9 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
   if (e == hipSuccess) e = dalloc(c, &ptr, (cnt));
   A(c->nd.x, 3 * N) A(c->nd.v, 3 * N) A(c->nd.a, 3 * N) A(c->nd.u, 3 * N) A(c->nd.u_dt, 3 * N)
   A(c->nd.prev_a, 3 * N) A(c->nd.fi, 3 * N) A(c->nd.fe, 3 * N) A(c->nd.mdiag, N) A(c->nd.voln, N)
-  A(c->nd.voln0_sum, N) A(c->nd.anp_ratio, N) A(c->nd.T, N)
+  A(c->nd.voln0_sum, N) A(c->nd.anp_ratio, N) A(c->nd.T, N) A(c->nd.rho_avg, N)
   A(c->ms.elnod, n * E) A(c->ms.nodel, n * E) A(c->ms.nodel_loc, n * E) A(c->ms.nodel_offset, N)
-  A(c->ms.nodel_count, N) A(c->ms.nodel_pk, n * E) A(c->ms.nodel_pad, 8 * N) A(c->bc_slot, N)
+  A(c->ms.nodel_count, N) A(c->ms.nodel_pk, n * E) A(c->ms.nodel_pad, 8 * N) A(c->bc_word, N)
   A(c->scalars, 64) A(c->status, 16) A(c->ms.o2s, E)
   c->ms.ncl = plan.clusters();
   c->ms.nslot = plan.slots();
@@ -177,18 +250,27 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     free_all(c);
     return WFX_ERR_STATE;
   }
-  A(c->ms.cl_eoff, c->ms.ncl + 1) A(c->ms.cl_sbase, c->ms.ncl + 1) A(c->ms.cl_loff, c->ms.nslot + c->ms.ncl)
-  A(c->ms.cl_ent, n * E) A(c->ms.nsl_off, N + 1)
+  const EntryTables et = entry_tables(c, plan);
+  A(c->ms.cl_desc, c->ms.ncl) A(c->ms.cl_goff, c->ms.nslot + c->ms.ncl)
+  A(c->ms.cl_ent, et.ent.size()) A(c->ms.nsl_off, N + 1)
   A(c->ms.cl_snode, c->ms.nslot) A(c->ms.cl_lslot, n * E)
-  if (c->precision == WFX_FP64) {
-    A(c->ms.nsl, c->ms.nslot)
-  } else {
-    A(c->ms.spos, c->ms.nslot)
+  const PairTables pt = pair_tables(c, plan);
+  c->pair = pt.pw > 0;
+  if (c->precision == WFX_FP64) A(c->ms.nsl, c->ms.nslot)
+  if (c->precision == WFX_FP32_MIXED || c->pair) A(c->ms.spos, c->ms.nslot)
+  if (c->pair) {
+    double *t[3] = {nullptr, nullptr, nullptr};  // (doubles: enough for either nodal type)
+    A(c->ms.sbc, c->ms.nslot) A(c->ms.srec, c->ms.nslot) A(c->ms.sent, pt.ent.size()) A(c->x_b, 3 * N)
+    A(t[0], 3 * N) A(t[1], 3 * N) A(t[2], 3 * N)
+    c->v_b = t[0];
+    c->pa_b = t[1];
+    c->ud_b = t[2];
+    c->ms.pw = pt.pw;
   }
   // partial minima of the volume pass (one per element cluster) and of the
   // per-step kernels at block size >= 64
   c->cfl_cap_min = (int)std::max<size_t>((E + 63) / 64 + 1, (size_t)c->ms.ncl + 1);
-  A(c->cfl_part, c->cfl_cap_min + (N + 63) / 64 + 1)
+  A(c->cfl_part, c->cfl_cap_min + std::max<size_t>((N + 63) / 64, (size_t)c->ms.ncl) + 1)
   if (e == hipSuccess) e = (c->precision == WFX_FP64) ? alloc_elem(c, c->e64) : alloc_elem(c, c->e32);
   A(c->x_start, 3 * N)
   if (c->precision == WFX_FP32_MIXED) {
@@ -220,15 +302,18 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_loc, c->nodel_loc_h.data(), n * E * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_offset, c->nodel_offset_h.data(), N * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_count, c->nodel_count_h.data(), N * sizeof(int), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_eoff, plan.eoff.data(), plan.eoff.size() * sizeof(int), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_sbase, plan.sbase.data(), plan.sbase.size() * sizeof(int), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_loff, plan.loff.data(), plan.loff.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_ent, plan.ent.data(), plan.ent.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_desc, et.desc.data(), et.desc.size() * sizeof(int4), hipMemcpyHostToDevice));
+  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_goff, et.goff.data(), et.goff.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_ent, et.ent.data(), et.ent.size() * sizeof(uint2), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.nsl_off, plan.nsl_off.data(), plan.nsl_off.size() * sizeof(int), hipMemcpyHostToDevice));
   if (c->ms.nsl)
     WFX_CHECK_HIP(hipMemcpy(c->ms.nsl, plan.nsl.data(), plan.nsl.size() * sizeof(int), hipMemcpyHostToDevice));
   if (c->ms.spos)
     WFX_CHECK_HIP(hipMemcpy(c->ms.spos, plan.spos.data(), plan.spos.size() * sizeof(int), hipMemcpyHostToDevice));
+  if (c->pair) {
+    WFX_CHECK_HIP(hipMemcpy(c->ms.srec, pt.rec.data(), pt.rec.size() * sizeof(int4), hipMemcpyHostToDevice));
+    WFX_CHECK_HIP(hipMemcpy(c->ms.sent, pt.ent.data(), pt.ent.size() * sizeof(int), hipMemcpyHostToDevice));
+  }
   WFX_CHECK_HIP(hipMemcpy(c->ms.cl_snode, plan.snode.data(), plan.snode.size() * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.cl_lslot, plan.lslot.data(), plan.lslot.size() * sizeof(uint16_t),
                           hipMemcpyHostToDevice));
@@ -241,7 +326,6 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
   for (size_t i = 0; i < N; ++i)
     for (int j = 0; j < std::min(8, c->nodel_count_h[i]); ++j) pad[j * N + i] = pk[c->nodel_offset_h[i] + j];
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_pad, pad.data(), 8 * N * sizeof(int), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemset(c->bc_slot, 0xff, N * sizeof(int)));  // -1: no boundary condition
   WFX_CHECK_HIP(hipMemcpy(c->scalars + kCflDt, &c->prm.dt, sizeof(double), hipMemcpyHostToDevice));
   {
     std::vector<double> t0(N, c->prm.mat.temp);  // setTemp (Domain_d.h:678-683)
@@ -271,6 +355,8 @@ static int finish_mesh(wfx_ctx *c) {
   c->el_o2s.swap(plan.o2s);
   int rc = setup_device(c, plan);
   if (rc) return rc;
+  c->slot_node_h.clear();
+  if (c->pair) c->slot_node_h.swap(plan.snode);
   c->prm.N = c->N;
   c->prm.E = c->E;
   c->prm.n = c->n;
@@ -422,6 +508,7 @@ static int scan_elements(wfx_ctx *c) {
   if (!rc) rc = download_real(c, v0.data(), f64 ? (void *)c->e64.vol0 : (void *)c->e32.vol0, v0.size(), true);
   if (rc) return rc;
   c->rho_uniform = 0.0;
+  c->rho_avg_valid = false;
   if (!r.empty() && r[0] > 0.0 &&
       std::all_of(r.begin(), r.end(), [&](double v) { return v == r[0]; }))
     c->rho_uniform = r[0];
@@ -983,16 +1070,18 @@ int wfx_allocate_bcs(wfx_ctx *c) {
     }
   }
   if (!mask.empty()) {
-    int *pm = nullptr;
     double *pt = nullptr;
-    WFX_CHECK_HIP(dalloc(c, &pm, mask.size()));
     WFX_CHECK_HIP(dalloc(c, &pt, tab.size()));
-    WFX_CHECK_HIP(hipMemcpy(pm, mask.data(), mask.size() * sizeof(int), hipMemcpyHostToDevice));
     WFX_CHECK_HIP(hipMemcpy(pt, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
-    c->bc_mask = pm;
     c->bc_tab = pt;
   }
-  WFX_CHECK_HIP(hipMemcpy(c->bc_slot, slot.data(), c->N * sizeof(int), hipMemcpyHostToDevice));
+  for (int &w : slot) w = w < 0 ? 0 : (w << 3) | mask[w];
+  WFX_CHECK_HIP(hipMemcpy(c->bc_word, slot.data(), c->N * sizeof(int), hipMemcpyHostToDevice));
+  if (c->pair) {
+    std::vector<int> sbc(c->slot_node_h.size());
+    for (size_t k = 0; k < sbc.size(); ++k) sbc[k] = slot[c->slot_node_h[k]];
+    WFX_CHECK_HIP(hipMemcpy(c->ms.sbc, sbc.data(), sbc.size() * sizeof(int), hipMemcpyHostToDevice));
+  }
   return WFX_OK;
 }
 
@@ -1234,6 +1323,7 @@ int wfx_calc_elem_density(wfx_ctx *c, wfx_stream s) {
   // evaluates the pressure terms in full
   c->rho_uniform = 0.0;
   c->elem_guard = 1;
+  c->rho_avg_valid = false;
   return WFX_OK;
 }
 STEP_FN(wfx_calc_nodal_vol, BY_PRECISION(c, launch_nodal_vol, c, st))
@@ -1628,7 +1718,7 @@ static uint64_t graph_signature(wfx_ctx *c) {
     mix(ci, sizeof(ci));
     mix(cptr, sizeof(cptr));
   }
-  const void *ptrs[] = {c->bc_nod[0], c->bc_nod[1], c->bc_nod[2], c->bc_slot, c->bc_mask, c->bc_tab,
+  const void *ptrs[] = {c->bc_nod[0], c->bc_nod[1], c->bc_nod[2], c->bc_word, c->bc_tab,
                         c->react, c->hist, c->e64.He, c->e32.He, c->temp_e, c->dt_hist};
   mix(ptrs, sizeof(ptrs));
   int ints[] = {c->N, c->E, c->n, c->has_fe, c->bc_count[0], c->bc_count[1], c->bc_count[2],

@@ -24,6 +24,10 @@
 //                                                   UpdateCorrection*,
 //                                                   UpdatePrediction)
 //
+// Meshes of at most 256 element clusters take two kernels per step instead
+// (paired passes): F2 becomes part of F3's staging, and F4 and the next F1
+// one cluster pass.
+//
 // Every expression is the one of the per-step kernels, so the FP64 fused path
 // differs from the per-step path only in the order of the nodal force sums:
 // the hourglass force is subtracted per element instead of after the
@@ -33,7 +37,7 @@
 //
 // Device inputs beyond the per-step state:
 //   nodel_pk[nnz]  packed CSR entry (element << 3) | local node
-//   bc_slot[N]     -1 or index into bc_mask / bc_val (per-node Dirichlet data)
+//   bc_word[N]     0, or (index into bc_val << 3) | mask (per-node Dirichlet data)
 //   anp_ratio[N]   V_n / V0_n,   vsum0[N] = V0_n (constant after init)
 #pragma once
 
@@ -75,19 +79,28 @@ __device__ __forceinline__ double anp_ratio_at(const double *ratio, int i) {
   else return 1.0 + (double)reinterpret_cast<const float *>(ratio)[i];
 }
 
-// V0_n: CSR-ordered sum of the initial volumes (calcElemPressure :698-705)
+// Once per run, V0_n: CSR-ordered sum of the initial volumes (calcElemPressure
+// :698-705), and the mean density of the node's elements.  Densities do not
+// change during a fused run, so CalcNodalMassFromVol's sum of rho V_n / c
+// over the c elements is this mean times V_n: a loop of c divisions less in
+// every step's nodal sums.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void f0_vsum0(int N, const int *__restrict__ off,
                                                    const int *__restrict__ cnt,
                                                    const int *__restrict__ nodel_pk,
-                                                   const T *__restrict__ vol0,
-                                                   double *__restrict__ vsum0) {
+                                                   const T *__restrict__ vol0, const T *__restrict__ rho,
+                                                   double *__restrict__ vsum0, double *__restrict__ rho_avg) {
   int i = gtid();
   if (i >= N) return;
   int o = off[i], c = cnt[i];
-  double s0 = 0.0;
-  for (int k = 0; k < c; ++k) s0 += (double)vol0[nodel_pk[o + k] >> 3];
-  vsum0[i] = s0;
+  double s0 = 0.0, r = 0.0;
+  for (int k = 0; k < c; ++k) {
+    const int e = nodel_pk[o + k] >> 3;
+    s0 += (double)vol0[e];
+    r += (double)rho[e];
+  }
+  if (vsum0) vsum0[i] = s0;
+  rho_avg[i] = r / (double)c;
 }
 
 // F2: nodal volume sum in CSR order; ratio for the ANP pressure and nodal
@@ -98,7 +111,7 @@ __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *_
                                                    const int *__restrict__ nodel_pk,
                                                    const int *__restrict__ pad,
                                                    const T *__restrict__ vol,
-                                                   const T *__restrict__ rho,
+                                                   const double *__restrict__ rho_avg,
                                                    const double *__restrict__ vsum0,
                                                    double *__restrict__ ratio,
                                                    double *__restrict__ mdiag, double rho_u) {
@@ -112,11 +125,9 @@ __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *_
   // CSR entries are taken eight at a time with independent loads, then
   // summed in CSR order (the order of the reference's serial loop); the
   // first eight come from the padded [8][N] table.
-  // The densities of the first chunk are loaded together with the volumes and
-  // kept in registers (every hexa node and most tet nodes have <= 8
-  // elements); with a uniform density (rho_u > 0) no density is loaded.
+  const double v0 = ld_stream(&vsum0[i]);
+  const double rho_n = rho_u > 0.0 ? rho_u : ld_stream(&rho_avg[i]);
   double s = 0.0;
-  double r0[kChunk];
   for (int k = 0; k < c; k += kChunk) {
     int e[kChunk];
     double vv[kChunk];
@@ -128,10 +139,6 @@ __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *_
     // would each be waited for on their own
 #pragma unroll
     for (int j = 0; j < kChunk; ++j) vv[j] = (double)vol[e[j] >= 0 ? e[j] : e[0]];
-    if (k == 0 && rho_u <= 0.0) {
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j) r0[j] = (double)rho[e[j] >= 0 ? e[j] : e[0]];
-    }
 #pragma unroll
     for (int j = 0; j < kChunk; ++j)
       if (k + j < c) s += vv[j];
@@ -139,32 +146,11 @@ __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *_
   // the ANP ratio V_n / V0_n: FP64 stores it; FP32-mixed stores its
   // deviation from 1 as a float in the same buffer (the element pass adds the
   // 1 back; the deviation keeps the float's relative precision)
-  const double v0 = ld_stream(&vsum0[i]);
   if constexpr (std::is_same<T, double>::value) ratio[i] = s / v0;
   else reinterpret_cast<float *>(ratio)[i] = (float)(s / v0 - 1.0);
   double vn = s;
-  vn /= nodxelem;
-  double dc = (double)c, mass = 0.0;
-  if (rho_u > 0.0) {  // every term is the same value: formed once, added c times
-    const double term = 1.0 * rho_u * vn / dc;
-    for (int k = 0; k < c; ++k) mass += term;
-    st_stream(&mdiag[i], mass);
-    return;
-  }
-  for (int k = 0; k < c; k += kChunk) {
-    double rr[kChunk];
-    if (k == 0) {
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j) rr[j] = r0[j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < kChunk; ++j) rr[j] = (k + j < c) ? (double)rho[nodel_pk[o + k + j] >> 3] : 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < kChunk; ++j)
-      if (k + j < c) mass += 1.0 * rr[j] * vn / dc;
-  }
-  mdiag[i] = mass;
+  vn *= 1.0 / nodxelem;  // 4 or 8: exact
+  st_stream(&mdiag[i], vn * rho_n);
 }
 
 // Nodes with many elements (tetrahedral meshes: about 23 per node) are
@@ -202,15 +188,20 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void f0_vsum0_lanes(int N, const int *__restrict__ off,
                                                          const int *__restrict__ cnt,
                                                          const int *__restrict__ nodel_pk,
-                                                         const T *__restrict__ vol0,
-                                                         double *__restrict__ vsum0) {
+                                                         const T *__restrict__ vol0, const T *__restrict__ rho,
+                                                         double *__restrict__ vsum0,
+                                                         double *__restrict__ rho_avg) {
   constexpr int L = kF2Lanes;
   const long g = (long)xcd_block() * kBlock + threadIdx.x;
   const long n = g / L;
   const int q = (int)(g % L), i = (int)(n < N ? n : N - 1);  // every lane reaches the butterfly
   const int o = off[i], c = cnt[i];
   const double s0 = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return (double)vol0[e]; });
-  if (q == 0 && n < N) vsum0[i] = s0;
+  const double r = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return (double)rho[e]; });
+  if (q == 0 && n < N) {
+    if (vsum0) vsum0[i] = s0;
+    rho_avg[i] = r / (double)c;
+  }
 }
 
 // F2 with kF2Lanes lanes per node: the nodal volume sum, ANP ratio and mass
@@ -219,7 +210,8 @@ template <typename T, int BS>
 __global__ __launch_bounds__(BS) void f2_nodal_lanes(int N, int nodxelem, const int *__restrict__ off,
                                                      const int *__restrict__ cnt,
                                                      const int *__restrict__ nodel_pk,
-                                                     const T *__restrict__ vol, const T *__restrict__ rho,
+                                                     const T *__restrict__ vol,
+                                                     const double *__restrict__ rho_avg,
                                                      const double *__restrict__ vsum0,
                                                      double *__restrict__ ratio, double *__restrict__ mdiag,
                                                      double rho_u) {
@@ -228,22 +220,13 @@ __global__ __launch_bounds__(BS) void f2_nodal_lanes(int N, int nodxelem, const 
   const long n = g / L;
   const int q = (int)(g % L), i = (int)(n < N ? n : N - 1);  // every lane reaches the butterflies
   const int o = off[i], c = cnt[i];
-  const double v0 = vsum0[i];  // loaded with the offsets, not after the sum
+  // loaded with the offsets, not after the sum
+  const double v0 = vsum0[i], rho_n = rho_u > 0.0 ? rho_u : rho_avg[i];
   const double s = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return (double)vol[e]; });
-  double vn = s;
-  vn /= nodxelem;
-  const double dc = (double)c;
-  double mass = 0.0;
-  if (rho_u > 0.0) {  // every term is the same value: formed once, added c times
-    const double term = 1.0 * rho_u * vn / dc;
-    for (int k = 0; k < c; ++k) mass += term;
-  } else {
-    mass = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return 1.0 * (double)rho[e] * vn / dc; });
-  }
   if (q != 0 || n >= N) return;
   if constexpr (std::is_same<T, double>::value) ratio[i] = s / v0;
   else reinterpret_cast<float *>(ratio)[i] = (float)(s / v0 - 1.0);
-  mdiag[i] = mass;
+  mdiag[i] = s * (1.0 / nodxelem) * rho_n;
 }
 
 struct FusedParams {
@@ -369,13 +352,32 @@ __device__ __forceinline__ void cofactors(const T (&J)[3][3], T (&C)[3][3], T &d
 }
 #undef WFX_COFACTORS
 
-// pow(vol, 0.6666666) of the hourglass coefficient (Mechanical.f90:299): the
-// FP64 path in double, FP32-mixed with the hardware base-2 logarithm and
-// exponential (the same NaN, zero and infinity cases)
+// pow(vol, 0.6666666) of the hourglass coefficient (Mechanical.f90:299).
+// FP64: vol^(2/3) exp(-d ln vol) with d = 2/3 - 0.6666666.  r = cbrt(vol), its
+// square in two parts and the residual vol - r^3 give vol^(2/3) to half a unit
+// in the last place; |d ln vol| < 5e-6, so that three terms of the exponential
+// leave 2e-23.  The library's pow carries a double-double logarithm and
+// exponential one after the other: 1450 of the 13200 cycles of the element
+// pass's chain on an idle chip; cbrt and log are shorter and independent of
+// each other.  Largest error over 1e-30..1e30: 0.6 ulp (pow 0.8).  Other volumes
+// (not positive, not finite, out of the float reciprocal's range) take pow.
+// FP32-mixed: the hardware base-2 logarithm and exponential.
+__device__ __forceinline__ double pow_hg(double vol) {
+  constexpr double d = 6.666666666858372e-08;
+  const double r = cbrt(vol), y = d * log(vol);
+  const double h = r * r, l = fma(r, r, -h);
+  const double res = fma(-r, l, fma(-r, h, vol));
+  const double t = (2.0 / 3.0) * res * (double)__builtin_amdgcn_rcpf((float)vol) - y * (1.0 - y * (0.5 - y * (1.0 / 6.0)));
+  return h + fma(h, t, l);
+}
 template <typename T>
 __device__ __forceinline__ T vol_pow_hg(T vol) {
-  if constexpr (std::is_same<T, double>::value) return pow(vol, 0.6666666);
-  else return exp2f(0.6666666f * log2f(vol));
+  if constexpr (std::is_same<T, double>::value) {
+    if (vol >= 1e-30 && vol <= 1e30) return pow_hg(vol);
+    return pow(vol, 0.6666666);
+  } else {
+    return exp2f(0.6666666f * log2f(vol));
+  }
 }
 
 // The cluster's slots staged in LDS by the element pass: positions (double),
@@ -602,7 +604,7 @@ constexpr int kStashVals = TH ? 25 : 22;
 
 template <typename T, int NN, int LAW, int BS, bool TH, class Sink>
 __device__ __forceinline__ void element_material(
-    int e, int E, const FusedParams &fp, ElemGeo<T, NN, TH> &G, const ElemState<T> &S,
+    int e, int E, const FusedParams &fp, T dt, ElemGeo<T, NN, TH> &G, const ElemState<T> &S,
     const T *__restrict__ vol0, const T *__restrict__ rho, const T *__restrict__ He, T *__restrict__ tau_io,
     T *__restrict__ eps_io, T *__restrict__ p_out, T *__restrict__ pl_strain, T *__restrict__ sigma_y,
     T *__restrict__ q_plheat, double *stash, Sink &&sink) {
@@ -656,7 +658,6 @@ __device__ __forceinline__ void element_material(
   if (fp.write_out) p_out[e] = pe;
 
   // ---- Jaumann update and J2 return (CalcStressStrain) -------------------
-  T dt = (T)(fp.dtp ? *fp.dtp : fp.dt);
   const MatParams &mp = fp.mp;
   T3<T> tau = t3_from_sym(S.tau[0], S.tau[1], S.tau[2], S.tau[3], S.tau[4], S.tau[5]);
   T3<T> D = t3_from_sym(s00, s11, s22, s01, s12, s02);
@@ -834,18 +835,36 @@ __device__ __forceinline__ void element_material(
 
 // Cluster tables of the fused element pass on the device (wfx_cluster.hpp)
 struct ClusterArgs {
-  const int *eoff;       // [C+1] first stored element of each cluster
-  const int *sbase;      // [C+1] first slot of each cluster
-  const uint16_t *loff;  // cluster c: its M+1 entry offsets at sbase[c] + c
-  const uint16_t *ent;   // element-node entries t * 8 + a grouped by slot, cluster c at eoff[c] * n
+  const int4 *desc;      // as DevMesh::cl_desc, cl_goff, cl_ent
+  const uint16_t *goff;
+  const uint2 *ent;
   const int *snode;      // [S] slot -> node
   const uint16_t *lslot; // [E][n] element-node -> slot within its cluster
-  const int *spos;       // [S] FP32-mixed: slot -> where its partial sum is stored (node-major)
+  const int *spos;       // [S] slot -> where its partial sum is stored when node-major
   long S;                // slots: the row length of the partial sums
+  int nm;                // partial sums node-major (FP32-mixed always, FP64 with the paired passes)
 };
 
-// Where the element pass stores a slot's partial sum.  FP64: in slot order
-// (a cluster's sums are one contiguous run; the node pass reads a node's
+// What the paired passes need beyond the four separate ones
+struct PairArgs {
+  const int4 *rec;       // per slot (DevMesh::srec)
+  const int *sent;       //   and its node's elements [S][pw]
+  const int *sbc;        //   and its boundary word
+  int pw, lanes;         // lanes: summed as f2_nodal_lanes sums, else in CSR order as f2_nodal
+  const void *vol;       // T[E]
+  const double *vsum0, *rho_avg;
+  double *ratio, *mdiag; // written by each node's first slot
+  // per-step CFL time step (cfl > 0): the partial extremes, and where the
+  // first work-group leaves the result
+  double cfl, K;
+  const double *minl, *vmax;
+  int nmin, nmax, step;
+  double *scal, *dt_hist;
+};
+
+// Where the element pass stores a slot's partial sum.  FP64 (but for the
+// paired passes of small meshes, where one dependent load less counts and
+// bandwidth does not): in slot order (a cluster's sums are one contiguous run; the node pass reads a node's
 // slots through their ids, and moves its bytes near the copy rate anyway).
 // FP32-mixed: node-major, at the slot's place in its node's slot list (the
 // node pass reads a node's sums contiguously from its offset, one dependent
@@ -860,14 +879,17 @@ template <bool TH>
 constexpr int kNodeVals = TH ? 4 : 3;
 
 // LDS of one work-group of the element pass, in turn: the cluster's staged
-// slots (SlotLds), then the element-node values [kNodeVals * n][kCluster]
-// and, in the same space (each thread only ever touches its own column, and
-// reloads its stash before it writes its values), the per-thread stash of
-// the FP64 hexahedral rate-law passes
+// slots (SlotLds), then the element-node values (kEntStride; the last
+// component without its unused cells) and, in the same space (each thread
+// only ever writes its own column, and reloads its stash before it writes its
+// values), the per-thread stash of the FP64 hexahedral rate-law passes.
+// FP64 hexahedra: 53,256 bytes, three work-groups on a CU.
+template <typename T, int NN, bool TH>
+constexpr int kEntLds = ((kNodeVals<TH> - 1) * kEntStride(NN) + NN * kCluster + 1) * (int)sizeof(T);
 template <typename T, int NN, int LAW, bool TH>
-constexpr int kF3Vals = (kStashLDS<T, NN, LAW> && kStashVals<TH> * 8 > kNodeVals<TH> * NN * (int)sizeof(T))
+constexpr int kF3Vals = (kStashLDS<T, NN, LAW> && kStashVals<TH> * 8 * kCluster > kEntLds<T, NN, TH>)
                             ? kStashVals<TH> * 8 * kCluster
-                            : kNodeVals<TH> * NN * (int)sizeof(T) * kCluster;
+                            : kEntLds<T, NN, TH>;
 template <typename T, int NN, int LAW, bool TH>
 constexpr int kF3Lds = kF3Vals<T, NN, LAW, TH> > SlotLds<T, NN>::bytes ? kF3Vals<T, NN, LAW, TH>
                                                                         : SlotLds<T, NN>::bytes;
@@ -884,6 +906,114 @@ __device__ __forceinline__ void load_lslot(const uint16_t *p, int (&ls)[NN]) {
   }
 }
 
+// The nodal volume sums of a thread's slots' nodes from the element volumes,
+// with the ANP ratio as F2 leaves it and, by a node's first slot, the ratio
+// and the mass stored: F2's sums in F2's orders (f2_nodal, or with lanes set
+// f2_nodal_lanes: eight strided sums and their butterfly), so that paired and
+// separate passes give the same bits.  In three parts, so that the entries
+// are loaded with the slot records and the volumes with the nodal state: as
+// one part after the staging's loads, slot after slot and with the mass
+// summed from the densities, it added 6300 (hexahedra) and 12000
+// (tetrahedra) cycles to the staging's 1000.
+template <typename T, int NN>
+struct PairSum {
+  // entries in flight: all of a structured hexahedral node's; up to 24 of a
+  // tetrahedral one's
+  static constexpr int W = NN == 8 ? 8 : 24, K = kSlotsPerThread<NN>;
+  long slot[K];
+  int4 en[K][W / 4];
+  T v[K][W];
+  double v0[K], rho_n[K];
+  __device__ __forceinline__ void entries(const PairArgs &pr, int k0) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int h = 0; h < W / 4; ++h)
+        en[k][h] = reinterpret_cast<const int4 *>(pr.sent + slot[k] * pr.pw)[min(k0 / 4 + h, pr.pw / 4 - 1)];
+  }
+  __device__ __forceinline__ void volumes(const PairArgs &pr) {
+    const T *vol = static_cast<const T *>(pr.vol);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int h = 0; h < W / 4; ++h) {
+        v[k][4 * h + 0] = vol[en[k][h].x];
+        v[k][4 * h + 1] = vol[en[k][h].y];
+        v[k][4 * h + 2] = vol[en[k][h].z];
+        v[k][4 * h + 3] = vol[en[k][h].w];
+      }
+  }
+  __device__ __forceinline__ void nodal(const PairArgs &pr, const int4 (&rec)[K], double rho_u) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      v0[k] = pr.vsum0[rec[k].x];
+      rho_n[k] = rho_u > 0.0 ? rho_u : pr.rho_avg[rec[k].x];
+    }
+  }
+  __device__ __forceinline__ void ratio(const PairArgs &pr, const int4 (&rec)[K], const bool (&mine)[K],
+                                        T (&out)[K]) {
+    double s[K], l[K][8];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      s[k] = 0.0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) l[k][j] = 0.0;
+    }
+    for (int k0 = 0;;) {
+      // entries past the node's count add zero
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int c = rec[k].w & 0xff;
+        if (pr.lanes) {
+#pragma unroll
+          for (int j = 0; j < W; ++j) l[k][j & 7] += k0 + j < c ? (double)v[k][j] : 0.0;
+        } else {
+#pragma unroll
+          for (int j = 0; j < W; ++j) s[k] += k0 + j < c ? (double)v[k][j] : 0.0;
+        }
+      }
+      k0 += W;
+      if (k0 >= pr.pw) break;
+      entries(pr, k0);
+      volumes(pr);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (pr.lanes)
+        s[k] = ((l[k][0] + l[k][1]) + (l[k][2] + l[k][3])) + ((l[k][4] + l[k][5]) + (l[k][6] + l[k][7]));
+      if constexpr (std::is_same<T, double>::value) out[k] = s[k] / v0[k];
+      else out[k] = (float)(s[k] / v0[k] - 1.0);
+      if (mine[k] && rec[k].w < 0) {
+        reinterpret_cast<T *>(pr.ratio)[rec[k].x] = out[k];
+        pr.mdiag[rec[k].x] = s[k] * (1.0 / NN) * rho_n[k];
+      }
+    }
+  }
+};
+
+// The step's dt from the partial extremes (k_cfl_reduce's arithmetic): every
+// work-group reduces them for itself, since a kernel for it costs 3 us and its
+// launch while the few partials of a small mesh take less than one; the first
+// work-group stores the result for the later kernels.
+template <typename T>
+__device__ __forceinline__ double pair_cfl_dt(const PairArgs &pr, const T *rho) {
+  double m = kMinEdgeInit, v = 0.0;
+  for (int k = threadIdx.x; k < pr.nmin; k += kCluster) m = fmin(m, pr.minl[k]);
+  for (int k = threadIdx.x; k < pr.nmax; k += kCluster) v = fmax(v, pr.vmax[k]);
+  m = block_extreme<kCluster, true>(m);
+  v = block_extreme<kCluster, false>(v);
+  const double cs = sqrt(pr.K / (double)rho[0]);
+  const double dt = pr.cfl * m / (cs + v);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    pr.scal[kCflMinl] = m;
+    pr.scal[kCflVmax] = v;
+    pr.scal[kCflCs] = cs;
+    pr.scal[kCflDt] = dt;
+    if (pr.dt_hist) pr.dt_hist[pr.step] = dt;
+  }
+  return dt;
+}
+
 // F3: one work-group per element cluster.  The work-group first stages its
 // cluster's slots (the distinct nodes of its elements: positions,
 // velocities, ANP ratio, ids) in LDS with one load per slot and field; each
@@ -892,22 +1022,26 @@ __device__ __forceinline__ void load_lslot(const uint16_t *p, int (&ls)[NN]) {
 // cluster node (the slot's entries, ascending element, in double) and writes
 // one partial sum per slot (assemblyForces, Matrices.C:42-87, for the
 // cluster's share of each node).
-template <typename T, int NN, int LAW, bool TH>
+// PAIR (small meshes, launch-bound): F2 is part of the staging, each slot's
+// thread summing its node's element volumes; slots of a node in several
+// clusters repeat the sum (1.7 times the work of F2), and a launch and F2's
+// round trip of the ratio are saved.
+template <typename T, int NN, int LAW, bool TH, bool PAIR>
 __global__ __launch_bounds__(kCluster) void f3_cluster(
-    int E, int N, FusedParams fp, ClusterArgs ca, const double *__restrict__ x, const T *__restrict__ v,
+    int E, int N, FusedParams fp, ClusterArgs ca, PairArgs pr, const double *__restrict__ x, const T *__restrict__ v,
     const double *__restrict__ ratio, const T *__restrict__ vol0, const T *__restrict__ rho,
     const T *__restrict__ sy0, const T *__restrict__ He, T *__restrict__ tau_io, T *__restrict__ eps_io,
     T *__restrict__ p_out, T *__restrict__ pl_strain, T *__restrict__ sigma_y, T *__restrict__ part,
     T *__restrict__ q_plheat) {
   constexpr int R = kNodeVals<TH>;
   __shared__ __align__(16) unsigned char lds_raw[kF3Lds<T, NN, LAW, TH>];
-  __shared__ uint32_t l_ent[kCluster * NN / 2];  // the cluster's entries, two per word
   T *lf = reinterpret_cast<T *>(lds_raw);
   const SlotLds<T, NN> L(lds_raw);
   const int c = xcd_block(), t = threadIdx.x;
-  const int e0 = ca.eoff[c], ne = ca.eoff[c + 1] - e0;
-  const int s0 = ca.sbase[c], M = ca.sbase[c + 1] - s0;  // M <= slot_cap(NN), checked at set-up
-  const uint16_t *lo = ca.loff + s0 + c;
+  const int4 cd = ca.desc[c];
+  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
+  const uint16_t *lo = ca.goff + s0 + c;
+  const uint2 *en = ca.ent + cd.w;  // the cluster's entry groups
   // the nodes of this thread's slots t and t + kCluster: first, as the
   // staging loads depend on them
   constexpr int kSl = kSlotsPerThread<NN>;
@@ -916,40 +1050,46 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   // elements, entries or slots repeating its last one (a cluster has at
   // least one element and NN slots), so that none is waited for on its own;
   // the values are used only where they are the thread's own.
-  // First the nodes of this thread's slots t and t + kCluster, which the
-  // staging loads depend on.
+  // Loads return in order, so the order is that of the waits: the nodes of
+  // this thread's slots t and t + kCluster (PAIR: with their elements), the
+  // slot tables and the element's slots; the nodal state; the element's own
+  // state last, which only the second part of the chain needs.
   int sn[kSl];
+  int4 rec[kSl];
+  bool mine[kSl];
+  PairSum<T, NN> ps;
 #pragma unroll
-  for (int k = 0; k < kSl; ++k) sn[k] = ca.snode[s0 + min(t + k * kCluster, M - 1)];
-  // The cluster's slot tables are loaded into registers before the element
-  // chain, so that the loads complete under its arithmetic: the entries
-  // (ne * NN uint16 from a 4-byte aligned start, since e0 * NN is even) go to
-  // LDS after it; the entry offsets of the thread's own slots t and
-  // t + kCluster stay in registers.
-  const uint32_t *en32 = reinterpret_cast<const uint32_t *>(ca.ent + (long)e0 * NN);
-  const int nw = ne * NN / 2;
-  uint32_t ew[NN / 2];
-#pragma unroll
-  for (int k = 0; k < NN / 2; ++k) ew[k] = en32[min(t + k * kCluster, nw - 1)];
+  for (int k = 0; k < kSl; ++k) {
+    const int j = t + k * kCluster, q = s0 + min(j, M - 1);
+    if constexpr (PAIR) {
+      rec[k] = pr.rec[q];
+      sn[k] = rec[k].x;
+      ps.slot[k] = q;
+      mine[k] = j < M;
+    } else {
+      sn[k] = ca.snode[q];
+    }
+  }
+  if constexpr (PAIR) ps.entries(pr, 0);
+  // The entry groups' range of the thread's own slots t and t + kCluster; the
+  // groups themselves follow once these are here.
   uint32_t ow[kSl];  // (end << 16) | start of slots t and t + kCluster
   int sp[kSl];       //   and where their sums go
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
     const int q = min(t + k * kCluster, M - 1);
-    ow[k] = ((uint32_t)lo[q + 1] << 16) | lo[q];
-    if constexpr (kNodeMajor<T>) sp[k] = ca.spos[s0 + q];
-    else sp[k] = s0 + q;
+    __builtin_memcpy(&ow[k], lo + q, 4);  // lo[q], lo[q + 1]
+    if constexpr (kNodeMajor<T> || PAIR) sp[k] = ca.spos[s0 + q];
+    else sp[k] = ca.nm ? ca.spos[s0 + q] : s0 + q;
   }
   int ls[NN];
-  ElemState<T> S;
-  {
-    const int e = e0 + min(t, ne - 1);
-    load_lslot<NN>(ca.lslot + (long)e * NN, ls);
-    load_elem_state<T>(e, E, tau_io, eps_io, pl_strain, sy0, He, S);
-  }
+  const int my_e = e0 + min(t, ne - 1);
+  load_lslot<NN>(ca.lslot + (long)my_e * NN, ls);
+  __builtin_amdgcn_sched_barrier(0);
   // stage the slots: all loads first, then the LDS stores
   double sx[kSl][3];
   T sv[kSl][3], sr[kSl];
+  if constexpr (PAIR) ps.volumes(pr);
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
     const int node = sn[k];
@@ -958,9 +1098,26 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
       sx[k][d] = x[(long)d * N + node];
       sv[k][d] = v[(long)d * N + node];
     }
-    if constexpr (std::is_same<T, double>::value) sr[k] = ratio[node];
-    else sr[k] = reinterpret_cast<const float *>(ratio)[node];
+    if constexpr (PAIR) {
+    } else if constexpr (std::is_same<T, double>::value) {
+      sr[k] = ratio[node];
+    } else {
+      sr[k] = reinterpret_cast<const float *>(ratio)[node];
+    }
   }
+  if constexpr (PAIR) ps.nodal(pr, rec, fp.rho_u);
+  __builtin_amdgcn_sched_barrier(0);
+  ElemState<T> S;
+  load_elem_state<T>(my_e, E, tau_io, eps_io, pl_strain, sy0, He, S);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (PAIR) ps.ratio(pr, rec, mine, sr);
+  double dt_step = fp.dt;
+  if constexpr (PAIR) {
+    if (pr.cfl > 0.0) dt_step = pair_cfl_dt<T>(pr, rho);
+  } else {
+    if (fp.dtp) dt_step = *fp.dtp;
+  }
+  const T dt = (T)dt_step;
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
     const int j = t + k * kCluster;  // < slot_cap
@@ -973,18 +1130,27 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
     L.r[j] = sr[k];
   }
   __syncthreads();
+  // The thread's slots' entries straight from the table: they arrive under
+  // the element chain.  (Staged in LDS, the eight 16-bit reads of a slot cost
+  // as many LDS passes as a third of its values.)
+  constexpr int kGr = NN == 8 ? 2 : 6;  // groups held in registers
+  uint2 ew[kSl][kGr];
+#pragma unroll
+  for (int k = 0; k < kSl; ++k)
+#pragma unroll
+    for (int h = 0; h < kGr; ++h) ew[k][h] = en[(ow[k] & 0xffffu) + h];
   ElemGeo<T, NN, TH> G;
   if (t < ne) element_geometry<T, NN, TH>(fp, L, ls, G);
   __syncthreads();  // the staged slots are read: their LDS takes the element-node values
   if (t < ne) {
     element_material<T, NN, LAW, kCluster, TH>(
-        e0 + t, E, fp, G, S, vol0, rho, He, tau_io, eps_io, p_out, pl_strain, sigma_y, q_plheat,
+        e0 + t, E, fp, dt, G, S, vol0, rho, He, tau_io, eps_io, p_out, pl_strain, sigma_y, q_plheat,
         reinterpret_cast<double *>(lds_raw) + t, [&](int a, int node, T f0, T f1, T f2, T th) {
-          lf[(a * R + 0) * kCluster + t] = f0;
-          lf[(a * R + 1) * kCluster + t] = f1;
-          lf[(a * R + 2) * kCluster + t] = f2;
+          lf[0 * kEntStride(NN) + a * kCluster + t] = f0;
+          lf[1 * kEntStride(NN) + a * kCluster + t] = f1;
+          lf[2 * kEntStride(NN) + a * kCluster + t] = f2;
           if constexpr (TH) {
-            lf[(a * R + 3) * kCluster + t] = th;
+            lf[3 * kEntStride(NN) + a * kCluster + t] = th;
             if (fp.dte_flat) {  // this step's rate at the flat index calcThermalExpansion reads
               const long q = (long)fp.flat_base[e0 + t] + a;
               if (q < N) static_cast<T *>(fp.dte_flat)[q] = (T)((double)th / fp.mdiag[node]);
@@ -992,13 +1158,11 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
           }
         });
   }
+  // the zero cells lie in thread 0's column, as its stash does: it is done with it
+  if (t == 0)
 #pragma unroll
-  for (int k = 0; k < NN / 2; ++k) {
-    const int w = t + k * kCluster;
-    if (w < nw) l_ent[w] = ew[k];
-  }
+    for (int u = 0; u < R; ++u) lf[u * kEntStride(NN) + NN * kCluster] = T(0);
   __syncthreads();
-  const uint16_t *en = reinterpret_cast<const uint16_t *>(l_ent);
 #pragma unroll
   for (int r = 0; r < kSl; ++r) {  // M <= kSl * kCluster
     const int j = t + r * kCluster;
@@ -1007,18 +1171,57 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
     double acc[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) acc[q] = 0.0;
-    for (int k = k0; k < k1; ++k) {
-      const int q = en[k];
-      const int tt = q >> 3, a = q & 7;
+    // Four entries at a time with their LDS reads in flight together, added in
+    // order.  One entry per pass waited for two dependent LDS reads each time:
+    // 2800 (hexahedra) and 4900 (tetrahedra) of the 13200 and 11700 cycles a
+    // work-group takes on an idle chip.
+    auto add4 = [&](uint2 w) {
+      T val[4][R];
 #pragma unroll
-      for (int u = 0; u < R; ++u) acc[u] += (double)lf[(a * R + u) * kCluster + tt];
-    }
+      for (int h = 0; h < 4; ++h) {
+        const unsigned o = h & 1 ? (h < 2 ? w.x : w.y) >> 16 : (h < 2 ? w.x : w.y) & 0xffffu;
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+          val[h][u] = *reinterpret_cast<const T *>(lds_raw + o + u * (kEntStride(NN) * (int)sizeof(T)));
+      }
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int u = 0; u < R; ++u) acc[u] += (double)val[h][u];
+    };
+#pragma unroll
+    for (int h = 0; h < kGr; ++h)
+      if (k0 + h < k1) add4(ew[r][h]);
+    for (int k = k0 + kGr; k < k1; ++k) add4(en[k]);  // more elements than the registers hold
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      if constexpr (kNodeMajor<T>) part[q * ca.S + sp[r]] = (T)acc[q];
+      if (kNodeMajor<T> || PAIR || ca.nm) part[q * ca.S + sp[r]] = (T)acc[q];
       else st_stream(&part[q * ca.S + sp[r]], (T)acc[q]);
     }
   }
+}
+
+// One element's volume from its staged positions, the inverted-element count
+// and (edges) its smallest edge
+template <typename T, int NN>
+__device__ __forceinline__ double element_volume(int e, const double *lx, int cap, const int (&ls)[NN], bool edges,
+                                                 T *__restrict__ vol, unsigned int *__restrict__ status) {
+  T J[3][3], C[3][3], det;
+  staged_jacobian<T, NN>(lx, cap, ls, J);
+  cofactors(J, C, det);
+  const T w = (NN == 4) ? T(1.0 / 6.0) : T(8.0);
+  vol[e] = det * w;  // CalcElemVol's 0 + detJ * w * 1 (the same value)
+  count_inverted(det, status);
+  if (!edges) return kMinEdgeInit;
+  T P[4][3];  // the first four nodes, as calcMinEdgeLength takes them
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      if constexpr (std::is_same<T, double>::value) P[a][d] = lx[d * cap + ls[a]];
+      else P[a][d] = T(lx[d * cap + ls[a]] - lx[d * cap + ls[0]]);
+    }
+  return min_edge4<T>(P);
 }
 
 // F1 as a cluster pass: one work-group per element cluster stages its
@@ -1038,8 +1241,8 @@ __global__ __launch_bounds__(kCluster) void f1_cluster(int E, ClusterArgs ca, co
   __shared__ double lx[3 * cap];
   __shared__ int lnode[cap];
   const int c = xcd_block(), t = threadIdx.x;
-  const int e0 = ca.eoff[c], ne = ca.eoff[c + 1] - e0;
-  const int s0 = ca.sbase[c], M = ca.sbase[c + 1] - s0;  // M <= slot_cap(NN), checked at set-up
+  const int4 cd = ca.desc[c];
+  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
   // every load is issued unconditionally (threads past the cluster's
   // elements or slots repeat its last one), as in the element pass
   constexpr int kSl = kSlotsPerThread<NN>;
@@ -1070,23 +1273,7 @@ __global__ __launch_bounds__(kCluster) void f1_cluster(int E, ClusterArgs ca, co
       for (int a = 0; a < NN; ++a) m += 1.0 / NN * (double)dte_flat[lnode[ls[a]]];
       texp[e] = (T)m;
     }
-    T J[3][3], C[3][3], det;
-    staged_jacobian<T, NN>(lx, cap, ls, J);
-    cofactors(J, C, det);
-    const T w = (NN == 4) ? T(1.0 / 6.0) : T(8.0);
-    vol[e] = det * w;  // CalcElemVol's 0 + detJ * w * 1 (the same value)
-    count_inverted(det, status);
-    if (minl_part) {  // the first four nodes, as calcMinEdgeLength takes them
-      T P[4][3];
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          if constexpr (std::is_same<T, double>::value) P[a][d] = lx[d * cap + ls[a]];
-          else P[a][d] = T(lx[d * cap + ls[a]] - lx[d * cap + ls[0]]);
-        }
-      medge = min_edge4<T>(P);
-    }
+    medge = element_volume<T, NN>(e, lx, cap, ls, minl_part != nullptr, vol, status);
   }
   if (minl_part) {
     medge = block_extreme<kCluster, true>(medge);
@@ -1235,10 +1422,11 @@ struct NodeParams {
 // share one word of bits, so the test costs one scalar load; storing every
 // node's force instead (and reading the reaction nodes' back) cost 24 B per
 // node and step.
-template <typename T>
+// (LANES: the lanes hold nodes of their own, each with its own word.)
+template <typename T, bool LANES>
 __device__ __forceinline__ void record_reaction(const NodeParams &np, int i, double fz) {
   if (!np.rz) return;
-  const int w = __builtin_amdgcn_readfirstlane(i >> 6);
+  const int w = LANES ? i >> 6 : __builtin_amdgcn_readfirstlane(i >> 6);
   const unsigned long long b = np.rbits[w];
   const int l = i & 63;
   if ((b >> l) & 1ull)
@@ -1261,13 +1449,14 @@ template <typename T, bool CONTACT>
 struct NodeIn {
   T v[3], pa[3], ud[3];
   float lo[3];
-  double x[3], u[3], xs[3], fe[3], cf[3], m;
-  int slot;
+  double x[3], u[3], xs[3], fe[3], cf[3], bv[3], m;
+  int mask;
 };
 template <typename T, bool CONTACT>
 __device__ __forceinline__ void load_node(int i, long Ns, const NodeParams &np, const double *__restrict__ cf,
                                           const double *__restrict__ fe, const double *__restrict__ mdiag,
-                                          const int *__restrict__ bc_slot, const T *__restrict__ v,
+                                          int word,
+                                          const double *__restrict__ bc_val, const T *__restrict__ v,
                                           const T *__restrict__ prev_a, const T *__restrict__ u_dt,
                                           const double *__restrict__ x, const double *__restrict__ u,
                                           NodeIn<T, CONTACT> &s) {
@@ -1302,7 +1491,17 @@ __device__ __forceinline__ void load_node(int i, long Ns, const NodeParams &np, 
     if constexpr (CONTACT) s.cf[d] = (cf + r)[ui];
   }
   s.m = mdiag[ui];
-  s.slot = bc_slot[ui];
+  // The boundary values here and not where they are used: six uses in a row,
+  // each behind its own branch, waited for their load one after the other and
+  // made the constrained nodes' wavefronts the last ones of the pass.
+  s.mask = word & 7;
+  s.bv[0] = s.bv[1] = s.bv[2] = 0.0;
+  if (word) {
+    const double *b = bc_val + 3L * (word >> 3);
+    s.bv[0] = b[0];
+    s.bv[1] = b[1];
+    s.bv[2] = b[2];
+  }
 }
 
 // The nodal update of one step for node i given its assembled internal
@@ -1327,20 +1526,22 @@ __device__ __forceinline__ void load_node(int i, long Ns, const NodeParams &np, 
 // run's last step stores the corrected increment, and with a per-step time
 // step (the previous step's length predicted it) it is read and stored
 // every step.
-template <typename T, bool CFL, bool CONTACT>
+// PAIR: the paired node pass, where several work-groups update the same node
+// and only the one that owns it (own) stores; xn_out receives the new
+// position in either case.
+template <typename T, bool CFL, bool CONTACT, bool PAIR>
 __device__ __forceinline__ double node_update(
     int i, long Ns, const NodeParams &np, double (&f)[3], const NodeIn<T, CONTACT> &s,
-    const int *__restrict__ bc_mask, const double *__restrict__ bc_val, T *__restrict__ fi, T *__restrict__ v,
-    T *__restrict__ prev_a, T *__restrict__ u_dt, double *__restrict__ x, double *__restrict__ u,
-    unsigned int *__restrict__ status) {
+    T *__restrict__ fi, T *__restrict__ v, T *__restrict__ prev_a, T *__restrict__ u_dt, double *__restrict__ x, double *__restrict__ u,
+    unsigned int *__restrict__ status, bool own, double *xn_out) {
+  const bool store = !PAIR || own;
   unsigned bad = 0;
 #pragma unroll
   for (int d = 0; d < 3; ++d)
     if (!isfinite(f[d])) { f[d] = 0.0; ++bad; }
-  if (bad) atomicAdd(status, bad);
-  record_reaction<T>(np, i, f[2]);
-  const int slot = s.slot;
-  const int mask = slot >= 0 ? bc_mask[slot] : 0;
+  if (bad && store) atomicAdd(status, bad);
+  if (store) record_reaction<T, PAIR>(np, i, f[2]);
+  const int mask = s.mask;
   const double m = s.m;
   double vs[3];
   const unsigned ui = (unsigned)i;
@@ -1349,26 +1550,28 @@ __device__ __forceinline__ double node_update(
     const long r = d * Ns;
     T &fi_d = (fi + r)[ui], &v_d = (v + r)[ui], &pa_d = (prev_a + r)[ui], &ud_d = (u_dt + r)[ui];
     double &x_d = (x + r)[ui];
-    if (np.write_fi) fi_d = (T)f[d];
+    if (np.write_fi && store) fi_d = (T)f[d];
     double a = (s.fe[d] - f[d]) / m;                    // calcAccel
     if constexpr (CONTACT) a += s.cf[d] / m;            //   + contact force
     if (mask & (1 << d)) a = 0.0;                       // ImposeBCA
     double pa = (double)s.pa[d];
     a = np.f * (a - np.alpha * pa);                     // UpdateCorrectionAccVel
     double vv = (double)s.v[d] + np.gdt * a;
-    if (mask & (1 << d)) vv = bc_val[3L * slot + d];    // ImposeBCV
+    if (mask & (1 << d)) vv = s.bv[d];    // ImposeBCV
     // the previous node pass's prediction, from its v' and a
     double v0 = (double)s.v[d];
     if (!(mask & (1 << d))) v0 = v0 - np.pred_v * pa;
     double ud = np.read_ud ? (double)s.ud[d] : np.dt * (v0 + np.pred_u * pa);
     ud = ud + np.bdt2 * a;                              // UpdateCorrectionPos
     const double xo = s.x[d], xn = xo + ud;
-    x_d = xn;
+    if (store) x_d = xn;
+    if constexpr (PAIR) xn_out[d] = xn;
     if constexpr (std::is_same<T, double>::value) {
       const double bb = xn - xo;
       const double err = (xo - (xn - bb)) + (ud - bb);  // xo + ud - xn, exactly
       const double lo = (np.run_first ? 0.0 : (double)s.lo[d]) + err;
-      if (np.run_last) {
+      if (!store) {
+      } else if (np.run_last) {
         (u + r)[ui] = s.u[d] + (np.run_first ? ud : ((xn - s.xs[d]) + lo));
       } else {
         if (np.run_first) (np.x_start + r)[ui] = xo;
@@ -1378,11 +1581,13 @@ __device__ __forceinline__ double node_update(
     if (np.predict) {                                   // UpdatePrediction
       ud = np.dt * (vv + np.pred_u * a);
       vv = vv + np.pred_v * a;
-      if (mask & (1 << d)) vv = bc_val[3L * slot + d];  // ImposeBCV
+      if (mask & (1 << d)) vv = s.bv[d];  // ImposeBCV
     }
-    if (np.write_ud || !np.predict) ud_d = (T)ud;
-    pa_d = (T)a;
-    v_d = (T)vv;
+    if (store) {
+      if (np.write_ud || !np.predict) ud_d = (T)ud;
+      pa_d = (T)a;
+      v_d = (T)vv;
+    }
     vs[d] = (double)(T)vv;
   }
   // speed of the predicted velocity, for the next step's CFL time step
@@ -1395,8 +1600,9 @@ __device__ __forceinline__ double node_update(
 // Matrices.C:42-87, completed across clusters), four at a time: FP64 through
 // the slot ids of the node's list, FP32-mixed directly from its offset (the
 // element pass stores those sums node-major).
-template <typename T, bool TH = false>
-__device__ __forceinline__ void gather_slots(int o, int c, const int *__restrict__ nsl, const T *__restrict__ part,
+// W: partial sums in flight together.
+template <typename T, bool TH, int W>
+__device__ __forceinline__ void gather_slots(int o, int c, bool nm, const int *__restrict__ nsl, const T *__restrict__ part,
                                              long S, double (&f)[TH ? 4 : 3]) {
   constexpr int R = TH ? 4 : 3;
 #pragma unroll
@@ -1404,21 +1610,21 @@ __device__ __forceinline__ void gather_slots(int o, int c, const int *__restrict
   // every load is issued (indices past the node's count repeat its last
   // slot) and only the node's own entries are added: conditional loads would
   // each be waited for on their own
-  for (int k = 0; k < c; k += 4) {
-    int sl[4];
+  for (int k = 0; k < c; k += W) {
+    int sl[W];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < W; ++j) {
       const int kk = min(k + j, c - 1);
-      if constexpr (kNodeMajor<T>) sl[j] = o + kk;
+      if (kNodeMajor<T> || nm) sl[j] = o + kk;
       else sl[j] = nsl[o + kk];
     }
-    T q[4][R];
+    T q[W][R];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < W; ++j)
 #pragma unroll
       for (int d = 0; d < R; ++d) q[j][d] = part[d * S + sl[j]];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < W; ++j)
       if (k + j < c)
 #pragma unroll
         for (int d = 0; d < R; ++d) f[d] += (double)q[j][d];
@@ -1430,10 +1636,10 @@ __device__ __forceinline__ void gather_slots(int o, int c, const int *__restrict
 // TH: thermal coupling, T += (sum of the node's thermal terms) / m * dt
 template <typename T, int BS, bool CFL, bool CONTACT, bool TH>
 __global__ __launch_bounds__(BS) void f4_node(
-    int N, NodeParams np, const double *__restrict__ cf, const int *__restrict__ nsl_off,
+    int N, NodeParams np, int nm, const double *__restrict__ cf, const int *__restrict__ nsl_off,
     const int *__restrict__ nsl, const T *__restrict__ part, long S,
-    const double *__restrict__ fe, const double *__restrict__ mdiag, const int *__restrict__ bc_slot,
-    const int *__restrict__ bc_mask, const double *__restrict__ bc_val, T *__restrict__ fi,
+    const double *__restrict__ fe, const double *__restrict__ mdiag, const int *__restrict__ bc_word,
+    const double *__restrict__ bc_val, T *__restrict__ fi,
     T *__restrict__ v, T *__restrict__ prev_a, T *__restrict__ u_dt,
     double *__restrict__ x, double *__restrict__ u, unsigned int *__restrict__ status,
     double *__restrict__ Tn) {
@@ -1445,12 +1651,12 @@ __global__ __launch_bounds__(BS) void f4_node(
     // the node's slot range first: the partial sums wait for it, not for
     // the state loads behind it
     const int o = nsl_off[i], c = nsl_off[i + 1] - o;
+    const int word = bc_word[i];  // and the boundary word: the boundary values wait for it
     NodeIn<T, CONTACT> st;
-    load_node<T, CONTACT>(i, N, q, cf, fe, mdiag, bc_slot, v, prev_a, u_dt, x, u, st);
+    load_node<T, CONTACT>(i, N, q, cf, fe, mdiag, word, bc_val, v, prev_a, u_dt, x, u, st);
     double f[TH ? 4 : 3];
-    gather_slots<T, TH>(o, c, nsl, part, S, f);
-    speed = node_update<T, CFL, CONTACT>(i, N, q, *reinterpret_cast<double(*)[3]>(f), st, bc_mask, bc_val, fi, v,
-                                         prev_a, u_dt, x, u, status);
+    gather_slots<T, TH, 4>(o, c, nm, nsl, part, S, f);
+    speed = node_update<T, CFL, CONTACT, false>(i, N, q, *reinterpret_cast<double(*)[3]>(f), st, fi, v, prev_a, u_dt, x, u, status, true, nullptr);
     if constexpr (TH) {  // T += (dTdt + q_cont / (m cp)) dt (Thermal.C:124)
       double r = f[3] / st.m;
       if (q.qcont) r += q.qcont[i] * 1.0 / (st.m * q.cp_T);
@@ -1466,6 +1672,74 @@ __global__ __launch_bounds__(BS) void f4_node(
 }
 
 
+
+// F4 and the next step's F1 in one cluster pass (small meshes, launch-bound):
+// each work-group updates all nodes its elements touch, one per thread, so
+// that it has the new positions its volumes need without waiting for other
+// work-groups; a node of several clusters is updated by each of them alike
+// and stored by its first slot's.  The new state goes to the other set of
+// buffers, since the other work-groups still read this one (x_lo and T, which
+// only the storing thread uses, stay in place).
+// Bound: two dependent rounds of loads (slot record and boundary word; sums,
+// state and boundary values), each near a microsecond since the last kernel's
+// results lie beyond this XCD's L2, the update and the launch; not bytes.
+struct NodeSet {  // the nodal arrays a paired node pass writes
+  double *x;
+  void *v, *pa, *ud;
+};
+template <typename T, int NN, bool CFL, bool CONTACT, bool TH>
+__global__ __launch_bounds__(slot_cap(NN)) void f41_cluster(
+    int N, NodeParams np, ClusterArgs ca, PairArgs pr, NodeSet out, const double *__restrict__ cf,
+    const T *__restrict__ part, const double *__restrict__ fe, const double *__restrict__ mdiag,
+    const double *__restrict__ bc_val, T *__restrict__ fi, const T *__restrict__ v, const T *__restrict__ prev_a,
+    const T *__restrict__ u_dt, const double *__restrict__ x, unsigned int *__restrict__ status,
+    double *__restrict__ Tn, T *__restrict__ vol, double *__restrict__ minl_part) {
+  constexpr int cap = slot_cap(NN);
+  __shared__ double lx[3 * cap];
+  const int c = xcd_block(), t = threadIdx.x;
+  const int4 cd = ca.desc[c];
+  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
+  NodeParams q = np;
+  if constexpr (CFL) set_step_length(q, *q.dtp);
+  // as in the element pass every load is issued unconditionally: threads past
+  // the cluster's slots or elements repeat its last one and store nothing
+  const int4 rec = pr.rec[s0 + min(t, M - 1)];
+  const int word = pr.sbc[s0 + min(t, M - 1)];
+  int ls[NN];
+  load_lslot<NN>(ca.lslot + (long)(e0 + min(t, ne - 1)) * NN, ls);
+  const int i = rec.x;
+  const bool own = t < M && rec.w < 0;
+  NodeIn<T, CONTACT> st;
+  load_node<T, CONTACT>(i, N, q, cf, fe, mdiag, word, bc_val, v, prev_a, u_dt, x, nullptr, st);
+  double f[TH ? 4 : 3];
+  // all of a node's sums in one round: up to 8 clusters meet in a corner of bricks
+  if (__any(rec.z > 4)) gather_slots<T, TH, 8>(rec.y, rec.z, true, nullptr, part, ca.S, f);
+  else gather_slots<T, TH, 4>(rec.y, rec.z, true, nullptr, part, ca.S, f);
+  double xn[3];
+  double speed = node_update<T, CFL, CONTACT, true>(
+      i, N, q, *reinterpret_cast<double(*)[3]>(f), st, fi, static_cast<T *>(out.v), static_cast<T *>(out.pa),
+      static_cast<T *>(out.ud), out.x, nullptr, status, own, xn);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) lx[d * cap + t] = xn[d];
+  if constexpr (TH) {
+    if (own) {
+      double r = f[3] / st.m;
+      if (q.qcont) r += q.qcont[i] * 1.0 / (st.m * q.cp_T);
+      Tn[i] += r * q.dt;
+    }
+  }
+  __syncthreads();
+  double medge = kMinEdgeInit;
+  if (t < ne) medge = element_volume<T, NN>(e0 + t, lx, cap, ls, CFL, vol, status);
+  if constexpr (CFL) {
+    medge = block_extreme<cap, true>(medge);
+    speed = block_extreme<cap, false>(speed);
+    if (t == 0) {
+      minl_part[blockIdx.x] = medge;
+      q.vmax_part[blockIdx.x] = speed;
+    }
+  }
+}
 
 // FP32-mixed fused runs keep v, prev_a, u_dt and fi in float between steps:
 // narrowed once when the run starts, widened back (and u advanced by the
@@ -1566,16 +1840,24 @@ hipError_t launch_rigid_update(wfx_ctx *c, bool device_dt, hipStream_t s) {
 
 }  // namespace
 
+// V0_n (v0) and the nodal mean densities
 template <typename T>
-hipError_t launch_vsum0(wfx_ctx *c, hipStream_t s) {
+hipError_t launch_run_sums(wfx_ctx *c, bool v0, hipStream_t s) {
   if (c->f2_lanes) {
     hipLaunchKernelGGL((f0_vsum0_lanes<T>), dim3(nblocks((long)c->N * kF2Lanes)), dim3(kBlock), 0, s, c->N,
-                       c->ms.nodel_offset, c->ms.nodel_count, c->ms.nodel_pk, elem<T>(c).vol0, c->nd.voln0_sum);
+                       c->ms.nodel_offset, c->ms.nodel_count, c->ms.nodel_pk, elem<T>(c).vol0, elem<T>(c).rho,
+                       v0 ? c->nd.voln0_sum : (double *)nullptr, c->nd.rho_avg);
   } else {
     hipLaunchKernelGGL((f0_vsum0<T>), dim3(nblocks(c->N)), dim3(kBlock), 0, s, c->N, c->ms.nodel_offset,
-                       c->ms.nodel_count, c->ms.nodel_pk, elem<T>(c).vol0, c->nd.voln0_sum);
+                       c->ms.nodel_count, c->ms.nodel_pk, elem<T>(c).vol0, elem<T>(c).rho,
+                       v0 ? c->nd.voln0_sum : (double *)nullptr, c->nd.rho_avg);
   }
+  c->rho_avg_valid = true;
   return hipGetLastError();
+}
+template <typename T>
+hipError_t launch_vsum0(wfx_ctx *c, hipStream_t s) {
+  return launch_run_sums<T>(c, true, s);
 }
 
 inline NodeParams node_params(wfx_ctx *c, int predict) {
@@ -1623,9 +1905,162 @@ hipError_t launch_thermal(wfx_ctx *c, hipStream_t s);
 
 // Launch one phase (1..4) of a fused step on the current state with block
 // size BS; launch_fused_phase picks BS from the context (autotuned or 256).
-template <typename T, int NN, int LAW>
+template <typename T, int NN, int LAW, bool PAIR>
 auto f3_pick(bool th) {
-  return th ? f3_cluster<T, NN, LAW, true> : f3_cluster<T, NN, LAW, false>;
+  return th ? f3_cluster<T, NN, LAW, true, PAIR> : f3_cluster<T, NN, LAW, false, PAIR>;
+}
+
+// the fused path's nodal arrays in the element real type
+template <typename T>
+void fused_node_arrays(wfx_ctx *c, T *&v, T *&pa, T *&ud, T *&fi) {
+  if constexpr (std::is_same<T, double>::value) {
+    v = c->nd.v; pa = c->nd.prev_a; ud = c->nd.u_dt; fi = c->nd.fi;
+  } else {
+    v = c->v32; pa = c->pa32; ud = c->ud32; fi = c->fi32;
+  }
+}
+inline ClusterArgs cluster_args(const wfx_ctx *c) {
+  return ClusterArgs{c->ms.cl_desc, c->ms.cl_goff, c->ms.cl_ent, c->ms.cl_snode,
+                     c->ms.cl_lslot, c->ms.spos,  c->ms.nslot,   c->ms.spos != nullptr};
+}
+
+// F3 (PAIR: with F2 in its staging); dtp: the step's dt on the device, or null
+template <typename T, bool PAIR>
+hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr, hipStream_t s) {
+  auto &el = elem<T>(c);
+  const auto &P = c->prm;
+  const auto &st = P.stab;
+  T *vN, *paN, *udN, *fiN;
+  fused_node_arrays<T>(c, vN, paN, udN, fiN);
+  FusedParams fp;
+  fp.dt = P.dt;
+  fp.mp = mat_params(c);
+  fp.pp = press_params(c);
+  fp.need_jlocal = press_needs_jlocal(fp.pp);
+  fp.av_al = st.artifvisc0;
+  fp.av_be = st.artifvisc1;
+  fp.avq = el.avq;
+  fp.hg_coeff = (c->n == 8) ? st.hg_coeff : 0.0;
+  fp.cs0 = P.mat.cs0;
+  fp.rho_u = c->rho_uniform;
+  fp.dtp = dtp;
+  fp.plheat_frac = c->thermal.plheat_frac;
+  fp.k_T = c->thermal.k_T;
+  fp.cp_T = c->thermal.cp_T;
+  const bool texp = c->thermal.on && c->thermal.exp_T != 0.0;
+  fp.exp_T = c->thermal.exp_T;
+  fp.texp = texp ? el.texp : nullptr;
+  fp.dte_flat = texp ? el.dte_flat : nullptr;
+  fp.flat_base = c->ms.flat_base;
+  fp.mdiag = c->nd.mdiag;
+  fp.write_out = c->fused_write_out;
+  const bool rate = law_class(fp.mp.model) == LAW_RATE, th = c->thermal.on;
+  auto kern = (c->n == 8) ? (rate ? f3_pick<T, 8, LAW_RATE, PAIR>(th) : f3_pick<T, 8, LAW_PLAIN, PAIR>(th))
+                          : (rate ? f3_pick<T, 4, LAW_RATE, PAIR>(th) : f3_pick<T, 4, LAW_PLAIN, PAIR>(th));
+  hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, c->E, c->N, fp, cluster_args(c), pr, c->nd.x, vN,
+                     c->nd.anp_ratio, el.vol0, el.rho, el.sy0, el.He, el.tau, el.eps, el.p, el.pl_strain,
+                     el.sigma_y, el.part, c->thermal.on ? el.q_plheat : (T *)nullptr);
+  return hipGetLastError();
+}
+
+// F1, with the edge minima of the per-step CFL time step when cfl
+template <typename T>
+hipError_t launch_volumes(wfx_ctx *c, bool cfl, hipStream_t s) {
+  auto &el = elem<T>(c);
+  const bool texp = c->thermal.on && c->thermal.exp_T != 0.0;
+  auto kern = c->n == 8 ? f1_cluster<T, 8> : f1_cluster<T, 4>;
+  hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, c->E, cluster_args(c), c->nd.x, c->N, el.vol,
+                     cfl ? c->cfl_part : (double *)nullptr, c->status, el.dte_flat, texp ? el.texp : (T *)nullptr);
+  return hipGetLastError();
+}
+
+// ---- paired passes: two kernels per step ------------------------------------
+template <typename T>
+PairArgs pair_args(wfx_ctx *c, int step) {
+  PairArgs pr{};
+  pr.rec = c->ms.srec;
+  pr.sent = c->ms.sent;
+  pr.pw = c->ms.pw;
+  pr.lanes = c->f2_lanes;
+  pr.vol = elem<T>(c).vol;
+  pr.vsum0 = c->nd.voln0_sum;
+  pr.rho_avg = c->nd.rho_avg;
+  pr.sbc = c->ms.sbc;
+  pr.ratio = c->nd.anp_ratio;
+  pr.mdiag = c->nd.mdiag;
+  pr.cfl = c->prm.cfl;
+  pr.K = c->prm.mat.K;
+  pr.minl = c->cfl_part;
+  pr.vmax = c->cfl_part + c->cfl_cap_min;
+  pr.nmin = c->ms.ncl;
+  pr.nmax = c->cfl_nvmax;
+  pr.step = step;
+  pr.scal = c->scalars;
+  pr.dt_hist = (step >= 0 && step < c->dt_cap) ? c->dt_hist : nullptr;
+  return pr;
+}
+
+// nodal sums and element pass of one step (F2 + F3), and the contact forces
+template <typename T>
+hipError_t launch_pair_element(wfx_ctx *c, int step, hipStream_t s) {
+  const bool cfl = c->prm.cfl > 0.0;
+  if (cfl && c->contact.on) {  // calcMinEdgeLength also refreshes the element heights contact uses
+    hipError_t e = launch_elem_length(c, s);
+    if (e != hipSuccess) return e;
+  }
+  hipError_t e = launch_element_pass<T, true>(c, nullptr, pair_args<T>(c, step), s);
+  if (e != hipSuccess || !c->contact.on) return e;
+  T *vN, *paN, *udN, *fiN;
+  fused_node_arrays<T>(c, vN, paN, udN, fiN);
+  return launch_contact<T>(c, vN, cfl, s);
+}
+
+template <typename T, int NN, bool CFL, bool CT>
+auto f41_pick(bool th) {
+  return th ? f41_cluster<T, NN, CFL, CT, true> : f41_cluster<T, NN, CFL, CT, false>;
+}
+template <typename T, int NN>
+auto f41_pick(bool cfl, bool ct, bool th) {
+  return cfl ? (ct ? f41_pick<T, NN, true, true>(th) : f41_pick<T, NN, true, false>(th))
+             : (ct ? f41_pick<T, NN, false, true>(th) : f41_pick<T, NN, false, false>(th));
+}
+
+// the context's nodal arrays and the other set change places
+template <typename T>
+void pair_swap(wfx_ctx *c) {
+  std::swap(c->nd.x, c->x_b);
+  auto swap_t = [](T *&a, void *&b) {
+    T *q = a;
+    a = static_cast<T *>(b);
+    b = q;
+  };
+  if constexpr (std::is_same<T, double>::value) {
+    swap_t(c->nd.v, c->v_b); swap_t(c->nd.prev_a, c->pa_b); swap_t(c->nd.u_dt, c->ud_b);
+  } else {
+    swap_t(c->v32, c->v_b); swap_t(c->pa32, c->pa_b); swap_t(c->ud32, c->ud_b);
+  }
+}
+
+// node pass of one step and the next one's volumes (F4 + F1), the rigid
+// surfaces' motion; the nodal arrays change places
+template <typename T>
+hipError_t launch_pair_node(wfx_ctx *c, hipStream_t s) {
+  const bool cfl = c->prm.cfl > 0.0, ct = c->contact.on, th = c->thermal.on;
+  auto &el = elem<T>(c);
+  T *vN, *paN, *udN, *fiN;
+  fused_node_arrays<T>(c, vN, paN, udN, fiN);
+  NodeParams np = node_params(c, 1);
+  np.dtp = cfl ? c->scalars + kCflDt : nullptr;
+  np.vmax_part = c->cfl_part + c->cfl_cap_min;
+  auto kern = c->n == 8 ? f41_pick<T, 8>(cfl, ct, th) : f41_pick<T, 4>(cfl, ct, th);
+  hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(slot_cap(c->n)), 0, s, c->N, np, cluster_args(c), pair_args<T>(c, -1),
+                     NodeSet{c->x_b, c->v_b, c->pa_b, c->ud_b}, c->contact.contforce, el.part, c->nd.fe,
+                     c->nd.mdiag, c->bc_tab, fiN, vN, paN, udN, c->nd.x, c->status, c->nd.T, el.vol, c->cfl_part);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (cfl) c->cfl_nvmax = c->ms.ncl;
+  pair_swap<T>(c);
+  return ct ? launch_rigid_update(c, cfl, s) : hipSuccess;
 }
 
 template <typename T, int BS, bool CFL, bool CT>
@@ -1639,71 +2074,39 @@ hipError_t launch_fused_phase_bs(wfx_ctx *c, int phase, int predict, int step, h
   const bool cfl = step >= 0 && c->prm.cfl > 0.0;
   const double *dtp = cfl ? c->scalars + kCflDt : nullptr;
   auto &el = elem<T>(c);
-  const auto &P = c->prm;
-  const auto &st = P.stab;
+  const auto &st = c->prm.stab;
   const int N = c->N, E = c->E;
   const int gN = (N + BS - 1) / BS;
-  // nodal arrays of the fused node pass in the element real type
   T *vN, *paN, *udN, *fiN;
-  if constexpr (std::is_same<T, double>::value) {
-    vN = c->nd.v; paN = c->nd.prev_a; udN = c->nd.u_dt; fiN = c->nd.fi;
-  } else {
-    vN = c->v32; paN = c->pa32; udN = c->ud32; fiN = c->fi32;
-  }
-  const ClusterArgs ca{c->ms.cl_eoff, c->ms.cl_sbase, c->ms.cl_loff,  c->ms.cl_ent,
-                       c->ms.cl_snode, c->ms.cl_lslot, c->ms.spos, c->ms.nslot};
+  fused_node_arrays<T>(c, vN, paN, udN, fiN);
+  const ClusterArgs ca = cluster_args(c);
   if (phase == 1) {
-    double *minl = cfl ? c->cfl_part : nullptr;
-    const bool texp = c->thermal.on && c->thermal.exp_T != 0.0;
-    auto kern = c->n == 8 ? f1_cluster<T, 8> : f1_cluster<T, 4>;
-    hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, E, ca, c->nd.x, N, el.vol, minl, c->status,
-                       el.dte_flat, texp ? el.texp : (T *)nullptr);
+    hipError_t e = launch_volumes<T>(c, cfl, s);
+    if (e != hipSuccess) return e;
     if (cfl) {
-      hipError_t e = launch_cfl_reduce<T>(c, c->ms.ncl, step, s);
+      e = launch_cfl_reduce<T>(c, c->ms.ncl, step, s);
       // calcMinEdgeLength also refreshes the element heights contact uses
       if (e == hipSuccess && c->contact.on) e = launch_elem_length(c, s);
       return e;
     }
   } else if (phase == 2) {
+    if (!c->rho_avg_valid) {  // outside a run, after the densities changed
+      hipError_t e = launch_run_sums<T>(c, false, s);
+      if (e != hipSuccess) return e;
+    }
     if (c->f2_lanes) {
       const int gL = (int)(((long)N * kF2Lanes + BS - 1) / BS);
       hipLaunchKernelGGL((f2_nodal_lanes<T, BS>), dim3(gL), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
-                         c->ms.nodel_count, c->ms.nodel_pk, el.vol, el.rho, c->nd.voln0_sum, c->nd.anp_ratio,
+                         c->ms.nodel_count, c->ms.nodel_pk, el.vol, c->nd.rho_avg, c->nd.voln0_sum, c->nd.anp_ratio,
                          c->nd.mdiag, c->rho_uniform);
     } else {
       hipLaunchKernelGGL((f2_nodal<T, BS>), dim3(gN), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
-                         c->ms.nodel_count, c->ms.nodel_pk, c->ms.nodel_pad, el.vol, el.rho, c->nd.voln0_sum,
+                         c->ms.nodel_count, c->ms.nodel_pk, c->ms.nodel_pad, el.vol, c->nd.rho_avg, c->nd.voln0_sum,
                          c->nd.anp_ratio, c->nd.mdiag, c->rho_uniform);
     }
   } else if (phase == 3) {
-    FusedParams fp;
-    fp.dt = P.dt;
-    fp.mp = mat_params(c);
-    fp.pp = press_params(c);
-    fp.need_jlocal = press_needs_jlocal(fp.pp);
-    fp.av_al = st.artifvisc0;
-    fp.av_be = st.artifvisc1;
-    fp.avq = el.avq;
-    fp.hg_coeff = (c->n == 8) ? st.hg_coeff : 0.0;
-    fp.cs0 = P.mat.cs0;
-    fp.rho_u = c->rho_uniform;
-    fp.dtp = dtp;
-    fp.plheat_frac = c->thermal.plheat_frac;
-    fp.k_T = c->thermal.k_T;
-    fp.cp_T = c->thermal.cp_T;
-    const bool texp = c->thermal.on && c->thermal.exp_T != 0.0;
-    fp.exp_T = c->thermal.exp_T;
-    fp.texp = texp ? el.texp : nullptr;
-    fp.dte_flat = texp ? el.dte_flat : nullptr;
-    fp.flat_base = c->ms.flat_base;
-    fp.mdiag = c->nd.mdiag;
-    fp.write_out = c->fused_write_out;
-    const bool rate = law_class(fp.mp.model) == LAW_RATE, th = c->thermal.on;
-    auto kern = (c->n == 8) ? (rate ? f3_pick<T, 8, LAW_RATE>(th) : f3_pick<T, 8, LAW_PLAIN>(th))
-                            : (rate ? f3_pick<T, 4, LAW_RATE>(th) : f3_pick<T, 4, LAW_PLAIN>(th));
-    hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, E, N, fp, ca, c->nd.x, vN,
-                       c->nd.anp_ratio, el.vol0, el.rho, el.sy0, el.He, el.tau, el.eps, el.p, el.pl_strain,
-                       el.sigma_y, el.part, c->thermal.on ? el.q_plheat : (T *)nullptr);
+    hipError_t e = launch_element_pass<T, false>(c, dtp, PairArgs{}, s);
+    if (e != hipSuccess) return e;
     // contact forces after the element forces, before the assembly
     if (c->contact.on) return launch_contact<T>(c, vN, cfl, s);
   } else if (phase == 4) {
@@ -1714,8 +2117,8 @@ hipError_t launch_fused_phase_bs(wfx_ctx *c, int phase, int predict, int step, h
     const bool ct = c->contact.on, th = c->thermal.on;
     auto kern = cfl ? (ct ? f4_pick<T, BS, true, true>(th) : f4_pick<T, BS, true, false>(th))
                     : (ct ? f4_pick<T, BS, false, true>(th) : f4_pick<T, BS, false, false>(th));
-    hipLaunchKernelGGL(kern, dim3(gN), dim3(BS), 0, s, N, np, c->contact.contforce, c->ms.nsl_off, c->ms.nsl,
-                       el.part, c->ms.nslot, c->nd.fe, c->nd.mdiag, c->bc_slot, c->bc_mask, c->bc_tab, fiN, vN,
+    hipLaunchKernelGGL(kern, dim3(gN), dim3(BS), 0, s, N, np, ca.nm, c->contact.contforce, c->ms.nsl_off, c->ms.nsl,
+                       el.part, c->ms.nslot, c->nd.fe, c->nd.mdiag, c->bc_word, c->bc_tab, fiN, vN,
                        paN, udN, c->nd.x, c->nd.u, c->status, c->nd.T);
     // the rigid surfaces move after the position update
     if (c->contact.on && step >= 0) return launch_rigid_update(c, cfl, s);
@@ -1833,6 +2236,20 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
     hipError_t e = launch_cfl_begin<T>(c, s, true);
     if (e != hipSuccess) return e;
   }
+  // Paired passes: the nodal arrays change places in every step but the
+  // last, whose node pass updates them in place; the first step's does too
+  // where that makes the changes even, so that a run ends in the arrays it
+  // started in (a captured run has their addresses in its kernels).  With
+  // events the four passes run separately.
+  const bool pair = c->pair && !ev && !(c->thermal.on && c->thermal.exp_T != 0.0);
+  struct Places {  // a failed launch leaves the arrays in their places
+    wfx_ctx *c;
+    double *x;
+    ~Places() {
+      if (c->nd.x != x) pair_swap<T>(c);
+    }
+  } places{c, c->nd.x};
+  bool have_vol = false;
   for (int k = 0; k < nsteps; ++k) {
     if (c->contact.on && (c->contact.step_count + k) % 10 == 0) {
       hipError_t e = launch_ext_face_areas(c, s);  // every 10 steps, at the step's start
@@ -1847,22 +2264,22 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
     c->fused_write_ud = c->prm.cfl > 0.0 ? 1 : 0;
     c->fused_run_first = k == 0 ? 1 : 0;
     c->fused_run_last = k + 1 == nsteps ? 1 : 0;
-    for (int ph = 1; ph <= 4; ++ph) {
-      if (ev) {
-        hipError_t e = hipEventRecord(ev[4 * k + ph - 1], s);
-        if (e != hipSuccess) return e;
-      }
+    const bool in_place = !pair || k + 1 == nsteps || (k == 0 && nsteps % 2 == 0);
+    hipError_t e = hipSuccess;
+    for (int ph = 1; ph <= 4 && e == hipSuccess; ++ph) {
+      if (ev) e = hipEventRecord(ev[4 * k + ph - 1], s);
+      if (e != hipSuccess || (ph == 1 && have_vol) || (ph == 2 && pair)) continue;
       c->fused_rz = ph == 4 ? rec.row(k) : nullptr;
-      hipError_t e = launch_fused_phase<T>(c, ph, k + 1 < nsteps, s, k);
-      c->fused_rz = nullptr;
-      if (e != hipSuccess) {
-        c->fused_write_fi = c->fused_write_out = c->fused_read_ud = c->fused_write_ud = 1;
-        c->fused_run_first = c->fused_run_last = 1;
-        return e;
-      }
+      if (ph == 1 && pair) e = launch_volumes<T>(c, c->prm.cfl > 0.0, s);
+      else if (ph == 3 && pair) e = launch_pair_element<T>(c, k, s);
+      else if (ph == 4 && !in_place) e = launch_pair_node<T>(c, s);
+      else e = launch_fused_phase<T>(c, ph, k + 1 < nsteps, s, k);
     }
+    have_vol = !in_place;
+    c->fused_rz = nullptr;
     c->fused_write_fi = c->fused_write_out = c->fused_read_ud = c->fused_write_ud = 1;
     c->fused_run_first = c->fused_run_last = 1;
+    if (e != hipSuccess) return e;
     if (ev && k + 1 == nsteps) {
       hipError_t e = hipEventRecord(ev[4 * nsteps], s);
       if (e != hipSuccess) return e;

@@ -65,6 +65,11 @@ struct Stab {
 
 // elements per cluster of the fused element pass (its work-group size)
 constexpr int kCluster = 256;
+// The element pass's element-node values in LDS: component u of node a of the
+// cluster's element t at u * kEntStride(n) + a * kCluster + t, and a cell that
+// holds zero at u * kEntStride(n) + n * kCluster, which the slots' unused entries
+// name
+constexpr int kEntStride(int n) { return (n + 1) * kCluster; }
 
 // slots of the context's device status counters (unsigned int[16])
 constexpr int kStatNonfinite = 0;  // non-finite internal-force entries scrubbed
@@ -127,6 +132,7 @@ struct DevNode {
   double *T = nullptr;  // nodal temperature (thermal coupling)
   double *mdiag = nullptr, *voln = nullptr, *voln0_sum = nullptr;
   double *anp_ratio = nullptr;  // fused path: V_n / V0_n
+  double *rho_avg = nullptr;    // fused path: mean density of the node's elements
 };
 
 struct DevMesh {
@@ -141,12 +147,25 @@ struct DevMesh {
   // partial sums are stored there, node-major)
   int ncl = 0;
   long nslot = 0;
-  int *cl_eoff = nullptr, *cl_sbase = nullptr;
-  uint16_t *cl_loff = nullptr, *cl_ent = nullptr;
+  // [C] {first element, first slot, elements | slots << 16, first entry group};
+  // per cluster its slots + 1 group offsets (cluster c at its first slot + c);
+  // the entry groups, four LDS byte offsets of element-node values each
+  // (kEntStride), a slot's last one filled up with the zero cell's
+  int4 *cl_desc = nullptr;
+  uint16_t *cl_goff = nullptr;
+  uint2 *cl_ent = nullptr;
   int *nsl_off = nullptr, *nsl = nullptr, *spos = nullptr;
   // slot -> node [S]; each stored element's nodes as slot indices of its cluster [E][n]
   int *cl_snode = nullptr;
   uint16_t *cl_lslot = nullptr;
+  // paired passes (small meshes): per slot {node, its first position in the
+  // node's slot list, the list's length, the node's element count | (first
+  // slot of the node) << 31}, and the node's stored elements in CSR order,
+  // padded to pw entries with repeats of the last one [S][pw]
+  int4 *srec = nullptr;
+  int *sent = nullptr;
+  int pw = 0;
+  int *sbc = nullptr;  // and the slot's boundary word (wfx_ctx::bc_word of its node)
   int *o2s = nullptr;        // original element -> stored element (field transfers)
   int *flat_base = nullptr;  // thermal expansion: original element * n of each stored element
 };
@@ -175,6 +194,7 @@ struct wfx_ctx {
   // original element el_s2o[s]; every element field crosses the boundary in
   // the original order
   std::vector<int> el_s2o, el_o2s;
+  std::vector<int> slot_node_h;  // paired passes: the node of each slot
   std::vector<int> nodel_h, nodel_loc_h, nodel_offset_h, nodel_count_h;
   std::vector<double> sy0_h;     // per element
   std::vector<int> bc_nod_h[3];
@@ -200,15 +220,18 @@ struct wfx_ctx {
   int react_n = 0, react_rows = 0;
   void *react_ring = nullptr;
   void *fused_rz = nullptr;  // the row the next fused node pass fills (set inside runs)
-  // per-node Dirichlet data for the fused node pass: slot or -1, bit mask of
-  // constrained directions and the three prescribed values per slot
-  int *bc_slot = nullptr, *bc_mask = nullptr;
+  // per-node Dirichlet data for the fused node pass, and the three prescribed
+  // values per slot
+  int *bc_word = nullptr;  // [N] (slot << 3) | mask of the constrained directions; 0: none
   double *bc_tab = nullptr;
   // FP32-mixed fused path: narrowed nodal state during a run, start positions
   float *v32 = nullptr, *pa32 = nullptr, *ud32 = nullptr, *fi32 = nullptr;
   double *x_start = nullptr;  // (both precisions)
   float *x_lo = nullptr;      // FP64 fused runs: rounding error of the position updates
   int has_fe = 0;            // external nodal forces set (non-zero)
+  // rho_avg holds the present densities' means (a run forms them anew; a
+  // single node pass outside one does when this is not set)
+  bool rho_avg_valid = false;
   double rho_uniform = 0.0;  // > 0: every element density equals this value
   // host scan of vol0 and rho (wfx_init, wfx_set_field): elem_guard 1 when an
   // initial volume is not finite or (nearly) zero or a density is not positive
@@ -235,6 +258,13 @@ struct wfx_ctx {
   int fused_write_ud = 1;    // and stores it every step (cleared inside runs of a fixed time step)
   int fused_run_first = 1;   // the fused step is the first of a run
   int fused_run_last = 1;    // the fused step is the last of a run
+  // Paired passes: a run takes two kernels per step (nodal sums with the
+  // element pass, node pass with the next volumes); the node pass writes
+  // x, v, prev_a and u_dt to the other of two sets of buffers (the b set here;
+  // v, prev_a and u_dt in the fused path's nodal type)
+  int pair = 0;
+  double *x_b = nullptr;
+  void *v_b = nullptr, *pa_b = nullptr, *ud_b = nullptr;
   int f2_lanes = 0;          // the nodal volume sums take several lanes per node (many elements per node)
   double *scalars = nullptr;      // device scratch for reductions (reaction force)
   // this context's device's address of the library's static scratch array
