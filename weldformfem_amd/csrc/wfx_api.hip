@@ -50,6 +50,32 @@ static hipError_t dalloc(wfx_ctx *c, T **p, size_t count) {
   return e;
 }
 
+// The buffers a mesh needs, asked for one by one and taken from one
+// allocation, cleared by one memset: some 60 allocations and memsets of their own
+// were half of the set-up of a small mesh.
+class Arena {
+ public:
+  template <typename T>
+  void want(T *&p, size_t count) {
+    want_bytes((void **)&p, count * sizeof(T));
+  }
+  void want_bytes(void **p, size_t bytes) {
+    asked_.push_back({p, total_});
+    total_ += (std::max<size_t>(bytes, 1) + 255) / 256 * 256;  // hipMalloc's own alignment
+  }
+  hipError_t take(wfx_ctx *c) {
+    char *base = nullptr;
+    hipError_t e = dalloc(c, &base, total_);
+    if (e == hipSuccess)
+      for (auto &a : asked_) *a.first = base + a.second;
+    return e;
+  }
+
+ private:
+  std::vector<std::pair<void **, size_t>> asked_;
+  size_t total_ = 0;
+};
+
 static void drop_graph(wfx_ctx *c) {
   if (c->graph_exec) (void)hipGraphExecDestroy(c->graph_exec);
   if (c->graph) (void)hipGraphDestroy(c->graph);
@@ -98,11 +124,9 @@ static void free_all(wfx_ctx *c) {
 }
 
 template <typename T>
-static hipError_t alloc_elem(wfx_ctx *c, DevElem<T> &el) {
+static void want_elem(wfx_ctx *c, DevElem<T> &el, Arena &arena) {
   const size_t E = c->E, n = c->n;
-  hipError_t e = hipSuccess;
-#define A(ptr, cnt) \
-  if (e == hipSuccess) e = dalloc(c, &el.ptr, (cnt));
+#define A(ptr, cnt) arena.want(el.ptr, (cnt));
   A(detJ, E) A(dH, 3 * n * E) A(vol, E) A(vol0, E) A(rho, E) A(rho0, E) A(p, E) A(pl_strain, E)
   A(sigma_y, E) A(sy0, E) A(str_rate, 6 * E) A(rot_rate, 3 * E) A(sigma, 6 * E) A(tau, 6 * E)
   // f_elem is padded to whole 64-element tiles (the fused path may tile it);
@@ -110,7 +134,6 @@ static hipError_t alloc_elem(wfx_ctx *c, DevElem<T> &el) {
   A(eps, 6 * E) A(strain_pl_incr, 6 * E) A(f_elem, (std::is_same<T, float>::value ? 4 : 3) * n * ((E + 63) / 64 * 64))
   A(f_hg, 3 * n * E) A(avq, E) A(part, 4 * (c->ms.nslot > 0 ? c->ms.nslot : 1))
 #undef A
-  return e;
 }
 
 // ---- static scratch of the allocation-free entry point ----------------------
@@ -199,27 +222,23 @@ static EntryTables entry_tables(const wfx_ctx *c, const ClusterPlan &plan) {
 // separate passes never take less than the 17 us their four launches cost.
 constexpr int kPairMaxClusters = 256;
 constexpr int kPairMaxElems = 32;  // elements of a node
-struct PairTables {
-  int pw = 0;
-  std::vector<int4> rec;
-  std::vector<int> ent;
-};
-static PairTables pair_tables(const wfx_ctx *c, const ClusterPlan &plan) {
-  PairTables t;
-  const int most = c->nodel_count_h.empty() ? 0 : *std::max_element(c->nodel_count_h.begin(), c->nodel_count_h.end());
-  if (plan.clusters() > kPairMaxClusters || most > kPairMaxElems) return t;
+// Entries per slot of the paired passes' table, or 0
+static int pair_width(const wfx_ctx *c, const ClusterPlan &plan) {
+  if (plan.clusters() > kPairMaxClusters || c->nodel_count_h.empty()) return 0;
+  const auto mm = std::minmax_element(c->nodel_count_h.begin(), c->nodel_count_h.end());
   // a node of no element has no slot: only the separate node pass reaches it
-  if (*std::min_element(c->nodel_count_h.begin(), c->nodel_count_h.end()) == 0) return t;
-  t.pw = (most + 7) / 8 * 8;
-  const long S = plan.slots();
-  t.rec.resize(S);
-  t.ent.resize((size_t)S * t.pw);
-  for (long s = 0; s < S; ++s) {
-    const int i = plan.snode[s], o = plan.nsl_off[i], cnt = c->nodel_count_h[i], co = c->nodel_offset_h[i];
-    t.rec[s] = make_int4(i, o, plan.nsl_off[i + 1] - o, (int)((unsigned)cnt | (plan.nsl[o] == s ? 0x80000000u : 0u)));
-    for (int k = 0; k < t.pw; ++k) t.ent[(size_t)s * t.pw + k] = c->el_o2s[c->nodel_h[co + std::min(k, cnt - 1)]];
-  }
-  return t;
+  if (*mm.second > kPairMaxElems || *mm.first == 0) return 0;
+  return (*mm.second + 7) / 8 * 8;
+}
+// the tables themselves from the ones already on the device, one thread per slot
+__global__ __launch_bounds__(256) void k_pair_tables(long S, int pw, const int *snode, const int *spos,
+                                                     const int *nsl_off, const int *off, const int *cnt,
+                                                     const int *nodel, int4 *rec, int *ent) {
+  const long s = blockIdx.x * 256L + threadIdx.x;
+  if (s >= S) return;
+  const int i = snode[s], o = nsl_off[i], c = cnt[i], co = off[i];
+  rec[s] = make_int4(i, o, nsl_off[i + 1] - o, (int)((unsigned)c | (spos[s] == o ? 0x80000000u : 0u)));
+  for (int k = 0; k < pw; ++k) ent[s * pw + k] = nodel[co + min(k, c - 1)];
 }
 
 // Allocates every device buffer for the mesh held on the host and uploads
@@ -231,9 +250,8 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     if (rc) return rc;
   }
   const size_t N = c->N, E = c->E, n = c->n;
-  hipError_t e = hipSuccess;
-#define A(ptr, cnt) \
-  if (e == hipSuccess) e = dalloc(c, &ptr, (cnt));
+  Arena arena;
+#define A(ptr, cnt) arena.want(ptr, (cnt));
   A(c->nd.x, 3 * N) A(c->nd.v, 3 * N) A(c->nd.a, 3 * N) A(c->nd.u, 3 * N) A(c->nd.u_dt, 3 * N)
   A(c->nd.prev_a, 3 * N) A(c->nd.fi, 3 * N) A(c->nd.fe, 3 * N) A(c->nd.mdiag, N) A(c->nd.voln, N)
   A(c->nd.voln0_sum, N) A(c->nd.anp_ratio, N) A(c->nd.T, N) A(c->nd.rho_avg, N)
@@ -254,24 +272,24 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
   A(c->ms.cl_desc, c->ms.ncl) A(c->ms.cl_goff, c->ms.nslot + c->ms.ncl)
   A(c->ms.cl_ent, et.ent.size()) A(c->ms.nsl_off, N + 1)
   A(c->ms.cl_snode, c->ms.nslot) A(c->ms.cl_lslot, n * E)
-  const PairTables pt = pair_tables(c, plan);
-  c->pair = pt.pw > 0;
+  const int pw = pair_width(c, plan);
+  c->pair = pw > 0;
   if (c->precision == WFX_FP64) A(c->ms.nsl, c->ms.nslot)
   if (c->precision == WFX_FP32_MIXED || c->pair) A(c->ms.spos, c->ms.nslot)
   if (c->pair) {
-    double *t[3] = {nullptr, nullptr, nullptr};  // (doubles: enough for either nodal type)
-    A(c->ms.sbc, c->ms.nslot) A(c->ms.srec, c->ms.nslot) A(c->ms.sent, pt.ent.size()) A(c->x_b, 3 * N)
-    A(t[0], 3 * N) A(t[1], 3 * N) A(t[2], 3 * N)
-    c->v_b = t[0];
-    c->pa_b = t[1];
-    c->ud_b = t[2];
-    c->ms.pw = pt.pw;
+    A(c->ms.sbc, c->ms.nslot) A(c->ms.srec, c->ms.nslot) A(c->ms.sent, (size_t)c->ms.nslot * pw) A(c->x_b, 3 * N)
+    const size_t nv = 3 * N * (c->precision == WFX_FP64 ? sizeof(double) : sizeof(float));
+    arena.want_bytes(&c->v_b, nv);
+    arena.want_bytes(&c->pa_b, nv);
+    arena.want_bytes(&c->ud_b, nv);
+    c->ms.pw = pw;
   }
   // partial minima of the volume pass (one per element cluster) and of the
   // per-step kernels at block size >= 64
   c->cfl_cap_min = (int)std::max<size_t>((E + 63) / 64 + 1, (size_t)c->ms.ncl + 1);
   A(c->cfl_part, c->cfl_cap_min + std::max<size_t>((N + 63) / 64, (size_t)c->ms.ncl) + 1)
-  if (e == hipSuccess) e = (c->precision == WFX_FP64) ? alloc_elem(c, c->e64) : alloc_elem(c, c->e32);
+  if (c->precision == WFX_FP64) want_elem(c, c->e64, arena);
+  else want_elem(c, c->e32, arena);
   A(c->x_start, 3 * N)
   if (c->precision == WFX_FP32_MIXED) {
     A(c->v32, 3 * N) A(c->pa32, 3 * N) A(c->ud32, 3 * N) A(c->fi32, 3 * N)
@@ -279,6 +297,7 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     A(c->x_lo, 3 * N)
   }
 #undef A
+  const hipError_t e = arena.take(c);
   if (e != hipSuccess) {
     set_error(std::string("device allocation: ") + hipGetErrorString(e));
     free_all(c);
@@ -310,13 +329,15 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     WFX_CHECK_HIP(hipMemcpy(c->ms.nsl, plan.nsl.data(), plan.nsl.size() * sizeof(int), hipMemcpyHostToDevice));
   if (c->ms.spos)
     WFX_CHECK_HIP(hipMemcpy(c->ms.spos, plan.spos.data(), plan.spos.size() * sizeof(int), hipMemcpyHostToDevice));
-  if (c->pair) {
-    WFX_CHECK_HIP(hipMemcpy(c->ms.srec, pt.rec.data(), pt.rec.size() * sizeof(int4), hipMemcpyHostToDevice));
-    WFX_CHECK_HIP(hipMemcpy(c->ms.sent, pt.ent.data(), pt.ent.size() * sizeof(int), hipMemcpyHostToDevice));
-  }
   WFX_CHECK_HIP(hipMemcpy(c->ms.cl_snode, plan.snode.data(), plan.snode.size() * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.cl_lslot, plan.lslot.data(), plan.lslot.size() * sizeof(uint16_t),
                           hipMemcpyHostToDevice));
+  if (c->pair) {
+    hipLaunchKernelGGL(k_pair_tables, dim3((unsigned)((c->ms.nslot + 255) / 256)), dim3(256), 0, nullptr, c->ms.nslot,
+                       pw, c->ms.cl_snode, c->ms.spos, c->ms.nsl_off, c->ms.nodel_offset, c->ms.nodel_count,
+                       c->ms.nodel, c->ms.srec, c->ms.sent);
+    WFX_CHECK_HIP(hipGetLastError());
+  }
   std::vector<int> pk(n * E);
   for (size_t k = 0; k < n * E; ++k) pk[k] = (nodel_s[k] << 3) | c->nodel_loc_h[k];
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_pk, pk.data(), n * E * sizeof(int), hipMemcpyHostToDevice));
@@ -363,49 +384,19 @@ static int finish_mesh(wfx_ctx *c) {
   return WFX_OK;
 }
 
-// host <-> device element-real conversion for the two precisions
-template <typename T>
-static int upload_elem_real(T *dst, const double *src, size_t count) {
-  if constexpr (std::is_same<T, double>::value) {
-    WFX_CHECK_HIP(hipMemcpy(dst, src, count * sizeof(double), hipMemcpyHostToDevice));
-  } else {
-    std::vector<float> tmp(src, src + count);
-    WFX_CHECK_HIP(hipMemcpy(dst, tmp.data(), count * sizeof(float), hipMemcpyHostToDevice));
-  }
-  return WFX_OK;
-}
-
-static int upload_real(wfx_ctx *c, void *dst, const double *src, size_t count, bool elem_type) {
-  if (!elem_type || c->precision == WFX_FP64) return upload_elem_real<double>((double *)dst, src, count);
-  return upload_elem_real<float>((float *)dst, src, count);
-}
-
-static int download_real(wfx_ctx *c, double *dst, const void *src, size_t count, bool elem_type) {
-  if (!elem_type || c->precision == WFX_FP64) {
-    WFX_CHECK_HIP(hipMemcpy(dst, src, count * sizeof(double), hipMemcpyDeviceToHost));
-  } else {
-    std::vector<float> tmp(count);
-    WFX_CHECK_HIP(hipMemcpy(tmp.data(), src, count * sizeof(float), hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < count; ++i) dst[i] = tmp[i];
-  }
-  return WFX_OK;
-}
-
-// Element rows [E][rows] between the original order (host) and the stored
-// order (device rows [rows][E]): transposed and permuted in one pass.
-static void elem_rows_to_device(const wfx_ctx *c, const double *h, int rows, double *dev_rows) {
-  const long E = c->E;
-  for (long o = 0; o < E; ++o) {
-    const long st = c->el_o2s[o];
-    for (int r = 0; r < rows; ++r) dev_rows[(long)r * E + st] = h[o * rows + r];
-  }
-}
-
 // one value per element, original order -> stored order, uploaded
 static int upload_elem_values(wfx_ctx *c, void *dst, const double *h, long count) {
-  std::vector<double> t((size_t)count);
-  elem_rows_to_device(c, h, 1, t.data());
-  return upload_real(c, dst, t.data(), t.size(), true);
+  WFX_CHECK_HIP(hipDeviceSynchronize());
+  return field_from_host(c, FieldMove{dst, count, 1, 0, c->precision == WFX_FP32_MIXED, c->ms.o2s}, h);
+}
+
+// n equal values (in the element type, or double), there when this returns
+static int fill_values(wfx_ctx *c, void *dst, size_t n, double v, bool elem_type) {
+  FillList f;
+  f.add_value(dst, n, v, elem_type && c->precision == WFX_FP32_MIXED);
+  WFX_CHECK_HIP(launch_fill(f, nullptr));
+  WFX_CHECK_HIP(hipStreamSynchronize(nullptr));
+  return WFX_OK;
 }
 
 // Description of one transferable field.  Host layout is [cnt][rows] (the
@@ -501,25 +492,26 @@ static hipStream_t as_stream(wfx_stream s) { return (hipStream_t)s; }
 // that is not finite or below 1e-200 (J_local = vol/vol0 not finite) or a
 // density that is not positive and finite sets the guard under which the
 // fused pass evaluates every pressure and viscosity term in full.
-static int scan_elements(wfx_ctx *c) {
-  std::vector<double> r(c->E), v0(c->E);
+// On the device, four words in the context's scalars (cleared first): read
+// back whole, the two arrays took as long as 40 steps of a small mesh.
+static unsigned long long *scan_words(wfx_ctx *c) { return (unsigned long long *)(c->scalars + kScan); }
+static void clear_scan(wfx_ctx *c, FillList &f) {
+  f.add(scan_words(c), 16);
+  f.add(scan_words(c) + 2, 8, 0xffffffffu);
+}
+static int scan_elements(wfx_ctx *c, hipStream_t st) {
   const bool f64 = c->precision == WFX_FP64;
-  int rc = download_real(c, r.data(), f64 ? (void *)c->e64.rho : (void *)c->e32.rho, r.size(), true);
-  if (!rc) rc = download_real(c, v0.data(), f64 ? (void *)c->e64.vol0 : (void *)c->e32.vol0, v0.size(), true);
-  if (rc) return rc;
-  c->rho_uniform = 0.0;
+  unsigned long long h[4];
+  WFX_CHECK_HIP(f64 ? launch_scan_elem<double>(c, scan_words(c), st) : launch_scan_elem<float>(c, scan_words(c), st));
+  WFX_CHECK_HIP(hipMemcpyAsync(h, scan_words(c), sizeof(h), hipMemcpyDeviceToHost, st));
+  WFX_CHECK_HIP(hipStreamSynchronize(st));
+  double first, rmin;
+  std::memcpy(&first, &h[3], sizeof(first));
+  std::memcpy(&rmin, &h[2], sizeof(rmin));
+  c->rho_uniform = h[0] == 0 && first > 0.0 ? first : 0.0;
   c->rho_avg_valid = false;
-  if (!r.empty() && r[0] > 0.0 &&
-      std::all_of(r.begin(), r.end(), [&](double v) { return v == r[0]; }))
-    c->rho_uniform = r[0];
-  bool bad = false;
-  double rmin = DBL_MAX;
-  for (long e = 0; e < c->E; ++e) {
-    bad = bad || !(r[e] > 0.0 && r[e] <= DBL_MAX) || !(std::fabs(v0[e]) >= 1e-200 && std::fabs(v0[e]) <= DBL_MAX);
-    rmin = std::min(rmin, r[e]);
-  }
-  c->elem_guard = bad ? 1 : 0;
-  c->rho_min = (c->E > 0 && !bad) ? rmin : 0.0;
+  c->elem_guard = h[1] ? 1 : 0;
+  c->rho_min = h[1] ? 0.0 : rmin;
   return WFX_OK;
 }
 
@@ -623,9 +615,7 @@ int wfx_get_sizes(wfx_ctx *c, int *N, int *E, int *n) {
 
 int wfx_set_density(wfx_ctx *c, double rho) {
   REQUIRE_MESH(c);
-  std::vector<double> h(c->E, rho);
-  void *dst = c->precision == WFX_FP64 ? (void *)c->e64.rho0 : (void *)c->e32.rho0;
-  return upload_real(c, dst, h.data(), h.size(), true);
+  return fill_values(c, c->precision == WFX_FP64 ? (void *)c->e64.rho0 : (void *)c->e32.rho0, c->E, rho, true);
 }
 
 // Elastic_ (Material.cuh:22-27) and the fields every law shares.  The
@@ -652,8 +642,7 @@ static int assign_material(wfx_ctx *c, const Material &m) {
   c->prm.mat = m;
   if (c->has_mesh) {
     c->sy0_h.assign(c->E, m.sy0);
-    void *dst = c->precision == WFX_FP64 ? (void *)c->e64.sy0 : (void *)c->e32.sy0;
-    return upload_elem_values(c, dst, c->sy0_h.data(), (long)c->sy0_h.size());
+    return fill_values(c, c->precision == WFX_FP64 ? (void *)c->e64.sy0 : (void *)c->e32.sy0, c->E, m.sy0, true);
   }
   return WFX_OK;
 }
@@ -727,8 +716,7 @@ int wfx_set_temperature(wfx_ctx *c, double T) {
   REQUIRE(std::isfinite(T), WFX_ERR_ARG, "temperature must be finite");
   c->prm.mat.temp = T;
   if (c->has_mesh) {  // setTemp: every node as well
-    std::vector<double> t0(c->N, T);
-    WFX_CHECK_HIP(hipMemcpy(c->nd.T, t0.data(), t0.size() * sizeof(double), hipMemcpyHostToDevice));
+    return fill_values(c, c->nd.T, c->N, T, false);
   }
   return WFX_OK;
 }
@@ -991,11 +979,9 @@ int wfx_set_elem_temperature(wfx_ctx *c, const double *T, int count) {
   }
   REQUIRE(count == c->E, WFX_ERR_ARG, "temperature needs one value per element");
   if (!c->temp_buf) WFX_CHECK_HIP(dalloc(c, &c->temp_buf, c->E));
-  {
-    std::vector<double> t((size_t)count);
-    elem_rows_to_device(c, T, 1, t.data());
-    WFX_CHECK_HIP(hipMemcpy(c->temp_buf, t.data(), sizeof(double) * (size_t)count, hipMemcpyHostToDevice));
-  }
+  WFX_CHECK_HIP(hipDeviceSynchronize());
+  int rc = field_from_host(c, FieldMove{c->temp_buf, count, 1, 0, 0, c->ms.o2s}, T);
+  if (rc) return rc;
   c->temp_e = c->temp_buf;
   return WFX_OK;
 }
@@ -1090,8 +1076,7 @@ int wfx_set_dt(wfx_ctx *c, double dt) {
   REQUIRE(dt > 0.0 && std::isfinite(dt), WFX_ERR_ARG, "dt must be positive");
   c->prm.dt = dt;
   // the device copy the first prediction of a per-step-CFL run reads
-  if (c->scalars) WFX_CHECK_HIP(hipMemcpy(c->scalars + kCflDt, &dt, sizeof(double), hipMemcpyHostToDevice));
-  return WFX_OK;
+  return c->scalars ? fill_values(c, c->scalars + kCflDt, 1, dt, false) : WFX_OK;
 }
 
 int wfx_set_cfl(wfx_ctx *c, double cfl_factor) {
@@ -1252,55 +1237,44 @@ int wfx_init(wfx_ctx *c, wfx_stream s) {
   const size_t N = c->N, E = c->E;
   // InitValues (Domain_d.C:393-416) plus zero state; every buffer the
   // reference leaves uninitialised starts at zero here.
-  for (double *p : {c->nd.v, c->nd.a, c->nd.u, c->nd.u_dt, c->nd.prev_a, c->nd.fi})
-    WFX_CHECK_HIP(hipMemsetAsync(p, 0, 3 * N * sizeof(double), st));
-  size_t es = c->precision == WFX_FP64 ? sizeof(double) : sizeof(float);
-  auto zero_e = [&](void *p, size_t rows) { return hipMemsetAsync(p, 0, rows * E * es, st); };
-  if (c->precision == WFX_FP64) {
-    auto &el = c->e64;
-    for (auto pr : {std::make_pair((void *)el.p, 1), {(void *)el.pl_strain, 1}, {(void *)el.tau, 6},
-                    {(void *)el.eps, 6}, {(void *)el.sigma, 6}, {(void *)el.strain_pl_incr, 6},
-                    {(void *)el.f_hg, 3 * c->n}})
-      WFX_CHECK_HIP(zero_e(pr.first, pr.second));
-    WFX_CHECK_HIP(hipMemcpyAsync(el.sigma_y, el.sy0, E * es, hipMemcpyDeviceToDevice, st));
-  } else {
-    auto &el = c->e32;
-    for (auto pr : {std::make_pair((void *)el.p, 1), {(void *)el.pl_strain, 1}, {(void *)el.tau, 6},
-                    {(void *)el.eps, 6}, {(void *)el.sigma, 6}, {(void *)el.strain_pl_incr, 6},
-                    {(void *)el.f_hg, 3 * c->n}})
-      WFX_CHECK_HIP(zero_e(pr.first, pr.second));
-    WFX_CHECK_HIP(hipMemcpyAsync(el.sigma_y, el.sy0, E * es, hipMemcpyDeviceToDevice, st));
+  const bool f64 = c->precision == WFX_FP64;
+  const size_t es = f64 ? sizeof(double) : sizeof(float);
+  FillList clear;
+  for (double *p : {c->nd.v, c->nd.a, c->nd.u, c->nd.u_dt, c->nd.prev_a, c->nd.fi}) clear.add(p, 3 * N * sizeof(double));
+#define EL(f) (f64 ? (void *)c->e64.f : (void *)c->e32.f)
+  for (void *p : {EL(p), EL(pl_strain)}) clear.add(p, E * es);
+  for (void *p : {EL(tau), EL(eps), EL(sigma), EL(strain_pl_incr)}) clear.add(p, 6 * E * es);
+  clear.add(EL(f_hg), 3 * (size_t)c->n * E * es);
+  clear.add(c->status, 16 * sizeof(unsigned int));
+  clear.add(EL(dte_flat), N * es);  // the temperature rates thermal expansion reads
+#undef EL
+  if (c->contact.on) {  // contact state starts clear
+    auto &ct = c->contact;
+    clear.add(ct.contforce, 3 * N * sizeof(double));
+    clear.add(ct.ut_prev, 3 * N * sizeof(double));
+    clear.add(ct.cfn, N * sizeof(double));
+    clear.add(ct.mesh_in_contact, N * sizeof(int), 0xffffffffu);
   }
-  for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, false, st));
+  clear_scan(c, clear);
+  // before the counters are cleared: inverted elements of the initial mesh
+  // are counted by the first step
   LAUNCH(BY_PRECISION(c, launch_elem_jacobians, c, st));
-  LAUNCH(BY_PRECISION(c, launch_elem_vol, c, st));
-  void *vol = c->precision == WFX_FP64 ? (void *)c->e64.vol : (void *)c->e32.vol;
-  void *vol0 = c->precision == WFX_FP64 ? (void *)c->e64.vol0 : (void *)c->e32.vol0;
-  WFX_CHECK_HIP(hipMemcpyAsync(vol0, vol, E * es, hipMemcpyDeviceToDevice, st));
-  LAUNCH(BY_PRECISION(c, launch_elem_density, c, st));
+  LAUNCH(launch_fill(clear, st));
+  for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, false, st));
+  LAUNCH(BY_PRECISION(c, launch_init_elem, c, st));
   LAUNCH(BY_PRECISION(c, launch_nodal_vol, c, st));
   LAUNCH(BY_PRECISION(c, launch_nodal_mass, c, st));
-  WFX_CHECK_HIP(hipMemsetAsync(c->status, 0, 16 * sizeof(unsigned int), st));
   c->status_seen[0] = c->status_seen[1] = 0;
-  {  // the temperature rates thermal expansion reads start at zero
-    void *dte = c->precision == WFX_FP64 ? (void *)c->e64.dte_flat : (void *)c->e32.dte_flat;
-    if (dte) WFX_CHECK_HIP(hipMemsetAsync(dte, 0, N * (c->precision == WFX_FP64 ? sizeof(double) : sizeof(float)), st));
-  }
   if (c->contact.on) {
-    // contact state starts clear; calcMinEdgeLength before the solve
-    // (main.C:862) gives the element heights
-    auto &ct = c->contact;
-    WFX_CHECK_HIP(hipMemsetAsync(ct.contforce, 0, 3 * N * sizeof(double), st));
-    WFX_CHECK_HIP(hipMemsetAsync(ct.ut_prev, 0, 3 * N * sizeof(double), st));
-    WFX_CHECK_HIP(hipMemsetAsync(ct.cfn, 0, N * sizeof(double), st));
-    WFX_CHECK_HIP(hipMemsetAsync(ct.mesh_in_contact, 0xff, N * sizeof(int), st));
+    // calcMinEdgeLength before the solve (main.C:862) gives the element heights
     LAUNCH(contact_elem_length(c, st));
     LAUNCH(contact_face_areas(c, st));
-    ct.step_count = 0;
+    c->contact.step_count = 0;
   }
-  WFX_CHECK_HIP(hipStreamSynchronize(st));
+  int rc = scan_elements(c, st);  // synchronises
+  if (rc) return rc;
   c->initialized = true;
-  return scan_elements(c);
+  return WFX_OK;
 }
 
 // ---- per-step API -----------------------------------------------------------
@@ -2003,7 +1977,12 @@ int wfx_set_field(wfx_ctx *c, const char *name, const void *host, long count) {
   const double *h = (const double *)host;
   if (!std::strcmp(name, "fe")) c->has_fe = std::any_of(h, h + count, [](double v) { return v != 0.0; });
   int rc = field_from_host(c, field_move(c, f), h);
-  if (rc == WFX_OK && (!std::strcmp(name, "rho") || !std::strcmp(name, "vol0"))) rc = scan_elements(c);
+  if (rc == WFX_OK && (!std::strcmp(name, "rho") || !std::strcmp(name, "vol0"))) {
+    FillList f;
+    clear_scan(c, f);
+    WFX_CHECK_HIP(launch_fill(f, nullptr));
+    rc = scan_elements(c, nullptr);
+  }
   return rc;
 }
 

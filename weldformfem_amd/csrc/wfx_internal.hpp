@@ -42,6 +42,8 @@ enum Model { BILINEAR = 0, HOLLOMON = 1, JOHNSON_COOK = 2, GMT = 3 };
 // scalars: minimum edge length, maximum speed, sound speed sqrt(K / rho[0])
 // and dt of the last step
 constexpr int kCflMinl = 16, kCflVmax = 17, kCflCs = 18, kCflDt = 20;
+// and of the host's scan of densities and initial volumes (four words; 16-byte aligned)
+constexpr int kScan = 24;
 
 struct Material {
   int model = BILINEAR;

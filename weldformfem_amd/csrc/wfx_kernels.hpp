@@ -407,6 +407,46 @@ __global__ __launch_bounds__(kBlock) void k_elem_density(int E, const T *__restr
   rho[e] = rho0[e] * vol0[e] / vol[e];
 }
 
+// wfx_init: CalcElemVol, the initial volumes, calcElemDensity and the
+// initial yield stresses in one pass
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_init_elem(int E, const T *__restrict__ detJ, T w,
+                                                      const T *__restrict__ rho0, const T *__restrict__ sy0,
+                                                      T *__restrict__ vol, T *__restrict__ vol0,
+                                                      T *__restrict__ rho, T *__restrict__ sigma_y) {
+  const int e = gtid();
+  if (e >= E) return;
+  T v = T(0);
+  v += detJ[e] * w * T(1);
+  vol[e] = vol0[e] = v;
+  rho[e] = rho0[e] * v / v;
+  sigma_y[e] = sy0[e];
+}
+
+// What the host has to know of the densities and initial volumes: scan[0]
+// whether a density differs from the first one, scan[1] whether a density is
+// not positive and finite or an initial volume not finite or (nearly) zero,
+// the smallest density as ordered bits (positive doubles; scan[1] 0) and the
+// first one.  The first three cleared to {0, 0, all ones} by the caller.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_scan_elem(int E, const T *__restrict__ rho, const T *__restrict__ vol0,
+                                                      unsigned long long *__restrict__ scan) {
+  const int e = gtid();
+  const double first = (double)rho[0];
+  double r = first;
+  bool bad = false;
+  if (e < E) {
+    r = (double)rho[e];
+    const double v = fabs((double)vol0[e]);
+    bad = !(r > 0.0 && r <= DBL_MAX) || !(v >= 1e-200 && v <= DBL_MAX);
+  }
+  if (__any(!(r == first)) && (threadIdx.x & 63) == 0) atomicOr(scan, 1ull);
+  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(scan + 1, 1ull);
+  if (e == 0) scan[3] = (unsigned long long)__double_as_longlong(first);
+  const double m = block_extreme<kBlock, true>(r);
+  if (threadIdx.x == 0) atomicMin(scan + 2, (unsigned long long)__double_as_longlong(m));
+}
+
 // Walk of node i's CSR entries [o, o + c) in batches of kCsrBatch, over the
 // packed entries (element << 3) | local node: the first eight come from the
 // padded table pad[j * N + i] (unit stride across a wavefront, one or two
@@ -1264,6 +1304,9 @@ template <typename T> hipError_t launch_hourglass(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_assembly(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_energies(wfx_ctx *c, double *dev_out2, double *partial, hipStream_t s);
 
+template <typename T> hipError_t launch_init_elem(wfx_ctx *c, hipStream_t s);
+template <typename T> hipError_t launch_scan_elem(wfx_ctx *c, unsigned long long *scan, hipStream_t s);
+
 #define WFX_DEFINE_LAUNCHERS(T)                                                                    \
   template <> hipError_t launch_elem_jacobians<T>(wfx_ctx * c, hipStream_t s) {                    \
     auto &el = elem<T>(c);                                                                         \
@@ -1280,6 +1323,20 @@ template <typename T> hipError_t launch_energies(wfx_ctx *c, double *dev_out2, d
     T w = (c->n == 4) ? T(1.0 / 6.0) : T(8.0);                                                     \
     hipLaunchKernelGGL((k_elem_vol<T>), dim3(nblocks(c->E)), dim3(kBlock), 0, s, c->E, el.detJ,    \
                        el.vol, w);                                                                 \
+    return hipGetLastError();                                                                      \
+  }                                                                                                \
+  template <> hipError_t launch_init_elem<T>(wfx_ctx * c, hipStream_t s) {                         \
+    auto &el = elem<T>(c);                                                                         \
+    T w = (c->n == 4) ? T(1.0 / 6.0) : T(8.0);                                                     \
+    hipLaunchKernelGGL((k_init_elem<T>), dim3(nblocks(c->E)), dim3(kBlock), 0, s, c->E, el.detJ,   \
+                       w, el.rho0, el.sy0, el.vol, el.vol0, el.rho, el.sigma_y);                   \
+    return hipGetLastError();                                                                      \
+  }                                                                                                \
+  template <> hipError_t launch_scan_elem<T>(wfx_ctx * c, unsigned long long *scan,                \
+                                             hipStream_t s) {                                      \
+    auto &el = elem<T>(c);                                                                         \
+    hipLaunchKernelGGL((k_scan_elem<T>), dim3(nblocks(c->E)), dim3(kBlock), 0, s, c->E, el.rho,    \
+                       el.vol0, scan);                                                             \
     return hipGetLastError();                                                                      \
   }                                                                                                \
   template <> hipError_t launch_elem_density<T>(wfx_ctx * c, hipStream_t s) {                      \

@@ -10,6 +10,8 @@ namespace wfx {
 template <typename T> hipError_t launch_elem_jacobians(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_elem_vol(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_elem_density(wfx_ctx *c, hipStream_t s);
+template <typename T> hipError_t launch_init_elem(wfx_ctx *c, hipStream_t s);
+template <typename T> hipError_t launch_scan_elem(wfx_ctx *c, unsigned long long *scan, hipStream_t s);
 template <typename T> hipError_t launch_nodal_vol(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_nodal_mass(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_strain_rates(wfx_ctx *c, hipStream_t s);
@@ -25,6 +27,8 @@ template <typename T> hipError_t launch_energies(wfx_ctx *c, double *dev_out2, d
   template <> hipError_t launch_elem_jacobians<T>(wfx_ctx *, hipStream_t);                       \
   template <> hipError_t launch_elem_vol<T>(wfx_ctx *, hipStream_t);                             \
   template <> hipError_t launch_elem_density<T>(wfx_ctx *, hipStream_t);                         \
+  template <> hipError_t launch_init_elem<T>(wfx_ctx *, hipStream_t);                            \
+  template <> hipError_t launch_scan_elem<T>(wfx_ctx *, unsigned long long *, hipStream_t);      \
   template <> hipError_t launch_nodal_vol<T>(wfx_ctx *, hipStream_t);                            \
   template <> hipError_t launch_nodal_mass<T>(wfx_ctx *, hipStream_t);                           \
   template <> hipError_t launch_strain_rates<T>(wfx_ctx *, hipStream_t);                         \
@@ -115,6 +119,33 @@ hipError_t contact_rigid_update(wfx_ctx *c, double dt, hipStream_t s);
 // and around the adjoint's recomputation)
 std::vector<std::pair<void *, size_t>> fused_state_buffers(wfx_ctx *c);
 void adjoint_free(wfx_ctx *c);
+
+// Fills device buffers with a 4-byte word each (8-byte values for a double
+// fill) in one launch.
+struct FillList {
+  static constexpr int kMost = 24;
+  int count = 0;
+  struct {
+    void *p;
+    size_t words;          // 4-byte words
+    unsigned lo, hi;       // even and odd words
+  } buf[kMost];
+  void add(void *p, size_t bytes, unsigned word = 0) { add2(p, bytes, word, word); }
+  void add2(void *p, size_t bytes, unsigned lo, unsigned hi) {
+    if (p && bytes) buf[count++] = {p, bytes / 4, lo, hi};
+  }
+  void add_value(void *p, size_t n, double v, bool f32) {
+    union { double d; float f; unsigned u[2]; } b;
+    if (f32) {
+      b.f = (float)v;
+      add(p, n * 4, b.u[0]);
+    } else {
+      b.d = v;
+      add2(p, n * 8, b.u[0], b.u[1]);
+    }
+  }
+};
+hipError_t launch_fill(const FillList &f, hipStream_t s);
 
 // A real field's transfer: host [cnt][rows] double, device [rows][cnt]
 // (spin: 3 device rows for host columns 3..5 of 6, the others zero), float
