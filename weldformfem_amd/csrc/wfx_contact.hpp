@@ -103,6 +103,7 @@ __global__ __launch_bounds__(kBlock) void k_contact(
   const int i = ext_nodes[k];
   const double dt = cp.dtp ? *cp.dtp : cp.dt;
   mesh_in_contact[i] = -1;
+  const int o = off[i], c = cnt[i];
   const R3 xi = r3_soa(x, N, i);
   const R3 vi = r3((double)v[i], (double)v[N + i], (double)v[2L * N + i]);
   for (int j = 0; j < cp.rt; ++j) {
@@ -118,8 +119,19 @@ __global__ __launch_bounds__(kBlock) void k_contact(
     }
     if (!inside) continue;
     double nodlen = 0.0;
-    const int o = off[i], c = cnt[i];
-    for (int q = 0; q < c; ++q) nodlen += elem_length[nodel[o + q]];
+    // eight elements at a time, added in order: one by one each waited for two
+    // dependent loads (tetrahedral nodes have about 23)
+    for (int q = 0; q < c; q += 8) {
+      int el[8];
+      double h[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) el[k] = nodel[o + min(q + k, c - 1)];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) h[k] = elem_length[el[k]];
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (q + k < c) nodlen += h[k];
+    }
     nodlen /= c;
     const double m = mdiag[i];
     const double v_reln = dot(vi, nj);
@@ -163,26 +175,31 @@ __global__ __launch_bounds__(kBlock) void k_contact(
   }
 }
 
+// The rigid surfaces' arrays for their motion; rn 0: none
+struct RigidArgs {
+  int rn, rt;
+  double *rnode;
+  const double *rvel;
+  const int *rtri;
+  double *rnormal, *rpplane;
+};
 // rigid surfaces after the position update: node += v dt, then normals and
 // plane offsets (nfar = 2); one block
-__global__ __launch_bounds__(kBlock) void k_rigid_update(int rn, int rt, double *__restrict__ rnode,
-                                                         const double *__restrict__ rvel,
-                                                         const int *__restrict__ rtri,
-                                                         double *__restrict__ rnormal,
-                                                         double *__restrict__ rpplane, double dt,
-                                                         const double *__restrict__ dtp) {
-  if (dtp) dt = *dtp;
-  for (int k = threadIdx.x; k < 3 * rn; k += blockDim.x) rnode[k] = rnode[k] + rvel[k] * dt;
+__device__ __forceinline__ void rigid_move(const RigidArgs &r, double dt) {
+  for (int k = threadIdx.x; k < 3 * r.rn; k += blockDim.x) r.rnode[k] = r.rnode[k] + r.rvel[k] * dt;
   __syncthreads();
-  for (int e = threadIdx.x; e < rt; e += blockDim.x) {
-    const int *t = rtri + 3 * e;
-    const R3 w = cross(r3_aos(rnode, t[1]) - r3_aos(rnode, t[0]), r3_aos(rnode, t[2]) - r3_aos(rnode, t[0]));
+  for (int e = threadIdx.x; e < r.rt; e += blockDim.x) {
+    const int *t = r.rtri + 3 * e;
+    const R3 w = cross(r3_aos(r.rnode, t[1]) - r3_aos(r.rnode, t[0]), r3_aos(r.rnode, t[2]) - r3_aos(r.rnode, t[0]));
     const R3 nrm = w / len(w);
-    rnormal[3 * e] = nrm.x;
-    rnormal[3 * e + 1] = nrm.y;
-    rnormal[3 * e + 2] = nrm.z;
-    rpplane[e] = dot(r3_aos(rnode, t[2]), nrm);
+    r.rnormal[3 * e] = nrm.x;
+    r.rnormal[3 * e + 1] = nrm.y;
+    r.rnormal[3 * e + 2] = nrm.z;
+    r.rpplane[e] = dot(r3_aos(r.rnode, t[2]), nrm);
   }
+}
+__global__ __launch_bounds__(kBlock) void k_rigid_update(RigidArgs r, double dt, const double *__restrict__ dtp) {
+  rigid_move(r, dtp ? *dtp : dt);
 }
 
 }  // namespace

@@ -114,8 +114,16 @@ __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *_
                                                    const double *__restrict__ rho_avg,
                                                    const double *__restrict__ vsum0,
                                                    double *__restrict__ ratio,
-                                                   double *__restrict__ mdiag, double rho_u) {
-  int i = gtid();
+                                                   double *__restrict__ mdiag, double rho_u, CflReduce cr,
+                                                   const T *__restrict__ rho) {
+  // per-step CFL time step: one more block reduces it beside the nodes, which do
+  // not need it (a kernel of its own took 3 us and its launch)
+  const int nb = gridDim.x - (cr.cfl > 0.0 ? 1 : 0);
+  if ((int)blockIdx.x == nb) {
+    cfl_reduce<BS>(cr, rho, true);
+    return;
+  }
+  int i = xcd_block(nb) * BS + threadIdx.x;
   if (i >= N) return;
   const int c = ld_stream(&cnt[i]), o = c > kChunk ? off[i] : 0;
   // The table, count and V0_n are read once per step: non-temporal loads, so
@@ -214,9 +222,14 @@ __global__ __launch_bounds__(BS) void f2_nodal_lanes(int N, int nodxelem, const 
                                                      const double *__restrict__ rho_avg,
                                                      const double *__restrict__ vsum0,
                                                      double *__restrict__ ratio, double *__restrict__ mdiag,
-                                                     double rho_u) {
+                                                     double rho_u, CflReduce cr, const T *__restrict__ rho) {
   constexpr int L = kF2Lanes;
-  const long g = (long)xcd_block() * BS + threadIdx.x;
+  const int nb = gridDim.x - (cr.cfl > 0.0 ? 1 : 0);  // as in f2_nodal
+  if ((int)blockIdx.x == nb) {
+    cfl_reduce<BS>(cr, rho, true);
+    return;
+  }
+  const long g = (long)xcd_block(nb) * BS + threadIdx.x;
   const long n = g / L;
   const int q = (int)(g % L), i = (int)(n < N ? n : N - 1);  // every lane reaches the butterflies
   const int o = off[i], c = cnt[i];
@@ -854,12 +867,7 @@ struct PairArgs {
   const void *vol;       // T[E]
   const double *vsum0, *rho_avg;
   double *ratio, *mdiag; // written by each node's first slot
-  // per-step CFL time step (cfl > 0): the partial extremes, and where the
-  // first work-group leaves the result
-  double cfl, K;
-  const double *minl, *vmax;
-  int nmin, nmax, step;
-  double *scal, *dt_hist;
+  CflReduce cr;          // per-step CFL time step
 };
 
 // Where the element pass stores a slot's partial sum.  FP64 (but for the
@@ -991,29 +999,6 @@ struct PairSum {
   }
 };
 
-// The step's dt from the partial extremes (k_cfl_reduce's arithmetic): every
-// work-group reduces them for itself, since a kernel for it costs 3 us and its
-// launch while the few partials of a small mesh take less than one; the first
-// work-group stores the result for the later kernels.
-template <typename T>
-__device__ __forceinline__ double pair_cfl_dt(const PairArgs &pr, const T *rho) {
-  double m = kMinEdgeInit, v = 0.0;
-  for (int k = threadIdx.x; k < pr.nmin; k += kCluster) m = fmin(m, pr.minl[k]);
-  for (int k = threadIdx.x; k < pr.nmax; k += kCluster) v = fmax(v, pr.vmax[k]);
-  m = block_extreme<kCluster, true>(m);
-  v = block_extreme<kCluster, false>(v);
-  const double cs = sqrt(pr.K / (double)rho[0]);
-  const double dt = pr.cfl * m / (cs + v);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    pr.scal[kCflMinl] = m;
-    pr.scal[kCflVmax] = v;
-    pr.scal[kCflCs] = cs;
-    pr.scal[kCflDt] = dt;
-    if (pr.dt_hist) pr.dt_hist[pr.step] = dt;
-  }
-  return dt;
-}
-
 // F3: one work-group per element cluster.  The work-group first stages its
 // cluster's slots (the distinct nodes of its elements: positions,
 // velocities, ANP ratio, ids) in LDS with one load per slot and field; each
@@ -1113,7 +1098,10 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   if constexpr (PAIR) ps.ratio(pr, rec, mine, sr);
   double dt_step = fp.dt;
   if constexpr (PAIR) {
-    if (pr.cfl > 0.0) dt_step = pair_cfl_dt<T>(pr, rho);
+    // every work-group reduces the step's dt for itself, since a kernel for it
+    // takes 3 us and the few partials of a small mesh less than one; the first
+    // work-group stores it for the later kernels
+    if (pr.cr.cfl > 0.0) dt_step = cfl_reduce<kCluster>(pr.cr, rho, blockIdx.x == 0);
   } else {
     if (fp.dtp) dt_step = *fp.dtp;
   }
@@ -1642,10 +1630,20 @@ __global__ __launch_bounds__(BS) void f4_node(
     const double *__restrict__ bc_val, T *__restrict__ fi,
     T *__restrict__ v, T *__restrict__ prev_a, T *__restrict__ u_dt,
     double *__restrict__ x, double *__restrict__ u, unsigned int *__restrict__ status,
-    double *__restrict__ Tn) {
-  int i = gtid();
+    double *__restrict__ Tn, RigidArgs rg) {
   NodeParams q = np;
   if constexpr (CFL) set_step_length(q, *q.dtp);
+  // contact: one more block moves the rigid surfaces beside the nodes (a
+  // kernel of its own took 2 us and its launch)
+  int nb = gridDim.x;
+  if constexpr (CONTACT) {
+    nb -= rg.rn > 0 ? 1 : 0;
+    if ((int)blockIdx.x == nb) {
+      rigid_move(rg, q.dt);
+      return;
+    }
+  }
+  const int i = xcd_block(nb) * BS + threadIdx.x;
   double speed = 0.0;
   if (i < N) {
     // the node's slot range first: the partial sums wait for it, not for
@@ -1693,14 +1691,22 @@ __global__ __launch_bounds__(slot_cap(NN)) void f41_cluster(
     const T *__restrict__ part, const double *__restrict__ fe, const double *__restrict__ mdiag,
     const double *__restrict__ bc_val, T *__restrict__ fi, const T *__restrict__ v, const T *__restrict__ prev_a,
     const T *__restrict__ u_dt, const double *__restrict__ x, unsigned int *__restrict__ status,
-    double *__restrict__ Tn, T *__restrict__ vol, double *__restrict__ minl_part) {
+    double *__restrict__ Tn, T *__restrict__ vol, double *__restrict__ minl_part, RigidArgs rg) {
   constexpr int cap = slot_cap(NN);
   __shared__ double lx[3 * cap];
-  const int c = xcd_block(), t = threadIdx.x;
-  const int4 cd = ca.desc[c];
-  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
   NodeParams q = np;
   if constexpr (CFL) set_step_length(q, *q.dtp);
+  int nb = gridDim.x;
+  if constexpr (CONTACT) {  // one more block, as in f4_node
+    nb -= 1;
+    if ((int)blockIdx.x == nb) {
+      rigid_move(rg, q.dt);
+      return;
+    }
+  }
+  const int c = xcd_block(nb), t = threadIdx.x;
+  const int4 cd = ca.desc[c];
+  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
   // as in the element pass every load is issued unconditionally: threads past
   // the cluster's slots or elements repeat its last one and store nothing
   const int4 rec = pr.rec[s0 + min(t, M - 1)];
@@ -1831,10 +1837,13 @@ hipError_t launch_contact(wfx_ctx *c, const T *v, bool device_dt, hipStream_t s)
                      ct.node_area, ct.contforce, ct.ut_prev, ct.mesh_in_contact, ct.cfn);
   return hipGetLastError();
 }
+inline RigidArgs rigid_args(const wfx_ctx *c, bool move) {
+  const auto &ct = c->contact;
+  return RigidArgs{move ? ct.rn : 0, ct.rt, ct.rnode, ct.rvel, ct.rtri, ct.rnormal, ct.rpplane};
+}
 hipError_t launch_rigid_update(wfx_ctx *c, bool device_dt, hipStream_t s) {
-  auto &ct = c->contact;
-  hipLaunchKernelGGL(k_rigid_update, dim3(1), dim3(kBlock), 0, s, ct.rn, ct.rt, ct.rnode, ct.rvel, ct.rtri,
-                     ct.rnormal, ct.rpplane, c->prm.dt, device_dt ? c->scalars + kCflDt : nullptr);
+  hipLaunchKernelGGL(k_rigid_update, dim3(1), dim3(kBlock), 0, s, rigid_args(c, true), c->prm.dt,
+                     device_dt ? c->scalars + kCflDt : nullptr);
   return hipGetLastError();
 }
 
@@ -1892,12 +1901,9 @@ inline NodeParams node_params(wfx_ctx *c, int predict) {
 }
 
 // dt of step `step` of a run from the partial extremes (per-step CFL time step)
-template <typename T>
-hipError_t launch_cfl_reduce(wfx_ctx *c, int nmin, int step, hipStream_t s) {
-  hipLaunchKernelGGL((k_cfl_reduce<T>), dim3(1), dim3(kCflReduceBlock), 0, s, c->cfl_part, nmin,
-                     c->cfl_part + c->cfl_cap_min, c->cfl_nvmax, elem<T>(c).rho, c->prm.mat.K, c->prm.cfl,
-                     c->scalars, (step >= 0 && step < c->dt_cap) ? c->dt_hist : nullptr, step);
-  return hipGetLastError();
+inline CflReduce cfl_args(const wfx_ctx *c, double cfl, int nmin, int step) {
+  return CflReduce{cfl,  c->prm.mat.K, c->cfl_part,   c->cfl_part + c->cfl_cap_min, nmin, c->cfl_nvmax,
+                   step, c->scalars,   (step >= 0 && step < c->dt_cap) ? c->dt_hist : nullptr};
 }
 
 template <typename T>
@@ -1988,15 +1994,7 @@ PairArgs pair_args(wfx_ctx *c, int step) {
   pr.sbc = c->ms.sbc;
   pr.ratio = c->nd.anp_ratio;
   pr.mdiag = c->nd.mdiag;
-  pr.cfl = c->prm.cfl;
-  pr.K = c->prm.mat.K;
-  pr.minl = c->cfl_part;
-  pr.vmax = c->cfl_part + c->cfl_cap_min;
-  pr.nmin = c->ms.ncl;
-  pr.nmax = c->cfl_nvmax;
-  pr.step = step;
-  pr.scal = c->scalars;
-  pr.dt_hist = (step >= 0 && step < c->dt_cap) ? c->dt_hist : nullptr;
+  pr.cr = cfl_args(c, c->prm.cfl, c->ms.ncl, step);
   return pr;
 }
 
@@ -2053,14 +2051,15 @@ hipError_t launch_pair_node(wfx_ctx *c, hipStream_t s) {
   np.dtp = cfl ? c->scalars + kCflDt : nullptr;
   np.vmax_part = c->cfl_part + c->cfl_cap_min;
   auto kern = c->n == 8 ? f41_pick<T, 8>(cfl, ct, th) : f41_pick<T, 4>(cfl, ct, th);
-  hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(slot_cap(c->n)), 0, s, c->N, np, cluster_args(c), pair_args<T>(c, -1),
+  hipLaunchKernelGGL(kern, dim3(c->ms.ncl + (ct ? 1 : 0)), dim3(slot_cap(c->n)), 0, s, c->N, np, cluster_args(c), pair_args<T>(c, -1),
                      NodeSet{c->x_b, c->v_b, c->pa_b, c->ud_b}, c->contact.contforce, el.part, c->nd.fe,
-                     c->nd.mdiag, c->bc_tab, fiN, vN, paN, udN, c->nd.x, c->status, c->nd.T, el.vol, c->cfl_part);
+                     c->nd.mdiag, c->bc_tab, fiN, vN, paN, udN, c->nd.x, c->status, c->nd.T, el.vol, c->cfl_part,
+                     rigid_args(c, ct));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (cfl) c->cfl_nvmax = c->ms.ncl;
   pair_swap<T>(c);
-  return ct ? launch_rigid_update(c, cfl, s) : hipSuccess;
+  return hipSuccess;
 }
 
 template <typename T, int BS, bool CFL, bool CT>
@@ -2083,26 +2082,24 @@ hipError_t launch_fused_phase_bs(wfx_ctx *c, int phase, int predict, int step, h
   if (phase == 1) {
     hipError_t e = launch_volumes<T>(c, cfl, s);
     if (e != hipSuccess) return e;
-    if (cfl) {
-      e = launch_cfl_reduce<T>(c, c->ms.ncl, step, s);
-      // calcMinEdgeLength also refreshes the element heights contact uses
-      if (e == hipSuccess && c->contact.on) e = launch_elem_length(c, s);
-      return e;
-    }
+    // calcMinEdgeLength also refreshes the element heights contact uses
+    if (cfl && c->contact.on) return launch_elem_length(c, s);
   } else if (phase == 2) {
     if (!c->rho_avg_valid) {  // outside a run, after the densities changed
       hipError_t e = launch_run_sums<T>(c, false, s);
       if (e != hipSuccess) return e;
     }
+    const CflReduce cr = cfl_args(c, cfl ? c->prm.cfl : 0.0, c->ms.ncl, step);
+    const int more = cfl ? 1 : 0;
     if (c->f2_lanes) {
       const int gL = (int)(((long)N * kF2Lanes + BS - 1) / BS);
-      hipLaunchKernelGGL((f2_nodal_lanes<T, BS>), dim3(gL), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
+      hipLaunchKernelGGL((f2_nodal_lanes<T, BS>), dim3(gL + more), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
                          c->ms.nodel_count, c->ms.nodel_pk, el.vol, c->nd.rho_avg, c->nd.voln0_sum, c->nd.anp_ratio,
-                         c->nd.mdiag, c->rho_uniform);
+                         c->nd.mdiag, c->rho_uniform, cr, el.rho);
     } else {
-      hipLaunchKernelGGL((f2_nodal<T, BS>), dim3(gN), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
+      hipLaunchKernelGGL((f2_nodal<T, BS>), dim3(gN + more), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
                          c->ms.nodel_count, c->ms.nodel_pk, c->ms.nodel_pad, el.vol, c->nd.rho_avg, c->nd.voln0_sum,
-                         c->nd.anp_ratio, c->nd.mdiag, c->rho_uniform);
+                         c->nd.anp_ratio, c->nd.mdiag, c->rho_uniform, cr, el.rho);
     }
   } else if (phase == 3) {
     hipError_t e = launch_element_pass<T, false>(c, dtp, PairArgs{}, s);
@@ -2117,11 +2114,10 @@ hipError_t launch_fused_phase_bs(wfx_ctx *c, int phase, int predict, int step, h
     const bool ct = c->contact.on, th = c->thermal.on;
     auto kern = cfl ? (ct ? f4_pick<T, BS, true, true>(th) : f4_pick<T, BS, true, false>(th))
                     : (ct ? f4_pick<T, BS, false, true>(th) : f4_pick<T, BS, false, false>(th));
-    hipLaunchKernelGGL(kern, dim3(gN), dim3(BS), 0, s, N, np, ca.nm, c->contact.contforce, c->ms.nsl_off, c->ms.nsl,
+    const RigidArgs rg = rigid_args(c, ct && step >= 0);  // the rigid surfaces move after the position update
+    hipLaunchKernelGGL(kern, dim3(gN + (rg.rn > 0 ? 1 : 0)), dim3(BS), 0, s, N, np, ca.nm, c->contact.contforce, c->ms.nsl_off, c->ms.nsl,
                        el.part, c->ms.nslot, c->nd.fe, c->nd.mdiag, c->bc_word, c->bc_tab, fiN, vN,
-                       paN, udN, c->nd.x, c->nd.u, c->status, c->nd.T);
-    // the rigid surfaces move after the position update
-    if (c->contact.on && step >= 0) return launch_rigid_update(c, cfl, s);
+                       paN, udN, c->nd.x, c->nd.u, c->status, c->nd.T, rg);
   } else if (phase == 5) {
     const bool av = st.artifvisc0 != 0.0 || st.artifvisc1 != 0.0 || press_params(c).guard;
     hipLaunchKernelGGL((f_sigma<T>), dim3(nblocks(E)), dim3(kBlock), 0, s, E, el.p, el.tau, el.avq, el.vol,
@@ -2172,7 +2168,9 @@ hipError_t launch_cfl_step(wfx_ctx *c, int step, hipStream_t s) {
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_cfl_min_edge, dim3(nblocks(c->E)), dim3(kBlock), 0, s, c->E, c->N, c->ms.elnod, c->nd.x,
                      c->cfl_part);
-  return launch_cfl_reduce<T>(c, nblocks(c->E), -1, s);
+  hipLaunchKernelGGL((k_cfl_reduce<T>), dim3(1), dim3(kCflReduceBlock), 0, s,
+                     cfl_args(c, c->prm.cfl, nblocks(c->E), -1), elem<T>(c).rho);
+  return hipGetLastError();
 }
 
 // ThermalCalcs of one per-step API step: element rates from the stored

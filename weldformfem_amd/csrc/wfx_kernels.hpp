@@ -26,11 +26,12 @@ namespace {
 // b % 8), and each XCD has its own L2.  Remap so that every XCD walks one
 // contiguous range of logical blocks: neighbouring elements share nodes, so
 // their gathers then hit the same L2.
-__device__ __forceinline__ int xcd_block() {
-  const int nb = gridDim.x, b = blockIdx.x;
+__device__ __forceinline__ int xcd_block(int nb) {  // nb logical blocks, blockIdx.x one of them
+  const int b = blockIdx.x;
   const int per = nb >> 3, rem = nb & 7, xcd = b & 7, idx = b >> 3;
   return xcd * per + (xcd < rem ? xcd : rem) + idx;
 }
+__device__ __forceinline__ int xcd_block() { return xcd_block(gridDim.x); }
 __device__ __forceinline__ int gtid() { return xcd_block() * blockDim.x + threadIdx.x; }
 
 // ---------------------------------------------------------------------------
@@ -110,27 +111,46 @@ __global__ __launch_bounds__(kBlock) void k_cfl_max_speed(int N, const T *__rest
   if (threadIdx.x == 0) part[blockIdx.x] = sp;
 }
 
-// dt of a step from the partial extremes (one block)
+// dt of a step from the partial extremes, by one block; store: whether this
+// block leaves it (and the extremes) in the scalars.  Eight loads in flight a
+// thread: the partials of a large mesh are tens of thousands.
+struct CflReduce {
+  double cfl, K;  // cfl 0: no reduction
+  const double *minl, *vmax;
+  int nmin, nmax, step;
+  double *scal, *dt_hist;
+};
+template <int BS, typename T>
+__device__ __forceinline__ double cfl_reduce(const CflReduce &r, const T *rho, bool store) {
+  double m = kMinEdgeInit, v = 0.0;
+  auto walk = [&](const double *p, int n, auto take) {
+    for (int k = threadIdx.x; k < n; k += 8 * BS) {
+      double q[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = p[min(k + j * BS, n - 1)];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) take(q[j]);
+    }
+  };
+  walk(r.minl, r.nmin, [&](double q) { m = fmin(m, q); });
+  walk(r.vmax, r.nmax, [&](double q) { v = fmax(v, q); });
+  m = block_extreme<BS, true>(m);
+  v = block_extreme<BS, false>(v);
+  const double cs = sqrt(r.K / (double)rho[0]);
+  const double dt = r.cfl * m / (cs + v);
+  if (store && threadIdx.x == 0) {
+    r.scal[kCflMinl] = m;
+    r.scal[kCflVmax] = v;
+    r.scal[kCflCs] = cs;
+    r.scal[kCflDt] = dt;
+    if (r.dt_hist) r.dt_hist[r.step] = dt;
+  }
+  return dt;
+}
 constexpr int kCflReduceBlock = 1024;
 template <typename T>
-__global__ __launch_bounds__(kCflReduceBlock) void k_cfl_reduce(
-    const double *__restrict__ minl_part, int nmin, const double *__restrict__ vmax_part, int nmax,
-    const T *__restrict__ rho, double K, double cfl, double *__restrict__ s, double *__restrict__ dt_hist,
-    int step) {
-  double m = kMinEdgeInit, v = 0.0;
-  for (int k = threadIdx.x; k < nmin; k += kCflReduceBlock) m = fmin(m, minl_part[k]);
-  for (int k = threadIdx.x; k < nmax; k += kCflReduceBlock) v = fmax(v, vmax_part[k]);
-  m = block_extreme<kCflReduceBlock, true>(m);
-  v = block_extreme<kCflReduceBlock, false>(v);
-  if (threadIdx.x == 0) {
-    const double cs = sqrt(K / (double)rho[0]);
-    const double dt = cfl * m / (cs + v);
-    s[kCflMinl] = m;
-    s[kCflVmax] = v;
-    s[kCflCs] = cs;
-    s[kCflDt] = dt;
-    if (dt_hist) dt_hist[step] = dt;
-  }
+__global__ __launch_bounds__(kCflReduceBlock) void k_cfl_reduce(CflReduce r, const T *__restrict__ rho) {
+  cfl_reduce<kCflReduceBlock>(r, rho, true);
 }
 
 // ---------------------------------------------------------------------------
