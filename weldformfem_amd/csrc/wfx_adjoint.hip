@@ -20,13 +20,19 @@
 // steps (checkpoints).  Backward: for each segment, last first, the state is
 // restored from its checkpoint, the K steps are recomputed while their
 // inputs (x, v', tau, ep) and node-pass values (fi, m, r) are recorded, and
-// the segment is then reversed step by step with five kernels:
-//   a_node1   node-pass reverse: prediction, correction, BC masks, accel,
-//             reaction cotangent -> fi and m cotangents
-//   a_elem1   element reverse (recomputes the element forward first)
-//   a_node2   gathers the r cotangents; volume cotangent per node
-//   a_elem2   element volume cotangent -> positions
-//   a_node3   gathers the element position/velocity cotangents
+// the segment is then reversed step by step with two kernels, each one
+// work-group per element cluster over the nodes its elements touch (slots), as
+// the paired forward passes:
+//   a_element  node: the later step's position and velocity cotangents gathered
+//              from the clusters' sums, then the node-pass reverse
+//              (prediction, correction, BC masks, accel, reaction cotangent ->
+//              fi and m cotangents); element reverse (recomputes the element
+//              forward first); its position, velocity and ratio cotangents
+//              summed per slot
+//   a_volume   node: the ratio cotangents gathered, volume cotangent; element
+//              volume cotangent -> positions, summed per slot
+// A node of several clusters is worked on by each of them alike and stored by
+// its first slot's, to a second set of buffers since the others still read.
 // All adjoint arithmetic is FP64; the forward runs in the context's precision.
 #include <algorithm>
 #include <cmath>
@@ -35,6 +41,7 @@
 
 #include "../../include/wfx.h"
 #include "wfx_adjoint.hpp"
+#include "wfx_fused.hpp"
 #include "wfx_internal.hpp"
 #include "wfx_launch.hpp"
 
@@ -46,9 +53,10 @@ struct Adjoint {
   size_t ck_stride = 0, slot_stride = 0;
   std::vector<void *> mem;
   double *ck = nullptr, *slot = nullptr, *hist = nullptr, *hbar = nullptr;
-  double *xb = nullptr, *vb = nullptr, *udb = nullptr, *pab = nullptr;
-  double *taub = nullptr, *epb = nullptr, *fib = nullptr, *mb = nullptr, *w = nullptr;
-  double *contrib = nullptr, *volb = nullptr, *grad = nullptr;
+  double *bars[2] = {nullptr, nullptr};  // the state cotangents [x v ud pa][3][N], two sets
+  double *taub = nullptr, *epb = nullptr, *mb = nullptr;
+  double *p1[2] = {nullptr, nullptr}, *p2 = nullptr;  // per-slot sums (SlotSums)
+  double *volb = nullptr, *grad = nullptr;
   double *sy0d = nullptr, *Hd = nullptr, *rhod = nullptr, *rho_avg = nullptr, *sums = nullptr;
   int *rgroup = nullptr;
   std::vector<std::pair<void *, size_t>> final_bufs;
@@ -158,50 +166,76 @@ struct NodeAdj {
   int has_fe, ng;
 };
 
-// node-pass reverse of step k; Z-bar of boundary k+1 in, of boundary k out
-// (partial: the element gathers are added by a_node3).  dtb (per-step CFL
-// time step, else null): node i's share of the step length's cotangent, from
-// vv = v' + gamma dt ac, ud = ud + beta dt^2 ac and the prediction
-// ud' = dt (vv + (0.5 - beta) dt ac), v'' = vv + (1 - gamma) dt ac, with ac the
-// corrected acceleration (1/(1-alpha)) (a - alpha pa)
-__global__ void a_node1(int N, int E, NodeAdj P, const double *rec, const double *fe, const int *bc_word,
-                        const int *rgroup, const double *hbar_k, double *xb, double *vb,
-                        double *udb, double *pab, double *fib, double *mb, double *dtb) {
-  int i = (int)tid();
-  if (i >= N) return;
-  const long Ns = N;
-  const double *fi = rec + 6 * Ns, m = rec[9 * Ns + i];
-  const double *vrec = rec + 3 * Ns, *parec = rec + 11 * Ns + 7L * E;
-  const int mask = bc_word[i] & 7;
-  const double dt = P.dt, ia = 1.0 / (1.0 - P.alpha);
+// the state cotangents [3][N] at a step boundary
+struct Bars {
+  double *x, *v, *ud, *pa;
+};
+
+// the slots' lists and the sums over them: P1 [7][S] of a_element (position,
+// velocity, ratio), P2 [3][S] of a_volume (position); a slot's place is its own
+// index or, node-major (nm), its place in its node's list
+struct SlotSums {
+  const int *nsl_off, *nsl, *spos;
+  int nm, shift;  // shift: the entry table's byte offsets are for 4-byte values (1) or doubles (0)
+  long S;
+};
+__device__ __forceinline__ int slot_at(const SlotSums &q, int o) { return q.nm ? o : q.nsl[o]; }
+__device__ __forceinline__ bool first_slot(const SlotSums &q, int o, int slot) {
+  return q.nm ? q.spos[slot] == o : q.nsl[o] == slot;
+}
+
+// node-pass reverse of step k for node i; Z-bar of boundary k+1 in, of
+// boundary k out (partial: the element sums of this step are added by the
+// next earlier step's call).  dtbar (per-step CFL time step): the node's share
+// of the step length's cotangent, from vv = v' + gamma dt ac, ud = ud + beta
+// dt^2 ac and the prediction ud' = dt (vv + (0.5 - beta) dt ac), v'' = vv +
+// (1 - gamma) dt ac, with ac the corrected acceleration (1/(1-alpha)) (a - alpha pa)
+struct NodeBack {
+  double x[3], v[3], ud[3], pa[3], fib[3], mb, dtb;
+};
+__device__ __forceinline__ void node_reverse(int i, long Ns, long Es, const NodeAdj &P, const double *rec,
+                                             const double *fe, int mask, double hbar, bool cfl, const Bars &in,
+                                             const double (&dx)[3], const double (&dv)[3], NodeBack &B) {
+  const double *fi = rec + 6 * Ns, *vrec = rec + 3 * Ns, *parec = rec + 11 * Ns + 7L * Es;
+  const double m = rec[9 * Ns + i], dt = P.dt, ia = 1.0 / (1.0 - P.alpha);
+  double f[3], xb[3], vb[3], udb[3], pab[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const long id = d * Ns + i;
+    f[d] = fi[id];
+    xb[d] = in.x[id] + dx[d];
+    vb[d] = in.v[id] + dv[d];
+    udb[d] = in.ud[id];
+    pab[d] = in.pa[id];
+  }
   double mbar = 0.0, dtbar = 0.0;
+#pragma unroll
   for (int d = 0; d < 3; ++d) {
     const long id = d * Ns + i;
     const bool free_d = !((mask >> d) & 1);
-    const double vp = vb[id], udp = udb[id], pa_in = pab[id], xbar = xb[id];
+    const double vp = vb[d], udp = udb[d], pa_in = pab[d], xbar = xb[d];
     const double vpm = free_d ? vp : 0.0;
     const double vpp = dt * udp + vpm;       // v'' after its boundary values
     const double vppr = free_d ? vpp : 0.0;  // v'' before them
     const double app = dt * dt * (0.5 - P.beta) * udp + (1.0 - P.gamma) * dt * vpm + pa_in +
                        P.gamma * dt * vppr + P.beta * dt * dt * xbar;
-    udb[id] = xbar;
-    vb[id] = vppr;
-    pab[id] = -P.alpha * ia * app;
+    B.x[d] = xbar;
+    B.ud[d] = xbar;
+    B.v[d] = vppr;
+    B.pa[d] = -P.alpha * ia * app;
     const double abar = free_d ? app * ia : 0.0;
-    const double a = ((P.has_fe ? fe[id] : 0.0) - fi[id]) / m;
-    double fb = -abar / m;
-    if (d == 2 && rgroup[i] >= 0) fb += hbar_k[rgroup[i]];
-    fib[id] = fb;
+    const double a = ((P.has_fe ? fe[id] : 0.0) - f[d]) / m;
+    B.fib[d] = -abar / m + (d == 2 ? hbar : 0.0);
     mbar -= abar * a / m;
-    if (dtb) {
+    if (cfl) {
       const double ac = ia * ((free_d ? a : 0.0) - P.alpha * parec[id]);
       const double vv = free_d ? vrec[id] + P.gamma * dt * ac : vrec[id];  // an imposed v' is its value
       dtbar += udp * (vv + 2.0 * (0.5 - P.beta) * dt * ac) + vpm * (1.0 - P.gamma) * ac +
                vppr * P.gamma * ac + xbar * 2.0 * P.beta * dt * ac;
     }
   }
-  mb[i] = mbar;
-  if (dtb) dtb[i] = dtbar;
+  B.mb = mbar;
+  B.dtb = dtbar;
 }
 
 // Per-step CFL time step dt = cfl m / (cs + v), m the smallest edge of the
@@ -325,118 +359,238 @@ __global__ void k_law_temps(int E, int law, const double *Te, double T_t, double
   }
 }
 
-template <int NN>
-__global__ __launch_bounds__(kB) void a_elem1(int E, int N, adj::ElemConst K, const int *elnod,
-                                              const double *rec, const double *fib, const double *sy0d,
-                                              const double *Hd, const double *rhod, double *taub,
-                                              double *epb, double *contrib, double *volb, double *grad,
-                                              double *dtb_e, const double *lawc) {
-  int e = (int)tid();
-  if (e >= E) return;
-  if (lawc) {  // the element's own temperature factors
-    if (K.law == 2) {
-      K.jsoft = lawc[e];
-    } else {
-      K.ga = lawc[e];
-      K.gexp = lawc[E + e];
-      K.gn = lawc[2L * E + e];
-      K.gm = lawc[3L * E + e];
-      K.gi = lawc[4L * E + e];
+// Sums of R components per slot of the work-group's cluster from the
+// element-node values in LDS (kEntStride), to P[R][S] (the element pass's sums)
+template <int NN, int R>
+__device__ __forceinline__ void slot_sums(const unsigned char *lds, const ClusterArgs &ca, const SlotSums &q,
+                                          int c, const int4 &cd, double *P) {
+  const int s0 = cd.y, M = cd.z >> 16;
+  const uint16_t *lo = ca.goff + s0 + c;
+  const uint2 *en = ca.ent + cd.w;
+  for (int j = threadIdx.x; j < M; j += kCluster) {
+    const int at = q.nm ? q.spos[s0 + j] : s0 + j;
+    double acc[R];
+#pragma unroll
+    for (int u = 0; u < R; ++u) acc[u] = 0.0;
+    const int k1 = lo[j + 1];
+    for (int k = lo[j]; k < k1; ++k) {
+      const uint2 w = en[k];
+      double v[4][R];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const unsigned o = ((h < 2 ? w.x : w.y) >> (16 * (h & 1)) & 0xffffu) << q.shift;
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+          v[h][u] = *reinterpret_cast<const double *>(lds + o + u * (kEntStride(NN) * 8));
+      }
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int u = 0; u < R; ++u) acc[u] += v[h][u];
     }
+#pragma unroll
+    for (int u = 0; u < R; ++u) P[u * q.S + at] = acc[u];
   }
+}
+
+// The reverse step's first kernel.  LDS: the slots' nodal data (x, v', r and
+// the fi cotangent), then the 7 n element-node values; 127 KB (hexahedra), so
+// that every component is summed in one round: one work-group on a CU, which
+// its registers (256 and 224 accumulation registers: the element's forward and
+// reverse live together) allow no more of anyway.
+// Before (node, element, node, element and node kernels with the element-node
+// values in memory, 30^3 hexahedra): 5.0 + 17.7 + 6.0 + 9.9 + 8.0 us.
+template <int NN>
+__global__ __launch_bounds__(kCluster) void a_element(
+    int E, int N, NodeAdj P, adj::ElemConst K, ClusterArgs ca, SlotSums q, const double *rec, const double *fe,
+    const int *bc_word, const int *rgroup, const double *hbar_k, Bars in, Bars out, const double *P1in,
+    const double *P2in, int pending, double *mb, double *dtb_n, const double *sy0d, const double *Hd,
+    const double *rhod, double *taub, double *epb, double *P1, double *volb, double *grad, double *dtb_e,
+    const double *lawc) {
+  constexpr int cap = slot_cap(NN), kSl = kSlotsPerThread<NN>;
+  __shared__ __align__(16) double lds[6 * kEntStride(NN) + NN * kCluster + 1];
+  static_assert(10 * cap <= 6 * kEntStride(NN) + NN * kCluster, "the staged slots fit");
+  const int c = xcd_block(), t = threadIdx.x;
+  const int4 cd = ca.desc[c];
+  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;
   const long Es = E, Ns = N;
   const double *x = rec, *v = rec + 3 * Ns, *r = rec + 10 * Ns, *tau = rec + 11 * Ns, *ep = tau + 6 * Es;
-  adj::ElemIn<NN> in;
+  const int e = e0 + min(t, ne - 1);
+  int ls[NN];
+  load_lslot<NN>(ca.lslot + (long)e * NN, ls);
+  int node[kSl], o[kSl], n[kSl];
+#pragma unroll
+  for (int k = 0; k < kSl; ++k) node[k] = ca.snode[s0 + min(t + k * kCluster, M - 1)];
+#pragma unroll
+  for (int k = 0; k < kSl; ++k) {
+    o[k] = q.nsl_off[node[k]];
+    n[k] = q.nsl_off[node[k] + 1] - o[k];
+  }
+#pragma unroll
+  for (int k = 0; k < kSl; ++k) {
+    const int j = t + k * kCluster, i = node[k];
+    const bool own = j < M && first_slot(q, o[k], s0 + min(j, M - 1));
+    double dx[3] = {0.0, 0.0, 0.0}, dv[3] = {0.0, 0.0, 0.0};
+    if (pending)  // the later step's element sums, clusters in order
+      for (int h = 0; h < n[k]; h += 4) {
+        double p[4][9];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int at = slot_at(q, o[k] + min(h + g, n[k] - 1));
+#pragma unroll
+          for (int u = 0; u < 6; ++u) p[g][u] = P1in[u * q.S + at];
+#pragma unroll
+          for (int u = 0; u < 3; ++u) p[g][6 + u] = P2in[u * q.S + at];
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          if (h + g < n[k])
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+              dx[u] += p[g][u] + p[g][6 + u];
+              dv[u] += p[g][3 + u];
+            }
+      }
+    const int rg = rgroup[i];
+    NodeBack B;
+    node_reverse(i, Ns, Es, P, rec, fe, bc_word[i] & 7, rg >= 0 ? hbar_k[rg] : 0.0, dtb_n != nullptr, in, dx, dv, B);
+    if (own) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const long id = d * Ns + i;
+        out.x[id] = B.x[d];
+        out.v[id] = B.v[d];
+        out.ud[id] = B.ud[d];
+        out.pa[id] = B.pa[d];
+      }
+      mb[i] = B.mb;
+      if (dtb_n) dtb_n[i] = B.dtb;
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      lds[d * cap + j] = x[d * Ns + i];
+      lds[(3 + d) * cap + j] = v[d * Ns + i];
+      lds[(7 + d) * cap + j] = B.fib[d];
+    }
+    lds[6 * cap + j] = r[i];
+  }
+  __syncthreads();
+  adj::ElemIn<NN> ei;
   double fb[NN][3];
+#pragma unroll
   for (int a = 0; a < NN; ++a) {
-    const int g = elnod[a * Es + e];
-    for (int c = 0; c < 3; ++c) {
-      in.X[a][c] = x[c * Ns + g];
-      in.V[a][c] = v[c * Ns + g];
-      fb[a][c] = fib[c * Ns + g];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      ei.X[a][d] = lds[d * cap + ls[a]];
+      ei.V[a][d] = lds[(3 + d) * cap + ls[a]];
+      fb[a][d] = lds[(7 + d) * cap + ls[a]];
     }
-    in.r[a] = r[g];
+    ei.r[a] = lds[6 * cap + ls[a]];
   }
-  double tb[6];
-  for (int q = 0; q < 6; ++q) {
-    in.tau[q] = tau[q * Es + e];
-    tb[q] = taub[q * Es + e];
-  }
-  in.ep = ep[e];
-  in.rho = rhod[e];
-  in.sy0 = sy0d[e];
-  in.H = Hd[e];
-  adj::ElemFwd<NN> F;
-  adj::elem_forward<NN>(K, in, F);
-  adj::ElemBar<NN> B;
-  adj::elem_reverse<NN>(K, in, F, fb, tb, epb[e], B);
-  for (int q = 0; q < 6; ++q) taub[q * Es + e] = B.tau[q];
-  epb[e] = B.ep;
-  for (int a = 0; a < NN; ++a) {
-    for (int c = 0; c < 3; ++c) {
-      contrib[(a * 7 + c) * Es + e] = B.X[a][c];
-      contrib[(a * 7 + 3 + c) * Es + e] = B.V[a][c];
+  __syncthreads();
+  if (t < ne) {
+    if (lawc) {  // the element's own temperature factors
+      if (K.law == 2) {
+        K.jsoft = lawc[e];
+      } else {
+        K.ga = lawc[e];
+        K.gexp = lawc[E + e];
+        K.gn = lawc[2L * E + e];
+        K.gm = lawc[3L * E + e];
+        K.gi = lawc[4L * E + e];
+      }
     }
-    contrib[(a * 7 + 6) * Es + e] = B.r[a];
+    double tb[6];
+    for (int k = 0; k < 6; ++k) {
+      ei.tau[k] = tau[k * Es + e];
+      tb[k] = taub[k * Es + e];
+    }
+    ei.ep = ep[e];
+    ei.rho = rhod[e];
+    ei.sy0 = sy0d[e];
+    ei.H = Hd[e];
+    adj::ElemFwd<NN> F;
+    adj::elem_forward<NN>(K, ei, F);
+    adj::ElemBar<NN> B;
+    adj::elem_reverse<NN>(K, ei, F, fb, tb, epb[e], B);
+    for (int k = 0; k < 6; ++k) taub[k * Es + e] = B.tau[k];
+    epb[e] = B.ep;
+    volb[e] = B.volb;
+    if (dtb_e) dtb_e[e] = B.dt;
+    // rows: the law's two parameters (bilinear sy0, H; Hollomon Kh, mh;
+    // Johnson-Cook A, B; GMT C1, n2), hg
+    grad[e] += K.law == 1 ? B.Kh : B.sy0;
+    grad[Es + e] += K.law == 1 ? B.mh : B.H;
+    grad[2 * Es + e] += B.hg;
+#pragma unroll
+    for (int a = 0; a < NN; ++a) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        lds[d * kEntStride(NN) + a * kCluster + t] = B.X[a][d];
+        lds[(3 + d) * kEntStride(NN) + a * kCluster + t] = B.V[a][d];
+      }
+      lds[6 * kEntStride(NN) + a * kCluster + t] = B.r[a];
+    }
   }
-  volb[e] = B.volb;
-  if (dtb_e) dtb_e[e] = B.dt;
-  // rows: the law's two parameters (bilinear sy0, H; Hollomon Kh, mh;
-  // Johnson-Cook A, B; GMT C1, n2), hg
-  grad[e] += K.law == 1 ? B.Kh : B.sy0;
-  grad[Es + e] += K.law == 1 ? B.mh : B.H;
-  grad[2 * Es + e] += B.hg;
+  if (t < 7) lds[t * kEntStride(NN) + NN * kCluster] = 0.0;
+  __syncthreads();
+  slot_sums<NN, 7>(reinterpret_cast<const unsigned char *>(lds), ca, q, c, cd, P1);
 }
 
-__global__ void a_node2(int N, int E, int n, const int *off, const int *cnt, const int *pk, const double *contrib,
-                        const double *vsum0, const double *mb, const double *rho_avg, double *w) {
-  int i = (int)tid();
-  if (i >= N) return;
-  const long Es = E;
-  double rs = 0.0;
-  for (int k = 0; k < cnt[i]; ++k) {
-    const int q = pk[off[i] + k];
-    rs += contrib[((q & 7) * 7 + 6) * Es + (q >> 3)];
-  }
-  w[i] = rs / vsum0[i] + mb[i] * rho_avg[i] / n;
-}
-
+// The reverse step's second kernel: the nodes' volume cotangents w (the ratio
+// cotangents over S0_i, and the mass cotangent through rho V / n), each
+// element's volume cotangent to its positions
 template <int NN>
-__global__ __launch_bounds__(kB) void a_elem2(int E, int N, const int *elnod, const double *rec,
-                                              const double *volb, const double *w, double *contrib) {
-  int e = (int)tid();
-  if (e >= E) return;
-  const long Es = E, Ns = N;
-  double X[NN][3], vb = volb[e];
-  for (int a = 0; a < NN; ++a) {
-    const int g = elnod[a * Es + e];
-    for (int c = 0; c < 3; ++c) X[a][c] = rec[c * Ns + g];
-    vb += w[g];
-  }
-  double Xb[NN][3];
-  adj::vol_reverse<NN>(X, vb, Xb);
-  for (int a = 0; a < NN; ++a)
-    for (int c = 0; c < 3; ++c) contrib[(a * 7 + c) * Es + e] += Xb[a][c];
-}
-
-__global__ void a_node3(int N, int E, const int *off, const int *cnt, const int *pk, const double *contrib,
-                        double *xb, double *vb) {
-  int i = (int)tid();
-  if (i >= N) return;
-  const long Es = E, Ns = N;
-  double sx[3] = {0, 0, 0}, sv[3] = {0, 0, 0};
-  for (int k = 0; k < cnt[i]; ++k) {
-    const int q = pk[off[i] + k];
-    const long base = (long)(q & 7) * 7, e = q >> 3;
-    for (int c = 0; c < 3; ++c) {
-      sx[c] += contrib[(base + c) * Es + e];
-      sv[c] += contrib[(base + 3 + c) * Es + e];
+__global__ __launch_bounds__(kCluster) void a_volume(int E, int N, ClusterArgs ca, SlotSums q, const double *rec,
+                                                     const double *P1, const double *vsum0, const double *mb,
+                                                     const double *rho_avg, const double *volb, double *P2) {
+  constexpr int cap = slot_cap(NN), kSl = kSlotsPerThread<NN>;
+  __shared__ __align__(16) double lds[2 * kEntStride(NN) + NN * kCluster + 1];
+  const int c = xcd_block(), t = threadIdx.x;
+  const int4 cd = ca.desc[c];
+  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;
+  const long Ns = N;
+  const int e = e0 + min(t, ne - 1);
+  int ls[NN];
+  load_lslot<NN>(ca.lslot + (long)e * NN, ls);
+  double vb = volb[e];
+#pragma unroll
+  for (int k = 0; k < kSl; ++k) {
+    const int j = t + k * kCluster, i = ca.snode[s0 + min(j, M - 1)];
+    const int o = q.nsl_off[i], n = q.nsl_off[i + 1] - o;
+    double rs = 0.0;
+    for (int h = 0; h < n; h += 4) {
+      double p[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) p[g] = P1[6 * q.S + slot_at(q, o + min(h + g, n - 1))];
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        if (h + g < n) rs += p[g];
     }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) lds[d * cap + j] = rec[d * Ns + i];
+    lds[3 * cap + j] = rs / vsum0[i] + mb[i] * rho_avg[i] / NN;
   }
-  for (int c = 0; c < 3; ++c) {
-    xb[c * Ns + i] += sx[c];
-    vb[c * Ns + i] += sv[c];
+  __syncthreads();
+  double X[NN][3];
+#pragma unroll
+  for (int a = 0; a < NN; ++a) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) X[a][d] = lds[d * cap + ls[a]];
+    vb += lds[3 * cap + ls[a]];
   }
+  __syncthreads();
+  if (t < ne) {
+    double Xb[NN][3];
+    adj::vol_reverse<NN>(X, vb, Xb);
+#pragma unroll
+    for (int a = 0; a < NN; ++a)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) lds[d * kEntStride(NN) + a * kCluster + t] = Xb[a][d];
+  }
+  if (t < 3) lds[t * kEntStride(NN) + NN * kCluster] = 0.0;
+  __syncthreads();
+  slot_sums<NN, 3>(reinterpret_cast<const unsigned char *>(lds), ca, q, c, cd, P2);
 }
 
 // parameter gradients: one work-group per parameter row, fixed order; for
@@ -547,9 +701,10 @@ static int adj_alloc(wfx_ctx *c, int nsteps, int every) {
     get(&A->slot, A->slot_stride * every);
     get(&A->hist, (size_t)nsteps * ng);
     get(&A->hbar, (size_t)nsteps * ng);
-    get(&A->xb, 3 * N); get(&A->vb, 3 * N); get(&A->udb, 3 * N); get(&A->pab, 3 * N);
-    get(&A->taub, 6 * E); get(&A->epb, E); get(&A->fib, 3 * N); get(&A->mb, N); get(&A->w, N);
-    get(&A->contrib, 7 * n * E); get(&A->volb, E); get(&A->grad, 3 * E);
+    const long S = c->ms.nslot;
+    get(&A->bars[0], 12 * N); get(&A->bars[1], 12 * N);
+    get(&A->taub, 6 * E); get(&A->epb, E); get(&A->mb, N);
+    get(&A->p1[0], 7 * S); get(&A->p1[1], 7 * S); get(&A->p2, 3 * S); get(&A->volb, E); get(&A->grad, 3 * E);
     get(&A->sy0d, E); get(&A->Hd, E); get(&A->rhod, E); get(&A->rho_avg, N); get(&A->sums, 8 + E);
     get(&A->dts, nsteps); get(&A->dtb, N + E); get(&A->cfl_loc, 8); get(&A->lawc, 5 * E);
     if (err == hipSuccess) {
@@ -674,8 +829,7 @@ static int adjoint_backward(wfx_ctx *c, hipStream_t st) {
   const int N = c->N, E = c->E, n = c->n;
   auto &el = el_of<T>(c);
   const auto &P = c->prm;
-  for (double *p : {A->xb, A->vb, A->udb, A->pab, A->fib})
-    hipLaunchKernelGGL(k_zero, dim3(nb(3L * N)), dim3(kB), 0, st, 3L * N, p);
+  hipLaunchKernelGGL(k_zero, dim3(nb(12L * N)), dim3(kB), 0, st, 12L * N, A->bars[0]);
   hipLaunchKernelGGL(k_zero, dim3(nb(6L * E)), dim3(kB), 0, st, 6L * E, A->taub);
   hipLaunchKernelGGL(k_zero, dim3(nb(E)), dim3(kB), 0, st, (long)E, A->epb);
   hipLaunchKernelGGL(k_zero, dim3(nb(3L * E)), dim3(kB), 0, st, 3L * E, A->grad);
@@ -727,6 +881,14 @@ static int adjoint_backward(wfx_ctx *c, hipStream_t st) {
     lawc = A->lawc;
   }
   NodeAdj NP{P.dt, P.alpha, P.beta, P.gamma, c->has_fe, A->ng};
+  const ClusterArgs ca = cluster_args(c);
+  const SlotSums sums{c->ms.nsl_off, c->ms.nsl, c->ms.spos, c->ms.spos != nullptr, c->precision == WFX_FP64 ? 0 : 1,
+                      c->ms.nslot};
+  auto bars = [&](int k) {
+    double *b = A->bars[k];
+    return Bars{b, b + 3L * N, b + 6L * N, b + 9L * N};
+  };
+  int cur = 0, pending = 0;
   for (int seg = A->nck - 1; seg >= 0; --seg) {
     const int k0 = seg * A->every, k1 = std::min(A->nsteps, k0 + A->every);
     LAUNCH(load_ck<T>(c, seg, st));
@@ -738,29 +900,28 @@ static int adjoint_backward(wfx_ctx *c, hipStream_t st) {
       const double *rec = A->slot + (size_t)(k - k0) * A->slot_stride;
       if (A->cfl) NP.dt = K.dt = A->dts_h[k];
       double *dtb_n = A->cfl ? A->dtb : nullptr, *dtb_e = A->cfl ? A->dtb + N : nullptr;
-      hipLaunchKernelGGL(a_node1, dim3(nb(N)), dim3(kB), 0, st, N, E, NP, rec, c->nd.fe, c->bc_word,
-                         A->rgroup, A->hbar + (size_t)k * A->ng, A->xb, A->vb, A->udb, A->pab, A->fib, A->mb,
-                         dtb_n);
-      if (n == 8)
-        hipLaunchKernelGGL((a_elem1<8>), dim3(nb(E)), dim3(kB), 0, st, E, N, K, c->ms.elnod, rec, A->fib,
-                           A->sy0d, A->Hd, A->rhod, A->taub, A->epb, A->contrib, A->volb, A->grad, dtb_e, lawc);
-      else
-        hipLaunchKernelGGL((a_elem1<4>), dim3(nb(E)), dim3(kB), 0, st, E, N, K, c->ms.elnod, rec, A->fib,
-                           A->sy0d, A->Hd, A->rhod, A->taub, A->epb, A->contrib, A->volb, A->grad, dtb_e, lawc);
-      hipLaunchKernelGGL(a_node2, dim3(nb(N)), dim3(kB), 0, st, N, E, n, c->ms.nodel_offset, c->ms.nodel_count,
-                         c->ms.nodel_pk, A->contrib, c->nd.voln0_sum, A->mb, A->rho_avg, A->w);
-      if (n == 8)
-        hipLaunchKernelGGL((a_elem2<8>), dim3(nb(E)), dim3(kB), 0, st, E, N, c->ms.elnod, rec, A->volb, A->w,
-                           A->contrib);
-      else
-        hipLaunchKernelGGL((a_elem2<4>), dim3(nb(E)), dim3(kB), 0, st, E, N, c->ms.elnod, rec, A->volb, A->w,
-                           A->contrib);
-      hipLaunchKernelGGL(a_node3, dim3(nb(N)), dim3(kB), 0, st, N, E, c->ms.nodel_offset, c->ms.nodel_count,
-                         c->ms.nodel_pk, A->contrib, A->xb, A->vb);
+      const Bars in = bars(cur), out = bars(1 - cur);
+      if (n == 8) {
+        hipLaunchKernelGGL((a_element<8>), dim3(c->ms.ncl), dim3(kCluster), 0, st, E, N, NP, K, ca, sums, rec,
+                           c->nd.fe, c->bc_word, A->rgroup, A->hbar + (size_t)k * A->ng, in, out, A->p1[1 - cur],
+                           A->p2, pending, A->mb, dtb_n, A->sy0d, A->Hd, A->rhod, A->taub, A->epb, A->p1[cur],
+                           A->volb, A->grad, dtb_e, lawc);
+        hipLaunchKernelGGL((a_volume<8>), dim3(c->ms.ncl), dim3(kCluster), 0, st, E, N, ca, sums, rec, A->p1[cur],
+                           c->nd.voln0_sum, A->mb, A->rho_avg, A->volb, A->p2);
+      } else {
+        hipLaunchKernelGGL((a_element<4>), dim3(c->ms.ncl), dim3(kCluster), 0, st, E, N, NP, K, ca, sums, rec,
+                           c->nd.fe, c->bc_word, A->rgroup, A->hbar + (size_t)k * A->ng, in, out, A->p1[1 - cur],
+                           A->p2, pending, A->mb, dtb_n, A->sy0d, A->Hd, A->rhod, A->taub, A->epb, A->p1[cur],
+                           A->volb, A->grad, dtb_e, lawc);
+        hipLaunchKernelGGL((a_volume<4>), dim3(c->ms.ncl), dim3(kCluster), 0, st, E, N, ca, sums, rec, A->p1[cur],
+                           c->nd.voln0_sum, A->mb, A->rho_avg, A->volb, A->p2);
+      }
+      cur = 1 - cur;  // the cotangents and sums just written are the next step's inputs
+      pending = 1;
       if (A->cfl) {  // the step length's dependence on x and v' at the step's start
         hipLaunchKernelGGL(a_cfl_locate, dim3(1), dim3(kCflB), 0, st, E, N, c->ms.elnod, rec, A->cfl_loc);
         hipLaunchKernelGGL(a_cfl_apply, dim3(1), dim3(kCflB), 0, st, N, E, A->dts_h[k], P.cfl, A->dtb, A->cfl_loc,
-                           c->ms.elnod, rec, A->xb, A->vb);
+                           c->ms.elnod, rec, out.x, out.v);
       }
       LAUNCH(hipGetLastError());
     }
