@@ -41,9 +41,10 @@
 
 #include "../../include/wfx.h"
 #include "wfx_adjoint.hpp"
-#include "wfx_fused.hpp"
 #include "wfx_internal.hpp"
+#include "wfx_kernels.hpp"
 #include "wfx_launch.hpp"
+#include "wfx_slots.hpp"
 
 namespace wfx {
 
@@ -698,7 +699,7 @@ static int adj_alloc(wfx_ctx *c, int nsteps, int every) {
       if (err == hipSuccess) { A->mem.push_back(q); *p = (double *)q; }
     };
     get(&A->ck, A->ck_stride * nck);
-    get(&A->slot, A->slot_stride * every);
+    get(&A->slot, A->slot_stride * (every + 1));  // and the state after a segment's last step
     get(&A->hist, (size_t)nsteps * ng);
     get(&A->hbar, (size_t)nsteps * ng);
     const long S = c->ms.nslot;
@@ -797,6 +798,23 @@ static hipError_t fused_step(wfx_ctx *c, int predict, int k, bool last, double *
   return hipGetLastError();
 }
 
+// The two sets of nodal arrays in the places they had (a run of paired steps
+// ends so by itself; a failed one, or one record by record, does not)
+struct KeepPlaces {
+  wfx_ctx *c;
+  double *x, *v, *pa, *ud, *x_b;
+  float *v32, *pa32, *ud32;
+  void *v_b, *pa_b, *ud_b;
+  explicit KeepPlaces(wfx_ctx *q)
+      : c(q), x(q->nd.x), v(q->nd.v), pa(q->nd.prev_a), ud(q->nd.u_dt), x_b(q->x_b), v32(q->v32), pa32(q->pa32),
+        ud32(q->ud32), v_b(q->v_b), pa_b(q->pa_b), ud_b(q->ud_b) {}
+  ~KeepPlaces() {
+    c->nd.x = x; c->nd.v = v; c->nd.prev_a = pa; c->nd.u_dt = ud; c->x_b = x_b;
+    c->v32 = v32; c->pa32 = pa32; c->ud32 = ud32;
+    c->v_b = v_b; c->pa_b = pa_b; c->ud_b = ud_b;
+  }
+};
+
 template <typename T>
 static int adjoint_forward(wfx_ctx *c, int nsteps, bool want_hist, hipStream_t st) {
   Adjoint *A = c->adj;
@@ -806,12 +824,12 @@ static int adjoint_forward(wfx_ctx *c, int nsteps, bool want_hist, hipStream_t s
   LAUNCH(launch_fused_pack<T>(c, st));
   if (A->cfl) LAUNCH(launch_cfl_begin<T>(c, st, true));
   const ReactRecord rec(c, want_hist ? A->hist : nullptr, nsteps, sizeof(T));
+  const KeepPlaces places(c);
+  const bool pair = run_paired(c);
+  bool have_vol = false;
   for (int k = 0; k < nsteps; ++k) {
     if (k % A->every == 0) LAUNCH(save_ck<T>(c, k / A->every, st));
-    c->fused_rz = rec.row(k);
-    const hipError_t e = fused_step<T>(c, k + 1 < nsteps, k, k + 1 == nsteps, nullptr, st);
-    c->fused_rz = nullptr;
-    LAUNCH(e);
+    LAUNCH(launch_run_step<T>(c, k, nsteps, pair, have_vol, rec.row(k), st, nullptr));
     if (rec.full(k)) LAUNCH(launch_reaction_rows<T>(c, rec, k, st));
   }
   LAUNCH(launch_fused_unpack<T>(c, st));
@@ -888,14 +906,32 @@ static int adjoint_backward(wfx_ctx *c, hipStream_t st) {
     double *b = A->bars[k];
     return Bars{b, b + 3L * N, b + 6L * N, b + 9L * N};
   };
+  const KeepPlaces places(c);
+  auto record = [&](int j) {
+    double *p = A->slot + (size_t)j * A->slot_stride;
+    const long n3 = 3L * N, o = 11L * N;
+    return StepRecord{p, p + n3, p + o + 7L * E, p + 2 * n3, p + 9L * N, p + 10L * N, p + o, p + o + 6L * E};
+  };
   int cur = 0, pending = 0;
   for (int seg = A->nck - 1; seg >= 0; --seg) {
     const int k0 = seg * A->every, k1 = std::min(A->nsteps, k0 + A->every);
     LAUNCH(load_ck<T>(c, seg, st));
     if (A->cfl) LAUNCH(launch_cfl_begin<T>(c, st, true));  // the first recomputed step's largest speed
-    for (int k = k0; k < k1; ++k)
-      LAUNCH(fused_step<T>(c, k + 1 < A->nsteps, k, k + 1 == A->nsteps, A->slot + (size_t)(k - k0) * A->slot_stride,
-                           st));
+    if constexpr (std::is_same<T, double>::value) {
+      if (run_paired(c)) {
+        // the checkpoint's state into the first record, then from record to record
+        const StepRecord r0 = record(0);
+        hipLaunchKernelGGL((k_rec_pre<T>), dim3(nb(9L * N + 7L * E)), dim3(kB), 0, st, N, E, c->nd.x, c->nd.v, el.tau,
+                           el.pl_strain, c->nd.prev_a, r0.x);
+        LAUNCH(hipGetLastError());
+        for (int k = k0; k < k1; ++k)
+          LAUNCH(launch_recorded_step<T>(c, k, k == k0, record(k - k0), record(k - k0 + 1), st));
+      }
+    }
+    if (!std::is_same<T, double>::value || !run_paired(c))
+      for (int k = k0; k < k1; ++k)
+        LAUNCH(fused_step<T>(c, k + 1 < A->nsteps, k, k + 1 == A->nsteps, A->slot + (size_t)(k - k0) * A->slot_stride,
+                             st));
     for (int k = k1 - 1; k >= k0; --k) {
       const double *rec = A->slot + (size_t)(k - k0) * A->slot_stride;
       if (A->cfl) NP.dt = K.dt = A->dts_h[k];

@@ -11,6 +11,9 @@ namespace wfx {
 template hipError_t launch_vsum0<double>(wfx_ctx *, hipStream_t);
 template hipError_t launch_fused_phase<double>(wfx_ctx *, int, int, hipStream_t, int);
 template hipError_t launch_fused_steps<double>(wfx_ctx *, int, double *, hipStream_t, hipEvent_t *);
+template hipError_t launch_run_step<double>(wfx_ctx *, int, int, bool, bool &, void *, hipStream_t, hipEvent_t *);
+template hipError_t launch_recorded_step<double>(wfx_ctx *, int, bool, const StepRecord &, const StepRecord &,
+                                                 hipStream_t);
 template hipError_t launch_fused_pack<double>(wfx_ctx *, hipStream_t);
 template hipError_t launch_fused_unpack<double>(wfx_ctx *, hipStream_t);
 template hipError_t launch_cfl_begin<double>(wfx_ctx *, hipStream_t, bool);

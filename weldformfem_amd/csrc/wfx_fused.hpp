@@ -45,6 +45,7 @@
 #include "wfx_contact.hpp"
 #include "wfx_kernels.hpp"
 #include "wfx_launch.hpp"
+#include "wfx_slots.hpp"
 
 namespace wfx {
 namespace {
@@ -410,13 +411,6 @@ struct SlotLds {
         node(reinterpret_cast<int *>(base + (3 * 8 + 4 * (int)sizeof(T)) * cap)) {}
 };
 
-// Slots each thread of a cluster pass stages (slot_cap = kSlotsPerThread *
-// kCluster): the staging rows past the cluster's slot count are written with
-// a repeat of its last slot and never read, so that no load or store of the
-// staging waits behind a branch
-template <int NN>
-constexpr int kSlotsPerThread = slot_cap(NN) / kCluster;
-
 // What the first part of the element chain leaves for the second: geometry,
 // strain rate and spin, hourglass amplitudes, the nodal ANP average and,
 // with thermal coupling, the element's temperature terms.
@@ -594,8 +588,8 @@ struct ElemState {
   T tau[6], eps[6], ep, sy0, He;
 };
 template <typename T>
-__device__ __forceinline__ void load_elem_state(int e, int E, const T *__restrict__ tau_io,
-                                                const T *__restrict__ eps_io, const T *__restrict__ pl_strain,
+__device__ __forceinline__ void load_elem_state(int e, int E, const T *tau_io,
+                                                const T *__restrict__ eps_io, const T *pl_strain,
                                                 const T *__restrict__ sy0, const T *__restrict__ He,
                                                 ElemState<T> &S) {
   const long Es = E;
@@ -618,8 +612,8 @@ constexpr int kStashVals = TH ? 25 : 22;
 template <typename T, int NN, int LAW, int BS, bool TH, class Sink>
 __device__ __forceinline__ void element_material(
     int e, int E, const FusedParams &fp, T dt, ElemGeo<T, NN, TH> &G, const ElemState<T> &S,
-    const T *__restrict__ vol0, const T *__restrict__ rho, const T *__restrict__ He, T *__restrict__ tau_io,
-    T *__restrict__ eps_io, T *__restrict__ p_out, T *__restrict__ pl_strain, T *__restrict__ sigma_y,
+    const T *__restrict__ vol0, const T *__restrict__ rho, const T *__restrict__ He, T *tau_out,
+    T *__restrict__ eps_io, T *__restrict__ p_out, T *pl_out, bool pl_all, T *__restrict__ sigma_y,
     T *__restrict__ q_plheat, double *stash, Sink &&sink) {
   const long Es = E;
   T s00 = G.s00, s11 = G.s11, s22 = G.s22, s01 = G.s01, s12 = G.s12, s02 = G.s02;
@@ -718,8 +712,10 @@ __device__ __forceinline__ void element_material(
     T dgamma = (sig_trial - sy) / (T(3) * Gm + H);
     T factor = T(1) - (T(3) * Gm * dgamma) / sig_trial;
     tau = t3_scale(s, factor);
-    pl_strain[e] = ep + dgamma;
+    pl_out[e] = ep + dgamma;
     dep = dgamma;
+  } else if (pl_all) {  // not in place: every element's
+    pl_out[e] = ep;
   }
   T3<T> sig = t3_add(pI, tau);
   double heat = 0.0;  // thermal coupling: the element's heat per node and cp
@@ -758,9 +754,9 @@ __device__ __forceinline__ void element_material(
   st_stream(&eps_io[3 * Es + e], S.eps[3] + D.xy * dt);
   st_stream(&eps_io[4 * Es + e], S.eps[4] + D.yz * dt);
   st_stream(&eps_io[5 * Es + e], S.eps[5] + D.xz * dt);
-  st_stream(&tau_io[0 * Es + e], tau.xx); st_stream(&tau_io[1 * Es + e], tau.yy);
-  st_stream(&tau_io[2 * Es + e], tau.zz); st_stream(&tau_io[3 * Es + e], tau.xy);
-  st_stream(&tau_io[4 * Es + e], tau.yz); st_stream(&tau_io[5 * Es + e], tau.xz);
+  st_stream(&tau_out[0 * Es + e], tau.xx); st_stream(&tau_out[1 * Es + e], tau.yy);
+  st_stream(&tau_out[2 * Es + e], tau.zz); st_stream(&tau_out[3 * Es + e], tau.xy);
+  st_stream(&tau_out[4 * Es + e], tau.yz); st_stream(&tau_out[5 * Es + e], tau.xz);
 
   T C[3][3], hm[3][4];
   double gT0 = G.gT0, gT1 = G.gT1, gT2 = G.gT2;
@@ -846,18 +842,6 @@ __device__ __forceinline__ void element_material(
   }
 }
 
-// Cluster tables of the fused element pass on the device (wfx_cluster.hpp)
-struct ClusterArgs {
-  const int4 *desc;      // as DevMesh::cl_desc, cl_goff, cl_ent
-  const uint16_t *goff;
-  const uint2 *ent;
-  const int *snode;      // [S] slot -> node
-  const uint16_t *lslot; // [E][n] element-node -> slot within its cluster
-  const int *spos;       // [S] slot -> where its partial sum is stored when node-major
-  long S;                // slots: the row length of the partial sums
-  int nm;                // partial sums node-major (FP32-mixed always, FP64 with the paired passes)
-};
-
 // What the paired passes need beyond the four separate ones
 struct PairArgs {
   const int4 *rec;       // per slot (DevMesh::srec)
@@ -901,18 +885,6 @@ constexpr int kF3Vals = (kStashLDS<T, NN, LAW> && kStashVals<TH> * 8 * kCluster 
 template <typename T, int NN, int LAW, bool TH>
 constexpr int kF3Lds = kF3Vals<T, NN, LAW, TH> > SlotLds<T, NN>::bytes ? kF3Vals<T, NN, LAW, TH>
                                                                         : SlotLds<T, NN>::bytes;
-
-// One element's nodes as slot indices of its cluster (a 16- or 8-byte load)
-template <int NN>
-__device__ __forceinline__ void load_lslot(const uint16_t *p, int (&ls)[NN]) {
-  typedef unsigned int u32v __attribute__((ext_vector_type(NN / 2)));
-  const u32v w = __builtin_nontemporal_load(reinterpret_cast<const u32v *>(p));
-#pragma unroll
-  for (int k = 0; k < NN / 2; ++k) {
-    ls[2 * k] = (int)(w[k] & 0xffffu);
-    ls[2 * k + 1] = (int)(w[k] >> 16);
-  }
-}
 
 // The nodal volume sums of a thread's slots' nodes from the element volumes,
 // with the ANP ratio as F2 leaves it and, by a node's first slot, the ratio
@@ -1015,8 +987,8 @@ template <typename T, int NN, int LAW, bool TH, bool PAIR>
 __global__ __launch_bounds__(kCluster) void f3_cluster(
     int E, int N, FusedParams fp, ClusterArgs ca, PairArgs pr, const double *__restrict__ x, const T *__restrict__ v,
     const double *__restrict__ ratio, const T *__restrict__ vol0, const T *__restrict__ rho,
-    const T *__restrict__ sy0, const T *__restrict__ He, T *__restrict__ tau_io, T *__restrict__ eps_io,
-    T *__restrict__ p_out, T *__restrict__ pl_strain, T *__restrict__ sigma_y, T *__restrict__ part,
+    const T *__restrict__ sy0, const T *__restrict__ He, const T *tau_in, T *tau_out, T *__restrict__ eps_io,
+    T *__restrict__ p_out, const T *pl_in, T *pl_out, T *__restrict__ sigma_y, T *__restrict__ part,
     T *__restrict__ q_plheat) {
   constexpr int R = kNodeVals<TH>;
   __shared__ __align__(16) unsigned char lds_raw[kF3Lds<T, NN, LAW, TH>];
@@ -1093,7 +1065,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   if constexpr (PAIR) ps.nodal(pr, rec, fp.rho_u);
   __builtin_amdgcn_sched_barrier(0);
   ElemState<T> S;
-  load_elem_state<T>(my_e, E, tau_io, eps_io, pl_strain, sy0, He, S);
+  load_elem_state<T>(my_e, E, tau_in, eps_io, pl_in, sy0, He, S);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (PAIR) ps.ratio(pr, rec, mine, sr);
   double dt_step = fp.dt;
@@ -1132,7 +1104,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   __syncthreads();  // the staged slots are read: their LDS takes the element-node values
   if (t < ne) {
     element_material<T, NN, LAW, kCluster, TH>(
-        e0 + t, E, fp, dt, G, S, vol0, rho, He, tau_io, eps_io, p_out, pl_strain, sigma_y, q_plheat,
+        e0 + t, E, fp, dt, G, S, vol0, rho, He, tau_out, eps_io, p_out, pl_out, pl_in != pl_out, sigma_y, q_plheat,
         reinterpret_cast<double *>(lds_raw) + t, [&](int a, int node, T f0, T f1, T f2, T th) {
           lf[0 * kEntStride(NN) + a * kCluster + t] = f0;
           lf[1 * kEntStride(NN) + a * kCluster + t] = f1;
@@ -1925,11 +1897,6 @@ void fused_node_arrays(wfx_ctx *c, T *&v, T *&pa, T *&ud, T *&fi) {
     v = c->v32; pa = c->pa32; ud = c->ud32; fi = c->fi32;
   }
 }
-inline ClusterArgs cluster_args(const wfx_ctx *c) {
-  return ClusterArgs{c->ms.cl_desc, c->ms.cl_goff, c->ms.cl_ent, c->ms.cl_snode,
-                     c->ms.cl_lslot, c->ms.spos,  c->ms.nslot,   c->ms.spos != nullptr};
-}
-
 // F3 (PAIR: with F2 in its staging); dtp: the step's dt on the device, or null
 template <typename T, bool PAIR>
 hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr, hipStream_t s) {
@@ -1964,8 +1931,9 @@ hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr
   auto kern = (c->n == 8) ? (rate ? f3_pick<T, 8, LAW_RATE, PAIR>(th) : f3_pick<T, 8, LAW_PLAIN, PAIR>(th))
                           : (rate ? f3_pick<T, 4, LAW_RATE, PAIR>(th) : f3_pick<T, 4, LAW_PLAIN, PAIR>(th));
   hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, c->E, c->N, fp, cluster_args(c), pr, c->nd.x, vN,
-                     c->nd.anp_ratio, el.vol0, el.rho, el.sy0, el.He, el.tau, el.eps, el.p, el.pl_strain,
-                     el.sigma_y, el.part, c->thermal.on ? el.q_plheat : (T *)nullptr);
+                     c->nd.anp_ratio, el.vol0, el.rho, el.sy0, el.He, el.tau,
+                     c->fused_tau_out ? (T *)c->fused_tau_out : el.tau, el.eps, el.p, el.pl_strain,
+                     c->fused_pl_out ? (T *)c->fused_pl_out : el.pl_strain, el.sigma_y, el.part, c->thermal.on ? el.q_plheat : (T *)nullptr);
   return hipGetLastError();
 }
 
@@ -2060,6 +2028,41 @@ hipError_t launch_pair_node(wfx_ctx *c, hipStream_t s) {
   if (cfl) c->cfl_nvmax = c->ms.ncl;
   pair_swap<T>(c);
   return hipSuccess;
+}
+
+// Step k by the paired passes from one step record to the next (the adjoint's
+// recomputation, FP64): the nodal arrays, stress and plastic strain are read
+// in `in` and written in `out`, the step's internal force, mass and nodal
+// ratios go to `in`, so that nothing is copied.  first: the step's volumes are
+// not there yet.
+template <typename T>
+hipError_t launch_recorded_step(wfx_ctx *c, int k, bool first, const StepRecord &in, const StepRecord &out,
+                                hipStream_t s) {
+  static_assert(std::is_same<T, double>::value, "the records hold doubles");
+  auto &el = c->e64;
+  DevNode nd = c->nd;
+  double *x_b = c->x_b, *tau = el.tau, *ep = el.pl_strain;
+  void *v_b = c->v_b, *pa_b = c->pa_b;
+  c->nd.x = in.x; c->nd.v = in.v; c->nd.prev_a = in.pa;
+  c->nd.fi = in.fi; c->nd.mdiag = in.m; c->nd.anp_ratio = in.r;
+  c->x_b = out.x; c->v_b = out.v; c->pa_b = out.pa;
+  el.tau = in.tau; el.pl_strain = in.ep;
+  c->fused_tau_out = out.tau; c->fused_pl_out = out.ep;
+  c->fused_write_out = 0;
+  c->fused_read_ud = (k == 0 || c->prm.cfl > 0.0) ? 1 : 0;
+  c->fused_write_ud = c->prm.cfl > 0.0 ? 1 : 0;
+  c->fused_run_first = k == 0 ? 1 : 0;
+  c->fused_run_last = 0;
+  hipError_t e = first ? launch_volumes<T>(c, c->prm.cfl > 0.0, s) : hipSuccess;
+  if (e == hipSuccess) e = launch_pair_element<T>(c, k, s);
+  if (e == hipSuccess) e = launch_pair_node<T>(c, s);
+  c->fused_write_out = c->fused_read_ud = c->fused_write_ud = c->fused_run_first = c->fused_run_last = 1;
+  c->fused_tau_out = c->fused_pl_out = nullptr;
+  el.tau = tau; el.pl_strain = ep;
+  nd.u_dt = c->nd.u_dt;  // the increment's two buffers stay where the step left them
+  c->nd = nd;
+  c->x_b = x_b; c->v_b = v_b; c->pa_b = pa_b;
+  return e;
 }
 
 template <typename T, int BS, bool CFL, bool CT>
@@ -2223,6 +2226,58 @@ hipError_t launch_fused_unpack(wfx_ctx *c, hipStream_t s) {
   return hipGetLastError();
 }
 
+// The nodal arrays change places in every paired step but a run's last, whose
+// node pass updates them in place; the first step's does too where that makes
+// the changes even, so that a run ends in the arrays it started in (a captured
+// run has their addresses in its kernels).
+inline bool step_in_place(bool pair, int k, int nsteps) {
+  return !pair || k + 1 == nsteps || (k == 0 && nsteps % 2 == 0);
+}
+
+// A failed launch leaves the nodal arrays in their places
+template <typename T>
+struct NodalPlaces {
+  wfx_ctx *c;
+  double *x;
+  explicit NodalPlaces(wfx_ctx *c_) : c(c_), x(c_->nd.x) {}
+  ~NodalPlaces() {
+    if (c->nd.x != x) pair_swap<T>(c);
+  }
+};
+
+// Step k of a run of nsteps; have_vol: the step before left this one's
+// volumes (and whether this one leaves the next one's).  rz: the step's
+// reaction record, or null.  ev: an event before each pass (separate passes).
+template <typename T>
+hipError_t launch_run_step(wfx_ctx *c, int k, int nsteps, bool pair, bool &have_vol, void *rz, hipStream_t s,
+                           hipEvent_t *ev) {
+  // the internal force and the element outputs are observed after the run
+  c->fused_write_fi = (k + 1 == nsteps) ? 1 : 0;
+  c->fused_write_out = (k + 1 == nsteps) ? 1 : 0;
+  // the increment is predicted again from v' and prev_a after the first
+  // step, unless each step has its own length
+  c->fused_read_ud = (k == 0 || c->prm.cfl > 0.0) ? 1 : 0;
+  c->fused_write_ud = c->prm.cfl > 0.0 ? 1 : 0;
+  c->fused_run_first = k == 0 ? 1 : 0;
+  c->fused_run_last = k + 1 == nsteps ? 1 : 0;
+  const bool in_place = step_in_place(pair, k, nsteps);
+  hipError_t e = hipSuccess;
+  for (int ph = 1; ph <= 4 && e == hipSuccess; ++ph) {
+    if (ev) e = hipEventRecord(ev[4 * k + ph - 1], s);
+    if (e != hipSuccess || (ph == 1 && have_vol) || (ph == 2 && pair)) continue;
+    c->fused_rz = ph == 4 ? rz : nullptr;
+    if (ph == 1 && pair) e = launch_volumes<T>(c, c->prm.cfl > 0.0, s);
+    else if (ph == 3 && pair) e = launch_pair_element<T>(c, k, s);
+    else if (ph == 4 && !in_place) e = launch_pair_node<T>(c, s);
+    else e = launch_fused_phase<T>(c, ph, k + 1 < nsteps, s, k);
+  }
+  have_vol = !in_place;
+  c->fused_rz = nullptr;
+  c->fused_write_fi = c->fused_write_out = c->fused_read_ud = c->fused_write_ud = 1;
+  c->fused_run_first = c->fused_run_last = 1;
+  return e;
+}
+
 template <typename T>
 hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t s, hipEvent_t *ev) {
   const ReactRecord rec(c, hist, nsteps, sizeof(T));
@@ -2234,49 +2289,15 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
     hipError_t e = launch_cfl_begin<T>(c, s, true);
     if (e != hipSuccess) return e;
   }
-  // Paired passes: the nodal arrays change places in every step but the
-  // last, whose node pass updates them in place; the first step's does too
-  // where that makes the changes even, so that a run ends in the arrays it
-  // started in (a captured run has their addresses in its kernels).  With
-  // events the four passes run separately.
-  const bool pair = c->pair && !ev && !(c->thermal.on && c->thermal.exp_T != 0.0);
-  struct Places {  // a failed launch leaves the arrays in their places
-    wfx_ctx *c;
-    double *x;
-    ~Places() {
-      if (c->nd.x != x) pair_swap<T>(c);
-    }
-  } places{c, c->nd.x};
+  const bool pair = run_paired(c) && !ev;  // with events the four passes run separately
+  const NodalPlaces<T> places(c);
   bool have_vol = false;
   for (int k = 0; k < nsteps; ++k) {
     if (c->contact.on && (c->contact.step_count + k) % 10 == 0) {
       hipError_t e = launch_ext_face_areas(c, s);  // every 10 steps, at the step's start
       if (e != hipSuccess) return e;
     }
-    // the internal force and the element outputs are observed after the run
-    c->fused_write_fi = (k + 1 == nsteps) ? 1 : 0;
-    c->fused_write_out = (k + 1 == nsteps) ? 1 : 0;
-    // the increment is predicted again from v' and prev_a after the first
-    // step, unless each step has its own length
-    c->fused_read_ud = (k == 0 || c->prm.cfl > 0.0) ? 1 : 0;
-    c->fused_write_ud = c->prm.cfl > 0.0 ? 1 : 0;
-    c->fused_run_first = k == 0 ? 1 : 0;
-    c->fused_run_last = k + 1 == nsteps ? 1 : 0;
-    const bool in_place = !pair || k + 1 == nsteps || (k == 0 && nsteps % 2 == 0);
-    hipError_t e = hipSuccess;
-    for (int ph = 1; ph <= 4 && e == hipSuccess; ++ph) {
-      if (ev) e = hipEventRecord(ev[4 * k + ph - 1], s);
-      if (e != hipSuccess || (ph == 1 && have_vol) || (ph == 2 && pair)) continue;
-      c->fused_rz = ph == 4 ? rec.row(k) : nullptr;
-      if (ph == 1 && pair) e = launch_volumes<T>(c, c->prm.cfl > 0.0, s);
-      else if (ph == 3 && pair) e = launch_pair_element<T>(c, k, s);
-      else if (ph == 4 && !in_place) e = launch_pair_node<T>(c, s);
-      else e = launch_fused_phase<T>(c, ph, k + 1 < nsteps, s, k);
-    }
-    have_vol = !in_place;
-    c->fused_rz = nullptr;
-    c->fused_write_fi = c->fused_write_out = c->fused_read_ud = c->fused_write_ud = 1;
-    c->fused_run_first = c->fused_run_last = 1;
+    const hipError_t e = launch_run_step<T>(c, k, nsteps, pair, have_vol, rec.row(k), s, ev);
     if (e != hipSuccess) return e;
     if (ev && k + 1 == nsteps) {
       hipError_t e = hipEventRecord(ev[4 * nsteps], s);

@@ -221,6 +221,9 @@ struct wfx_ctx {
   int *react_base = nullptr, *react_rank = nullptr;
   int react_n = 0, react_rows = 0;
   void *react_ring = nullptr;
+  // where the element pass leaves stress and plastic strain (null: in place;
+  // the adjoint's recomputation writes each step's into its record)
+  void *fused_tau_out = nullptr, *fused_pl_out = nullptr;
   void *fused_rz = nullptr;  // the row the next fused node pass fills (set inside runs)
   // per-node Dirichlet data for the fused node pass, and the three prescribed
   // values per slot

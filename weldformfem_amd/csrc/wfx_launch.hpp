@@ -72,6 +72,23 @@ hipError_t launch_reaction_gather(wfx_ctx *c, double *row, hipStream_t s);
 // the context's ring of recorded rows, allocated once per set of reaction nodes
 int ensure_react_ring(wfx_ctx *c);
 
+// Whether a run takes the paired passes.  Thermal expansion does not: its
+// flat array divides by the masses the paired element pass is still forming.
+inline bool run_paired(const wfx_ctx *c) { return c->pair && !(c->thermal.on && c->thermal.exp_T != 0.0); }
+template <typename T>
+hipError_t launch_run_step(wfx_ctx *c, int k, int nsteps, bool pair, bool &have_vol, void *rz, hipStream_t s,
+                           hipEvent_t *ev);
+extern template hipError_t launch_run_step<double>(wfx_ctx *, int, int, bool, bool &, void *, hipStream_t, hipEvent_t *);
+extern template hipError_t launch_run_step<float>(wfx_ctx *, int, int, bool, bool &, void *, hipStream_t, hipEvent_t *);
+struct StepRecord {  // one step of the adjoint's record
+  double *x, *v, *pa, *fi, *m, *r, *tau, *ep;
+};
+template <typename T>
+hipError_t launch_recorded_step(wfx_ctx *c, int k, bool first, const StepRecord &in, const StepRecord &out,
+                                hipStream_t s);
+extern template hipError_t launch_recorded_step<double>(wfx_ctx *, int, bool, const StepRecord &, const StepRecord &,
+                                                        hipStream_t);
+
 template <typename T> hipError_t launch_vsum0(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_fused_phase(wfx_ctx *c, int phase, int predict, hipStream_t s, int step);
 template <typename T> hipError_t launch_cfl_step(wfx_ctx *c, int step, hipStream_t s);
