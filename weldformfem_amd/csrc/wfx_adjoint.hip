@@ -194,27 +194,47 @@ __device__ __forceinline__ bool first_slot(const SlotSums &q, int o, int slot) {
 struct NodeBack {
   double x[3], v[3], ud[3], pa[3], fib[3], mb, dtb;
 };
-__device__ __forceinline__ void node_reverse(int i, long Ns, long Es, const NodeAdj &P, const double *rec,
-                                             const double *fe, int mask, double hbar, bool cfl, const Bars &in,
-                                             const double (&dx)[3], const double (&dv)[3], NodeBack &B) {
-  const double *fi = rec + 6 * Ns, *vrec = rec + 3 * Ns, *parec = rec + 11 * Ns + 7L * Es;
-  const double m = rec[9 * Ns + i], dt = P.dt, ia = 1.0 / (1.0 - P.alpha);
-  double f[3], xb[3], vb[3], udb[3], pab[3];
+struct NodeVals {
+  double x[3], v[3], fi[3], fe[3], xb[3], vb[3], ud[3], pab[3], pa[3], m, r;
+  int mask, rg;
+};
+__device__ __forceinline__ void load_node_vals(int i, long Ns, long Es, const NodeAdj &P, const double *rec,
+                                               const double *fe, const int *bc_word, const int *rgroup, bool cfl,
+                                               const Bars &in, NodeVals &s) {
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     const long id = d * Ns + i;
-    f[d] = fi[id];
-    xb[d] = in.x[id] + dx[d];
-    vb[d] = in.v[id] + dv[d];
-    udb[d] = in.ud[id];
-    pab[d] = in.pa[id];
+    s.x[d] = rec[id];
+    s.v[d] = rec[3 * Ns + id];
+    s.fi[d] = rec[6 * Ns + id];
+    s.pa[d] = cfl ? rec[11 * Ns + 7 * Es + id] : 0.0;
+    s.fe[d] = P.has_fe ? fe[id] : 0.0;
+    s.xb[d] = in.x[id];
+    s.vb[d] = in.v[id];
+    s.ud[d] = in.ud[id];
+    s.pab[d] = in.pa[id];
   }
+  s.m = rec[9 * Ns + i];
+  s.r = rec[10 * Ns + i];
+  s.mask = bc_word[i] & 7;
+  s.rg = rgroup[i];
+}
+// the sums of one slot: position, velocity (P1) and position (P2)
+__device__ __forceinline__ void load_sums(const SlotSums &q, const double *P1, const double *P2, int at,
+                                          double (&p)[9]) {
+#pragma unroll
+  for (int u = 0; u < 6; ++u) p[u] = P1[u * q.S + at];
+#pragma unroll
+  for (int u = 0; u < 3; ++u) p[6 + u] = P2[u * q.S + at];
+}
+__device__ __forceinline__ void node_reverse(const NodeAdj &P, const NodeVals &s, double hbar, bool cfl,
+                                             const double (&dx)[3], const double (&dv)[3], NodeBack &B) {
+  const double m = s.m, dt = P.dt, ia = 1.0 / (1.0 - P.alpha);
   double mbar = 0.0, dtbar = 0.0;
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const long id = d * Ns + i;
-    const bool free_d = !((mask >> d) & 1);
-    const double vp = vb[d], udp = udb[d], pa_in = pab[d], xbar = xb[d];
+    const bool free_d = !((s.mask >> d) & 1);
+    const double vp = s.vb[d] + dv[d], udp = s.ud[d], pa_in = s.pab[d], xbar = s.xb[d] + dx[d];
     const double vpm = free_d ? vp : 0.0;
     const double vpp = dt * udp + vpm;       // v'' after its boundary values
     const double vppr = free_d ? vpp : 0.0;  // v'' before them
@@ -225,12 +245,12 @@ __device__ __forceinline__ void node_reverse(int i, long Ns, long Es, const Node
     B.v[d] = vppr;
     B.pa[d] = -P.alpha * ia * app;
     const double abar = free_d ? app * ia : 0.0;
-    const double a = ((P.has_fe ? fe[id] : 0.0) - f[d]) / m;
+    const double a = (s.fe[d] - s.fi[d]) / m;
     B.fib[d] = -abar / m + (d == 2 ? hbar : 0.0);
     mbar -= abar * a / m;
     if (cfl) {
-      const double ac = ia * ((free_d ? a : 0.0) - P.alpha * parec[id]);
-      const double vv = free_d ? vrec[id] + P.gamma * dt * ac : vrec[id];  // an imposed v' is its value
+      const double ac = ia * ((free_d ? a : 0.0) - P.alpha * s.pa[d]);
+      const double vv = free_d ? s.v[d] + P.gamma * dt * ac : s.v[d];  // an imposed v' is its value
       dtbar += udp * (vv + 2.0 * (0.5 - P.beta) * dt * ac) + vpm * (1.0 - P.gamma) * ac +
                vppr * P.gamma * ac + xbar * 2.0 * P.beta * dt * ac;
     }
@@ -415,7 +435,7 @@ __global__ __launch_bounds__(kCluster) void a_element(
   const int4 cd = ca.desc[c];
   const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;
   const long Es = E, Ns = N;
-  const double *x = rec, *v = rec + 3 * Ns, *r = rec + 10 * Ns, *tau = rec + 11 * Ns, *ep = tau + 6 * Es;
+  const double *tau = rec + 11 * Ns, *ep = tau + 6 * Es;
   const int e = e0 + min(t, ne - 1);
   int ls[NN];
   load_lslot<NN>(ca.lslot + (long)e * NN, ls);
@@ -427,34 +447,39 @@ __global__ __launch_bounds__(kCluster) void a_element(
     o[k] = q.nsl_off[node[k]];
     n[k] = q.nsl_off[node[k] + 1] - o[k];
   }
+  // every slot's loads before the first slot's arithmetic: the nodal values
+  // and the first four of the later step's element sums (clusters in order)
+  NodeVals nv[kSl];
+  double p[kSl][4][9];
+#pragma unroll
+  for (int k = 0; k < kSl; ++k) {
+    load_node_vals(node[k], Ns, Es, P, rec, fe, bc_word, rgroup, dtb_n != nullptr, in, nv[k]);
+    if (pending)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) load_sums(q, P1in, P2in, slot_at(q, o[k] + min(g, n[k] - 1)), p[k][g]);
+  }
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
     const int j = t + k * kCluster, i = node[k];
     const bool own = j < M && first_slot(q, o[k], s0 + min(j, M - 1));
     double dx[3] = {0.0, 0.0, 0.0}, dv[3] = {0.0, 0.0, 0.0};
-    if (pending)  // the later step's element sums, clusters in order
-      for (int h = 0; h < n[k]; h += 4) {
-        double p[4][9];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int at = slot_at(q, o[k] + min(h + g, n[k] - 1));
-#pragma unroll
-          for (int u = 0; u < 6; ++u) p[g][u] = P1in[u * q.S + at];
-#pragma unroll
-          for (int u = 0; u < 3; ++u) p[g][6 + u] = P2in[u * q.S + at];
-        }
+    if (pending)
+      for (int h = 0;;) {
 #pragma unroll
         for (int g = 0; g < 4; ++g)
           if (h + g < n[k])
 #pragma unroll
             for (int u = 0; u < 3; ++u) {
-              dx[u] += p[g][u] + p[g][6 + u];
-              dv[u] += p[g][3 + u];
+              dx[u] += p[k][g][u] + p[k][g][6 + u];
+              dv[u] += p[k][g][3 + u];
             }
+        h += 4;
+        if (h >= n[k]) break;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) load_sums(q, P1in, P2in, slot_at(q, o[k] + min(h + g, n[k] - 1)), p[k][g]);
       }
-    const int rg = rgroup[i];
     NodeBack B;
-    node_reverse(i, Ns, Es, P, rec, fe, bc_word[i] & 7, rg >= 0 ? hbar_k[rg] : 0.0, dtb_n != nullptr, in, dx, dv, B);
+    node_reverse(P, nv[k], nv[k].rg >= 0 ? hbar_k[nv[k].rg] : 0.0, dtb_n != nullptr, dx, dv, B);
     if (own) {
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
@@ -469,11 +494,11 @@ __global__ __launch_bounds__(kCluster) void a_element(
     }
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      lds[d * cap + j] = x[d * Ns + i];
-      lds[(3 + d) * cap + j] = v[d * Ns + i];
+      lds[d * cap + j] = nv[k].x[d];
+      lds[(3 + d) * cap + j] = nv[k].v[d];
       lds[(7 + d) * cap + j] = B.fib[d];
     }
-    lds[6 * cap + j] = r[i];
+    lds[6 * cap + j] = nv[k].r;
   }
   __syncthreads();
   adj::ElemIn<NN> ei;
@@ -555,22 +580,42 @@ __global__ __launch_bounds__(kCluster) void a_volume(int E, int N, ClusterArgs c
   int ls[NN];
   load_lslot<NN>(ca.lslot + (long)e * NN, ls);
   double vb = volb[e];
+  // as in a_element: every slot's loads first
+  int node[kSl], o[kSl], n[kSl];
+#pragma unroll
+  for (int k = 0; k < kSl; ++k) node[k] = ca.snode[s0 + min(t + k * kCluster, M - 1)];
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
-    const int j = t + k * kCluster, i = ca.snode[s0 + min(j, M - 1)];
-    const int o = q.nsl_off[i], n = q.nsl_off[i + 1] - o;
-    double rs = 0.0;
-    for (int h = 0; h < n; h += 4) {
-      double p[4];
+    o[k] = q.nsl_off[node[k]];
+    n[k] = q.nsl_off[node[k] + 1] - o[k];
+  }
+  double x[kSl][3], v0[kSl], mbk[kSl], ra[kSl], p[kSl][4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) p[g] = P1[6 * q.S + slot_at(q, o + min(h + g, n - 1))];
+  for (int k = 0; k < kSl; ++k) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) x[k][d] = rec[d * Ns + node[k]];
+    v0[k] = vsum0[node[k]];
+    mbk[k] = mb[node[k]];
+    ra[k] = rho_avg[node[k]];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) p[k][g] = P1[6 * q.S + slot_at(q, o[k] + min(g, n[k] - 1))];
+  }
+#pragma unroll
+  for (int k = 0; k < kSl; ++k) {
+    const int j = t + k * kCluster;
+    double rs = 0.0;
+    for (int h = 0;;) {
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        if (h + g < n) rs += p[g];
+        if (h + g < n[k]) rs += p[k][g];
+      h += 4;
+      if (h >= n[k]) break;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) p[k][g] = P1[6 * q.S + slot_at(q, o[k] + min(h + g, n[k] - 1))];
     }
 #pragma unroll
-    for (int d = 0; d < 3; ++d) lds[d * cap + j] = rec[d * Ns + i];
-    lds[3 * cap + j] = rs / vsum0[i] + mb[i] * rho_avg[i] / NN;
+    for (int d = 0; d < 3; ++d) lds[d * cap + j] = x[k][d];
+    lds[3 * cap + j] = rs / v0[k] + mbk[k] * ra[k] / NN;
   }
   __syncthreads();
   double X[NN][3];
