@@ -384,10 +384,10 @@ __global__ void k_law_temps(int E, int law, const double *Te, double T_t, double
 // element-node values in LDS (kEntStride), to P[R][S] (the element pass's sums)
 template <int NN, int R>
 __device__ __forceinline__ void slot_sums(const unsigned char *lds, const ClusterArgs &ca, const SlotSums &q,
-                                          int c, const int4 &cd, double *P) {
-  const int s0 = cd.y, M = cd.z >> 16;
-  const uint16_t *lo = ca.goff + s0 + c;
-  const uint2 *en = ca.ent + cd.w;
+                                          const ClusterDesc &cd, double *P) {
+  const int s0 = cd.s0, M = cd.em >> 16;
+  const uint16_t *lo = ca.goff + cd.goff;
+  const uint2 *en = ca.ent + cd.ent;
   for (int j = threadIdx.x; j < M; j += kCluster) {
     const int at = q.nm ? q.spos[s0 + j] : s0 + j;
     double acc[R];
@@ -432,13 +432,13 @@ __global__ __launch_bounds__(kCluster) void a_element(
   __shared__ __align__(16) double lds[6 * kEntStride(NN) + NN * kCluster + 1];
   static_assert(10 * cap <= 6 * kEntStride(NN) + NN * kCluster, "the staged slots fit");
   const int c = xcd_block(), t = threadIdx.x;
-  const int4 cd = ca.desc[c];
-  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;
+  const ClusterDesc cd = ca.desc[c];
+  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;
   const long Es = E, Ns = N;
   const double *tau = rec + 11 * Ns, *ep = tau + 6 * Es;
   const int e = e0 + min(t, ne - 1);
   int ls[NN];
-  load_lslot<NN>(ca.lslot + (long)e * NN, ls);
+  load_lslot<NN>(ca.lslot + (long)(cd.lslot + min(t, ne - 1)) * NN, ls);
   int node[kSl], o[kSl], n[kSl];
 #pragma unroll
   for (int k = 0; k < kSl; ++k) node[k] = ca.snode[s0 + min(t + k * kCluster, M - 1)];
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(kCluster) void a_element(
   }
   if (t < 7) lds[t * kEntStride(NN) + NN * kCluster] = 0.0;
   __syncthreads();
-  slot_sums<NN, 7>(reinterpret_cast<const unsigned char *>(lds), ca, q, c, cd, P1);
+  slot_sums<NN, 7>(reinterpret_cast<const unsigned char *>(lds), ca, q, cd, P1);
 }
 
 // The reverse step's second kernel: the nodes' volume cotangents w (the ratio
@@ -573,12 +573,12 @@ __global__ __launch_bounds__(kCluster) void a_volume(int E, int N, ClusterArgs c
   constexpr int cap = slot_cap(NN), kSl = kSlotsPerThread<NN>;
   __shared__ __align__(16) double lds[2 * kEntStride(NN) + NN * kCluster + 1];
   const int c = xcd_block(), t = threadIdx.x;
-  const int4 cd = ca.desc[c];
-  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;
+  const ClusterDesc cd = ca.desc[c];
+  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;
   const long Ns = N;
   const int e = e0 + min(t, ne - 1);
   int ls[NN];
-  load_lslot<NN>(ca.lslot + (long)e * NN, ls);
+  load_lslot<NN>(ca.lslot + (long)(cd.lslot + min(t, ne - 1)) * NN, ls);
   double vb = volb[e];
   // as in a_element: every slot's loads first
   int node[kSl], o[kSl], n[kSl];
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(kCluster) void a_volume(int E, int N, ClusterArgs c
   }
   if (t < 3) lds[t * kEntStride(NN) + NN * kCluster] = 0.0;
   __syncthreads();
-  slot_sums<NN, 3>(reinterpret_cast<const unsigned char *>(lds), ca, q, c, cd, P2);
+  slot_sums<NN, 3>(reinterpret_cast<const unsigned char *>(lds), ca, q, cd, P2);
 }
 
 // parameter gradients: one work-group per parameter row, fixed order; for

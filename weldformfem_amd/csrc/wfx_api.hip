@@ -8,6 +8,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/wfx.h"
@@ -175,38 +176,97 @@ static int scratch_address(double **out) {
   return WFX_OK;
 }
 
-// The plan's slot entries as the element pass reads them: groups of four LDS
-// byte offsets, so that the pass extracts an address with one instruction and
-// adds without a test per entry.
-struct EntryTables {
-  std::vector<int4> desc;
-  std::vector<uint16_t> goff;
+// The plan's tables as the cluster passes read them.  The slot entries become
+// groups of four LDS byte offsets, so that the pass extracts an address with
+// one instruction and adds without a test per entry.  A cluster's entries
+// follow from its elements' slot indices, and clusters with equal indices
+// share both (the bricks of a structured block have a handful of shapes), as
+// clusters whose nodes differ by a constant share the node pattern: the
+// tables then stay in the caches instead of being streamed every step.
+// Element pass and volume pass, us, before / with sharing: 4M FP64 hexahedra
+// 282 + 51.5 / 258 + 45.9, 1.1M FP32-mixed 55.7 + 17.1 / 52.5 + 12.7; 1.2M
+// tetrahedra of an irregular mesh, which share nothing, 61 + 12.3 / 60 + 10.7.
+struct ClusterTables {
+  std::vector<ClusterDesc> desc;
+  std::vector<uint16_t> goff, lslot;
   std::vector<uint2> ent;
+  std::vector<int> nrel;
 };
-static EntryTables entry_tables(const wfx_ctx *c, const ClusterPlan &plan) {
-  EntryTables t;
+static uint64_t mix64(uint64_t h, uint64_t v) {
+  h = (h ^ v) * 0x9e3779b97f4a7c15ULL;
+  return h ^ (h >> 29);
+}
+static ClusterTables cluster_tables(const wfx_ctx *c, const ClusterPlan &plan) {
+  ClusterTables t;
   const int C = plan.clusters(), n = c->n;
   const unsigned es = c->precision == WFX_FP64 ? 8 : 4, zero = (unsigned)(n * kCluster) * es;
   t.desc.resize(C);
-  t.goff.resize(plan.slots() + C);
-  t.ent.reserve((size_t)c->E * n / 3);
+  // clusters seen so far by the hash of their tables
+  std::unordered_multimap<uint64_t, int> topo, nodes;
+  const auto shared = [](const std::unordered_multimap<uint64_t, int> &seen, uint64_t h, auto &&same) {
+    const auto r = seen.equal_range(h);
+    for (auto it = r.first; it != r.second; ++it)
+      if (same(it->second)) return it->second;
+    return -1;
+  };
   for (int k = 0; k < C; ++k) {
-    const int e0 = plan.eoff[k], s0 = plan.sbase[k], ne = plan.eoff[k + 1] - e0, m = plan.sbase[k + 1] - s0;
-    const size_t g0 = t.ent.size();
-    t.desc[k] = make_int4(e0, s0, ne | m << 16, (int)g0);
-    const uint16_t *lo = plan.loff.data() + s0 + k, *en = plan.ent.data() + (size_t)e0 * n;
-    for (int j = 0; j < m; ++j) {
-      t.goff[s0 + k + j] = (uint16_t)(t.ent.size() - g0);
-      for (int q = lo[j]; q < lo[j + 1]; q += 4) {
-        unsigned v[4];
-        for (int h = 0; h < 4; ++h) {
-          const int e = q + h < lo[j + 1] ? en[q + h] : -1;
-          v[h] = e < 0 ? zero : (unsigned)((e & 7) * kCluster + (e >> 3)) * es;
-        }
-        t.ent.push_back(make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16));
-      }
+    ClusterDesc &d = t.desc[k];
+    const int ne = plan.eoff[k + 1] - plan.eoff[k], m = plan.sbase[k + 1] - plan.sbase[k];
+    d.e0 = plan.eoff[k];
+    d.s0 = plan.sbase[k];
+    d.em = ne | m << 16;
+    const uint16_t *ls = plan.lslot.data() + (size_t)d.e0 * n;
+    uint64_t h = (uint64_t)d.em;
+    for (int q = 0; q < ne * n; q += 4) {
+      uint64_t w;
+      std::memcpy(&w, ls + q, 8);
+      h = mix64(h, w);
     }
-    t.goff[s0 + k + m] = (uint16_t)(t.ent.size() - g0);
+    int o = shared(topo, h, [&](int r) {
+      return t.desc[r].em == d.em &&
+             std::memcmp(plan.lslot.data() + (size_t)t.desc[r].e0 * n, ls, (size_t)ne * n * 2) == 0;
+    });
+    if (o >= 0) {
+      d.goff = t.desc[o].goff;
+      d.ent = t.desc[o].ent;
+      d.lslot = t.desc[o].lslot;
+    } else {
+      topo.emplace(h, k);
+      d.goff = (int)t.goff.size();
+      d.ent = (int)t.ent.size();
+      d.lslot = (int)(t.lslot.size() / n);
+      t.lslot.insert(t.lslot.end(), ls, ls + (size_t)ne * n);
+      const uint16_t *lo = plan.loff.data() + d.s0 + k, *en = plan.ent.data() + (size_t)d.e0 * n;
+      for (int j = 0; j < m; ++j) {
+        t.goff.push_back((uint16_t)(t.ent.size() - d.ent));
+        for (int q = lo[j]; q < lo[j + 1]; q += 4) {
+          unsigned v[4];
+          for (int i = 0; i < 4; ++i) {
+            const int e = q + i < lo[j + 1] ? en[q + i] : -1;
+            v[i] = e < 0 ? zero : (unsigned)((e & 7) * kCluster + (e >> 3)) * es;
+          }
+          t.ent.push_back(make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16));
+        }
+      }
+      t.goff.push_back((uint16_t)(t.ent.size() - d.ent));
+    }
+    const int *sn = plan.snode.data() + d.s0;
+    d.node0 = sn[0];
+    h = (uint64_t)m;
+    for (int j = 0; j < m; ++j) h = mix64(h, (uint64_t)(uint32_t)(sn[j] - sn[0]));
+    o = shared(nodes, h, [&](int r) {
+      if (t.desc[r].em >> 16 != m) return false;
+      for (int j = 0; j < m; ++j)
+        if (t.nrel[t.desc[r].nrel + j] != sn[j] - sn[0]) return false;
+      return true;
+    });
+    if (o >= 0) {
+      d.nrel = t.desc[o].nrel;
+    } else {
+      nodes.emplace(h, k);
+      d.nrel = (int)t.nrel.size();
+      for (int j = 0; j < m; ++j) t.nrel.push_back(sn[j] - sn[0]);
+    }
   }
   t.ent.resize(t.ent.size() + 8, make_uint2(0, 0));  // a slot's first six groups are read whatever their number
   return t;
@@ -268,10 +328,10 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     free_all(c);
     return WFX_ERR_STATE;
   }
-  const EntryTables et = entry_tables(c, plan);
-  A(c->ms.cl_desc, c->ms.ncl) A(c->ms.cl_goff, c->ms.nslot + c->ms.ncl)
-  A(c->ms.cl_ent, et.ent.size()) A(c->ms.nsl_off, N + 1)
-  A(c->ms.cl_snode, c->ms.nslot) A(c->ms.cl_lslot, n * E)
+  const ClusterTables ct = cluster_tables(c, plan);
+  A(c->ms.cl_desc, c->ms.ncl) A(c->ms.cl_goff, ct.goff.size()) A(c->ms.cl_ent, ct.ent.size())
+  A(c->ms.cl_lslot, ct.lslot.size()) A(c->ms.cl_nrel, ct.nrel.size()) A(c->ms.nsl_off, N + 1)
+  A(c->ms.cl_snode, c->ms.nslot)
   const int pw = pair_width(c, plan);
   c->pair = pw > 0;
   if (c->precision == WFX_FP64) A(c->ms.nsl, c->ms.nslot)
@@ -321,17 +381,20 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_loc, c->nodel_loc_h.data(), n * E * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_offset, c->nodel_offset_h.data(), N * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.nodel_count, c->nodel_count_h.data(), N * sizeof(int), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_desc, et.desc.data(), et.desc.size() * sizeof(int4), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_goff, et.goff.data(), et.goff.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_ent, et.ent.data(), et.ent.size() * sizeof(uint2), hipMemcpyHostToDevice));
+  const auto put = [](auto *dst, const auto &v) {
+    return hipMemcpy(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice);
+  };
+  WFX_CHECK_HIP(put(c->ms.cl_desc, ct.desc));
+  WFX_CHECK_HIP(put(c->ms.cl_goff, ct.goff));
+  WFX_CHECK_HIP(put(c->ms.cl_ent, ct.ent));
+  WFX_CHECK_HIP(put(c->ms.cl_lslot, ct.lslot));
+  WFX_CHECK_HIP(put(c->ms.cl_nrel, ct.nrel));
   WFX_CHECK_HIP(hipMemcpy(c->ms.nsl_off, plan.nsl_off.data(), plan.nsl_off.size() * sizeof(int), hipMemcpyHostToDevice));
   if (c->ms.nsl)
     WFX_CHECK_HIP(hipMemcpy(c->ms.nsl, plan.nsl.data(), plan.nsl.size() * sizeof(int), hipMemcpyHostToDevice));
   if (c->ms.spos)
     WFX_CHECK_HIP(hipMemcpy(c->ms.spos, plan.spos.data(), plan.spos.size() * sizeof(int), hipMemcpyHostToDevice));
   WFX_CHECK_HIP(hipMemcpy(c->ms.cl_snode, plan.snode.data(), plan.snode.size() * sizeof(int), hipMemcpyHostToDevice));
-  WFX_CHECK_HIP(hipMemcpy(c->ms.cl_lslot, plan.lslot.data(), plan.lslot.size() * sizeof(uint16_t),
-                          hipMemcpyHostToDevice));
   if (c->pair) {
     hipLaunchKernelGGL(k_pair_tables, dim3((unsigned)((c->ms.nslot + 255) / 256)), dim3(256), 0, nullptr, c->ms.nslot,
                        pw, c->ms.cl_snode, c->ms.spos, c->ms.nsl_off, c->ms.nodel_offset, c->ms.nodel_count,

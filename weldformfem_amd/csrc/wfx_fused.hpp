@@ -995,10 +995,10 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   T *lf = reinterpret_cast<T *>(lds_raw);
   const SlotLds<T, NN> L(lds_raw);
   const int c = xcd_block(), t = threadIdx.x;
-  const int4 cd = ca.desc[c];
-  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
-  const uint16_t *lo = ca.goff + s0 + c;
-  const uint2 *en = ca.ent + cd.w;  // the cluster's entry groups
+  const ClusterDesc cd = ca.desc[c];
+  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;  // M <= slot_cap(NN), checked at set-up
+  const uint16_t *lo = ca.goff + cd.goff;
+  const uint2 *en = ca.ent + cd.ent;  // the cluster's entry groups
   // the nodes of this thread's slots t and t + kCluster: first, as the
   // staging loads depend on them
   constexpr int kSl = kSlotsPerThread<NN>;
@@ -1028,7 +1028,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
       ps.slot[k] = q;
       mine[k] = j < M;
     } else {
-      sn[k] = ca.snode[q];
+      sn[k] = cd.node0 + ca.nrel[cd.nrel + min(j, M - 1)];
     }
   }
   if constexpr (PAIR) ps.entries(pr, 0);
@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   }
   int ls[NN];
   const int my_e = e0 + min(t, ne - 1);
-  load_lslot<NN>(ca.lslot + (long)my_e * NN, ls);
+  load_lslot<NN>(ca.lslot + (long)(cd.lslot + min(t, ne - 1)) * NN, ls);
   ElemState<T> S;
   if constexpr (PAIR) __builtin_amdgcn_sched_barrier(0);
   else load_elem_state<T>(my_e, E, tau_in, eps_io, pl_in, sy0, He, S);
@@ -1206,16 +1206,16 @@ __global__ __launch_bounds__(kCluster) void f1_cluster(int E, ClusterArgs ca, co
   __shared__ double lx[3 * cap];
   __shared__ int lnode[cap];
   const int c = xcd_block(), t = threadIdx.x;
-  const int4 cd = ca.desc[c];
-  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
+  const ClusterDesc cd = ca.desc[c];
+  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;  // M <= slot_cap(NN), checked at set-up
   // every load is issued unconditionally (threads past the cluster's
   // elements or slots repeat its last one), as in the element pass
   constexpr int kSl = kSlotsPerThread<NN>;
   int sn[kSl];
 #pragma unroll
-  for (int k = 0; k < kSl; ++k) sn[k] = ca.snode[s0 + min(t + k * kCluster, M - 1)];
+  for (int k = 0; k < kSl; ++k) sn[k] = cd.node0 + ca.nrel[cd.nrel + min(t + k * kCluster, M - 1)];
   int ls[NN];
-  load_lslot<NN>(ca.lslot + (long)(e0 + min(t, ne - 1)) * NN, ls);
+  load_lslot<NN>(ca.lslot + (long)(cd.lslot + min(t, ne - 1)) * NN, ls);
   double sx[kSl][3];
 #pragma unroll
   for (int k = 0; k < kSl; ++k)
@@ -1682,14 +1682,14 @@ __global__ __launch_bounds__(slot_cap(NN)) void f41_cluster(
     }
   }
   const int c = xcd_block(nb), t = threadIdx.x;
-  const int4 cd = ca.desc[c];
-  const int e0 = cd.x, s0 = cd.y, ne = cd.z & 0xffff, M = cd.z >> 16;  // M <= slot_cap(NN), checked at set-up
+  const ClusterDesc cd = ca.desc[c];
+  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;  // M <= slot_cap(NN), checked at set-up
   // as in the element pass every load is issued unconditionally: threads past
   // the cluster's slots or elements repeat its last one and store nothing
   const int4 rec = pr.rec[s0 + min(t, M - 1)];
   const int word = pr.sbc[s0 + min(t, M - 1)];
   int ls[NN];
-  load_lslot<NN>(ca.lslot + (long)(e0 + min(t, ne - 1)) * NN, ls);
+  load_lslot<NN>(ca.lslot + (long)(cd.lslot + min(t, ne - 1)) * NN, ls);
   const int i = rec.x;
   const bool own = t < M && rec.w < 0;
   NodeIn<T, CONTACT> st;

@@ -137,6 +137,16 @@ struct DevNode {
   double *rho_avg = nullptr;    // fused path: mean density of the node's elements
 };
 
+// One element cluster on the device: its elements and slots, and the start of
+// its tables (in groups, offsets, elements and nodes)
+struct alignas(32) ClusterDesc {
+  int e0, s0;     // first stored element, first slot
+  int em;         // elements | slots << 16
+  int goff, ent;  // group offsets and entry groups
+  int lslot;      // elements' slot indices
+  int node0, nrel;  // first slot's node, the slots' nodes less it
+};
+
 struct DevMesh {
   int *elnod = nullptr;
   int *nodel = nullptr, *nodel_loc = nullptr, *nodel_offset = nullptr, *nodel_count = nullptr;
@@ -149,17 +159,19 @@ struct DevMesh {
   // partial sums are stored there, node-major)
   int ncl = 0;
   long nslot = 0;
-  // [C] {first element, first slot, elements | slots << 16, first entry group};
-  // per cluster its slots + 1 group offsets (cluster c at its first slot + c);
-  // the entry groups, four LDS byte offsets of element-node values each
-  // (kEntStride), a slot's last one filled up with the zero cell's
-  int4 *cl_desc = nullptr;
+  // [C] where each cluster's elements, slots and tables are; per table set of
+  // m slots its m + 1 group offsets; the entry groups, four LDS byte offsets
+  // of element-node values each (kEntStride), a slot's last one filled up with
+  // the zero cell's; each element's nodes as slot indices [n]; the slots'
+  // nodes less the cluster's first slot's.  Clusters with the same tables
+  // share them.
+  ClusterDesc *cl_desc = nullptr;
   uint16_t *cl_goff = nullptr;
   uint2 *cl_ent = nullptr;
-  int *nsl_off = nullptr, *nsl = nullptr, *spos = nullptr;
-  // slot -> node [S]; each stored element's nodes as slot indices of its cluster [E][n]
-  int *cl_snode = nullptr;
   uint16_t *cl_lslot = nullptr;
+  int *cl_nrel = nullptr;
+  int *nsl_off = nullptr, *nsl = nullptr, *spos = nullptr;
+  int *cl_snode = nullptr;  // slot -> node [S]
   // paired passes (small meshes): per slot {node, its first position in the
   // node's slot list, the list's length, the node's element count | (first
   // slot of the node) << 31}, and the node's stored elements in CSR order,
