@@ -49,10 +49,33 @@ uint64_t brick_key(const uint64_t q[3], const int bits[3]) {
   return ((spread3(b[0]) | (spread3(b[1]) << 1) | (spread3(b[2]) << 2)) << sh) | local;
 }
 
+// Distinct nodes of stored elements [q0, q1)
+class NodeCounter {
+ public:
+  NodeCounter(int N, int n, const int *elnod, const std::vector<int> &s2o) : n_(n), elnod_(elnod), s2o_(s2o), seen_(N, 0) {}
+  int operator()(int q0, int q1) {
+    ++mark_;
+    int cnt = 0;
+    for (int q = q0; q < q1; ++q) {
+      const int *en = elnod_ + (size_t)s2o_[q] * n_;
+      for (int a = 0; a < n_; ++a) {
+        cnt += seen_[en[a]] != mark_;
+        seen_[en[a]] = mark_;
+      }
+    }
+    return cnt;
+  }
+
+ private:
+  int n_, mark_ = 0;
+  const int *elnod_;
+  const std::vector<int> &s2o_;
+  std::vector<int> seen_;
+};
+
 // Slot tables of clusters [c0, c1): per cluster its sorted (node, t*8 + a)
 // pairs give the slots (distinct nodes) and the entries grouped by slot.
-// With write = false only the slot counts m[c] are taken.
-void slot_tables(int n, const int *elnod, ClusterPlan &p, int c0, int c1, bool write, std::vector<int> &m) {
+void slot_tables(int n, const int *elnod, ClusterPlan &p, int c0, int c1) {
   std::vector<uint64_t> pairs;
   for (int c = c0; c < c1; ++c) {
     const int e0 = p.eoff[c], ne = p.eoff[c + 1] - e0;
@@ -62,13 +85,6 @@ void slot_tables(int n, const int *elnod, ClusterPlan &p, int c0, int c1, bool w
       for (int a = 0; a < n; ++a) pairs[(size_t)t * n + a] = ((uint64_t)en[a] << 16) | (uint64_t)(t * 8 + a);
     }
     std::sort(pairs.begin(), pairs.end());
-    if (!write) {
-      int cnt = 0;
-      for (size_t k = 0; k < pairs.size(); ++k)
-        if (k == 0 || (pairs[k] >> 16) != (pairs[k - 1] >> 16)) ++cnt;
-      m[c] = cnt;
-      continue;
-    }
     uint16_t *lo = p.loff.data() + p.sbase[c] + c;
     uint16_t *en = p.ent.data() + (size_t)e0 * n;
     int *sn = p.snode.data() + p.sbase[c];
@@ -102,9 +118,69 @@ void parallel_ranges(int count, F &&f) {
   for (auto &t : th) t.join();
 }
 
+// A block of n[0] x n[1] x n[2] cells in k[0] x k[1] x k[2] bricks whose edges
+// differ by at most one cell, each brick a cluster.
+struct BlockSplit {
+  int n[3], k[3];
+  uint64_t key(const uint64_t q[3]) const {
+    uint64_t b[3];
+    for (int d = 0; d < 3; ++d) b[d] = q[d] * (uint64_t)k[d] / (uint64_t)n[d];
+    return spread3(b[0]) | (spread3(b[1]) << 1) | (spread3(b[2]) << 2);
+  }
+  double clusters() const { return (double)k[0] * k[1] * k[2]; }
+  double slots() const { return (double)(n[0] + k[0]) * (n[1] + k[1]) * (n[2] + k[2]); }
+};
+
+// The split with the least traffic: a slot's nodal values, per row of a
+// brick's nodes along x the ends of its cache lines (worth eight slots), and
+// per cluster the lanes its elements leave idle.  Step of 151 x 119 x 61
+// hexahedra in FP64 by brick: 30.2 x 4 x 2 cells (this rule) 152.4 us, 15.1 x 4 x
+// 3.8 153.4, 7.9 x 7.9 x 3.8 153.9; 200 x 200 x 100 without the rows' weight
+// (11.8 x 5.9 x 3) 641, with it 585.
+BlockSplit split_block(const int n[3], int cs, int cap) {
+  BlockSplit best{{n[0], n[1], n[2]}, {n[0], n[1], n[2]}};  // one cell each
+  double least = 1e300;
+  for (int bx = 1; bx <= std::min(n[0], cs); ++bx)
+    for (int by = 1; by <= std::min(n[1], cs / bx); ++by)
+      for (int bz = 1; bz <= std::min(n[2], cs / (bx * by)); ++bz) {
+        if ((bx + 1) * (by + 1) * (bz + 1) > cap) continue;
+        const BlockSplit s{{n[0], n[1], n[2]}, {(n[0] + bx - 1) / bx, (n[1] + by - 1) / by, (n[2] + bz - 1) / bz}};
+        const double rows = (double)s.k[0] * (n[1] + s.k[1]) * (n[2] + s.k[2]);
+        const double cost = s.slots() + 8.0 * rows + 100.0 * s.clusters();
+        if (cost < least) {
+          least = cost;
+          best = s;
+        }
+      }
+  return best;
+}
+
+// Clusters and slots of stored elements [a, b) cut into runs of cs, runs of
+// more than cap nodes halved until none is
+void count_runs(NodeCounter &nodes, int a, int b, int cs, int cap, double &clusters, double &slots) {
+  clusters = slots = 0.0;
+  std::vector<std::pair<int, int>> todo;
+  for (int q = a; q < b; q += cs) {
+    todo.push_back({q, std::min(b, q + cs)});
+    while (!todo.empty()) {
+      const auto [q0, q1] = todo.back();
+      todo.pop_back();
+      const int m = nodes(q0, q1);
+      if (m > cap) {
+        todo.push_back({q0, q0 + (q1 - q0) / 2});
+        todo.push_back({q0 + (q1 - q0) / 2, q1});
+      } else {
+        clusters += 1.0;
+        slots += m;
+      }
+    }
+  }
+}
+
 }  // namespace
 
-int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs, ClusterPlan &p) {
+int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs, ClusterPlan &p,
+                  bool even) {
   // connected components (elements sharing a node), ordered by their first element
   std::vector<int> parent(N);
   std::iota(parent.begin(), parent.end(), 0);
@@ -153,6 +229,7 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
   p.s2o.resize(E);
   p.eoff.assign(1, 0);
   std::vector<std::pair<uint64_t, int>> key;
+  NodeCounter nodes(N, n, elnod, p.s2o);
   for (int k = 0; k < ncomp; ++k) {
     const int a = coff[k], b = coff[k + 1];
     double lo[3] = {1e300, 1e300, 1e300}, hs = 0.0;
@@ -165,12 +242,14 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
     if (!(h > 0.0) || !std::isfinite(h)) h = 1.0;
     key.resize(b - a);
     std::vector<uint64_t> cells(b - a);
+    int ext[3] = {0, 0, 0};  // cells of the component's bounding block
     const int nobits[3] = {0, 0, 0};
     for (int q = a; q < b; ++q) {
       const int e = byc[q];
       const uint64_t qc[3] = {quantize(cen[3 * (size_t)e], lo[0], h), quantize(cen[3 * (size_t)e + 1], lo[1], h),
                               quantize(cen[3 * (size_t)e + 2], lo[2], h)};
       cells[q - a] = brick_key(qc, nobits);
+      for (int d = 0; d < 3; ++d) ext[d] = std::max(ext[d], (int)qc[d] + 1);
     }
     // a brick holds about cs elements: 2^bits cells of the component's
     // occupancy (elements per occupied cell), half of the bits along x so
@@ -192,8 +271,34 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
       const int r = std::min(b, q + cs);
       for (int t = q; t < r; ++t) p.s2o[t] = key[t - a].second;
       std::sort(p.s2o.begin() + q, p.s2o.begin() + r);  // ascending original order within a cluster
-      p.eoff.push_back(r);
     }
+    // A block whose edges are no multiples of the brick's leaves runs that
+    // straddle bricks (151 x 119 x 61 cells: 219 elements a cluster after the
+    // halving, 1.91 slots an element).  Such a block is split evenly instead
+    // when that takes fewer slots and clusters, a cluster counted as the work
+    // of its 256 elements: FP64 step of that block 158.5 -> 149.7 us, 48 blocks
+    // of 6 to 40 cells a side 102 -> 96.8; where the runs are the better cut
+    // they win by 1% (100 x 99 x 51, 200 x 200 x 100).
+    if (even && b - a > cs && per_cell == 1.0 && (double)ext[0] * ext[1] * ext[2] == (double)(b - a)) {
+      double clusters, slots;
+      count_runs(nodes, a, b, cs, slot_cap(n), clusters, slots);
+      const BlockSplit sp = split_block(ext, cs, slot_cap(n));
+      if (sp.slots() + 250.0 * sp.clusters() < slots + 250.0 * clusters) {
+        for (int q = a; q < b; ++q) {
+          const int e = byc[q];
+          const uint64_t qc[3] = {quantize(cen[3 * (size_t)e], lo[0], h), quantize(cen[3 * (size_t)e + 1], lo[1], h),
+                                  quantize(cen[3 * (size_t)e + 2], lo[2], h)};
+          key[q - a] = {sp.key(qc), e};
+        }
+        std::sort(key.begin(), key.end());  // ascending original order within a brick
+        for (int q = a; q < b; ++q) {
+          p.s2o[q] = key[q - a].second;
+          if (q + 1 == b || key[q + 1 - a].first != key[q - a].first) p.eoff.push_back(q + 1);
+        }
+        continue;
+      }
+    }
+    for (int q = a; q < b; q += cs) p.eoff.push_back(std::min(b, q + cs));
   }
   p.o2s.resize(E);
   for (int s = 0; s < E; ++s) p.o2s[p.s2o[s]] = s;
@@ -203,7 +308,10 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
   for (;;) {
     const int C = p.clusters();
     m.assign(C, 0);
-    parallel_ranges(C, [&](int c0, int c1) { slot_tables(n, elnod, p, c0, c1, false, m); });
+    parallel_ranges(C, [&](int c0, int c1) {
+      NodeCounter count(N, n, elnod, p.s2o);
+      for (int c = c0; c < c1; ++c) m[c] = count(p.eoff[c], p.eoff[c + 1]);
+    });
     std::vector<int> eoff(1, 0);
     bool split = false;
     for (int c = 0; c < C; ++c) {
@@ -225,7 +333,7 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
   p.ent.assign((size_t)E * n, 0);
   p.snode.assign((size_t)S, 0);
   p.lslot.assign((size_t)E * n, 0);
-  parallel_ranges(C, [&](int c0, int c1) { slot_tables(n, elnod, p, c0, c1, true, m); });
+  parallel_ranges(C, [&](int c0, int c1) { slot_tables(n, elnod, p, c0, c1); });
   // node -> slots, in cluster order
   p.nsl_off.assign((size_t)N + 1, 0);
   for (int c = 0; c < C; ++c) {

@@ -3,8 +3,9 @@
 // The elements are stored in cluster order: each connected component of the
 // mesh is laid out brick by brick (bricks of about `cs` elements, longest
 // along x, in Morton order) by its element centroids and cut into runs of at
-// most `cs` elements; within a run the elements keep their ascending
-// original order.  One work-group of the fused element pass
+// most `cs` elements, or, a structured block of elements that such runs would
+// cut badly, split evenly into bricks; within a cluster the elements keep their
+// ascending original order.  One work-group of the fused element pass
 // handles one cluster and adds the forces of its element-nodes per cluster
 // node in LDS, in that order, so each (cluster, node) pair, a "slot", gets
 // one partial sum; the node pass adds a node's slots in ascending cluster
@@ -41,7 +42,8 @@ struct ClusterPlan {
 constexpr int slot_cap(int n) { return n == 8 ? 512 : 256; }
 
 // Plan for elnod [E][n] (original order, nodes in [0, N)) with node
-// coordinates x [N][3]; cs <= 256 elements per cluster.  Returns 0.
-int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs, ClusterPlan &p);
+// coordinates x [N][3]; cs <= 256 elements per cluster; even: a structured block
+// may be split evenly.  Returns 0.
+int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs, ClusterPlan &p, bool even = true);
 
 }  // namespace wfx
