@@ -478,15 +478,27 @@ __device__ __forceinline__ void staged_jacobian(const double *lx, int cap, const
   }
 }
 
+// The element's mean of its nodes' ANP ratios (calcElemPressure)
+template <typename T, int NN>
+__device__ __forceinline__ double element_ratio(const T *r, const int (&ls)[NN]) {
+  double J_avg = 0.0;
+#pragma unroll
+  for (int a = 0; a < NN; ++a) {
+    if constexpr (std::is_same<T, double>::value) J_avg += r[ls[a]];
+    else J_avg += 1.0 + (double)r[ls[a]];
+  }
+  return J_avg / NN;
+}
+
 // F3, first part: everything that reads the staged nodal data of element
 // `ls` (its nodes as slot indices): Jacobian, cofactors and determinant
 // (calcElemJAndDerivatives), the velocity gradient and from it the strain
-// rate and spin (calcElemStrainRates), the hourglass amplitudes, the ANP
-// average of the nodal ratios (calcElemPressure) and the contact test.
+// rate and spin (calcElemStrainRates), the hourglass amplitudes, with RATIO the
+// ANP average of the nodal ratios (calcElemPressure) and the contact test.
 // sum_a dH(d,a) y_a = sum_i C[i][d] (0.125 m_i(y)) for a hexahedron
 // (dH(d,a) = 0.125 sum_i s_i(a) C[i][d], Domain_d.C:1843-1850), and
 // sum_i C[i][d] (y_{i+1} - y_0) for a tetrahedron (:1866-1887).
-template <typename T, int NN, bool TH>
+template <typename T, int NN, bool TH, bool RATIO>
 __device__ __forceinline__ void element_geometry(const FusedParams &fp, const SlotLds<T, NN> &L,
                                                  const int (&ls)[NN], ElemGeo<T, NN, TH> &G) {
   T J[3][3];
@@ -540,13 +552,7 @@ __device__ __forceinline__ void element_geometry(const FusedParams &fp, const Sl
   G.w02 = qh * (Gv[2][0] - Gv[0][2]);
   // div v times detJ for the pressure's stabilisation terms
   G.div_v = (NN == 8 ? 0.125 : 1.0) * ((double)Gv[0][0] + (double)Gv[1][1] + (double)Gv[2][2]);
-  double J_avg = 0.0;
-#pragma unroll
-  for (int a = 0; a < NN; ++a) {
-    if constexpr (std::is_same<T, double>::value) J_avg += L.r[ls[a]];
-    else J_avg += 1.0 + (double)L.r[ls[a]];
-  }
-  G.J_avg = J_avg / NN;
+  if constexpr (RATIO) G.J_avg = element_ratio<T, NN>(L.r, ls);
   G.is_contact = elem_in_contact<NN>(fp.pp, [&](int a) { return L.node[ls[a]]; });
   // thermal coupling (ThermalCalcs, Thermal.C:27-115): the conduction matrix
   // applied through the element's temperature gradient,
@@ -895,11 +901,11 @@ constexpr int kF3Lds = kF3Vals<T, NN, LAW, TH> > SlotLds<T, NN>::bytes ? kF3Vals
 // one part after the staging's loads, slot after slot and with the mass
 // summed from the densities, it added 6300 (hexahedra) and 12000
 // (tetrahedra) cycles to the staging's 1000.
-template <typename T, int NN>
+template <typename T, int NN, int SLOTS = kSlotsPerThread<NN>>
 struct PairSum {
   // entries in flight: all of a structured hexahedral node's; up to 24 of a
   // tetrahedral one's
-  static constexpr int W = NN == 8 ? 8 : 24, K = kSlotsPerThread<NN>;
+  static constexpr int W = NN == 8 ? 8 : 24, K = SLOTS;
   long slot[K];
   int4 en[K][W / 4];
   T v[K][W];
@@ -911,8 +917,8 @@ struct PairSum {
       for (int h = 0; h < W / 4; ++h)
         en[k][h] = reinterpret_cast<const int4 *>(pr.sent + slot[k] * pr.pw)[min(k0 / 4 + h, pr.pw / 4 - 1)];
   }
-  __device__ __forceinline__ void volumes(const PairArgs &pr) {
-    const T *vol = static_cast<const T *>(pr.vol);
+  // vol: the volumes of the elements from the pass's first one on
+  __device__ __forceinline__ void volumes(const T *vol) {
 #pragma unroll
     for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -930,9 +936,9 @@ struct PairSum {
       rho_n[k] = rho_u > 0.0 ? rho_u : pr.rho_avg[rec[k].x];
     }
   }
-  __device__ __forceinline__ void ratio(const PairArgs &pr, const int4 (&rec)[K], const bool (&mine)[K],
-                                        T (&out)[K]) {
-    double s[K], l[K][8];
+  // the nodes' sums, their further volumes from vol
+  __device__ __forceinline__ void sums(const PairArgs &pr, const int4 (&rec)[K], const T *vol, double (&s)[K]) {
+    double l[K][8];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       s[k] = 0.0;
@@ -955,21 +961,46 @@ struct PairSum {
       k0 += W;
       if (k0 >= pr.pw) break;
       entries(pr, k0);
-      volumes(pr);
+      volumes(vol);
     }
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
+    for (int k = 0; k < K; ++k)
       if (pr.lanes)
         s[k] = ((l[k][0] + l[k][1]) + (l[k][2] + l[k][3])) + ((l[k][4] + l[k][5]) + (l[k][6] + l[k][7]));
-      if constexpr (std::is_same<T, double>::value) out[k] = s[k] / v0[k];
-      else out[k] = (float)(s[k] / v0[k] - 1.0);
-      if (mine[k] && rec[k].w < 0) {
-        reinterpret_cast<T *>(pr.ratio)[rec[k].x] = out[k];
-        pr.mdiag[rec[k].x] = s[k] * (1.0 / NN) * rho_n[k];
-      }
-    }
   }
+  __device__ __forceinline__ T ratio(int k, double s) const {
+    if constexpr (std::is_same<T, double>::value) return s / v0[k];
+    else return (float)(s / v0[k] - 1.0);
+  }
+  __device__ __forceinline__ double mass(int k, double s) const { return s * (1.0 / NN) * rho_n[k]; }
 };
+
+// One slot's sums of R components: its entry groups [k0, k1), the first G of
+// them in registers.  Four entries at a time with their LDS reads in flight
+// together, added in order.  One entry per pass waited for two dependent LDS
+// reads each time: 2800 (hexahedra) and 4900 (tetrahedra) of the 13200 and
+// 11700 cycles a work-group takes on an idle chip.
+template <typename T, int NN, int R, int G>
+__device__ __forceinline__ void add_entries(const unsigned char *lds, const uint2 (&ew)[G], const uint2 *en, int k0, int k1,
+                                            double (&acc)[R]) {
+  auto add4 = [&](uint2 w) {
+    T val[4][R];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      const unsigned o = h & 1 ? (h < 2 ? w.x : w.y) >> 16 : (h < 2 ? w.x : w.y) & 0xffffu;
+#pragma unroll
+      for (int u = 0; u < R; ++u) val[h][u] = *reinterpret_cast<const T *>(lds + o + u * (kEntStride(NN) * (int)sizeof(T)));
+    }
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+      for (int u = 0; u < R; ++u) acc[u] += (double)val[h][u];
+  };
+#pragma unroll
+  for (int h = 0; h < G; ++h)
+    if (k0 + h < k1) add4(ew[h]);
+  for (int k = k0 + G; k < k1; ++k) add4(en[k]);  // more elements than the registers hold
+}
 
 // F3: one work-group per element cluster.  The work-group first stages its
 // cluster's slots (the distinct nodes of its elements: positions,
@@ -1052,7 +1083,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   // stage the slots: all loads first, then the LDS stores
   double sx[kSl][3];
   T sv[kSl][3], sr[kSl];
-  if constexpr (PAIR) ps.volumes(pr);
+  if constexpr (PAIR) ps.volumes(static_cast<const T *>(pr.vol));
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
     const int node = sn[k];
@@ -1072,7 +1103,18 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (PAIR) load_elem_state<T>(my_e, E, tau_in, eps_io, pl_in, sy0, He, S);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (PAIR) ps.ratio(pr, rec, mine, sr);
+  if constexpr (PAIR) {
+    double vs[kSl];
+    ps.sums(pr, rec, static_cast<const T *>(pr.vol), vs);
+#pragma unroll
+    for (int k = 0; k < kSl; ++k) {
+      sr[k] = ps.ratio(k, vs[k]);
+      if (mine[k] && rec[k].w < 0) {
+        reinterpret_cast<T *>(pr.ratio)[rec[k].x] = sr[k];
+        pr.mdiag[rec[k].x] = ps.mass(k, vs[k]);
+      }
+    }
+  }
   double dt_step = fp.dt;
   if constexpr (PAIR) {
     // every work-group reduces the step's dt for itself, since a kernel for it
@@ -1105,7 +1147,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
 #pragma unroll
     for (int h = 0; h < kGr; ++h) ew[k][h] = en[(ow[k] & 0xffffu) + h];
   ElemGeo<T, NN, TH> G;
-  if (t < ne) element_geometry<T, NN, TH>(fp, L, ls, G);
+  if (t < ne) element_geometry<T, NN, TH, true>(fp, L, ls, G);
   __syncthreads();  // the staged slots are read: their LDS takes the element-node values
   if (t < ne) {
     element_material<T, NN, LAW, kCluster, TH>(
@@ -1136,33 +1178,9 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
     double acc[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) acc[q] = 0.0;
-    // Four entries at a time with their LDS reads in flight together, added in
-    // order.  One entry per pass waited for two dependent LDS reads each time:
-    // 2800 (hexahedra) and 4900 (tetrahedra) of the 13200 and 11700 cycles a
-    // work-group takes on an idle chip.
-    auto add4 = [&](uint2 w) {
-      T val[4][R];
+    add_entries<T, NN, R, kGr>(lds_raw, ew[r], en, k0, k1, acc);
 #pragma unroll
-      for (int h = 0; h < 4; ++h) {
-        const unsigned o = h & 1 ? (h < 2 ? w.x : w.y) >> 16 : (h < 2 ? w.x : w.y) & 0xffffu;
-#pragma unroll
-        for (int u = 0; u < R; ++u)
-          val[h][u] = *reinterpret_cast<const T *>(lds_raw + o + u * (kEntStride(NN) * (int)sizeof(T)));
-      }
-#pragma unroll
-      for (int h = 0; h < 4; ++h)
-#pragma unroll
-        for (int u = 0; u < R; ++u) acc[u] += (double)val[h][u];
-    };
-#pragma unroll
-    for (int h = 0; h < kGr; ++h)
-      if (k0 + h < k1) add4(ew[r][h]);
-    for (int k = k0 + kGr; k < k1; ++k) add4(en[k]);  // more elements than the registers hold
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      if (kNodeMajor<T> || PAIR || ca.nm) part[q * ca.S + sp[r]] = (T)acc[q];
-      else st_stream(&part[q * ca.S + sp[r]], (T)acc[q]);
-    }
+    for (int q = 0; q < R; ++q) part[q * ca.S + sp[r]] = (T)acc[q];  // cached: the node pass reads them next
   }
 }
 
@@ -1491,21 +1509,23 @@ __device__ __forceinline__ void load_node(int i, long Ns, const NodeParams &np, 
 // run's last step stores the corrected increment, and with a per-step time
 // step (the previous step's length predicted it) it is read and stored
 // every step.
-// PAIR: the paired node pass, where several work-groups update the same node
-// and only the one that owns it (own) stores; xn_out receives the new
-// position in either case.
-template <typename T, bool CFL, bool CONTACT, bool PAIR>
+// BY: the node pass (a thread per node); the paired node pass, where several
+// work-groups update the same node, only the one that owns it (own) stores
+// and xn_out receives the new position in either case; or the solo pass, which
+// keeps the state in s from step to step.
+enum NodeBy { BY_NODE, BY_SLOT, IN_PLACE };
+template <typename T, bool CFL, bool CONTACT, int BY>
 __device__ __forceinline__ double node_update(
-    int i, long Ns, const NodeParams &np, double (&f)[3], const NodeIn<T, CONTACT> &s,
+    int i, long Ns, const NodeParams &np, double (&f)[3], NodeIn<T, CONTACT> &s,
     T *__restrict__ fi, T *__restrict__ v, T *__restrict__ prev_a, T *__restrict__ u_dt, double *__restrict__ x, double *__restrict__ u,
     unsigned int *__restrict__ status, bool own, double *xn_out) {
-  const bool store = !PAIR || own;
+  const bool store = BY != BY_SLOT || own;
   unsigned bad = 0;
 #pragma unroll
   for (int d = 0; d < 3; ++d)
     if (!isfinite(f[d])) { f[d] = 0.0; ++bad; }
   if (bad && store) atomicAdd(status, bad);
-  if (store) record_reaction<T, PAIR>(np, i, f[2]);
+  if (store) record_reaction<T, BY != BY_NODE>(np, i, f[2]);
   const int mask = s.mask;
   const double m = s.m;
   double vs[3];
@@ -1529,8 +1549,9 @@ __device__ __forceinline__ double node_update(
     double ud = np.read_ud ? (double)s.ud[d] : np.dt * (v0 + np.pred_u * pa);
     ud = ud + np.bdt2 * a;                              // UpdateCorrectionPos
     const double xo = s.x[d], xn = xo + ud;
-    if (store) x_d = xn;
-    if constexpr (PAIR) xn_out[d] = xn;
+    if constexpr (BY == IN_PLACE) s.x[d] = xn;
+    else if (store) x_d = xn;
+    if constexpr (BY == BY_SLOT) xn_out[d] = xn;
     if constexpr (std::is_same<T, double>::value) {
       const double bb = xn - xo;
       const double err = (xo - (xn - bb)) + (ud - bb);  // xo + ud - xn, exactly
@@ -1540,7 +1561,8 @@ __device__ __forceinline__ double node_update(
         (u + r)[ui] = s.u[d] + (np.run_first ? ud : ((xn - s.xs[d]) + lo));
       } else {
         if (np.run_first) (np.x_start + r)[ui] = xo;
-        (np.x_lo + r)[ui] = (float)lo;
+        if constexpr (BY == IN_PLACE) s.lo[d] = (float)lo;
+        else (np.x_lo + r)[ui] = (float)lo;
       }
     }
     if (np.predict) {                                   // UpdatePrediction
@@ -1548,7 +1570,10 @@ __device__ __forceinline__ double node_update(
       vv = vv + np.pred_v * a;
       if (mask & (1 << d)) vv = s.bv[d];  // ImposeBCV
     }
-    if (store) {
+    if constexpr (BY == IN_PLACE) {
+      s.pa[d] = (T)a;
+      s.v[d] = (T)vv;
+    } else if (store) {
       if (np.write_ud || !np.predict) ud_d = (T)ud;
       pa_d = (T)a;
       v_d = (T)vv;
@@ -1631,7 +1656,7 @@ __global__ __launch_bounds__(BS) void f4_node(
     load_node<T, CONTACT>(i, N, q, cf, fe, mdiag, word, bc_val, v, prev_a, u_dt, x, u, st);
     double f[TH ? 4 : 3];
     gather_slots<T, TH, 4>(o, c, nm, nsl, part, S, f);
-    speed = node_update<T, CFL, CONTACT, false>(i, N, q, *reinterpret_cast<double(*)[3]>(f), st, fi, v, prev_a, u_dt, x, u, status, true, nullptr);
+    speed = node_update<T, CFL, CONTACT, BY_NODE>(i, N, q, *reinterpret_cast<double(*)[3]>(f), st, fi, v, prev_a, u_dt, x, u, status, true, nullptr);
     if constexpr (TH) {  // T += (dTdt + q_cont / (m cp)) dt (Thermal.C:124)
       double r = f[3] / st.m;
       if (q.qcont) r += q.qcont[i] * 1.0 / (st.m * q.cp_T);
@@ -1699,7 +1724,7 @@ __global__ __launch_bounds__(slot_cap(NN)) void f41_cluster(
   if (__any(rec.z > 4)) gather_slots<T, TH, 8>(rec.y, rec.z, true, nullptr, part, ca.S, f);
   else gather_slots<T, TH, 4>(rec.y, rec.z, true, nullptr, part, ca.S, f);
   double xn[3];
-  double speed = node_update<T, CFL, CONTACT, true>(
+  double speed = node_update<T, CFL, CONTACT, BY_SLOT>(
       i, N, q, *reinterpret_cast<double(*)[3]>(f), st, fi, static_cast<T *>(out.v), static_cast<T *>(out.pa),
       static_cast<T *>(out.ud), out.x, nullptr, status, own, xn);
 #pragma unroll
@@ -1721,6 +1746,152 @@ __global__ __launch_bounds__(slot_cap(NN)) void f41_cluster(
       minl_part[blockIdx.x] = medge;
       q.vmax_part[blockIdx.x] = speed;
     }
+  }
+}
+
+// Many steps of a mesh whose clusters share no node, in one launch: each
+// work-group's elements and nodes meet no other's, so that it steps alone, the
+// nodal state in registers (the thread of a slot is its node's), positions,
+// volumes and ratios in LDS.  Same arithmetic in the same order as the paired
+// passes, bit for bit.  The element state goes through memory as there (a
+// thread reads what it wrote; the loads lead the step and are not waited for
+// until the stress update).
+// Bound: the chain of one element and four barriers, on one CU: latency.  The
+// two launches a step and their round trips were three fifths of it.  Measured,
+// us a step, launched: one hexahedron 11.5 by the paired passes, 4.7 here; 216
+// hexahedra 5.9, with Johnson-Cook's law 10.4; the smallest tetrahedral cylinder 4.0.
+template <typename T, int NN, int LAW>
+__global__ __launch_bounds__(slot_cap(NN)) void f_solo(
+    int E, int N, int nsteps, size_t rz_row, FusedParams fp, NodeParams np, ClusterArgs ca, PairArgs pr,
+    double *x, T *v, T *prev_a, const T *__restrict__ u_dt, const double *__restrict__ fe,
+    const double *__restrict__ bc_val, const T *__restrict__ vol0, const T *__restrict__ rho,
+    const T *__restrict__ sy0, const T *__restrict__ He, T *tau, T *eps, T *pl, unsigned int *status) {
+  constexpr int cap = slot_cap(NN), R = 3;
+  __shared__ __align__(16) unsigned char staged[SlotLds<T, NN>::bytes];
+  __shared__ __align__(16) unsigned char lds_raw[kF3Vals<T, NN, LAW, false>];  // element-node values and stash, as in F3
+  __shared__ T lvol[kCluster], lpa[3 * cap];  // volumes; each thread's node's previous acceleration,
+  __shared__ double lbv[3 * cap];             //   boundary values and
+  __shared__ float llo[3 * cap];              //   position error terms
+  const SlotLds<T, NN> L(staged);
+  T *lf = reinterpret_cast<T *>(lds_raw);
+  const int t = threadIdx.x;
+  const ClusterDesc cd = ca.desc[blockIdx.x];
+  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;  // M <= slot_cap(NN), checked at set-up
+  const uint16_t *lo = ca.goff + cd.goff;
+  const uint2 *en = ca.ent + cd.ent;
+  // a thread per slot; as in F3, threads past the cluster's slots or elements
+  // repeat its last one
+  const int j = min(t, M - 1), te = min(t, ne - 1);
+  PairSum<T, NN, 1> ps;
+  int ls[NN];
+  load_lslot<NN>(ca.lslot + (long)(cd.lslot + te) * NN, ls);
+  const int4 rec[1] = {pr.rec[s0 + j]};
+  ps.slot[0] = s0 + j;
+  uint32_t ow;
+  __builtin_memcpy(&ow, lo + j, 4);
+  const int k0 = ow & 0xffffu, k1 = ow >> 16, i = rec[0].x, mask = pr.sbc[s0 + j] & 7;
+  np.predict = 1;
+  np.run_last = np.write_fi = np.write_ud = 0;
+  {
+    NodeIn<T, false> st;
+    load_node<T, false>(i, N, np, nullptr, fe, pr.mdiag, pr.sbc[s0 + j], bc_val, v, prev_a, u_dt, x, nullptr, st);
+    L.node[t] = i;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      L.x[d * cap + t] = st.x[d];
+      L.v[d * cap + t] = st.v[d];
+      lpa[d * cap + t] = st.pa[d];
+      lbv[d * cap + t] = st.bv[d];
+      llo[d * cap + t] = st.lo[d];
+    }
+  }
+  ps.nodal(pr, rec, fp.rho_u);
+  constexpr int kGr = NN == 8 ? 2 : 6;
+  uint2 ew[kGr];
+#pragma unroll
+  for (int h = 0; h < kGr; ++h) ew[h] = en[k0 + h];
+  const T dt = (T)fp.dt;
+  for (int step = 0; step < nsteps; ++step) {
+    // opaque, or the addresses of every row and entry are kept from step to
+    // step, in more registers than there are
+    int e = e0 + te;
+    asm volatile("" : "+v"(e));
+#pragma unroll
+    for (int h = 0; h < kGr; ++h) asm volatile("" : "+v"(ew[h].x), "+v"(ew[h].y));
+#pragma unroll
+    for (int a = 0; a < NN; ++a) asm volatile("" : "+v"(ls[a]));
+    ps.entries(pr, 0);
+    __syncthreads();
+    ElemGeo<T, NN, false> G;
+    if (t < ne) {
+      element_geometry<T, NN, false, false>(fp, L, ls, G);
+      count_inverted(G.detJ, status);
+      lvol[t] = G.volv;
+    }
+    ElemState<T> S;
+    load_elem_state<T>(e, E, tau, eps, pl, sy0, He, S);
+    __syncthreads();
+    double vs[1];
+    ps.volumes(lvol - e0);
+    ps.sums(pr, rec, lvol - e0, vs);
+    L.r[t] = ps.ratio(0, vs[0]);
+    const double m = ps.mass(0, vs[0]);
+    __syncthreads();
+    if (t < ne) {
+      G.J_avg = element_ratio<T, NN>(L.r, ls);
+      element_material<T, NN, LAW, kCluster, false>(
+          e, E, fp, dt, G, S, vol0, rho, He, tau, eps, nullptr, pl, false, nullptr, nullptr,
+          reinterpret_cast<double *>(lds_raw) + t, [&](int a, int, T f0, T f1, T f2, T) {
+            lf[0 * kEntStride(NN) + a * kCluster + t] = f0;
+            lf[1 * kEntStride(NN) + a * kCluster + t] = f1;
+            lf[2 * kEntStride(NN) + a * kCluster + t] = f2;
+          });
+    }
+    if (t == 0)  // the zero cells, as in F3
+#pragma unroll
+      for (int u = 0; u < R; ++u) lf[u * kEntStride(NN) + NN * kCluster] = T(0);
+    __syncthreads();
+    if (t < M) {
+      double acc[R] = {0.0, 0.0, 0.0}, f[3];
+      add_entries<T, NN, R, kGr>(lds_raw, ew, en, k0, k1, acc);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) f[d] = 0.0 + (double)(T)acc[d];
+      NodeIn<T, false> st;
+      st.m = m;
+      st.mask = mask;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const long r = (long)d * N;
+        st.x[d] = L.x[d * cap + t];
+        st.v[d] = L.v[d * cap + t];
+        st.pa[d] = lpa[d * cap + t];
+        st.bv[d] = lbv[d * cap + t];
+        st.lo[d] = llo[d * cap + t];
+        st.fe[d] = np.has_fe ? (fe + r)[(unsigned)i] : 0.0;
+        st.ud[d] = T(0);
+        if (np.read_ud) st.ud[d] = (u_dt + r)[(unsigned)i];
+      }
+      node_update<T, false, false, IN_PLACE>(i, N, np, f, st, nullptr, v, prev_a, nullptr, x, nullptr, status, true,
+                                             nullptr);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        L.x[d * cap + t] = st.x[d];
+        L.v[d * cap + t] = st.v[d];
+        lpa[d * cap + t] = st.pa[d];
+        llo[d * cap + t] = st.lo[d];
+      }
+    }
+    np.run_first = np.read_ud = 0;
+    if (np.rz) np.rz = static_cast<char *>(np.rz) + rz_row;
+  }
+  if (t >= M) return;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const long r = (long)d * N;
+    (x + r)[(unsigned)i] = L.x[d * cap + t];
+    (v + r)[(unsigned)i] = L.v[d * cap + t];
+    (prev_a + r)[(unsigned)i] = lpa[d * cap + t];
+    if constexpr (std::is_same<T, double>::value) (np.x_lo + r)[(unsigned)i] = llo[d * cap + t];
   }
 }
 
@@ -1902,14 +2073,11 @@ void fused_node_arrays(wfx_ctx *c, T *&v, T *&pa, T *&ud, T *&fi) {
     v = c->v32; pa = c->pa32; ud = c->ud32; fi = c->fi32;
   }
 }
-// F3 (PAIR: with F2 in its staging); dtp: the step's dt on the device, or null
-template <typename T, bool PAIR>
-hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr, hipStream_t s) {
+template <typename T>
+FusedParams element_params(wfx_ctx *c, const double *dtp) {
   auto &el = elem<T>(c);
   const auto &P = c->prm;
   const auto &st = P.stab;
-  T *vN, *paN, *udN, *fiN;
-  fused_node_arrays<T>(c, vN, paN, udN, fiN);
   FusedParams fp;
   fp.dt = P.dt;
   fp.mp = mat_params(c);
@@ -1932,6 +2100,15 @@ hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr
   fp.flat_base = c->ms.flat_base;
   fp.mdiag = c->nd.mdiag;
   fp.write_out = c->fused_write_out;
+  return fp;
+}
+// F3 (PAIR: with F2 in its staging); dtp: the step's dt on the device, or null
+template <typename T, bool PAIR>
+hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr, hipStream_t s) {
+  auto &el = elem<T>(c);
+  T *vN, *paN, *udN, *fiN;
+  fused_node_arrays<T>(c, vN, paN, udN, fiN);
+  const FusedParams fp = element_params<T>(c, dtp);
   const bool rate = law_class(fp.mp.model) == LAW_RATE, th = c->thermal.on;
   auto kern = (c->n == 8) ? (rate ? f3_pick<T, 8, LAW_RATE, PAIR>(th) : f3_pick<T, 8, LAW_PLAIN, PAIR>(th))
                           : (rate ? f3_pick<T, 4, LAW_RATE, PAIR>(th) : f3_pick<T, 4, LAW_PLAIN, PAIR>(th));
@@ -2250,6 +2427,28 @@ struct NodalPlaces {
   }
 };
 
+// Steps [k, k + n) of a run, n > 0 and none of them the last, by the solo pass;
+// rz: the first one's reaction record, or null
+template <typename T>
+hipError_t launch_solo_steps(wfx_ctx *c, int k, int n, void *rz, hipStream_t s) {
+  auto &el = elem<T>(c);
+  T *vN, *paN, *udN, *fiN;
+  fused_node_arrays<T>(c, vN, paN, udN, fiN);
+  FusedParams fp = element_params<T>(c, nullptr);
+  fp.write_out = 0;
+  NodeParams np = node_params(c, 1);
+  np.write_fi = np.write_ud = np.run_last = 0;
+  np.run_first = np.read_ud = k == 0 ? 1 : 0;
+  np.rz = rz;
+  const bool rate = law_class(fp.mp.model) == LAW_RATE;
+  auto kern = c->n == 8 ? (rate ? f_solo<T, 8, LAW_RATE> : f_solo<T, 8, LAW_PLAIN>)
+                        : (rate ? f_solo<T, 4, LAW_RATE> : f_solo<T, 4, LAW_PLAIN>);
+  hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(slot_cap(c->n)), 0, s, c->E, c->N, n, (size_t)c->react_n * sizeof(T), fp, np,
+                     cluster_args(c), pair_args<T>(c, -1), c->nd.x, vN, paN, udN, c->nd.fe, c->bc_tab, el.vol0, el.rho,
+                     el.sy0, el.He, el.tau, el.eps, el.pl_strain, c->status);
+  return hipGetLastError();
+}
+
 // Step k of a run of nsteps; have_vol: the step before left this one's
 // volumes (and whether this one leaves the next one's).  rz: the step's
 // reaction record, or null.  ev: an event before each pass (separate passes).
@@ -2297,7 +2496,18 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
   const bool pair = run_paired(c) && !ev;  // with events the four passes run separately
   const NodalPlaces<T> places(c);
   bool have_vol = false;
-  for (int k = 0; k < nsteps; ++k) {
+  int k = 0;
+  if constexpr (std::is_same<T, double>::value)
+    while (pair && run_solo(c) && k + 1 < nsteps) {  // all steps but the last
+      // up to the row at which the reaction record is full
+      int n = std::min(nsteps - 1 - k, kSoloSteps);
+      if (rec.hist) n = std::min(n, c->react_rows - k % c->react_rows);
+      hipError_t e = launch_solo_steps<T>(c, k, n, rec.row(k), s);
+      k += n;
+      if (e == hipSuccess && rec.full(k - 1)) e = launch_reaction_rows<T>(c, rec, k - 1, s);
+      if (e != hipSuccess) return e;
+    }
+  for (; k < nsteps; ++k) {
     if (c->contact.on && (c->contact.step_count + k) % 10 == 0) {
       hipError_t e = launch_ext_face_areas(c, s);  // every 10 steps, at the step's start
       if (e != hipSuccess) return e;
