@@ -272,6 +272,26 @@ static ClusterTables cluster_tables(const wfx_ctx *c, const ClusterPlan &plan) {
   return t;
 }
 
+// Bytes a step of the separate passes touches: element state, partial sums,
+// nodal state, tables.
+static double step_bytes(const wfx_ctx *c, const ClusterTables &ct) {
+  const double es = c->precision == WFX_FP64 ? 8 : 4, E = c->E, N = c->N, S = c->ms.nslot;
+  const double tables = 2.0 * ct.goff.size() + 2.0 * ct.lslot.size() + 8.0 * ct.ent.size() + 4.0 * ct.nrel.size();
+  // stress, strain, plastic strain, yield stress, volume; the sums and where they go;
+  // x, v, a, rounding terms, mass, ratio, V0, density; the element lists
+  return E * 15 * es + S * (3 * es + 4) + N * (24 + 6 * es + (es == 8 ? 12 : 0) + 8 + es + 16 + 12) +
+         4.0 * (c->f2_lanes ? E * c->n : 8 * N) + tables;
+}
+// The line between cached and non-temporal accesses, of the 256 MB last-level
+// cache.  Step of the separate passes, us, cached / non-temporal, by MB:
+// FP64 hexahedra 170 79.6 / 85.3, 217 93.6 / 101.8, 246 118.8 / 112.5, 372 165 /
+// 153, 1319 576 / 549; FP64 tetrahedra 161 73.2 / 77.6, 219 88.9 / 94.3, 241
+// 108.7 / 100.7; FP32-mixed hexahedra 218 92.6 / 102.9, 237 107.2 / 110.9, 278
+// 128.7 / 123.7, 363 162 / 149; tetrahedra 196 85.1 / 91.1, 252 120 / 106.
+// (Between the two, the strains alone non-temporal: 99.4 at 241 MB, 92.1 at 219,
+// 109.2 at 252: no better than the better of the two by more than a percent.)
+constexpr double kCachedStepBytes = 240e6;
+
 // Tables of the paired passes; pw 0: the mesh takes the separate ones.
 // The line: 256 clusters, one work-group on each of the 256 CUs.  Below it the
 // launches and dependent loads count and the repeated node updates (1.7 times,
@@ -329,6 +349,7 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     return WFX_ERR_STATE;
   }
   const ClusterTables ct = cluster_tables(c, plan);
+  c->stream_step = step_bytes(c, ct) > kCachedStepBytes;
   A(c->ms.cl_desc, c->ms.ncl) A(c->ms.cl_goff, ct.goff.size()) A(c->ms.cl_ent, ct.ent.size())
   A(c->ms.cl_lslot, ct.lslot.size()) A(c->ms.cl_nrel, ct.nrel.size()) A(c->ms.nsl_off, N + 1)
   A(c->ms.cl_snode, c->ms.nslot)

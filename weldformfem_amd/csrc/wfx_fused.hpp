@@ -57,19 +57,20 @@ constexpr int kChunk = 8;  // also the width of the padded first-entries table
 __device__ __forceinline__ long fidx(int row, long e, long Es, int nrow) {
   return (e >> 6) * ((long)nrow * 64) + (long)row * 64 + (e & 63);
 }
-// Element streams written once per step: non-temporal stores.
-template <typename T>
+// Data a pass reads or writes once per step (stress, strain, yield stress; F2's
+// tables).  NT: a step touches more than the last-level cache keeps until the
+// next (wfx_ctx::stream_step), and non-temporal accesses keep these out of the
+// way of what the gathers and the next pass read again; a smaller mesh finds
+// them there in the next step.
+template <bool NT, typename T>
 __device__ __forceinline__ void st_stream(T *p, T v) {
-  __builtin_nontemporal_store(v, p);
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
 }
-// Element data the element pass reads once per step (connectivity, stress,
-// strain, yield stress): non-temporal loads, so that they do not displace the
-// nodal arrays its gathers reuse from L2 (measured: element pass -2%; the
-// same loads in the volume and node passes made those slower, so they stay
-// plain there).
-template <typename T>
+template <bool NT, typename T>
 __device__ __forceinline__ T ld_stream(const T *p) {
-  return __builtin_nontemporal_load(p);
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  else return *p;
 }
 
 // The nodal ANP ratio F2 leaves for the element pass: double, or (FP32-mixed)
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(kBlock) void f0_vsum0(int N, const int *__restrict_
 
 // F2: nodal volume sum in CSR order; ratio for the ANP pressure and nodal
 // mass (the nodal volume field itself is written once per run, in phase 5).
-template <typename T, int BS>
+template <typename T, int BS, bool NT>
 __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *__restrict__ off,
                                                    const int *__restrict__ cnt,
                                                    const int *__restrict__ nodel_pk,
@@ -126,23 +127,22 @@ __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *_
   }
   int i = xcd_block(nb) * BS + threadIdx.x;
   if (i >= N) return;
-  const int c = ld_stream(&cnt[i]), o = c > kChunk ? off[i] : 0;
-  // The table, count and V0_n are read once per step: non-temporal loads, so
-  // that the element volumes the gathers reuse stay in L2 (measured on the
-  // 200x200x100 block: 89 -> 80 us FP64).  The ratio is stored plainly: the
-  // element pass gathers it next.
+  const int c = ld_stream<NT>(&cnt[i]), o = c > kChunk ? off[i] : 0;
+  // The table, count and V0_n are read once per step (4M FP64 hexahedra 68.4
+  // us with plain loads, 60.8 with NT; 1.1M FP32-mixed 14.7 and 16.9).  The ratio
+  // is stored plainly: the element pass gathers it next.
   // CSR entries are taken eight at a time with independent loads, then
   // summed in CSR order (the order of the reference's serial loop); the
   // first eight come from the padded [8][N] table.
-  const double v0 = ld_stream(&vsum0[i]);
-  const double rho_n = rho_u > 0.0 ? rho_u : ld_stream(&rho_avg[i]);
+  const double v0 = ld_stream<NT>(&vsum0[i]);
+  const double rho_n = rho_u > 0.0 ? rho_u : ld_stream<NT>(&rho_avg[i]);
   double s = 0.0;
   for (int k = 0; k < c; k += kChunk) {
     int e[kChunk];
     double vv[kChunk];
 #pragma unroll
     for (int j = 0; j < kChunk; ++j)
-      e[j] = (k == 0) ? (ld_stream(&pad[(long)j * N + i]) >> 3) : ((k + j < c) ? (nodel_pk[o + k + j] >> 3) : -1);
+      e[j] = (k == 0) ? (ld_stream<NT>(&pad[(long)j * N + i]) >> 3) : ((k + j < c) ? (nodel_pk[o + k + j] >> 3) : -1);
     // every load is issued (entries past the count read the chunk's first
     // element) and only the node's own entries are added: conditional loads
     // would each be waited for on their own
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(BS) void f2_nodal(int N, int nodxelem, const int *_
   else reinterpret_cast<float *>(ratio)[i] = (float)(s / v0 - 1.0);
   double vn = s;
   vn *= 1.0 / nodxelem;  // 4 or 8: exact
-  st_stream(&mdiag[i], vn * rho_n);
+  st_stream<NT>(&mdiag[i], vn * rho_n);
 }
 
 // Nodes with many elements (tetrahedral meshes: about 23 per node) are
@@ -593,7 +593,7 @@ template <typename T>
 struct ElemState {
   T tau[6], eps[6], ep, sy0, He;
 };
-template <typename T>
+template <typename T, bool NT>
 __device__ __forceinline__ void load_elem_state(int e, int E, const T *tau_io,
                                                 const T *__restrict__ eps_io, const T *pl_strain,
                                                 const T *__restrict__ sy0, const T *__restrict__ He,
@@ -601,12 +601,12 @@ __device__ __forceinline__ void load_elem_state(int e, int E, const T *tau_io,
   const long Es = E;
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
-    S.tau[k] = ld_stream(&tau_io[k * Es + e]);
-    S.eps[k] = ld_stream(&eps_io[k * Es + e]);
+    S.tau[k] = ld_stream<NT>(&tau_io[k * Es + e]);
+    S.eps[k] = ld_stream<NT>(&eps_io[k * Es + e]);
   }
-  S.ep = ld_stream(&pl_strain[e]);
-  S.sy0 = ld_stream(&sy0[e]);
-  S.He = He ? ld_stream(&He[e]) : T(0);
+  S.ep = ld_stream<NT>(&pl_strain[e]);
+  S.sy0 = ld_stream<NT>(&sy0[e]);
+  S.He = He ? ld_stream<NT>(&He[e]) : T(0);
 }
 
 template <typename T, int NN, int LAW>
@@ -615,7 +615,7 @@ constexpr bool kStashLDS = NN == 8 && LAW == LAW_RATE && std::is_same<T, double>
 template <bool TH>
 constexpr int kStashVals = TH ? 25 : 22;
 
-template <typename T, int NN, int LAW, int BS, bool TH, class Sink>
+template <typename T, int NN, int LAW, int BS, bool TH, bool NT, class Sink>
 __device__ __forceinline__ void element_material(
     int e, int E, const FusedParams &fp, T dt, ElemGeo<T, NN, TH> &G, const ElemState<T> &S,
     const T *__restrict__ vol0, const T *__restrict__ rho, const T *__restrict__ He, T *tau_out,
@@ -754,15 +754,15 @@ __device__ __forceinline__ void element_material(
     }
     if (fp.write_out) static_cast<T *>(fp.avq)[e] = (T)qs;
   }
-  st_stream(&eps_io[0 * Es + e], S.eps[0] + D.xx * dt);
-  st_stream(&eps_io[1 * Es + e], S.eps[1] + D.yy * dt);
-  st_stream(&eps_io[2 * Es + e], S.eps[2] + D.zz * dt);
-  st_stream(&eps_io[3 * Es + e], S.eps[3] + D.xy * dt);
-  st_stream(&eps_io[4 * Es + e], S.eps[4] + D.yz * dt);
-  st_stream(&eps_io[5 * Es + e], S.eps[5] + D.xz * dt);
-  st_stream(&tau_out[0 * Es + e], tau.xx); st_stream(&tau_out[1 * Es + e], tau.yy);
-  st_stream(&tau_out[2 * Es + e], tau.zz); st_stream(&tau_out[3 * Es + e], tau.xy);
-  st_stream(&tau_out[4 * Es + e], tau.yz); st_stream(&tau_out[5 * Es + e], tau.xz);
+  st_stream<NT>(&eps_io[0 * Es + e], S.eps[0] + D.xx * dt);
+  st_stream<NT>(&eps_io[1 * Es + e], S.eps[1] + D.yy * dt);
+  st_stream<NT>(&eps_io[2 * Es + e], S.eps[2] + D.zz * dt);
+  st_stream<NT>(&eps_io[3 * Es + e], S.eps[3] + D.xy * dt);
+  st_stream<NT>(&eps_io[4 * Es + e], S.eps[4] + D.yz * dt);
+  st_stream<NT>(&eps_io[5 * Es + e], S.eps[5] + D.xz * dt);
+  st_stream<NT>(&tau_out[0 * Es + e], tau.xx); st_stream<NT>(&tau_out[1 * Es + e], tau.yy);
+  st_stream<NT>(&tau_out[2 * Es + e], tau.zz); st_stream<NT>(&tau_out[3 * Es + e], tau.xy);
+  st_stream<NT>(&tau_out[4 * Es + e], tau.yz); st_stream<NT>(&tau_out[5 * Es + e], tau.xz);
 
   T C[3][3], hm[3][4];
   double gT0 = G.gT0, gT1 = G.gT1, gT2 = G.gT2;
@@ -1014,7 +1014,7 @@ __device__ __forceinline__ void add_entries(const unsigned char *lds, const uint
 // thread summing its node's element volumes; slots of a node in several
 // clusters repeat the sum (1.7 times the work of F2), and a launch and F2's
 // round trip of the ratio are saved.
-template <typename T, int NN, int LAW, bool TH, bool PAIR>
+template <typename T, int NN, int LAW, bool TH, bool PAIR, bool NT>
 __global__ __launch_bounds__(kCluster) void f3_cluster(
     int E, int N, FusedParams fp, ClusterArgs ca, PairArgs pr, const double *__restrict__ x, const T *__restrict__ v,
     const double *__restrict__ ratio, const T *__restrict__ vol0, const T *__restrict__ rho,
@@ -1079,7 +1079,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   load_lslot<NN>(ca.lslot + (long)(cd.lslot + min(t, ne - 1)) * NN, ls);
   ElemState<T> S;
   if constexpr (PAIR) __builtin_amdgcn_sched_barrier(0);
-  else load_elem_state<T>(my_e, E, tau_in, eps_io, pl_in, sy0, He, S);
+  else load_elem_state<T, NT>(my_e, E, tau_in, eps_io, pl_in, sy0, He, S);
   // stage the slots: all loads first, then the LDS stores
   double sx[kSl][3];
   T sv[kSl][3], sr[kSl];
@@ -1101,7 +1101,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   }
   if constexpr (PAIR) ps.nodal(pr, rec, fp.rho_u);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (PAIR) load_elem_state<T>(my_e, E, tau_in, eps_io, pl_in, sy0, He, S);
+  if constexpr (PAIR) load_elem_state<T, NT>(my_e, E, tau_in, eps_io, pl_in, sy0, He, S);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (PAIR) {
     double vs[kSl];
@@ -1150,7 +1150,7 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   if (t < ne) element_geometry<T, NN, TH, true>(fp, L, ls, G);
   __syncthreads();  // the staged slots are read: their LDS takes the element-node values
   if (t < ne) {
-    element_material<T, NN, LAW, kCluster, TH>(
+    element_material<T, NN, LAW, kCluster, TH, NT>(
         e0 + t, E, fp, dt, G, S, vol0, rho, He, tau_out, eps_io, p_out, pl_out, pl_in != pl_out, sigma_y, q_plheat,
         reinterpret_cast<double *>(lds_raw) + t, [&](int a, int node, T f0, T f1, T f2, T th) {
           lf[0 * kEntStride(NN) + a * kCluster + t] = f0;
@@ -1829,7 +1829,7 @@ __global__ __launch_bounds__(slot_cap(NN)) void f_solo(
       lvol[t] = G.volv;
     }
     ElemState<T> S;
-    load_elem_state<T>(e, E, tau, eps, pl, sy0, He, S);
+    load_elem_state<T, false>(e, E, tau, eps, pl, sy0, He, S);
     __syncthreads();
     double vs[1];
     ps.volumes(lvol - e0);
@@ -1839,7 +1839,7 @@ __global__ __launch_bounds__(slot_cap(NN)) void f_solo(
     __syncthreads();
     if (t < ne) {
       G.J_avg = element_ratio<T, NN>(L.r, ls);
-      element_material<T, NN, LAW, kCluster, false>(
+      element_material<T, NN, LAW, kCluster, false, false>(
           e, E, fp, dt, G, S, vol0, rho, He, tau, eps, nullptr, pl, false, nullptr, nullptr,
           reinterpret_cast<double *>(lds_raw) + t, [&](int a, int, T f0, T f1, T f2, T) {
             lf[0 * kEntStride(NN) + a * kCluster + t] = f0;
@@ -2059,9 +2059,14 @@ hipError_t launch_thermal(wfx_ctx *c, hipStream_t s);
 
 // Launch one phase (1..4) of a fused step on the current state with block
 // size BS; launch_fused_phase picks BS from the context (autotuned or 256).
-template <typename T, int NN, int LAW, bool PAIR>
+template <typename T, int NN, int LAW, bool PAIR, bool NT>
 auto f3_pick(bool th) {
-  return th ? f3_cluster<T, NN, LAW, true, PAIR> : f3_cluster<T, NN, LAW, false, PAIR>;
+  return th ? f3_cluster<T, NN, LAW, true, PAIR, NT> : f3_cluster<T, NN, LAW, false, PAIR, NT>;
+}
+template <typename T, bool PAIR, bool NT>
+auto f3_pick(int n, bool rate, bool th) {
+  return n == 8 ? (rate ? f3_pick<T, 8, LAW_RATE, PAIR, NT>(th) : f3_pick<T, 8, LAW_PLAIN, PAIR, NT>(th))
+                : (rate ? f3_pick<T, 4, LAW_RATE, PAIR, NT>(th) : f3_pick<T, 4, LAW_PLAIN, PAIR, NT>(th));
 }
 
 // the fused path's nodal arrays in the element real type
@@ -2110,8 +2115,9 @@ hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr
   fused_node_arrays<T>(c, vN, paN, udN, fiN);
   const FusedParams fp = element_params<T>(c, dtp);
   const bool rate = law_class(fp.mp.model) == LAW_RATE, th = c->thermal.on;
-  auto kern = (c->n == 8) ? (rate ? f3_pick<T, 8, LAW_RATE, PAIR>(th) : f3_pick<T, 8, LAW_PLAIN, PAIR>(th))
-                          : (rate ? f3_pick<T, 4, LAW_RATE, PAIR>(th) : f3_pick<T, 4, LAW_PLAIN, PAIR>(th));
+  auto kern = f3_pick<T, PAIR, false>(c->n, rate, th);
+  if constexpr (!PAIR)
+    if (c->stream_step) kern = f3_pick<T, false, true>(c->n, rate, th);
   hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, c->E, c->N, fp, cluster_args(c), pr, c->nd.x, vN,
                      c->nd.anp_ratio, el.vol0, el.rho, el.sy0, el.He, el.tau,
                      c->fused_tau_out ? (T *)c->fused_tau_out : el.tau, el.eps, el.p, el.pl_strain,
@@ -2282,7 +2288,8 @@ hipError_t launch_fused_phase_bs(wfx_ctx *c, int phase, int predict, int step, h
                          c->ms.nodel_count, c->ms.nodel_pk, el.vol, c->nd.rho_avg, c->nd.voln0_sum, c->nd.anp_ratio,
                          c->nd.mdiag, c->rho_uniform, cr, el.rho);
     } else {
-      hipLaunchKernelGGL((f2_nodal<T, BS>), dim3(gN + more), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
+      auto kern = c->stream_step ? f2_nodal<T, BS, true> : f2_nodal<T, BS, false>;
+      hipLaunchKernelGGL(kern, dim3(gN + more), dim3(BS), 0, s, N, c->n, c->ms.nodel_offset,
                          c->ms.nodel_count, c->ms.nodel_pk, c->ms.nodel_pad, el.vol, c->nd.rho_avg, c->nd.voln0_sum,
                          c->nd.anp_ratio, c->nd.mdiag, c->rho_uniform, cr, el.rho);
     }
