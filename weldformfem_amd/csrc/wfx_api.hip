@@ -282,15 +282,18 @@ static double step_bytes(const wfx_ctx *c, const ClusterTables &ct) {
   return E * 15 * es + S * (3 * es + 4) + N * (24 + 6 * es + (es == 8 ? 12 : 0) + 8 + es + 16 + 12) +
          4.0 * (c->f2_lanes ? E * c->n : 8 * N) + tables;
 }
-// The line between cached and non-temporal accesses, of the 256 MB last-level
-// cache.  Step of the separate passes, us, cached / non-temporal, by MB:
+// The lines between cached and non-temporal accesses: a step's data fits the 256
+// MB last-level cache, and is more than the L2s (32 MB) lose little on anyway.
+// Step of the separate passes, us, cached / non-temporal, by MB: FP64 hexahedra
+// 29 36.5 / 36.5, 41 (thermal, Johnson-Cook) 48.8 / 48.3, 59 43.8 / 44.3, 81 51.3 /
+// 53.8; FP32-mixed 47 41.1 / 42.0, 74 49.2 / 51.6;
 // FP64 hexahedra 170 79.6 / 85.3, 217 93.6 / 101.8, 246 118.8 / 112.5, 372 165 /
 // 153, 1319 576 / 549; FP64 tetrahedra 161 73.2 / 77.6, 219 88.9 / 94.3, 241
 // 108.7 / 100.7; FP32-mixed hexahedra 218 92.6 / 102.9, 237 107.2 / 110.9, 278
 // 128.7 / 123.7, 363 162 / 149; tetrahedra 196 85.1 / 91.1, 252 120 / 106.
 // (Between the two, the strains alone non-temporal: 99.4 at 241 MB, 92.1 at 219,
 // 109.2 at 252: no better than the better of the two by more than a percent.)
-constexpr double kCachedStepBytes = 240e6;
+constexpr double kCachedStepBytes[2] = {45e6, 240e6};
 
 // Tables of the paired passes; pw 0: the mesh takes the separate ones.
 // The line: 256 clusters, one work-group on each of the 256 CUs.  Below it the
@@ -349,7 +352,8 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
     return WFX_ERR_STATE;
   }
   const ClusterTables ct = cluster_tables(c, plan);
-  c->stream_step = step_bytes(c, ct) > kCachedStepBytes;
+  const double touched = step_bytes(c, ct);
+  c->stream_step = touched < kCachedStepBytes[0] || touched > kCachedStepBytes[1];
   A(c->ms.cl_desc, c->ms.ncl) A(c->ms.cl_goff, ct.goff.size()) A(c->ms.cl_ent, ct.ent.size())
   A(c->ms.cl_lslot, ct.lslot.size()) A(c->ms.cl_nrel, ct.nrel.size()) A(c->ms.nsl_off, N + 1)
   A(c->ms.cl_snode, c->ms.nslot)

@@ -58,10 +58,9 @@ __device__ __forceinline__ long fidx(int row, long e, long Es, int nrow) {
   return (e >> 6) * ((long)nrow * 64) + (long)row * 64 + (e & 63);
 }
 // Data a pass reads or writes once per step (stress, strain, yield stress; F2's
-// tables).  NT: a step touches more than the last-level cache keeps until the
-// next (wfx_ctx::stream_step), and non-temporal accesses keep these out of the
-// way of what the gathers and the next pass read again; a smaller mesh finds
-// them there in the next step.
+// tables).  NT: non-temporal accesses keep these out of the way of what the
+// gathers and the next pass read again; else the next step finds them in the
+// last-level cache (wfx_ctx::stream_step says which).
 template <bool NT, typename T>
 __device__ __forceinline__ void st_stream(T *p, T v) {
   if constexpr (NT) __builtin_nontemporal_store(v, p);
@@ -2115,9 +2114,9 @@ hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr
   fused_node_arrays<T>(c, vN, paN, udN, fiN);
   const FusedParams fp = element_params<T>(c, dtp);
   const bool rate = law_class(fp.mp.model) == LAW_RATE, th = c->thermal.on;
-  auto kern = f3_pick<T, PAIR, false>(c->n, rate, th);
+  auto kern = f3_pick<T, PAIR, true>(c->n, rate, th);
   if constexpr (!PAIR)
-    if (c->stream_step) kern = f3_pick<T, false, true>(c->n, rate, th);
+    if (!c->stream_step) kern = f3_pick<T, false, false>(c->n, rate, th);
   hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, c->E, c->N, fp, cluster_args(c), pr, c->nd.x, vN,
                      c->nd.anp_ratio, el.vol0, el.rho, el.sy0, el.He, el.tau,
                      c->fused_tau_out ? (T *)c->fused_tau_out : el.tau, el.eps, el.p, el.pl_strain,
