@@ -900,7 +900,7 @@ constexpr int kF3Lds = kF3Vals<T, NN, LAW, TH> > SlotLds<T, NN>::bytes ? kF3Vals
 // one part after the staging's loads, slot after slot and with the mass
 // summed from the densities, it added 6300 (hexahedra) and 12000
 // (tetrahedra) cycles to the staging's 1000.
-template <typename T, int NN, int SLOTS = kSlotsPerThread<NN>>
+template <typename T, int NN, int SLOTS>
 struct PairSum {
   // entries in flight: all of a structured hexahedral node's; up to 24 of a
   // tetrahedral one's
@@ -1013,8 +1013,8 @@ __device__ __forceinline__ void add_entries(const unsigned char *lds, const uint
 // thread summing its node's element volumes; slots of a node in several
 // clusters repeat the sum (1.7 times the work of F2), and a launch and F2's
 // round trip of the ratio are saved.
-template <typename T, int NN, int LAW, bool TH, bool PAIR, bool NT>
-__global__ __launch_bounds__(kCluster) void f3_cluster(
+template <typename T, int NN, int LAW, bool TH, bool PAIR, bool NT, int SL, int BS>
+__global__ __launch_bounds__(BS) void f3_cluster(
     int E, int N, FusedParams fp, ClusterArgs ca, PairArgs pr, const double *__restrict__ x, const T *__restrict__ v,
     const double *__restrict__ ratio, const T *__restrict__ vol0, const T *__restrict__ rho,
     const T *__restrict__ sy0, const T *__restrict__ He, const T *tau_in, T *tau_out, T *__restrict__ eps_io,
@@ -1029,16 +1029,16 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;  // M <= slot_cap(NN), checked at set-up
   const uint16_t *lo = ca.goff + cd.goff;
   const uint2 *en = ca.ent + cd.ent;  // the cluster's entry groups
-  // the nodes of this thread's slots t and t + kCluster: first, as the
+  // the nodes of this thread's slots t and t + BS: first, as the
   // staging loads depend on them
-  constexpr int kSl = kSlotsPerThread<NN>;
-  static_assert(kSl * kCluster == slot_cap(NN) && kSl <= 2, "one or two slots per thread");
+  constexpr int kSl = SL;
+  static_assert(kSl * BS <= slot_cap(NN) && kSl <= 2, "one or two slots per thread");
   // Every load below is issued unconditionally, threads past the cluster's
   // elements, entries or slots repeating its last one (a cluster has at
   // least one element and NN slots), so that none is waited for on its own;
   // the values are used only where they are the thread's own.
   // Loads return in order, so the order is that of the waits: the nodes of
-  // this thread's slots t and t + kCluster (PAIR: with their elements), the
+  // this thread's slots t and t + BS (PAIR: with their elements), the
   // slot tables and the element's slots; the nodal state; the element's own
   // state last, which only the second part of the chain needs.  That is the
   // order of the paired passes, whose work-groups run alone on their CUs.  In
@@ -1048,10 +1048,10 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
   int sn[kSl];
   int4 rec[kSl];
   bool mine[kSl];
-  PairSum<T, NN> ps;
+  PairSum<T, NN, SL> ps;
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
-    const int j = t + k * kCluster, q = s0 + min(j, M - 1);
+    const int j = t + k * BS, q = s0 + min(j, M - 1);
     if constexpr (PAIR) {
       rec[k] = pr.rec[q];
       sn[k] = rec[k].x;
@@ -1062,13 +1062,13 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
     }
   }
   if constexpr (PAIR) ps.entries(pr, 0);
-  // The entry groups' range of the thread's own slots t and t + kCluster; the
+  // The entry groups' range of the thread's own slots t and t + BS; the
   // groups themselves follow once these are here.
-  uint32_t ow[kSl];  // (end << 16) | start of slots t and t + kCluster
+  uint32_t ow[kSl];  // (end << 16) | start of slots t and t + BS
   int sp[kSl];       //   and where their sums go
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
-    const int q = min(t + k * kCluster, M - 1);
+    const int q = min(t + k * BS, M - 1);
     __builtin_memcpy(&ow[k], lo + q, 4);  // lo[q], lo[q + 1]
     if constexpr (kNodeMajor<T> || PAIR) sp[k] = ca.spos[s0 + q];
     else sp[k] = ca.nm ? ca.spos[s0 + q] : s0 + q;
@@ -1119,14 +1119,14 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
     // every work-group reduces the step's dt for itself, since a kernel for it
     // takes 3 us and the few partials of a small mesh less than one; the first
     // work-group stores it for the later kernels
-    if (pr.cr.cfl > 0.0) dt_step = cfl_reduce<kCluster>(pr.cr, rho, blockIdx.x == 0);
+    if (pr.cr.cfl > 0.0) dt_step = cfl_reduce<BS>(pr.cr, rho, blockIdx.x == 0);
   } else {
     if (fp.dtp) dt_step = *fp.dtp;
   }
   const T dt = (T)dt_step;
 #pragma unroll
   for (int k = 0; k < kSl; ++k) {
-    const int j = t + k * kCluster;  // < slot_cap
+    const int j = t + k * BS;  // < slot_cap
     L.node[j] = sn[k];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -1170,8 +1170,8 @@ __global__ __launch_bounds__(kCluster) void f3_cluster(
     for (int u = 0; u < R; ++u) lf[u * kEntStride(NN) + NN * kCluster] = T(0);
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kSl; ++r) {  // M <= kSl * kCluster
-    const int j = t + r * kCluster;
+  for (int r = 0; r < kSl; ++r) {  // M <= kSl * BS
+    const int j = t + r * BS;
     if (j >= M) break;
     const int k0 = ow[r] & 0xffffu, k1 = ow[r] >> 16;
     double acc[R];
@@ -1686,14 +1686,14 @@ struct NodeSet {  // the nodal arrays a paired node pass writes
   double *x;
   void *v, *pa, *ud;
 };
-template <typename T, int NN, bool CFL, bool CONTACT, bool TH>
-__global__ __launch_bounds__(slot_cap(NN)) void f41_cluster(
+template <typename T, int NN, bool CFL, bool CONTACT, bool TH, int SL>
+__global__ __launch_bounds__(SL * kCluster) void f41_cluster(
     int N, NodeParams np, ClusterArgs ca, PairArgs pr, NodeSet out, const double *__restrict__ cf,
     const T *__restrict__ part, const double *__restrict__ fe, const double *__restrict__ mdiag,
     const double *__restrict__ bc_val, T *__restrict__ fi, const T *__restrict__ v, const T *__restrict__ prev_a,
     const T *__restrict__ u_dt, const double *__restrict__ x, unsigned int *__restrict__ status,
     double *__restrict__ Tn, T *__restrict__ vol, double *__restrict__ minl_part, RigidArgs rg) {
-  constexpr int cap = slot_cap(NN);
+  constexpr int cap = SL * kCluster;
   __shared__ double lx[3 * cap];
   NodeParams q = np;
   if constexpr (CFL) set_step_length(q, *q.dtp);
@@ -1707,7 +1707,7 @@ __global__ __launch_bounds__(slot_cap(NN)) void f41_cluster(
   }
   const int c = xcd_block(nb), t = threadIdx.x;
   const ClusterDesc cd = ca.desc[c];
-  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;  // M <= slot_cap(NN), checked at set-up
+  const int e0 = cd.e0, s0 = cd.s0, ne = cd.em & 0xffff, M = cd.em >> 16;  // M <= cap, checked at set-up
   // as in the element pass every load is issued unconditionally: threads past
   // the cluster's slots or elements repeat its last one and store nothing
   const int4 rec = pr.rec[s0 + min(t, M - 1)];
@@ -2058,14 +2058,21 @@ hipError_t launch_thermal(wfx_ctx *c, hipStream_t s);
 
 // Launch one phase (1..4) of a fused step on the current state with block
 // size BS; launch_fused_phase picks BS from the context (autotuned or 256).
-template <typename T, int NN, int LAW, bool PAIR, bool NT>
-auto f3_pick(bool th) {
-  return th ? f3_cluster<T, NN, LAW, true, PAIR, NT> : f3_cluster<T, NN, LAW, false, PAIR, NT>;
+template <typename T, int NN, bool PAIR, bool NT, int SL, int BS>
+auto f3_pick(bool rate, bool th) {
+  return rate ? (th ? f3_cluster<T, NN, LAW_RATE, true, PAIR, NT, SL, BS> : f3_cluster<T, NN, LAW_RATE, false, PAIR, NT, SL, BS>)
+              : (th ? f3_cluster<T, NN, LAW_PLAIN, true, PAIR, NT, SL, BS> : f3_cluster<T, NN, LAW_PLAIN, false, PAIR, NT, SL, BS>);
 }
 template <typename T, bool PAIR, bool NT>
-auto f3_pick(int n, bool rate, bool th) {
-  return n == 8 ? (rate ? f3_pick<T, 8, LAW_RATE, PAIR, NT>(th) : f3_pick<T, 8, LAW_PLAIN, PAIR, NT>(th))
-                : (rate ? f3_pick<T, 4, LAW_RATE, PAIR, NT>(th) : f3_pick<T, 4, LAW_PLAIN, PAIR, NT>(th));
+auto f3_pick(int n, bool one_slot, bool rate, bool th) {
+  if (n == 4) return f3_pick<T, 4, PAIR, NT, 1, kCluster>(rate, th);
+  if constexpr (PAIR) {
+    // a thread per slot: one work-group on a CU, the second slot's loads and
+    // sums would only lengthen its chain
+    return one_slot ? f3_pick<T, 8, PAIR, NT, 1, kCluster>(rate, th) : f3_pick<T, 8, PAIR, NT, 1, 2 * kCluster>(rate, th);
+  } else {
+    return f3_pick<T, 8, PAIR, NT, 2, kCluster>(rate, th);
+  }
 }
 
 // the fused path's nodal arrays in the element real type
@@ -2114,10 +2121,11 @@ hipError_t launch_element_pass(wfx_ctx *c, const double *dtp, const PairArgs &pr
   fused_node_arrays<T>(c, vN, paN, udN, fiN);
   const FusedParams fp = element_params<T>(c, dtp);
   const bool rate = law_class(fp.mp.model) == LAW_RATE, th = c->thermal.on;
-  auto kern = f3_pick<T, PAIR, true>(c->n, rate, th);
+  auto kern = f3_pick<T, PAIR, true>(c->n, c->one_slot, rate, th);
   if constexpr (!PAIR)
-    if (!c->stream_step) kern = f3_pick<T, false, false>(c->n, rate, th);
-  hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(kCluster), 0, s, c->E, c->N, fp, cluster_args(c), pr, c->nd.x, vN,
+    if (!c->stream_step) kern = f3_pick<T, false, false>(c->n, false, rate, th);
+  const int bs = PAIR && c->n == 8 && !c->one_slot ? 2 * kCluster : kCluster;
+  hipLaunchKernelGGL(kern, dim3(c->ms.ncl), dim3(bs), 0, s, c->E, c->N, fp, cluster_args(c), pr, c->nd.x, vN,
                      c->nd.anp_ratio, el.vol0, el.rho, el.sy0, el.He, el.tau,
                      c->fused_tau_out ? (T *)c->fused_tau_out : el.tau, el.eps, el.p, el.pl_strain,
                      c->fused_pl_out ? (T *)c->fused_pl_out : el.pl_strain, el.sigma_y, el.part, c->thermal.on ? el.q_plheat : (T *)nullptr);
@@ -2168,14 +2176,14 @@ hipError_t launch_pair_element(wfx_ctx *c, int step, hipStream_t s) {
   return launch_contact<T>(c, vN, cfl, s);
 }
 
-template <typename T, int NN, bool CFL, bool CT>
+template <typename T, int NN, bool CFL, bool CT, int SL>
 auto f41_pick(bool th) {
-  return th ? f41_cluster<T, NN, CFL, CT, true> : f41_cluster<T, NN, CFL, CT, false>;
+  return th ? f41_cluster<T, NN, CFL, CT, true, SL> : f41_cluster<T, NN, CFL, CT, false, SL>;
 }
-template <typename T, int NN>
+template <typename T, int NN, int SL>
 auto f41_pick(bool cfl, bool ct, bool th) {
-  return cfl ? (ct ? f41_pick<T, NN, true, true>(th) : f41_pick<T, NN, true, false>(th))
-             : (ct ? f41_pick<T, NN, false, true>(th) : f41_pick<T, NN, false, false>(th));
+  return cfl ? (ct ? f41_pick<T, NN, true, true, SL>(th) : f41_pick<T, NN, true, false, SL>(th))
+             : (ct ? f41_pick<T, NN, false, true, SL>(th) : f41_pick<T, NN, false, false, SL>(th));
 }
 
 // the context's nodal arrays and the other set change places
@@ -2205,8 +2213,10 @@ hipError_t launch_pair_node(wfx_ctx *c, hipStream_t s) {
   NodeParams np = node_params(c, 1);
   np.dtp = cfl ? c->scalars + kCflDt : nullptr;
   np.vmax_part = c->cfl_part + c->cfl_cap_min;
-  auto kern = c->n == 8 ? f41_pick<T, 8>(cfl, ct, th) : f41_pick<T, 4>(cfl, ct, th);
-  hipLaunchKernelGGL(kern, dim3(c->ms.ncl + (ct ? 1 : 0)), dim3(slot_cap(c->n)), 0, s, c->N, np, cluster_args(c), pair_args<T>(c, -1),
+  auto kern = c->n == 4      ? f41_pick<T, 4, 1>(cfl, ct, th)
+              : c->one_slot ? f41_pick<T, 8, 1>(cfl, ct, th)
+                            : f41_pick<T, 8, 2>(cfl, ct, th);
+  hipLaunchKernelGGL(kern, dim3(c->ms.ncl + (ct ? 1 : 0)), dim3(c->one_slot ? kCluster : slot_cap(c->n)), 0, s, c->N, np, cluster_args(c), pair_args<T>(c, -1),
                      NodeSet{c->x_b, c->v_b, c->pa_b, c->ud_b}, c->contact.contforce, el.part, c->nd.fe,
                      c->nd.mdiag, c->bc_tab, fiN, vN, paN, udN, c->nd.x, c->status, c->nd.T, el.vol, c->cfl_part,
                      rigid_args(c, ct));

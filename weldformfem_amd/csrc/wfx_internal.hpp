@@ -282,6 +282,7 @@ struct wfx_ctx {
   int pair = 0;
   double *x_b = nullptr;
   void *v_b = nullptr, *pa_b = nullptr, *ud_b = nullptr;
+  bool one_slot = false;     // no cluster has more slots than a work-group of the element pass threads
   bool stream_step = false;  // once-per-step data is accessed non-temporally
   int f2_lanes = 0;          // the nodal volume sums take several lanes per node (many elements per node)
   double *scalars = nullptr;      // device scratch for reductions (reaction force)
