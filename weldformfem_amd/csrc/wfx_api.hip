@@ -1487,22 +1487,26 @@ static int check_run_status(wfx_ctx *c, hipStream_t st) {
 
 // One SolveChungHulbert loop body (Solver_explicit.C:524-978, CPU order);
 // with react_row the reaction nodes' forces after assembly are recorded there.
-static int step_api(wfx_ctx *c, hipStream_t st, double *react_row) {
+// predicted: the step before has made this one's prediction; predict: make the
+// next one's (not with the per-step CFL time step, whose host value the next
+// step's reductions set).
+static int step_api(wfx_ctx *c, hipStream_t st, double *react_row, bool predicted, bool predict) {
   // external face areas every 10 steps, at the step's start (Solver_explicit.C:446-451)
   if (c->contact.on && c->contact.step_count % 10 == 0) LAUNCH(contact_face_areas(c, st));
-  LAUNCH(launch_update_prediction(c, st));
-  for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, false, st));
+  if (!predicted) {
+    LAUNCH(launch_update_prediction(c, st));
+    for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, false, st));
+  }
   LAUNCH(BY_PRECISION(c, launch_elem_jacobians, c, st));
   if (c->prm.cfl > 0.0) {
     int rc = cfl_step(c, st);
     if (rc) return rc;
   }
   LAUNCH(BY_PRECISION(c, launch_elem_vol, c, st));
-  LAUNCH(BY_PRECISION(c, launch_nodal_vol, c, st));
-  LAUNCH(BY_PRECISION(c, launch_nodal_mass, c, st));
+  LAUNCH(BY_PRECISION(c, launch_node_sums, c, st));
   LAUNCH(BY_PRECISION(c, launch_strain_rates, c, st));
   if (c->thermal.on) LAUNCH(BY_PRECISION(c, launch_thermal_expansion, c, st));  // Solver_explicit.C:719-720
-  LAUNCH(BY_PRECISION(c, launch_pressure, c, st));
+  LAUNCH(BY_PRECISION(c, launch_pressure_elem, c, st));
   LAUNCH(BY_PRECISION(c, launch_stress_strain, c, c->prm.dt, st));
   LAUNCH(BY_PRECISION(c, launch_artificial_viscosity, c, st));
   LAUNCH(BY_PRECISION(c, launch_elem_forces, c, st));
@@ -1510,11 +1514,7 @@ static int step_api(wfx_ctx *c, hipStream_t st, double *react_row) {
   if (c->contact.on) LAUNCH(contact_forces(c, st));  // CalcContactForces (Solver_explicit.C:769-770)
   LAUNCH(BY_PRECISION(c, launch_assembly, c, st));
   if (react_row) LAUNCH(launch_reaction_gather(c, react_row, st));
-  LAUNCH(launch_calc_accel(c, st));
-  for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, true, st));
-  LAUNCH(launch_correction_accvel(c, st));
-  for (int d = 0; d < 3; ++d) LAUNCH(launch_impose(c, d, false, st));
-  LAUNCH(launch_correction_pos(c, st));
+  LAUNCH(launch_node_step(c, predict, st));
   if (c->contact.on) LAUNCH(contact_rigid_update(c, c->prm.dt, st));  // TriMesh_d::Move (:996-1004)
   if (c->thermal.on) LAUNCH(BY_PRECISION(c, launch_thermal, c, st));  // ThermalCalcs
   c->contact.step_count++;
@@ -1576,7 +1576,7 @@ extern "C" {
 int wfx_step_api(wfx_ctx *c, wfx_stream s) {
   REQUIRE_MESH(c);
   REQUIRE(c->initialized, WFX_ERR_STATE, "call wfx_init first");
-  return step_api(c, as_stream(s), nullptr);
+  return step_api(c, as_stream(s), nullptr, false, false);
 }
 
 int wfx_run(wfx_ctx *c, int nsteps, double *reaction_hist, wfx_stream s) {
@@ -1594,7 +1594,8 @@ int wfx_run(wfx_ctx *c, int nsteps, double *reaction_hist, wfx_stream s) {
   c->dt_hist_h.clear();
   const ReactRecord rec(c, dh, nsteps, sizeof(double));
   for (int k = 0; k < nsteps; ++k) {
-    int rc = step_api(c, st, (double *)rec.row(k));
+    const bool ahead = !(c->prm.cfl > 0.0);
+    int rc = step_api(c, st, (double *)rec.row(k), ahead && k > 0, ahead && k + 1 < nsteps);
     if (rc) return rc;
     if (rec.full(k)) LAUNCH(launch_reaction_rows<double>(c, rec, k, st));
   }

@@ -68,6 +68,15 @@ hipError_t launch_correction_pos(wfx_ctx *c, hipStream_t s) {
   return hipGetLastError();
 }
 
+hipError_t launch_node_step(wfx_ctx *c, bool predict, hipStream_t s) {
+  const auto &p = c->prm;
+  const NodeStep q{p.dt, p.alpha, p.beta, p.gamma, 1.0 / (1.0 - p.alpha), p.gamma * p.dt, p.beta * p.dt * p.dt, predict};
+  hipLaunchKernelGGL(k_node_step, dim3(nblocks(c->N)), dim3(kBlock), 0, s, c->N, q, c->nd.fe, c->nd.fi, c->nd.mdiag,
+                     c->contact.on ? c->contact.contforce : nullptr, c->bc_word, c->bc_tab, c->nd.a, c->nd.prev_a,
+                     c->nd.v, c->nd.u_dt, c->nd.x, c->nd.u);
+  return hipGetLastError();
+}
+
 hipError_t launch_reaction(wfx_ctx *c, int dim, double *dev_out, hipStream_t s) {
   if (c->ngroups == 0) return hipSuccess;
   hipLaunchKernelGGL((k_reaction<double>), dim3(c->ngroups), dim3(kBlock), 0, s, c->react_off, c->react,

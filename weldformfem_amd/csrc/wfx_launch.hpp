@@ -16,6 +16,8 @@ template <typename T> hipError_t launch_nodal_vol(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_nodal_mass(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_strain_rates(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_pressure(wfx_ctx *c, hipStream_t s);
+template <typename T> hipError_t launch_node_sums(wfx_ctx *c, hipStream_t s);  // CalcNodalVol, CalcNodalMassFromVol, ANP ratios
+template <typename T> hipError_t launch_pressure_elem(wfx_ctx *c, hipStream_t s);  // the element part alone
 template <typename T> hipError_t launch_stress_strain(wfx_ctx *c, double dt, hipStream_t s);
 template <typename T> hipError_t launch_artificial_viscosity(wfx_ctx *c, hipStream_t s);
 template <typename T> hipError_t launch_elem_forces(wfx_ctx *c, hipStream_t s);
@@ -33,6 +35,8 @@ template <typename T> hipError_t launch_energies(wfx_ctx *c, double *dev_out2, d
   template <> hipError_t launch_nodal_mass<T>(wfx_ctx *, hipStream_t);                           \
   template <> hipError_t launch_strain_rates<T>(wfx_ctx *, hipStream_t);                         \
   template <> hipError_t launch_pressure<T>(wfx_ctx *, hipStream_t);                             \
+  template <> hipError_t launch_node_sums<T>(wfx_ctx *, hipStream_t);                            \
+  template <> hipError_t launch_pressure_elem<T>(wfx_ctx *, hipStream_t);                        \
   template <> hipError_t launch_stress_strain<T>(wfx_ctx *, double, hipStream_t);                \
   template <> hipError_t launch_artificial_viscosity<T>(wfx_ctx *, hipStream_t);                 \
   template <> hipError_t launch_elem_forces<T>(wfx_ctx *, hipStream_t);                          \
@@ -132,6 +136,7 @@ hipError_t launch_impose(wfx_ctx *c, int dim, bool accel, hipStream_t s);
 hipError_t launch_calc_accel(wfx_ctx *c, hipStream_t s);
 hipError_t launch_correction_accvel(wfx_ctx *c, hipStream_t s);
 hipError_t launch_correction_pos(wfx_ctx *c, hipStream_t s);
+hipError_t launch_node_step(wfx_ctx *c, bool predict, hipStream_t s);
 hipError_t launch_reaction(wfx_ctx *c, int dim, double *dev_out, hipStream_t s);
 hipError_t launch_min_edge(wfx_ctx *c, double *partial, double *dev_out, hipStream_t s);
 int min_edge_partial_count(wfx_ctx *c);
