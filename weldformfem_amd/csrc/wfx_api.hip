@@ -305,15 +305,6 @@ constexpr double kCachedStepBytes[2] = {45e6, 240e6};
 // separate passes never take less than the 17 us their four launches cost.
 constexpr int kPairMaxClusters = 256;
 constexpr int kPairMaxElems = 32;  // elements of a node
-// FP64 hexahedra: clusters of 64, or else 128, elements and at most 256 slots
-// while there is a CU for each.  Half the CUs or more are idle otherwise, and a
-// work-group's LDS passes and its second slot per thread are what its chain
-// waits for.  Eager / graph, us per step, at 256 elements a cluster and so: 8^3
-// 14.4 / 13.0 and 12.5 / 10.8, 20^3 15.0 / 13.5 and 12.8 / 11.6, 25^3 15.8 / 14.3
-// and 13.3 / 12.4, 32^3 (256 of 128) 16.0 / 15.8 and 13.6 / 13.7.  Tetrahedra, a
-// third of the slots and one a thread anyway: 12 cells 12.9 / 11.6 and 13.5 /
-// 12.0, 20 cells 13.5 / 12.5 and 17.8 / 16.5.
-constexpr int kSmallCluster = 64;
 // Entries per slot of the paired passes' table, or 0
 static int pair_width(const wfx_ctx *c, const ClusterPlan &plan) {
   if (plan.clusters() > kPairMaxClusters || c->nodel_count_h.empty()) return 0;
@@ -472,16 +463,7 @@ static int finish_mesh(wfx_ctx *c) {
   // FP32-mixed rounds each partial sum to a float, so that another cut gives
   // other results (1e-4 of the stresses after some hundred steps); FP64's differ
   // by rounding only
-  const bool fp64 = c->precision == WFX_FP64;
-  int cs = fp64 && c->n == 8 && c->E > kCluster ? kSmallCluster : kCluster;
-  for (;; cs *= 2) {
-    const bool small = cs < kCluster;
-    if (small && c->E > cs * kPairMaxClusters) continue;
-    plan = ClusterPlan();
-    plan_clusters(c->N, c->E, c->n, c->elnod_h.data(), c->x_h.data(), cs, plan, fp64, small ? kCluster : 0);
-    if (small && plan.max_component <= kCluster) cs = kCluster / 2;  // the solo pass takes whole components
-    else if (!small || plan.clusters() <= kPairMaxClusters) break;
-  }
+  plan_clusters(c->N, c->E, c->n, c->elnod_h.data(), c->x_h.data(), kCluster, plan, c->precision == WFX_FP64);
   c->el_s2o.swap(plan.s2o);
   c->el_o2s.swap(plan.o2s);
   int rc = setup_device(c, plan);

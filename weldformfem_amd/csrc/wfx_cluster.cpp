@@ -180,8 +180,7 @@ void count_runs(NodeCounter &nodes, int a, int b, int cs, int cap, double &clust
 }  // namespace
 
 int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs, ClusterPlan &p,
-                  bool even, int cap) {
-  if (cap <= 0) cap = slot_cap(n);
+                  bool even) {
   // connected components (elements sharing a node), ordered by their first element
   std::vector<int> parent(N);
   std::iota(parent.begin(), parent.end(), 0);
@@ -201,7 +200,6 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
   }
   std::vector<int> coff(ncomp + 1, 0);
   for (int e = 0; e < E; ++e) ++coff[comp[e] + 1];
-  p.max_component = ncomp ? *std::max_element(coff.begin(), coff.end()) : 0;
   for (int k = 0; k < ncomp; ++k) coff[k + 1] += coff[k];
   std::vector<int> byc(E);
   {
@@ -283,8 +281,8 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
     // they win by 1% (100 x 99 x 51, 200 x 200 x 100).
     if (even && b - a > cs && per_cell == 1.0 && (double)ext[0] * ext[1] * ext[2] == (double)(b - a)) {
       double clusters, slots;
-      count_runs(nodes, a, b, cs, cap, clusters, slots);
-      const BlockSplit sp = split_block(ext, cs, cap);
+      count_runs(nodes, a, b, cs, slot_cap(n), clusters, slots);
+      const BlockSplit sp = split_block(ext, cs, slot_cap(n));
       if (sp.slots() + 250.0 * sp.clusters() < slots + 250.0 * clusters) {
         for (int q = a; q < b; ++q) {
           const int e = byc[q];
@@ -304,8 +302,8 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
   }
   p.o2s.resize(E);
   for (int s = 0; s < E; ++s) p.o2s[p.s2o[s]] = s;
-  // slot counts; a cluster touching more than cap nodes is halved until none
-  // does (a single element has n <= cap nodes)
+  // slot counts; a cluster touching more than slot_cap(n) nodes is halved
+  // until none does (a single element has n <= slot_cap(n) nodes)
   std::vector<int> m;
   for (;;) {
     const int C = p.clusters();
@@ -317,7 +315,7 @@ int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs
     std::vector<int> eoff(1, 0);
     bool split = false;
     for (int c = 0; c < C; ++c) {
-      if (m[c] > cap) {
+      if (m[c] > slot_cap(n)) {
         eoff.push_back(p.eoff[c] + (p.eoff[c + 1] - p.eoff[c]) / 2);
         split = true;
       }

@@ -31,7 +31,6 @@ struct ClusterPlan {
   std::vector<int> spos;       // [S] slot -> its position k in nsl (nsl[spos[s]] = s)
   std::vector<int> snode;      // [S] slot -> its node (ascending node within a cluster)
   std::vector<uint16_t> lslot; // [E][n] stored element's nodes as slot indices within its cluster
-  int max_component = 0;       // elements of the largest connected component
   int max_slots = 0;           // largest slot count of a cluster (<= slot_cap(n))
   int clusters() const { return (int)eoff.size() - 1; }
   long slots() const { return sbase.empty() ? 0 : sbase.back(); }
@@ -43,9 +42,8 @@ struct ClusterPlan {
 constexpr int slot_cap(int n) { return n == 8 ? 512 : 256; }
 
 // Plan for elnod [E][n] (original order, nodes in [0, N)) with node
-// coordinates x [N][3]; cs <= 256 elements and at most cap slots per cluster (0:
-// slot_cap(n)); even: a structured block may be split evenly.  Returns 0.
-int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs, ClusterPlan &p, bool even = true,
-                  int cap = 0);
+// coordinates x [N][3]; cs <= 256 elements per cluster; even: a structured block
+// may be split evenly.  Returns 0.
+int plan_clusters(int N, int E, int n, const int *elnod, const double *x, int cs, ClusterPlan &p, bool even = true);
 
 }  // namespace wfx
