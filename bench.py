@@ -28,7 +28,7 @@ I4 = 4
 
 
 def fused_bytes(n, s, slots_per_elem, clusters_per_elem, hg=True, rho_uniform=True, over8_per_node=0.0,
-                f2_lanes=False):
+                f2_lanes=False, shared_tables=False):
     """Algorithmic bytes per element and per node of the fused kernels: each
     array a kernel touches is moved once, gathered nodal data once per node.
     s = element real size (8 FP64, 4 FP32-mixed); nodal positions are
@@ -43,7 +43,9 @@ def fused_bytes(n, s, slots_per_elem, clusters_per_elem, hg=True, rho_uniform=Tr
     slot's node id (int32), and gather the nodal data once per node.  The
     element pass writes one partial force per slot: FP64 in slot order (the
     node pass reads the node's slot ids), FP32-mixed node-major (it reads
-    each slot's position instead, the node pass none)."""
+    each slot's position instead, the node pass none).  shared_tables: clusters
+    with equal slot tables share them (the bricks of a structured block), which
+    then stay in the caches and are not counted."""
     rho = 1 if (hg and not rho_uniform) else 0
     sn = s
     spe, cpe = slots_per_elem, clusters_per_elem
@@ -51,15 +53,15 @@ def fused_bytes(n, s, slots_per_elem, clusters_per_elem, hg=True, rho_uniform=Tr
     # (u from it when a run ends); FP32-mixed recovers u from x alone
     u_rw = 2 * 3 * 4 if s == 8 else 0
     node_major = s == 4
-    stage = 2 * n + I4 * spe  # slot indices of the element's nodes, node id per slot
+    # slot indices of the element's nodes, node id per slot; slot entries (uint16
+    # per element-node), slot offsets (uint16 per slot and per cluster)
+    stage, entries = (0, 0) if shared_tables else (2 * n + I4 * spe, 2 * n + 2 * (spe + cpe))
     # tau, eps read and written; plastic strain read and written; sy0;
     # [rho] (pressure and yield stress are stored on a run's last step only)
     f3_reals = 12 + 12 + 2 + 1 + rho
-    # staging, element reals, slot entries (uint16 per element-node), slot
-    # offsets (uint16 per slot and per cluster), [slot positions], partial
-    # forces per slot
-    f3_elem = (stage + f3_reals * s + 2 * n + 2 * (spe + cpe) + (I4 * spe if node_major else 0)
-               + 3 * s * spe)
+    # staging, element reals, slot entries, [slot positions], partial forces
+    # per slot
+    f3_elem = stage + f3_reals * s + entries + (I4 * spe if node_major else 0) + 3 * s * spe
     return {
         "f1_volume": (stage + s, 3 * 8),
         # vol gathered (V_n once per run), [rho]; padded first-8 table, count,
@@ -79,11 +81,12 @@ def fused_bytes(n, s, slots_per_elem, clusters_per_elem, hg=True, rho_uniform=Tr
 
 
 def domain_fused_bytes(d, s, hg=True):
-    """fused_bytes for domain d (its slots, clusters and node valences)"""
+    """fused_bytes for domain d (its slots, clusters and node valences); the
+    hexahedral workloads are structured blocks"""
     N, E, n = d.sizes()
     cnt = d.field("nodel_count")
     return fused_bytes(n, s, d.get("slot_count") / E, d.get("cluster_count") / E, hg=hg,
-                       over8_per_node=float(np.mean(cnt > 8)), f2_lanes=n * E > 12 * N)
+                       over8_per_node=float(np.mean(cnt > 8)), f2_lanes=n * E > 12 * N, shared_tables=n == 8)
 
 
 def api_bytes(n, s, hg=True):

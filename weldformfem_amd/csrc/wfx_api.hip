@@ -299,9 +299,9 @@ constexpr double kCachedStepBytes[2] = {45e6, 240e6};
 // The line: 256 clusters, one work-group on each of the 256 CUs.  Below it the
 // launches and dependent loads count and the repeated node updates (1.7 times,
 // hexahedra) are free; above it they are not.  Measured in graph replay, us per
-// step, paired / separate: FP64 hexahedra 1 element 10.2 / 11.2, 20^3 13.4 /
-// 15.2, 30^3 (106 clusters) 15.5 / 16.9, 50^3 (489) 34.4 / 30.6; tetrahedra 8
-// cells 11.2 / 12.8, 27 cells (363) 17.8 / 17.9.  Launched one by one the
+// step, paired / separate: FP64 hexahedra 1 element 10.2 / 11.2 (now the solo
+// pass), 20^3 12.9 / 15.2, 30^3 (120 clusters) 15.4 / 16.9, 50^3 (489) 34.4 / 30.6;
+// tetrahedra 8 cells 11.2 / 12.8, 27 cells (363) 17.8 / 17.9.  Launched one by one the
 // separate passes never take less than the 17 us their four launches cost.
 constexpr int kPairMaxClusters = 256;
 constexpr int kPairMaxElems = 32;  // elements of a node

@@ -293,7 +293,7 @@ class Domain:
         return self._hist(nsteps, hist)
 
     def runFused(self, nsteps, reaction=True):
-        """nsteps steps through the four-kernel fused path (wfx_step_fused)"""
+        """nsteps steps through the fused path (wfx_step_fused)"""
         ng = max(self.reactionGroupCount(), 1)
         hist = np.zeros(max(int(nsteps), 1) * ng, dtype=np.float64)
         check(self._L.wfx_step_fused(self._h, int(nsteps), hist.ctypes.data if reaction else None,
