@@ -296,18 +296,21 @@ static double step_bytes(const wfx_ctx *c, const ClusterTables &ct) {
 constexpr double kCachedStepBytes[2] = {45e6, 240e6};
 
 // Tables of the paired passes; pw 0: the mesh takes the separate ones.
-// The line: 256 clusters, one work-group on each of the 256 CUs.  Below it the
-// launches and dependent loads count and the repeated node updates (1.7 times,
-// hexahedra) are free; above it they are not.  Measured in graph replay, us per
-// step, paired / separate: FP64 hexahedra 1 element 10.2 / 11.2 (now the solo
-// pass), 20^3 12.9 / 15.2, 30^3 (120 clusters) 15.4 / 16.9, 50^3 (489) 34.4 / 30.6;
-// tetrahedra 8 cells 11.2 / 12.8, 27 cells (363) 17.8 / 17.9.  Launched one by one the
-// separate passes never take less than the 17 us their four launches cost.
-constexpr int kPairMaxClusters = 256;
+// The line: in FP64 256 clusters, one work-group on each of the 256 CUs, in
+// FP32-mixed 512, two.  Below it the launches and dependent loads count and the
+// repeated node updates (1.7 times, hexahedra) are free; above it they are not.
+// us per step in graph replay, paired / separate: FP64 hexahedra 1 element 10.2 /
+// 11.2 (now the solo pass), 20^3 12.9 / 15.2, 40^3 (250 clusters) 17.4 / 20.9,
+// 42^3 (297) 26.2 / 24.1; tetrahedra 24 cells (255) 14.1 / 16.2, 32 cells 23.5 /
+// 21.6.  FP32-mixed hexahedra 40^3 14.6 / 18.4, 44^3 19.2 / 20.2, 48^3 (432) 19.2 /
+// 21.2, 50^3 (about 512) 27.1 / 24.5; tetrahedra 27 cells (363) 15.2 / 15.7, 30
+// cells (498) 15.9 / 16.5, 32 cells 18.5 / 17.9.  Launched one by one the separate
+// passes never take less than the 17 us their four launches cost.
+constexpr int kPairMaxClusters[2] = {256, 512};  // FP64, FP32-mixed
 constexpr int kPairMaxElems = 32;  // elements of a node
 // Entries per slot of the paired passes' table, or 0
 static int pair_width(const wfx_ctx *c, const ClusterPlan &plan) {
-  if (plan.clusters() > kPairMaxClusters || c->nodel_count_h.empty()) return 0;
+  if (plan.clusters() > kPairMaxClusters[c->precision == WFX_FP64 ? 0 : 1] || c->nodel_count_h.empty()) return 0;
   const auto mm = std::minmax_element(c->nodel_count_h.begin(), c->nodel_count_h.end());
   // a node of no element has no slot: only the separate node pass reaches it
   if (*mm.second > kPairMaxElems || *mm.first == 0) return 0;
