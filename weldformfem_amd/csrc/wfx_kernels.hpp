@@ -497,22 +497,25 @@ __global__ __launch_bounds__(kBlock) void k_init_elem(int E, const T *__restrict
 // not positive and finite or an initial volume not finite or (nearly) zero,
 // the smallest density as ordered bits (positive doubles; scan[1] 0) and the
 // first one.  The first three cleared to {0, 0, all ones} by the caller.
+// Bound: the atomics, 65 ns each on the one address, so few work-groups of
+// many elements (scan_blocks): 93k elements @S1, 4M @S2.
+inline int scan_blocks(int E) { return std::min(256, std::max(1, nblocks(E) / 8)); }
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_scan_elem(int E, const T *__restrict__ rho, const T *__restrict__ vol0,
                                                       unsigned long long *__restrict__ scan) {
-  const int e = gtid();
   const double first = (double)rho[0];
-  double r = first;
-  bool bad = false;
-  if (e < E) {
-    r = (double)rho[e];
-    const double v = fabs((double)vol0[e]);
-    bad = !(r > 0.0 && r <= DBL_MAX) || !(v >= 1e-200 && v <= DBL_MAX);
+  double m = first;
+  bool bad = false, differs = false;
+  for (int e = blockIdx.x * kBlock + threadIdx.x; e < E; e += gridDim.x * kBlock) {
+    const double r = (double)rho[e], v = fabs((double)vol0[e]);
+    differs |= !(r == first);
+    bad |= !(r > 0.0 && r <= DBL_MAX) || !(v >= 1e-200 && v <= DBL_MAX);
+    m = fmin(m, r);
   }
-  if (__any(!(r == first)) && (threadIdx.x & 63) == 0) atomicOr(scan, 1ull);
-  if (__any(bad) && (threadIdx.x & 63) == 0) atomicOr(scan + 1, 1ull);
-  if (e == 0) scan[3] = (unsigned long long)__double_as_longlong(first);
-  const double m = block_extreme<kBlock, true>(r);
+  if (__syncthreads_or(differs) && threadIdx.x == 0) atomicOr(scan, 1ull);
+  if (__syncthreads_or(bad) && threadIdx.x == 0) atomicOr(scan + 1, 1ull);
+  if (blockIdx.x == 0 && threadIdx.x == 0) scan[3] = (unsigned long long)__double_as_longlong(first);
+  m = block_extreme<kBlock, true>(m);
   if (threadIdx.x == 0) atomicMin(scan + 2, (unsigned long long)__double_as_longlong(m));
 }
 
@@ -1433,7 +1436,7 @@ template <typename T> hipError_t launch_scan_elem(wfx_ctx *c, unsigned long long
   template <> hipError_t launch_scan_elem<T>(wfx_ctx * c, unsigned long long *scan,                \
                                              hipStream_t s) {                                      \
     auto &el = elem<T>(c);                                                                         \
-    hipLaunchKernelGGL((k_scan_elem<T>), dim3(nblocks(c->E)), dim3(kBlock), 0, s, c->E, el.rho,    \
+    hipLaunchKernelGGL((k_scan_elem<T>), dim3(scan_blocks(c->E)), dim3(kBlock), 0, s, c->E, el.rho,\
                        el.vol0, scan);                                                             \
     return hipGetLastError();                                                                      \
   }                                                                                                \
