@@ -1,0 +1,299 @@
+// What the library's host code asks of the HIP runtime, without a GPU: this
+// program defines the runtime functions libwfx.so imports, so that the library
+// binds to them, and runs the C-ABI over them.  Device memory is host memory
+// filled with 0xff when allocated (a NaN in every double), memory copies and
+// fills are done, kernels are noted by name and not run but for the few below.
+// Usage: host_calls_check LIBRARY CHECK; prints what is wrong, exit code 0 if
+// nothing is.
+#include <dlfcn.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "../../include/wfx.h"
+
+namespace {
+
+struct Dim3 {
+  uint32_t x, y, z;
+};
+struct Kernel {
+  std::string name;
+  int device;
+  void *stream;
+  bool captured;
+};
+
+std::mutex mu;
+std::map<const void *, std::string> kernel_names;
+std::vector<Kernel> launched;
+std::function<void(const std::string &, void **)> on_launch;
+int current = 0;  // device
+bool capturing = false;
+std::map<void *, std::pair<size_t, int>> device_mem;  // bytes, device
+int wrong = 0;
+
+#define EXPECT(cond, ...)      \
+  do {                         \
+    if (!(cond)) {             \
+      ++wrong;                 \
+      std::printf(__VA_ARGS__); \
+      std::printf("\n");       \
+    }                          \
+  } while (0)
+
+bool is(const std::string &name, const char *kernel) { return name.find(kernel) != std::string::npos; }
+template <typename T>
+T arg(void **args, int k) {
+  T v;
+  std::memcpy(&v, args[k], sizeof(T));
+  return v;
+}
+
+thread_local struct {
+  Dim3 grid, block;
+  size_t shmem;
+  void *stream;
+} pushed;
+
+}  // namespace
+
+extern "C" {
+void **__hipRegisterFatBinary(const void *) {
+  static void *modules = nullptr;
+  return &modules;
+}
+void __hipUnregisterFatBinary(void **) {}
+void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *,
+                           void *, int *) {
+  kernel_names[host] = name;
+}
+void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
+int __hipPushCallConfiguration(Dim3 grid, Dim3 block, size_t shmem, void *stream) {
+  pushed = {grid, block, shmem, stream};
+  return 0;
+}
+int __hipPopCallConfiguration(Dim3 *grid, Dim3 *block, size_t *shmem, void **stream) {
+  *grid = pushed.grid;
+  *block = pushed.block;
+  *shmem = pushed.shmem;
+  *stream = pushed.stream;
+  return 0;
+}
+int hipLaunchKernel(const void *host, Dim3, Dim3, void **args, size_t, void *stream) {
+  std::lock_guard<std::mutex> l(mu);
+  const std::string &name = kernel_names[host];
+  launched.push_back({name, current, stream, capturing});
+  if (on_launch) on_launch(name, args);
+  return 0;
+}
+int hipGetDeviceCount(int *n) {
+  *n = 2;
+  return 0;
+}
+int hipGetDevice(int *d) {
+  *d = current;
+  return 0;
+}
+int hipSetDevice(int d) {
+  current = d;
+  return 0;
+}
+int hipMalloc(void **p, size_t bytes) {
+  *p = std::aligned_alloc(256, (bytes + 255) / 256 * 256);
+  std::memset(*p, 0xff, bytes);
+  device_mem[*p] = {bytes, current};
+  return 0;
+}
+int hipFree(void *p) {
+  device_mem.erase(p);
+  std::free(p);
+  return 0;
+}
+int hipHostMalloc(void **p, size_t bytes, unsigned) {
+  *p = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
+  return 0;
+}
+int hipHostFree(void *p) {
+  std::free(p);
+  return 0;
+}
+int hipMemset(void *p, int v, size_t bytes) {
+  std::memset(p, v, bytes);
+  return 0;
+}
+int hipMemcpy(void *d, const void *s, size_t bytes, int) {
+  std::memcpy(d, s, bytes);
+  return 0;
+}
+int hipMemcpyAsync(void *d, const void *s, size_t bytes, int, void *) {
+  std::memcpy(d, s, bytes);
+  return 0;
+}
+int hipGetSymbolAddress(void **p, const void *) {
+  static char scratch[1 << 20];
+  *p = scratch;
+  return 0;
+}
+int hipGetLastError() { return 0; }
+const char *hipGetErrorString(int) { return "error"; }
+int hipDeviceSynchronize() { return 0; }
+int hipStreamSynchronize(void *) { return 0; }
+int hipStreamWaitEvent(void *, void *, unsigned) { return 0; }
+int hipStreamCreate(void **s) {
+  *s = std::malloc(1);
+  return 0;
+}
+int hipStreamDestroy(void *s) {
+  std::free(s);
+  return 0;
+}
+int hipStreamIsCapturing(void *, int *status) {
+  *status = capturing ? 1 : 0;
+  return 0;
+}
+int hipStreamBeginCapture(void *, int) {
+  capturing = true;
+  return 0;
+}
+int hipStreamEndCapture(void *, void **graph) {
+  capturing = false;
+  *graph = std::malloc(1);
+  return 0;
+}
+int hipGraphInstantiate(void **exec, void *, void **, char *, size_t) {
+  *exec = std::malloc(1);
+  return 0;
+}
+int hipGraphLaunch(void *, void *) { return 0; }
+int hipGraphDestroy(void *g) {
+  std::free(g);
+  return 0;
+}
+int hipGraphExecDestroy(void *g) {
+  std::free(g);
+  return 0;
+}
+int hipEventCreateWithFlags(void **e, unsigned) {
+  *e = std::malloc(1);
+  return 0;
+}
+int hipEventCreate(void **e) { return hipEventCreateWithFlags(e, 0); }
+int hipEventDestroy(void *e) {
+  std::free(e);
+  return 0;
+}
+int hipEventRecord(void *, void *) { return 0; }
+int hipEventSynchronize(void *) { return 0; }
+int hipEventElapsedTime(float *ms, void *, void *) {
+  *ms = 1.0f;
+  return 0;
+}
+}  // extern "C"
+
+namespace {
+
+void *library;
+template <typename F>
+F *entry(const char *name) {
+  void *p = dlsym(library, name);
+  if (!p) {
+    std::printf("%s is not exported\n", name);
+    std::exit(2);
+  }
+  return reinterpret_cast<F *>(p);
+}
+// CALL(wfx_set_dt, c, dt): the entry point, which has to succeed
+#define CALL(fn, ...)                                                                                              \
+  do {                                                                                                             \
+    const int rc = entry<decltype(fn)>(#fn)(__VA_ARGS__);                                                          \
+    EXPECT(rc == 0, "%s returned %d: %s", #fn, rc, entry<decltype(wfx_last_error)>("wfx_last_error")());           \
+  } while (0)
+
+// n x n x n hexahedra and, with stray, a node of no element behind them
+struct Box {
+  std::vector<double> x;
+  std::vector<int> el;
+  int nodes, elems;
+  explicit Box(int n, bool stray = false) {
+    const int m = n + 1;
+    for (int k = 0; k < m; ++k)
+      for (int j = 0; j < m; ++j)
+        for (int i = 0; i < m; ++i) x.insert(x.end(), {0.1 * i, 0.1 * j, 0.1 * k});
+    for (int k = 0; k < n; ++k)
+      for (int j = 0; j < n; ++j)
+        for (int i = 0; i < n; ++i) {
+          const int a = (k * m + j) * m + i, b = a + m * m;
+          el.insert(el.end(), {a, a + 1, a + m + 1, a + m, b, b + 1, b + m + 1, b + m});
+        }
+    if (stray) x.insert(x.end(), {5.0, 5.0, 5.0});
+    nodes = (int)x.size() / 3;
+    elems = (int)el.size() / 8;
+  }
+};
+
+wfx_ctx *domain(const Box &b, int precision = WFX_FP64) {
+  wfx_ctx *c = nullptr;
+  CALL(wfx_create, &c, precision);
+  CALL(wfx_set_mesh, c, b.nodes, b.elems, 8, b.x.data(), b.el.data());
+  CALL(wfx_set_density, c, 7850.0);
+  CALL(wfx_set_material, c, WFX_BILINEAR, 200e9, 0.3, 7850.0, 300e6, 1e9, 0.0);
+  CALL(wfx_set_dt, c, 1e-6);
+  return c;
+}
+
+// Every entry of the step length's cotangent the gradient sums with a per-step
+// time step is one a kernel wrote or was cleared: a node of no element is in no
+// cluster, so that no cluster kernel writes its entry.
+void adjoint_stray() {
+  const Box b(3, true);
+  wfx_ctx *c = domain(b);
+  const int reaction[2] = {0, 1}, stray = b.nodes - 1;
+  for (int d = 0; d < 3; ++d) CALL(wfx_add_bc_vel_node, c, stray, d, 0.0);
+  CALL(wfx_allocate_bcs, c);
+  CALL(wfx_set_reaction_nodes, c, reaction, 2);
+  CALL(wfx_set_cfl, c, 0.3);
+  CALL(wfx_init, c, nullptr);
+  int summed = 0;
+  on_launch = [&](const std::string &name, void **args) {
+    if (!is(name, "a_cfl_apply")) return;
+    ++summed;
+    const double *dtb = arg<const double *>(args, 4);
+    EXPECT(dtb[stray] == 0.0, "the cotangent of the step length sums %g for the node of no element", dtb[stray]);
+  };
+  const int n = 3;
+  std::vector<double> hist(n), bar(n, 1.0), grad(3);
+  CALL(wfx_adjoint_forward, c, n, 2, hist.data(), nullptr);
+  CALL(wfx_adjoint_backward, c, bar.data(), grad.data(), nullptr, nullptr, nullptr, nullptr);
+  EXPECT(summed == n, "the cotangent of the step length was summed %d times in %d steps", summed, n);
+  CALL(wfx_destroy, c);
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const std::map<std::string, void (*)()> checks = {
+      {"adjoint_stray", adjoint_stray},
+  };
+  if (argc != 3 || !checks.count(argv[2])) return 2;
+  library = dlopen(argv[1], RTLD_NOW);
+  if (!library) {
+    std::printf("%s\n", dlerror());
+    return 2;
+  }
+  if (kernel_names.empty()) {  // the library bound to the HIP runtime itself
+    std::printf("the library did not register its kernels here\n");
+    return 2;
+  }
+  checks.at(argv[2])();
+  return wrong ? 1 : 0;
+}

@@ -1,0 +1,33 @@
+"""What the library's host code asks of the HIP runtime, over a stand-in for
+it (native/host_calls_check.cpp): runs without a GPU.
+
+* adjoint_stray: the gradient with a per-step time step sums no entry that
+  nothing wrote, also for a node of no element.
+"""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from weldformfem_amd import _lib
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SRC = os.path.join(HERE, "native", "host_calls_check.cpp")
+
+
+@pytest.fixture(scope="module")
+def checker(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if not gxx:
+        pytest.skip("g++ not available")
+    out = str(tmp_path_factory.mktemp("host_calls") / "host_calls_check")
+    subprocess.run([gxx, "-O1", "-std=c++17", "-pthread", "-rdynamic", SRC, "-ldl", "-o", out], check=True,
+                   capture_output=True)
+    return out
+
+
+@pytest.mark.parametrize("check", ["adjoint_stray"])
+def test_host_calls(checker, check):
+    r = subprocess.run([checker, _lib.LIB_PATH, check], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr

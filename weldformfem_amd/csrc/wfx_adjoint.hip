@@ -753,6 +753,9 @@ static int adj_alloc(wfx_ctx *c, int nsteps, int every) {
     get(&A->p1[0], 7 * S); get(&A->p1[1], 7 * S); get(&A->p2, 3 * S); get(&A->volb, E); get(&A->grad, 3 * E);
     get(&A->sy0d, E); get(&A->Hd, E); get(&A->rhod, E); get(&A->rho_avg, N); get(&A->sums, 8 + E);
     get(&A->dts, nsteps); get(&A->dtb, N + E); get(&A->cfl_loc, 8); get(&A->lawc, 5 * E);
+    // summed whole (a_cfl_apply), but written for the nodes of some cluster only:
+    // a node of no element has no share
+    if (err == hipSuccess) err = hipMemset(A->dtb, 0, (size_t)(N + E) * sizeof(double));
     if (err == hipSuccess) {
       void *q = nullptr;
       err = hipMalloc(&q, std::max<long>(N, 1) * sizeof(int));
