@@ -278,11 +278,47 @@ void adjoint_stray() {
   CALL(wfx_destroy, c);
 }
 
+// The nodal mean densities a phase-2 call reads belong to the present
+// densities: formed by an earlier kernel that ran, not by one that a capture
+// only recorded; once per captured run.
+void densities_captured() {
+  const Box b(3);
+  void *stream = nullptr;
+  hipStreamCreate(&stream);
+  wfx_ctx *c = domain(b);
+  CALL(wfx_init, c, nullptr);
+  CALL(wfx_step_fused, c, 3, nullptr, stream);
+  const std::vector<double> rho(b.elems, 7000.0);
+  CALL(wfx_set_field, c, "rho", rho.data(), (long)rho.size());
+  const auto formed = [&](bool captured) {
+    return std::count_if(launched.begin(), launched.end(), [&](const Kernel &k) {
+      return k.captured == captured && is(k.name, "f0_vsum0");
+    });
+  };
+  launched.clear();
+  CALL(wfx_graph_capture, c, 4, 0, stream);
+  EXPECT(formed(true) == 1, "the means are formed %ld times in a captured run", (long)formed(true));
+  CALL(wfx_fused_phase, c, 1, 0, stream);
+  CALL(wfx_fused_phase, c, 2, 0, stream);
+  EXPECT(formed(false) == 1, "phase 2 after a capture reads the means of the densities before it");
+  CALL(wfx_fused_phase, c, 2, 0, stream);
+  EXPECT(formed(false) == 1, "two phase-2 calls form the means %ld times", (long)formed(false));
+  // the caller's own capture: each replay meets the densities of its time
+  launched.clear();
+  hipStreamBeginCapture(stream, 0);
+  CALL(wfx_fused_phase, c, 2, 0, stream);
+  void *graph = nullptr;
+  hipStreamEndCapture(stream, &graph);
+  EXPECT(formed(true) == 1, "a captured phase 2 does not form the means");
+  CALL(wfx_destroy, c);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> checks = {
       {"adjoint_stray", adjoint_stray},
+      {"densities_captured", densities_captured},
   };
   if (argc != 3 || !checks.count(argv[2])) return 2;
   library = dlopen(argv[1], RTLD_NOW);

@@ -3,6 +3,8 @@ it (native/host_calls_check.cpp): runs without a GPU.
 
 * adjoint_stray: the gradient with a per-step time step sums no entry that
   nothing wrote, also for a node of no element.
+* densities_captured: the nodal mean densities are formed again after the
+  densities changed, whatever was captured in between.
 """
 import os
 import shutil
@@ -27,7 +29,7 @@ def checker(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["adjoint_stray"])
+@pytest.mark.parametrize("check", ["adjoint_stray", "densities_captured"])
 def test_host_calls(checker, check):
     r = subprocess.run([checker, _lib.LIB_PATH, check], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr

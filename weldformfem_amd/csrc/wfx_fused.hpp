@@ -1996,6 +1996,12 @@ hipError_t launch_rigid_update(wfx_ctx *c, bool device_dt, hipStream_t s) {
 
 }  // namespace
 
+// Whether what is launched on s is recorded, not run.  The null stream cannot be
+// captured (and asking about it fails while another thread captures).
+inline bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return s != nullptr && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
 // V0_n (v0) and the nodal mean densities
 template <typename T>
 hipError_t launch_run_sums(wfx_ctx *c, bool v0, hipStream_t s) {
@@ -2008,7 +2014,7 @@ hipError_t launch_run_sums(wfx_ctx *c, bool v0, hipStream_t s) {
                        c->ms.nodel_count, c->ms.nodel_pk, elem<T>(c).vol0, elem<T>(c).rho,
                        v0 ? c->nd.voln0_sum : (double *)nullptr, c->nd.rho_avg);
   }
-  c->rho_avg_valid = true;
+  if (!is_capturing(s)) c->rho_avg_valid = true;
   return hipGetLastError();
 }
 template <typename T>
@@ -2285,7 +2291,9 @@ hipError_t launch_fused_phase_bs(wfx_ctx *c, int phase, int predict, int step, h
     // calcMinEdgeLength also refreshes the element heights contact uses
     if (cfl && c->contact.on) return launch_elem_length(c, s);
   } else if (phase == 2) {
-    if (!c->rho_avg_valid) {  // outside a run, after the densities changed
+    // outside a run: after the densities changed, and in a capture, whose replays
+    // may follow another change (a run forms the means when it starts)
+    if (step < 0 && (!c->rho_avg_valid || is_capturing(s))) {
       hipError_t e = launch_run_sums<T>(c, false, s);
       if (e != hipSuccess) return e;
     }
