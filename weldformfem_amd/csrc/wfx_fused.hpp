@@ -84,7 +84,8 @@ __device__ __forceinline__ double anp_ratio_at(const double *ratio, int i) {
 // :698-705), and the mean density of the node's elements.  Densities do not
 // change during a fused run, so CalcNodalMassFromVol's sum of rho V_n / c
 // over the c elements is this mean times V_n: a loop of c divisions less in
-// every step's nodal sums.
+// every step's nodal sums.  (A node of no element: mean and mass 0, its empty
+// sum's.)
 template <typename T>
 __global__ __launch_bounds__(kBlock) void f0_vsum0(int N, const int *__restrict__ off,
                                                    const int *__restrict__ cnt,
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(kBlock) void f0_vsum0(int N, const int *__restrict_
     r += (double)rho[e];
   }
   if (vsum0) vsum0[i] = s0;
-  rho_avg[i] = r / (double)c;
+  rho_avg[i] = c > 0 ? r / (double)c : 0.0;
 }
 
 // F2: nodal volume sum in CSR order; ratio for the ANP pressure and nodal
@@ -208,7 +209,7 @@ __global__ __launch_bounds__(kBlock) void f0_vsum0_lanes(int N, const int *__res
   const double r = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return (double)rho[e]; });
   if (q == 0 && n < N) {
     if (vsum0) vsum0[i] = s0;
-    rho_avg[i] = r / (double)c;
+    rho_avg[i] = c > 0 ? r / (double)c : 0.0;
   }
 }
 
