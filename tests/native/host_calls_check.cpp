@@ -38,6 +38,7 @@ std::map<const void *, std::string> kernel_names;
 std::vector<Kernel> launched;
 std::function<void(const std::string &, void **)> on_launch;
 int current = 0;  // device
+int wanted = -1;  // >= 0: what follows the current device has to meet this one
 bool capturing = false;
 std::map<void *, std::pair<size_t, int>> device_mem;  // bytes, device
 int wrong = 0;
@@ -51,6 +52,10 @@ int wrong = 0;
     }                          \
   } while (0)
 
+// an allocation, an event or work on the null stream: where the current device is
+void at_current(const char *what, const std::string &name = "") {
+  EXPECT(wanted < 0 || current == wanted, "%s %s on device %d, the context is on %d", what, name.c_str(), current, wanted);
+}
 bool is(const std::string &name, const char *kernel) { return name.find(kernel) != std::string::npos; }
 template <typename T>
 T arg(void **args, int k) {
@@ -93,6 +98,7 @@ int hipLaunchKernel(const void *host, Dim3, Dim3, void **args, size_t, void *str
   std::lock_guard<std::mutex> l(mu);
   const std::string &name = kernel_names[host];
   launched.push_back({name, current, stream, capturing});
+  if (!stream) at_current("kernel", name);
   if (on_launch) on_launch(name, args);
   return 0;
 }
@@ -111,6 +117,7 @@ int hipSetDevice(int d) {
 int hipMalloc(void **p, size_t bytes) {
   *p = std::aligned_alloc(256, (bytes + 255) / 256 * 256);
   std::memset(*p, 0xff, bytes);
+  at_current("hipMalloc");
   device_mem[*p] = {bytes, current};
   return 0;
 }
@@ -146,8 +153,14 @@ int hipGetSymbolAddress(void **p, const void *) {
 }
 int hipGetLastError() { return 0; }
 const char *hipGetErrorString(int) { return "error"; }
-int hipDeviceSynchronize() { return 0; }
-int hipStreamSynchronize(void *) { return 0; }
+int hipDeviceSynchronize() {
+  at_current("hipDeviceSynchronize");
+  return 0;
+}
+int hipStreamSynchronize(void *s) {
+  if (!s) at_current("hipStreamSynchronize");
+  return 0;
+}
 int hipStreamWaitEvent(void *, void *, unsigned) { return 0; }
 int hipStreamCreate(void **s) {
   *s = std::malloc(1);
@@ -185,6 +198,7 @@ int hipGraphExecDestroy(void *g) {
 }
 int hipEventCreateWithFlags(void **e, unsigned) {
   *e = std::malloc(1);
+  at_current("hipEventCreate");
   return 0;
 }
 int hipEventCreate(void **e) { return hipEventCreateWithFlags(e, 0); }
@@ -192,7 +206,10 @@ int hipEventDestroy(void *e) {
   std::free(e);
   return 0;
 }
-int hipEventRecord(void *, void *) { return 0; }
+int hipEventRecord(void *, void *s) {
+  if (!s) at_current("hipEventRecord");
+  return 0;
+}
 int hipEventSynchronize(void *) { return 0; }
 int hipEventElapsedTime(float *ms, void *, void *) {
   *ms = 1.0f;
@@ -313,12 +330,50 @@ void densities_captured() {
   CALL(wfx_destroy, c);
 }
 
+// Calls without a stream work whichever device is current, on the context's
+// own, and leave the current one; so do the allocations of calls with a stream.
+void other_device(int precision) {
+  const Box b(4), large(60);  // large: more than one chunk of the transfers
+  void *stream = nullptr;
+  hipStreamCreate(&stream);
+  for (int own = 0; own < 2; ++own) {
+    wanted = -1;
+    current = own;
+    wfx_ctx *c = domain(b, precision), *l = domain(large, precision);
+    current = 1 - own;
+    wanted = own;
+    std::vector<double> v(3 * b.nodes), e(b.elems, 5e7), w(3 * large.nodes);
+    CALL(wfx_set_density, c, 7000.0);
+    CALL(wfx_set_material, c, WFX_BILINEAR, 200e9, 0.3, 7850.0, 300e6, 1e9, 0.0);
+    CALL(wfx_set_elem_sy0, c, e.data(), b.elems);
+    CALL(wfx_set_elem_tangent, c, e.data(), b.elems);
+    CALL(wfx_set_temperature, c, 30.0);
+    CALL(wfx_set_elem_temperature, c, e.data(), b.elems);
+    CALL(wfx_set_dt, c, 1e-6);
+    CALL(wfx_init, c, stream);
+    CALL(wfx_get_field, c, "x", v.data(), (long)v.size());
+    CALL(wfx_set_field, c, "v", v.data(), (long)v.size());
+    CALL(wfx_set_field, c, "rho", e.data(), (long)e.size());
+    CALL(wfx_get_field, l, "x", w.data(), (long)w.size());
+    CALL(wfx_set_field, l, "x", w.data(), (long)w.size());
+    const int nodes[2] = {0, 1};
+    CALL(wfx_set_reaction_nodes, c, nodes, 2);
+    std::vector<double> hist(4);
+    CALL(wfx_step_fused, c, 4, hist.data(), stream);
+    CALL(wfx_destroy, c);
+    CALL(wfx_destroy, l);
+    EXPECT(current == 1 - own, "the current device is %d, the caller's was %d", current, 1 - own);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> checks = {
       {"adjoint_stray", adjoint_stray},
       {"densities_captured", densities_captured},
+      {"other_device_fp64", [] { other_device(WFX_FP64); }},
+      {"other_device_mixed", [] { other_device(WFX_FP32_MIXED); }},
   };
   if (argc != 3 || !checks.count(argv[2])) return 2;
   library = dlopen(argv[1], RTLD_NOW);

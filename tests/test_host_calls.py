@@ -5,6 +5,8 @@ it (native/host_calls_check.cpp): runs without a GPU.
   nothing wrote, also for a node of no element.
 * densities_captured: the nodal mean densities are formed again after the
   densities changed, whatever was captured in between.
+* other_device: calls without a stream run on the context's device, whichever
+  is current.
 """
 import os
 import shutil
@@ -29,7 +31,10 @@ def checker(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["adjoint_stray", "densities_captured"])
+CHECKS = ["adjoint_stray", "densities_captured", "other_device_fp64", "other_device_mixed"]
+
+
+@pytest.mark.parametrize("check", CHECKS)
 def test_host_calls(checker, check):
     r = subprocess.run([checker, _lib.LIB_PATH, check], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -32,6 +32,7 @@ static void dfree(wfx_ctx *c, T *&p) {
   if (!p) return;
   auto it = std::find(c->allocations.begin(), c->allocations.end(), (void *)p);
   if (it != c->allocations.end()) {
+    const OnDevice on(c);
     (void)hipDeviceSynchronize();  // no queued work may still use it
     (void)hipFree(p);
     c->allocations.erase(it);
@@ -43,6 +44,8 @@ template <typename T>
 static hipError_t dalloc(wfx_ctx *c, T **p, size_t count) {
   void *q = nullptr;
   size_t bytes = (count > 0 ? count : 1) * sizeof(T);
+  const OnDevice on(c);
+  if (on.err != hipSuccess) return on.err;
   hipError_t e = hipMalloc(&q, bytes);
   if (e != hipSuccess) return e;
   c->allocations.push_back(q);
@@ -101,6 +104,7 @@ static void free_all(wfx_ctx *c) {
   c->react_base = c->react_rank = nullptr;
   c->react_ring = nullptr;
   c->react_n = c->react_rows = 0;
+  c->device = -1;
   c->bc_word = nullptr;
   c->bc_tab = nullptr;
   c->v32 = c->pa32 = c->ud32 = c->fi32 = nullptr;
@@ -334,6 +338,7 @@ static int setup_device(wfx_ctx *c, const ClusterPlan &plan) {
   {
     int rc = scratch_address(&c->scratch);  // the device this context's buffers live on
     if (rc) return rc;
+    WFX_CHECK_HIP(hipGetDevice(&c->device));
   }
   const size_t N = c->N, E = c->E, n = c->n;
   Arena arena;
@@ -481,12 +486,16 @@ static int finish_mesh(wfx_ctx *c) {
 
 // one value per element, original order -> stored order, uploaded
 static int upload_elem_values(wfx_ctx *c, void *dst, const double *h, long count) {
+  const OnDevice on(c);
+  WFX_CHECK_HIP(on.err);
   WFX_CHECK_HIP(hipDeviceSynchronize());
   return field_from_host(c, FieldMove{dst, count, 1, 0, c->precision == WFX_FP32_MIXED, c->ms.o2s}, h);
 }
 
 // n equal values (in the element type, or double), there when this returns
 static int fill_values(wfx_ctx *c, void *dst, size_t n, double v, bool elem_type) {
+  const OnDevice on(c);
+  WFX_CHECK_HIP(on.err);
   FillList f;
   f.add_value(dst, n, v, elem_type && c->precision == WFX_FP32_MIXED);
   WFX_CHECK_HIP(launch_fill(f, nullptr));
@@ -874,6 +883,8 @@ int wfx_set_rigid_mesh(wfx_ctx *c, int node_count, const double *nodes, const do
   std::vector<int> faces, ext, off, afc;
   external_faces(c, faces, ext, off, afc);
   REQUIRE(!ext.empty(), WFX_ERR_ARG, "the body has no external face");
+  const OnDevice on(c);
+  WFX_CHECK_HIP(on.err);
   auto &ct = c->contact;
   const size_t N = c->N;
   drop_graph(c);
@@ -1074,6 +1085,8 @@ int wfx_set_elem_temperature(wfx_ctx *c, const double *T, int count) {
   }
   REQUIRE(count == c->E, WFX_ERR_ARG, "temperature needs one value per element");
   if (!c->temp_buf) WFX_CHECK_HIP(dalloc(c, &c->temp_buf, c->E));
+  const OnDevice on(c);
+  WFX_CHECK_HIP(on.err);
   WFX_CHECK_HIP(hipDeviceSynchronize());
   int rc = field_from_host(c, FieldMove{c->temp_buf, count, 1, 0, 0, c->ms.o2s}, T);
   if (rc) return rc;
@@ -2045,6 +2058,8 @@ int wfx_get_field(wfx_ctx *c, const char *name, void *host, long count) {
   REQUIRE(!(c->fused_stale && fused_intermediate(name)), WFX_ERR_STATE,
           std::string(name) + " is a per-step intermediate not kept by wfx_step_fused; "
           "call the per-step entry point that produces it first");
+  const OnDevice on(c);
+  WFX_CHECK_HIP(on.err);
   WFX_CHECK_HIP(hipDeviceSynchronize());
   if (f.is_int) {
     const long cnt = f.cnt;
@@ -2069,6 +2084,8 @@ int wfx_set_field(wfx_ctx *c, const char *name, const void *host, long count) {
   REQUIRE(name && find_field(c, name, f), WFX_ERR_ARG, std::string("unknown field ") + (name ? name : ""));
   REQUIRE(host && count == f.cnt * f.rows, WFX_ERR_ARG, std::string("size mismatch for field ") + name);
   REQUIRE(!f.is_int, WFX_ERR_ARG, "connectivity and CSR are set through the mesh calls");
+  const OnDevice on(c);
+  WFX_CHECK_HIP(on.err);
   WFX_CHECK_HIP(hipDeviceSynchronize());
   const double *h = (const double *)host;
   if (!std::strcmp(name, "fe")) c->has_fe = std::any_of(h, h + count, [](double v) { return v != 0.0; });

@@ -198,6 +198,7 @@ struct StepParams {
 // The opaque context behind the C-ABI handle.
 struct wfx_ctx {
   int precision = 0;  // 0 FP64, 1 FP32-mixed
+  int device = -1;    // where the mesh's buffers are (the current one when the mesh was set)
   int N = 0, E = 0, n = 0, nnz = 0;
   bool has_mesh = false, initialized = false;
   wfx::StepParams prm;
@@ -305,3 +306,29 @@ struct wfx_ctx {
   wfx::Staging *stage = nullptr;  // owned, freed with the context
   wfx::Frames *frames = nullptr;  // owned, joined and freed with the context or a new mesh
 };
+
+namespace wfx {
+// Makes the context's device the current one while it lives.  Calls without a
+// stream need it for what follows the current device: allocations, events and
+// the null stream, whose kernels would run on another device beside the memory.
+class OnDevice {
+ public:
+  explicit OnDevice(const wfx_ctx *c) {
+    int now = -1;
+    if (c->device < 0) return;
+    err = hipGetDevice(&now);
+    if (err != hipSuccess || now == c->device) return;
+    err = hipSetDevice(c->device);
+    if (err == hipSuccess) back_ = now;
+  }
+  ~OnDevice() {
+    if (back_ >= 0) (void)hipSetDevice(back_);
+  }
+  OnDevice(const OnDevice &) = delete;
+  OnDevice &operator=(const OnDevice &) = delete;
+  hipError_t err = hipSuccess;
+
+ private:
+  int back_ = -1;
+};
+}  // namespace wfx
