@@ -8,7 +8,7 @@
 #include <dlfcn.h>
 
 #include <algorithm>
-#include <cmath>
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -17,6 +17,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/wfx.h"
@@ -40,8 +41,10 @@ std::function<void(const std::string &, void **)> on_launch;
 int current = 0;  // device
 int wanted = -1;  // >= 0: what follows the current device has to meet this one
 bool capturing = false;
-std::map<void *, std::pair<size_t, int>> device_mem;  // bytes, device
-int wrong = 0;
+std::map<void *, size_t> pinned;  // bytes
+size_t pinned_limit = SIZE_MAX;   // a larger request fails
+int last_error = 0;
+std::atomic<int> wrong{0};
 
 #define EXPECT(cond, ...)      \
   do {                         \
@@ -118,19 +121,22 @@ int hipMalloc(void **p, size_t bytes) {
   *p = std::aligned_alloc(256, (bytes + 255) / 256 * 256);
   std::memset(*p, 0xff, bytes);
   at_current("hipMalloc");
-  device_mem[*p] = {bytes, current};
   return 0;
 }
 int hipFree(void *p) {
-  device_mem.erase(p);
   std::free(p);
   return 0;
 }
 int hipHostMalloc(void **p, size_t bytes, unsigned) {
+  std::lock_guard<std::mutex> l(mu);
+  if (bytes > pinned_limit) return last_error = 2;
   *p = std::aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
+  pinned[*p] = bytes;
   return 0;
 }
 int hipHostFree(void *p) {
+  std::lock_guard<std::mutex> l(mu);
+  pinned.erase(p);
   std::free(p);
   return 0;
 }
@@ -151,7 +157,12 @@ int hipGetSymbolAddress(void **p, const void *) {
   *p = scratch;
   return 0;
 }
-int hipGetLastError() { return 0; }
+int hipGetLastError() {
+  std::lock_guard<std::mutex> l(mu);
+  const int e = last_error;
+  last_error = 0;
+  return e;
+}
 const char *hipGetErrorString(int) { return "error"; }
 int hipDeviceSynchronize() {
   at_current("hipDeviceSynchronize");
@@ -366,12 +377,80 @@ void other_device(int precision) {
   }
 }
 
+// the transfer kernels of a real field in double, on the host
+void run_transfers(const std::string &name, void **args) {
+  const bool out = is(name, "k_field_outIdLb0E");
+  if (!out && !is(name, "k_field_inIdLb0E")) return;
+  const long k0 = arg<long>(args, 0), n = arg<long>(args, 1), cnt = arg<long>(args, 3);
+  const int rows = arg<int>(args, 2);
+  const int *perm = arg<const int *>(args, 4);
+  double *p = arg<double *>(args, 5), *q = arg<double *>(args, 6);  // source, destination
+  for (long t = 0; t < n; ++t) {
+    const long i = (k0 + t) / rows, r = (k0 + t) % rows, at = r * cnt + (perm ? perm[i] : i);
+    if (out) q[t] = p[at];
+    else q[at] = p[t];
+  }
+}
+
+size_t pinned_bytes() {
+  size_t b = 0;
+  for (const auto &p : pinned) b += p.second;
+  return b;
+}
+
+// The pinned memory of the transfers: what transfers at the same time need, not
+// what every context once needed; none after the last context.
+void pinned_memory() {
+  const Box b(60);  // 680,943 nodal values: two chunks
+  std::vector<double> v(3 * b.nodes);
+  wfx_ctx *c[6];
+  for (auto &q : c) {
+    q = domain(b);
+    CALL(wfx_get_field, q, "x", v.data(), (long)v.size());
+    CALL(wfx_get_field, q, "T", v.data(), (long)b.nodes);
+    EXPECT(pinned_bytes() <= (68u << 20), "%zu MiB of pinned memory", pinned_bytes() >> 20);
+  }
+  for (auto &q : c) CALL(wfx_destroy, q);
+  EXPECT(pinned.empty(), "%zu MiB of pinned memory without a context", pinned_bytes() >> 20);
+}
+
+// Transfers without memory for the ring, and from several threads
+void transfers() {
+  on_launch = run_transfers;
+  const Box b(60);
+  const auto back_and_forth = [&](wfx_ctx *c, int seed) {
+    std::vector<double> v(3 * b.nodes), w(v.size(), 0.0);
+    for (size_t i = 0; i < v.size(); ++i) v[i] = (double)(i * 7 + seed);
+    CALL(wfx_set_field, c, "v", v.data(), (long)v.size());
+    CALL(wfx_get_field, c, "v", w.data(), (long)w.size());
+    EXPECT(v == w, "a field set and read back differs");
+  };
+  pinned_limit = 4u << 20;
+  wfx_ctx *c = domain(b);
+  back_and_forth(c, 1);
+  CALL(wfx_destroy, c);
+  pinned_limit = SIZE_MAX;
+  wfx_ctx *d[6];
+  for (auto &q : d) q = domain(b);
+  std::vector<std::thread> th;
+  for (int t = 0; t < 6; ++t)
+    th.emplace_back([&, t] {
+      for (int k = 0; k < 8; ++k) back_and_forth(d[t], 10 * t + k);
+    });
+  for (auto &t : th) t.join();
+  EXPECT(pinned_bytes() <= (4u * 68 << 20), "%zu MiB of pinned memory kept", pinned_bytes() >> 20);
+  for (auto &q : d) CALL(wfx_destroy, q);
+  EXPECT(pinned.empty(), "%zu MiB of pinned memory without a context", pinned_bytes() >> 20);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> checks = {
       {"adjoint_stray", adjoint_stray},
       {"densities_captured", densities_captured},
+      {"pinned_memory", pinned_memory},
+      {"transfers", transfers},
       {"other_device_fp64", [] { other_device(WFX_FP64); }},
       {"other_device_mixed", [] { other_device(WFX_FP32_MIXED); }},
   };

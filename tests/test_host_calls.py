@@ -7,6 +7,8 @@ it (native/host_calls_check.cpp): runs without a GPU.
   densities changed, whatever was captured in between.
 * other_device: calls without a stream run on the context's device, whichever
   is current.
+* pinned_memory, transfers: the transfers' pinned memory is shared, bounded and
+  given back; they work without memory for the ring and from several threads.
 """
 import os
 import shutil
@@ -31,7 +33,8 @@ def checker(tmp_path_factory):
     return out
 
 
-CHECKS = ["adjoint_stray", "densities_captured", "other_device_fp64", "other_device_mixed"]
+CHECKS = ["adjoint_stray", "densities_captured", "other_device_fp64", "other_device_mixed", "pinned_memory",
+          "transfers"]
 
 
 @pytest.mark.parametrize("check", CHECKS)

@@ -664,6 +664,7 @@ int wfx_create(wfx_ctx **out, int precision) {
   c->prm.alpha = (2.0 * rho_b - 1.0) / (1.0 + rho_b);
   c->prm.beta = (5.0 - 3.0 * rho_b) / ((1.0 + rho_b) * (1.0 + rho_b) * (2.0 - rho_b));
   c->prm.gamma = 1.5 - c->prm.alpha;
+  staging_open();
   *out = c;
   return WFX_OK;
 }
@@ -671,8 +672,8 @@ int wfx_create(wfx_ctx **out, int precision) {
 int wfx_destroy(wfx_ctx *c) {
   if (!c) return WFX_OK;
   free_all(c);
-  staging_free(c);
   delete c;
+  staging_close();
   return WFX_OK;
 }
 

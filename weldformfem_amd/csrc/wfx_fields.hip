@@ -34,29 +34,87 @@ constexpr size_t kChunkBytes = (size_t)4 << 20;
 constexpr int kSlots = 16, kCopyThreads = 8;
 
 struct Staging {
+  int device = -1;        // the events'
   char *small = nullptr;  // one chunk
   char *ring = nullptr;   // kSlots chunks, allocated by the first transfer that needs them
   hipEvent_t ev[kSlots] = {};
+  ~Staging() {
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (small) (void)hipHostFree(small);
+    if (ring) (void)hipHostFree(ring);
+  }
 };
 
-void staging_free(wfx_ctx *c) {
-  if (!c->stage) return;
-  for (hipEvent_t e : c->stage->ev)
-    if (e) (void)hipEventDestroy(e);
-  if (c->stage->small) (void)hipHostFree(c->stage->small);
-  if (c->stage->ring) (void)hipHostFree(c->stage->ring);
-  delete c->stage;
-  c->stage = nullptr;
+// The staging belongs to a transfer, not to a context: a transfer takes one that
+// is idle, or makes one, and leaves it for the next.  Many contexts in turn then
+// hold one (68 MiB of pinned memory), not one each; transfers at the same time
+// have their own.  At most kIdle stay, for as many threads that read fields all
+// the time, and none after the last context.
+constexpr int kIdle = 4;
+static std::mutex g_stage_mu;
+static Staging *g_idle[kIdle] = {};
+static long g_contexts = 0;
+
+void staging_open() {
+  std::lock_guard<std::mutex> l(g_stage_mu);
+  ++g_contexts;
+}
+void staging_close() {
+  Staging *drop[kIdle] = {};
+  {
+    std::lock_guard<std::mutex> l(g_stage_mu);
+    if (--g_contexts == 0) std::swap(drop, g_idle);
+  }
+  for (Staging *s : drop) delete s;
 }
 
-static int staging_ready(wfx_ctx *c, bool ring) {
-  if (!c->stage) c->stage = new Staging();
-  Staging &s = *c->stage;
-  if (!ring && !s.small) WFX_CHECK_HIP(hipHostMalloc((void **)&s.small, kChunkBytes, hipHostMallocPortable));
+// The current device is the transfer's.
+class StagingLease {
+ public:
+  explicit StagingLease(int device) {
+    {
+      std::lock_guard<std::mutex> l(g_stage_mu);
+      for (Staging *&q : g_idle)
+        if (!s_ && q && q->device == device) std::swap(s_, q);
+    }
+    if (!s_) s_ = new Staging();
+    s_->device = device;
+  }
+  ~StagingLease() {
+    {
+      std::lock_guard<std::mutex> l(g_stage_mu);
+      for (Staging *&q : g_idle)
+        if (s_ && !q) std::swap(s_, q);
+    }
+    delete s_;
+  }
+  StagingLease(const StagingLease &) = delete;
+  StagingLease &operator=(const StagingLease &) = delete;
+  Staging &operator*() const { return *s_; }
+
+ private:
+  Staging *s_ = nullptr;
+};
+
+// Allocates what is not there yet.  Without memory for a ring the transfer goes
+// chunk by chunk.
+static int staging_ready(Staging &s, bool ring) {
   if (ring && !s.ring) {
     for (hipEvent_t &e : s.ev)
       if (!e) WFX_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    WFX_CHECK_HIP(hipHostMalloc((void **)&s.ring, kChunkBytes * kSlots, hipHostMallocPortable));
+    if (hipHostMalloc((void **)&s.ring, kChunkBytes * kSlots, hipHostMallocPortable) != hipSuccess) {
+      s.ring = nullptr;
+      (void)hipGetLastError();  // or the next launch would report it
+    }
+  }
+  if (!(ring && s.ring) && !s.small) {
+    const hipError_t e = hipHostMalloc((void **)&s.small, kChunkBytes, hipHostMallocPortable);
+    if (e != hipSuccess) {
+      s.small = nullptr;
+      (void)hipGetLastError();
+    }
+    WFX_CHECK_HIP(e);
   }
   return WFX_OK;
 }
@@ -210,21 +268,26 @@ struct CopyJob {
   }
 };
 
-// The caller has synchronised the device.  Returns when the transfer is over.
+// The caller has synchronised the device and made it current.  Returns when the
+// transfer is over.
 template <bool OUT>
 int move_field(wfx_ctx *c, const FieldMove &f, double *user) {
   const long values = f.cnt * f.rows, per = (long)(kChunkBytes / sizeof(double));
   if (values == 0) return WFX_OK;
   const long chunks = (values + per - 1) / per;
-  int rc = staging_ready(c, chunks > 1);
+  const StagingLease lease(c->device);
+  Staging &s = *lease;
+  int rc = staging_ready(s, chunks > 1);
   if (rc) return rc;
-  Staging &s = *c->stage;
-  if (chunks == 1) {
+  if (chunks == 1 || !s.ring) {
     double *pin = (double *)s.small;
-    if (!OUT) std::memcpy(pin, user, values * sizeof(double));
-    WFX_CHECK_HIP(launch_chunk<OUT>(f, 0, values, pin));
-    WFX_CHECK_HIP(hipStreamSynchronize(nullptr));
-    if (OUT) std::memcpy(user, pin, values * sizeof(double));
+    for (long k = 0; k < chunks; ++k) {
+      const long n = std::min(per, values - k * per);
+      if (!OUT) std::memcpy(pin, user + k * per, n * sizeof(double));
+      WFX_CHECK_HIP(launch_chunk<OUT>(f, k * per, n, pin));
+      WFX_CHECK_HIP(hipStreamSynchronize(nullptr));
+      if (OUT) std::memcpy(user + k * per, pin, n * sizeof(double));
+    }
     return WFX_OK;
   }
   auto slot = [&](long k) { return (double *)(s.ring + (size_t)(k % kSlots) * kChunkBytes); };

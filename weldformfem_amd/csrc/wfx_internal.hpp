@@ -34,7 +34,6 @@ namespace wfx {
 void set_error(const std::string &msg);
 struct Adjoint;  // checkpointed adjoint run (wfx_adjoint.hip)
 struct Frames;   // asynchronous VTK frames (wfx_frames.hip)
-struct Staging;  // pinned host memory of the field transfers (wfx_fields.hip)
 
 enum Model { BILINEAR = 0, HOLLOMON = 1, JOHNSON_COOK = 2, GMT = 3 };
 
@@ -303,7 +302,6 @@ struct wfx_ctx {
   int hist_cap = 0;
   std::vector<void *> allocations;
   wfx::Adjoint *adj = nullptr;  // owned, freed with the context or a new mesh
-  wfx::Staging *stage = nullptr;  // owned, freed with the context
   wfx::Frames *frames = nullptr;  // owned, joined and freed with the context or a new mesh
 };
 

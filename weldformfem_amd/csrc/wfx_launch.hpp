@@ -182,7 +182,7 @@ hipError_t launch_fill(const FillList &f, hipStream_t s);
 // A real field's transfer: host [cnt][rows] double, device [rows][cnt]
 // (spin: 3 device rows for host columns 3..5 of 6, the others zero), float
 // when f32; perm maps a host item to its device column (null: the same).
-// The device must be idle; both return when the transfer is over.
+// The device must be current and idle; both return when the transfer is over.
 struct FieldMove {
   void *dev;
   long cnt;
@@ -191,7 +191,9 @@ struct FieldMove {
 };
 int field_to_host(wfx_ctx *c, const FieldMove &f, double *host);
 int field_from_host(wfx_ctx *c, const FieldMove &f, const double *host);
-void staging_free(wfx_ctx *c);
+// a context comes and goes: the transfers' pinned memory goes with the last one
+void staging_open();
+void staging_close();
 void frames_free(wfx_ctx *c);
 void frames_join(wfx_ctx *c);
 
