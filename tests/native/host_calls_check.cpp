@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -247,32 +248,38 @@ F *entry(const char *name) {
     EXPECT(rc == 0, "%s returned %d: %s", #fn, rc, entry<decltype(wfx_last_error)>("wfx_last_error")());           \
   } while (0)
 
-// n x n x n hexahedra and, with stray, a node of no element behind them
+// nx x ny x nz hexahedra (tets: six tetrahedra each) and, with stray, a node of
+// no element behind them
 struct Box {
   std::vector<double> x;
   std::vector<int> el;
-  int nodes, elems;
-  explicit Box(int n, bool stray = false) {
-    const int m = n + 1;
-    for (int k = 0; k < m; ++k)
-      for (int j = 0; j < m; ++j)
-        for (int i = 0; i < m; ++i) x.insert(x.end(), {0.1 * i, 0.1 * j, 0.1 * k});
-    for (int k = 0; k < n; ++k)
-      for (int j = 0; j < n; ++j)
-        for (int i = 0; i < n; ++i) {
-          const int a = (k * m + j) * m + i, b = a + m * m;
-          el.insert(el.end(), {a, a + 1, a + m + 1, a + m, b, b + 1, b + m + 1, b + m});
+  int nodes, elems, n;
+  explicit Box(int size, bool stray = false) : Box(size, size, size, false, stray) {}
+  Box(int nx, int ny, int nz, bool tets = false, bool stray = false) : n(tets ? 4 : 8) {
+    const int mx = nx + 1, my = ny + 1;
+    for (int k = 0; k <= nz; ++k)
+      for (int j = 0; j <= ny; ++j)
+        for (int i = 0; i <= nx; ++i) x.insert(x.end(), {0.1 * i, 0.1 * j, 0.1 * k});
+    const int part[6][4] = {{0, 1, 3, 5}, {1, 2, 3, 5}, {0, 5, 3, 4}, {4, 5, 3, 7}, {5, 6, 3, 7}, {5, 2, 3, 6}};
+    for (int k = 0; k < nz; ++k)
+      for (int j = 0; j < ny; ++j)
+        for (int i = 0; i < nx; ++i) {
+          const int a = (k * my + j) * mx + i, b = a + mx * my;
+          const int h[8] = {a, a + 1, a + mx + 1, a + mx, b, b + 1, b + mx + 1, b + mx};
+          if (!tets) el.insert(el.end(), h, h + 8);
+          for (int t = 0; tets && t < 6; ++t)
+            for (int q : part[t]) el.push_back(h[q]);
         }
-    if (stray) x.insert(x.end(), {5.0, 5.0, 5.0});
+    if (stray) x.insert(x.end(), {50.0, 50.0, 50.0});
     nodes = (int)x.size() / 3;
-    elems = (int)el.size() / 8;
+    elems = (int)el.size() / n;
   }
 };
 
 wfx_ctx *domain(const Box &b, int precision = WFX_FP64) {
   wfx_ctx *c = nullptr;
   CALL(wfx_create, &c, precision);
-  CALL(wfx_set_mesh, c, b.nodes, b.elems, 8, b.x.data(), b.el.data());
+  CALL(wfx_set_mesh, c, b.nodes, b.elems, b.n, b.x.data(), b.el.data());
   CALL(wfx_set_density, c, 7850.0);
   CALL(wfx_set_material, c, WFX_BILINEAR, 200e9, 0.3, 7850.0, 300e6, 1e9, 0.0);
   CALL(wfx_set_dt, c, 1e-6);
@@ -443,12 +450,123 @@ void transfers() {
   EXPECT(pinned.empty(), "%zu MiB of pinned memory without a context", pinned_bytes() >> 20);
 }
 
+// Which passes a run of seven steps takes: all of its steps but the last in the
+// solo pass, or in the paired ones, or every step in the separate ones (as the
+// last step's nodal update always is).  An odd run's paired steps all go to the
+// other set of buffers.
+enum Passes { SEPARATE, PAIRED, SOLO };
+void expect_passes(const char *what, wfx_ctx *c, Passes want) {
+  const int n = 7;
+  launched.clear();
+  CALL(wfx_step_fused, c, n, nullptr, nullptr);
+  const auto count = [](const char *kernel) {
+    return (int)std::count_if(launched.begin(), launched.end(), [&](const Kernel &k) { return is(k.name, kernel); });
+  };
+  const int solo = count("f_solo"), pair = count("f41_cluster"), node = count("f4_node"), sums = count("f2_nodal"),
+            elem = count("f3_cluster");
+  double clusters = 0.0;
+  CALL(wfx_get_param, c, "cluster_count", &clusters);
+  const bool ok = want == SOLO     ? solo == 1 && pair == 0 && node == 1 && sums == 0 && elem == 1
+                  : want == PAIRED ? solo == 0 && pair == n - 1 && node == 1 && sums == 0 && elem == n
+                                   : solo == 0 && pair == 0 && node == n && sums == n && elem == n;
+  EXPECT(ok, "%s, %g clusters: solo pass %d, paired node passes %d, node passes %d, nodal sums %d, element passes %d",
+         what, clusters, solo, pair, node, sums, elem);
+}
+// cells along x, y and z, precision, clusters of the plan (0: any), passes
+struct LineCase {
+  int x, y, z;
+  bool tets;
+  int precision, clusters;
+  Passes want;
+};
+void passes_by_size() {
+  const LineCase cases[] = {
+      {1, 1, 1, false, WFX_FP64, 1, SOLO},          {1, 1, 1, false, WFX_FP32_MIXED, 1, PAIRED},
+      {16, 4, 4, false, WFX_FP64, 1, SOLO},         {17, 4, 4, false, WFX_FP64, 2, PAIRED},
+      {20, 20, 20, false, WFX_FP64, 35, PAIRED},    {40, 40, 40, false, WFX_FP64, 250, PAIRED},
+      {40, 40, 41, false, WFX_FP64, 264, SEPARATE}, {40, 40, 40, false, WFX_FP32_MIXED, 250, PAIRED},
+      {48, 51, 50, false, WFX_FP32_MIXED, 480, PAIRED}, {49, 49, 49, false, WFX_FP32_MIXED, 574, SEPARATE},
+      {3, 3, 4, true, WFX_FP64, 1, SOLO},           {20, 20, 20, true, WFX_FP64, 0, PAIRED},
+      {27, 27, 27, true, WFX_FP64, 0, SEPARATE},    {27, 27, 27, true, WFX_FP32_MIXED, 0, PAIRED},
+      {28, 28, 28, true, WFX_FP32_MIXED, 515, SEPARATE}};
+  for (const LineCase &q : cases) {
+    const Box b(q.x, q.y, q.z, q.tets);
+    wfx_ctx *c = domain(b, q.precision);
+    CALL(wfx_init, c, nullptr);
+    double clusters = 0.0;
+    CALL(wfx_get_param, c, "cluster_count", &clusters);
+    EXPECT(q.clusters == 0 || clusters == q.clusters, "%d x %d x %d, precision %d: %g clusters", q.x, q.y, q.z,
+           q.precision, clusters);
+    char what[64];
+    std::snprintf(what, sizeof(what), "%d x %d x %d %s, precision %d", q.x, q.y, q.z, q.tets ? "tets" : "hexa",
+                  q.precision);
+    expect_passes(what, c, q.want);
+    CALL(wfx_destroy, c);
+  }
+}
+void passes_by_option() {
+  for (const int precision : {WFX_FP64, WFX_FP32_MIXED})
+    for (const bool small : {true, false}) {
+      const int n = small ? 2 : 9;
+      const Passes solo = small && precision == WFX_FP64 ? SOLO : PAIRED;
+      const Box hexa(n), tets(n, n, n, true), stray(n, true);
+      const auto fresh = [&](const Box &b) {
+        wfx_ctx *c = domain(b, precision);
+        CALL(wfx_init, c, nullptr);
+        return c;
+      };
+      wfx_ctx *c = fresh(hexa);
+      expect_passes("plain", c, solo);
+      CALL(wfx_set_cfl, c, 0.3);
+      expect_passes("per-step time step", c, PAIRED);
+      CALL(wfx_set_cfl, c, 0.0);
+      expect_passes("fixed time step again", c, solo);
+      CALL(wfx_set_thermal, c, 1, 50.0, 460.0, 0.9);
+      expect_passes("thermal", c, PAIRED);
+      CALL(wfx_set_thermal_expansion, c, 1e-5);
+      expect_passes("thermal expansion", c, SEPARATE);
+      CALL(wfx_destroy, c);
+      c = fresh(tets);
+      expect_passes("tetrahedra", c, solo);
+      const double die[9] = {0, 0, 9, 9, 0, 9, 0, 9, 9}, moving[9] = {0, 0, -1, 0, 0, -1, 0, 0, -1};
+      const int tri[3] = {0, 2, 1};
+      CALL(wfx_set_rigid_mesh, c, 3, die, moving, 1, tri, nullptr);
+      expect_passes("contact", c, PAIRED);
+      CALL(wfx_destroy, c);
+      c = fresh(stray);
+      expect_passes("a node of no element", c, SEPARATE);
+      CALL(wfx_destroy, c);
+    }
+  // 34 elements around an axis: more than the paired tables hold of a node
+  Box fan(0);
+  const int m = 34;
+  fan.x.clear();
+  for (int k = 0; k < 2; ++k) {
+    fan.x.insert(fan.x.end(), {0.0, 0.0, 0.1 * k});
+    for (int q = 0; q < m; ++q)
+      fan.x.insert(fan.x.end(), {std::cos(6.283185307179586 * q / m), std::sin(6.283185307179586 * q / m), 0.1 * k});
+  }
+  for (int q = 0; q < 17; ++q)
+    for (int half = 0; half < 2; ++half) {  // wedges as hexahedra with an edge of no length
+      const int a = 2 * q + half, b = (a + 1) % m;
+      fan.el.insert(fan.el.end(), {0, 1 + a, 1 + b, 0, m + 1, m + 2 + a, m + 2 + b, m + 1});
+    }
+  fan.nodes = 2 * (m + 1);
+  fan.elems = m;
+  wfx_ctx *c = domain(fan);
+  CALL(wfx_init, c, nullptr);
+  expect_passes("a node of 34 elements", c, SEPARATE);
+  CALL(wfx_destroy, c);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> checks = {
       {"adjoint_stray", adjoint_stray},
       {"densities_captured", densities_captured},
+      {"passes_by_size", passes_by_size},
+      {"passes_by_option", passes_by_option},
       {"pinned_memory", pinned_memory},
       {"transfers", transfers},
       {"other_device_fp64", [] { other_device(WFX_FP64); }},

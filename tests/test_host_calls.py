@@ -7,6 +7,9 @@ it (native/host_calls_check.cpp): runs without a GPU.
   densities changed, whatever was captured in between.
 * other_device: calls without a stream run on the context's device, whichever
   is current.
+* passes_by_size, passes_by_option: whether a run takes the separate, the paired
+  or the solo pass, on both sides of the lines and with every option that
+  excludes one.
 * pinned_memory, transfers: the transfers' pinned memory is shared, bounded and
   given back; they work without memory for the ring and from several threads.
 """
@@ -34,7 +37,7 @@ def checker(tmp_path_factory):
 
 
 CHECKS = ["adjoint_stray", "densities_captured", "other_device_fp64", "other_device_mixed", "pinned_memory",
-          "transfers"]
+          "transfers", "passes_by_size", "passes_by_option"]
 
 
 @pytest.mark.parametrize("check", CHECKS)

@@ -2456,6 +2456,7 @@ struct NodalPlaces {
 // rz: the first one's reaction record, or null
 template <typename T>
 hipError_t launch_solo_steps(wfx_ctx *c, int k, int n, void *rz, hipStream_t s) {
+  static_assert(std::is_same<T, double>::value, "run_solo: FP64 only (a template, so that only its unit holds the kernels)");
   auto &el = elem<T>(c);
   T *vN, *paN, *udN, *fiN;
   fused_node_arrays<T>(c, vN, paN, udN, fiN);
@@ -2523,7 +2524,7 @@ hipError_t launch_fused_steps(wfx_ctx *c, int nsteps, double *hist, hipStream_t 
   bool have_vol = false;
   int k = 0;
   if constexpr (std::is_same<T, double>::value)
-    while (pair && run_solo(c) && k + 1 < nsteps) {  // all steps but the last
+    while (!ev && run_solo(c) && k + 1 < nsteps) {  // all steps but the last
       // up to the row at which the reaction record is full
       int n = std::min(nsteps - 1 - k, kSoloSteps);
       if (rec.hist) n = std::min(n, c->react_rows - k % c->react_rows);

@@ -79,14 +79,16 @@ int ensure_react_ring(wfx_ctx *c);
 // Whether a run takes the paired passes.  Thermal expansion does not: its
 // flat array divides by the masses the paired element pass is still forming.
 inline bool run_paired(const wfx_ctx *c) { return c->pair && !(c->thermal.on && c->thermal.exp_T != 0.0); }
-// Whether a paired run takes the solo pass: no node belongs to two clusters
-// (meshes of up to 256 connected elements, or many such), and nothing outside
-// the nodes and elements moves with the steps.  FP64 only: its unit contracts
+// Whether a run takes the solo pass for all its steps but the last: a paired one
+// (whose tables it reads; every node then has a slot, so that as many slots as
+// nodes means no node of two clusters: meshes of up to 256 connected elements, or
+// many such) in which nothing outside the nodes and elements moves with the steps.  FP64 only: its unit contracts
 // within expressions; in the FP32-mixed unit the contractions the compiler picks
 // depend on the kernel around them, and a float rounded otherwise shows in the
 // results.
 inline bool run_solo(const wfx_ctx *c) {
-  return c->ms.nslot == c->N && !c->contact.on && !c->thermal.on && !(c->prm.cfl > 0.0);
+  return c->precision == 0 && run_paired(c) && c->ms.nslot == c->N && !c->contact.on && !c->thermal.on &&
+         !(c->prm.cfl > 0.0);
 }
 constexpr int kSoloSteps = 512;  // of one launch: a few milliseconds
 template <typename T>
