@@ -421,9 +421,18 @@ void pinned_memory() {
   EXPECT(pinned.empty(), "%zu MiB of pinned memory without a context", pinned_bytes() >> 20);
 }
 
-// Transfers without memory for the ring, and from several threads
+// Transfers by each way (kernels, copies, the ring), without memory for the ring,
+// and from several threads
 void transfers() {
   on_launch = run_transfers;
+  for (const int n : {1, 7, 8, 12, 13, 30, 60}) {  // 192 B to 5.4 MB of positions
+    const Box m(n);
+    wfx_ctx *c = domain(m);
+    std::vector<double> x(m.x.size());
+    CALL(wfx_get_field, c, "x", x.data(), (long)x.size());
+    EXPECT(x == m.x, "%d^3: the positions read differ from the mesh's", n);
+    CALL(wfx_destroy, c);
+  }
   const Box b(60);
   const auto back_and_forth = [&](wfx_ctx *c, int seed) {
     std::vector<double> v(3 * b.nodes), w(v.size(), 0.0);

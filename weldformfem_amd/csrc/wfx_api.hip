@@ -489,7 +489,7 @@ static int upload_elem_values(wfx_ctx *c, void *dst, const double *h, long count
   const OnDevice on(c);
   WFX_CHECK_HIP(on.err);
   WFX_CHECK_HIP(hipDeviceSynchronize());
-  return field_from_host(c, FieldMove{dst, count, 1, 0, c->precision == WFX_FP32_MIXED, c->ms.o2s}, h);
+  return field_from_host(c, FieldMove{dst, count, 1, 0, c->precision == WFX_FP32_MIXED, c->ms.o2s, c->el_o2s.data()}, h);
 }
 
 // n equal values (in the element type, or double), there when this returns
@@ -1089,7 +1089,7 @@ int wfx_set_elem_temperature(wfx_ctx *c, const double *T, int count) {
   const OnDevice on(c);
   WFX_CHECK_HIP(on.err);
   WFX_CHECK_HIP(hipDeviceSynchronize());
-  int rc = field_from_host(c, FieldMove{c->temp_buf, count, 1, 0, 0, c->ms.o2s}, T);
+  int rc = field_from_host(c, FieldMove{c->temp_buf, count, 1, 0, 0, c->ms.o2s, c->el_o2s.data()}, T);
   if (rc) return rc;
   c->temp_e = c->temp_buf;
   return WFX_OK;
@@ -2048,7 +2048,7 @@ static bool fused_intermediate(const char *name) {
 
 static FieldMove field_move(const wfx_ctx *c, const FieldDesc &f) {
   return FieldMove{f.dev, f.cnt, f.rows, f.kind == 1, f.elem && c->precision == WFX_FP32_MIXED,
-                   f.per_elem ? c->ms.o2s : nullptr};
+                   f.per_elem ? c->ms.o2s : nullptr, f.per_elem ? c->el_o2s.data() : nullptr};
 }
 
 int wfx_get_field(wfx_ctx *c, const char *name, void *host, long count) {

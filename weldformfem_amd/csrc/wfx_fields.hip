@@ -268,12 +268,44 @@ struct CopyJob {
   }
 };
 
+// Fields of more than kCopyFrom and up to kCopyTo bytes on the device, of at most
+// kCopyItems items: one hipMemcpy, the transposition, permutation and conversion
+// on the host.  The runtime copies up to 16 KiB by a way that takes 20 us, more in
+// 8; above the other two lines the host's loop takes longer than a kernel and the
+// wait for it.  us to read / set, this way and by the kernels: three components,
+// 12,288 B 23.1 / 22.2 and 15.5 / 15.2, 17,496 B 11.9 / 11.5 and 15.6 / 15.3,
+// 31,944 B 13.0 / 12.8 and 15.8 / 15.5, 52,728 B 15.0 / 14.7 and 16.5 / 15.9,
+// 81,000 B 17.6 / 17.2 and 17.7 / 16.8; one component, 4096 items 14.8 / 14.4 and
+// 16.2 / 15.7, 4913 items 15.9 / 16.4 and 16.3 / 15.6.
+constexpr size_t kCopyFrom = 16 << 10, kCopyTo = 64 << 10;
+constexpr long kCopyItems = 4500;
+template <bool OUT, typename T>
+int move_by_copy(const FieldMove &f, double *user) {
+  const int skip = f.spin ? 3 : 0, dr = f.rows - skip;  // the spin's zero diagonal
+  std::vector<T> t((size_t)dr * f.cnt);
+  if (OUT) WFX_CHECK_HIP(hipMemcpy(t.data(), f.dev, t.size() * sizeof(T), hipMemcpyDeviceToHost));
+  for (long i = 0; i < f.cnt; ++i) {
+    double *u = user + i * f.rows;
+    T *d = t.data() + (f.perm_h ? (long)f.perm_h[i] : i);
+    for (int r = 0; OUT && r < skip; ++r) u[r] = 0.0;
+    for (int r = 0; r < dr; ++r) {
+      if (OUT) u[skip + r] = (double)d[r * f.cnt];
+      else d[r * f.cnt] = (T)u[skip + r];
+    }
+  }
+  if (!OUT) WFX_CHECK_HIP(hipMemcpy(f.dev, t.data(), t.size() * sizeof(T), hipMemcpyHostToDevice));
+  return WFX_OK;
+}
+
 // The caller has synchronised the device and made it current.  Returns when the
 // transfer is over.
 template <bool OUT>
 int move_field(wfx_ctx *c, const FieldMove &f, double *user) {
   const long values = f.cnt * f.rows, per = (long)(kChunkBytes / sizeof(double));
   if (values == 0) return WFX_OK;
+  const size_t bytes = (size_t)f.cnt * (f.rows - (f.spin ? 3 : 0)) * (f.f32 ? sizeof(float) : sizeof(double));
+  if (bytes > kCopyFrom && bytes <= kCopyTo && f.cnt <= kCopyItems)
+    return f.f32 ? move_by_copy<OUT, float>(f, user) : move_by_copy<OUT, double>(f, user);
   const long chunks = (values + per - 1) / per;
   const StagingLease lease(c->device);
   Staging &s = *lease;

@@ -189,7 +189,8 @@ struct FieldMove {
   void *dev;
   long cnt;
   int rows, spin, f32;
-  const int *perm;
+  const int *perm;    // on the device
+  const int *perm_h;  // the same on the host
 };
 int field_to_host(wfx_ctx *c, const FieldMove &f, double *host);
 int field_from_host(wfx_ctx *c, const FieldMove &f, const double *host);
