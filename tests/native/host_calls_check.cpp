@@ -348,6 +348,34 @@ void densities_captured() {
   CALL(wfx_destroy, c);
 }
 
+// A uniform density needs no means: a run does not read the densities for them,
+// and forms them once the densities may differ.
+void densities_uniform() {
+  const Box b(3);
+  int formed = 0;
+  on_launch = [&](const std::string &name, void **args) {
+    if (is(name, "k_scan_elem")) {  // what it finds here
+      unsigned long long *scan = arg<unsigned long long *>(args, 3);
+      const double rho = 7850.0;
+      scan[0] = scan[1] = 0;
+      std::memcpy(&scan[2], &rho, 8);
+      std::memcpy(&scan[3], &rho, 8);
+    }
+    if (is(name, "f0_vsum0")) formed += arg<const double *>(args, 7) != nullptr;
+  };
+  wfx_ctx *c = domain(b);
+  CALL(wfx_init, c, nullptr);
+  CALL(wfx_step_fused, c, 1, nullptr, nullptr);
+  CALL(wfx_fused_phase, c, 2, 0, nullptr);
+  EXPECT(formed == 0, "means of a uniform density were formed");
+  CALL(wfx_calc_elem_density, c, nullptr);
+  CALL(wfx_fused_phase, c, 2, 0, nullptr);
+  EXPECT(formed == 1, "means formed %d times after the densities changed", formed);
+  CALL(wfx_step_fused, c, 1, nullptr, nullptr);
+  EXPECT(formed == 2, "a run did not form the means");
+  CALL(wfx_destroy, c);
+}
+
 // Calls without a stream work whichever device is current, on the context's
 // own, and leave the current one; so do the allocations of calls with a stream.
 void other_device(int precision) {
@@ -574,6 +602,7 @@ int main(int argc, char **argv) {
   const std::map<std::string, void (*)()> checks = {
       {"adjoint_stray", adjoint_stray},
       {"densities_captured", densities_captured},
+      {"densities_uniform", densities_uniform},
       {"passes_by_size", passes_by_size},
       {"passes_by_option", passes_by_option},
       {"pinned_memory", pinned_memory},

@@ -5,6 +5,7 @@ it (native/host_calls_check.cpp): runs without a GPU.
   nothing wrote, also for a node of no element.
 * densities_captured: the nodal mean densities are formed again after the
   densities changed, whatever was captured in between.
+* densities_uniform: means are formed only where densities may differ.
 * other_device: calls without a stream run on the context's device, whichever
   is current.
 * passes_by_size, passes_by_option: whether a run takes the separate, the paired
@@ -36,8 +37,8 @@ def checker(tmp_path_factory):
     return out
 
 
-CHECKS = ["adjoint_stray", "densities_captured", "other_device_fp64", "other_device_mixed", "pinned_memory",
-          "transfers", "passes_by_size", "passes_by_option"]
+CHECKS = ["adjoint_stray", "densities_captured", "densities_uniform", "other_device_fp64", "other_device_mixed",
+          "pinned_memory", "transfers", "passes_by_size", "passes_by_option"]
 
 
 @pytest.mark.parametrize("check", CHECKS)

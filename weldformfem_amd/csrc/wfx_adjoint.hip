@@ -946,6 +946,8 @@ static int adjoint_backward(wfx_ctx *c, hipStream_t st) {
     LAUNCH(hipGetLastError());
     lawc = A->lawc;
   }
+  // the recomputed steps read the nodal mean densities of the present densities
+  if (!(c->rho_uniform > 0.0) && !c->rho_avg_valid) LAUNCH(launch_vsum0<T>(c, st));
   NodeAdj NP{P.dt, P.alpha, P.beta, P.gamma, c->has_fe, A->ng};
   const ClusterArgs ca = cluster_args(c);
   const SlotSums sums{c->ms.nsl_off, c->ms.nsl, c->ms.spos, c->ms.spos != nullptr, c->precision == WFX_FP64 ? 0 : 1,

@@ -85,7 +85,8 @@ __device__ __forceinline__ double anp_ratio_at(const double *ratio, int i) {
 // change during a fused run, so CalcNodalMassFromVol's sum of rho V_n / c
 // over the c elements is this mean times V_n: a loop of c divisions less in
 // every step's nodal sums.  (A node of no element: mean and mass 0, its empty
-// sum's.)
+// sum's.)  Without rho_avg no density is read: the later passes take a uniform
+// density from their arguments.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void f0_vsum0(int N, const int *__restrict__ off,
                                                    const int *__restrict__ cnt,
@@ -99,10 +100,10 @@ __global__ __launch_bounds__(kBlock) void f0_vsum0(int N, const int *__restrict_
   for (int k = 0; k < c; ++k) {
     const int e = nodel_pk[o + k] >> 3;
     s0 += (double)vol0[e];
-    r += (double)rho[e];
+    if (rho_avg) r += (double)rho[e];
   }
   if (vsum0) vsum0[i] = s0;
-  rho_avg[i] = c > 0 ? r / (double)c : 0.0;
+  if (rho_avg) rho_avg[i] = c > 0 ? r / (double)c : 0.0;
 }
 
 // F2: nodal volume sum in CSR order; ratio for the ANP pressure and nodal
@@ -206,10 +207,11 @@ __global__ __launch_bounds__(kBlock) void f0_vsum0_lanes(int N, const int *__res
   const int q = (int)(g % L), i = (int)(n < N ? n : N - 1);  // every lane reaches the butterfly
   const int o = off[i], c = cnt[i];
   const double s0 = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return (double)vol0[e]; });
-  const double r = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return (double)rho[e]; });
+  double r = 0.0;
+  if (rho_avg) r = lane_csr_sum<L>(o, c, q, nodel_pk, [&](int e) { return (double)rho[e]; });
   if (q == 0 && n < N) {
     if (vsum0) vsum0[i] = s0;
-    rho_avg[i] = c > 0 ? r / (double)c : 0.0;
+    if (rho_avg) rho_avg[i] = c > 0 ? r / (double)c : 0.0;
   }
 }
 
@@ -2003,19 +2005,22 @@ inline bool is_capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return s != nullptr && hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
-// V0_n (v0) and the nodal mean densities
+// Whether the passes read the nodal mean densities
+inline bool reads_means(const wfx_ctx *c) { return !(c->rho_uniform > 0.0); }
+// V0_n (v0) and, where they are read, the nodal mean densities
 template <typename T>
 hipError_t launch_run_sums(wfx_ctx *c, bool v0, hipStream_t s) {
+  double *const avg = reads_means(c) ? c->nd.rho_avg : nullptr;
   if (c->f2_lanes) {
     hipLaunchKernelGGL((f0_vsum0_lanes<T>), dim3(nblocks((long)c->N * kF2Lanes)), dim3(kBlock), 0, s, c->N,
                        c->ms.nodel_offset, c->ms.nodel_count, c->ms.nodel_pk, elem<T>(c).vol0, elem<T>(c).rho,
-                       v0 ? c->nd.voln0_sum : (double *)nullptr, c->nd.rho_avg);
+                       v0 ? c->nd.voln0_sum : (double *)nullptr, avg);
   } else {
     hipLaunchKernelGGL((f0_vsum0<T>), dim3(nblocks(c->N)), dim3(kBlock), 0, s, c->N, c->ms.nodel_offset,
                        c->ms.nodel_count, c->ms.nodel_pk, elem<T>(c).vol0, elem<T>(c).rho,
-                       v0 ? c->nd.voln0_sum : (double *)nullptr, c->nd.rho_avg);
+                       v0 ? c->nd.voln0_sum : (double *)nullptr, avg);
   }
-  if (!is_capturing(s)) c->rho_avg_valid = true;
+  if (avg && !is_capturing(s)) c->rho_avg_valid = true;
   return hipGetLastError();
 }
 template <typename T>
@@ -2294,7 +2299,7 @@ hipError_t launch_fused_phase_bs(wfx_ctx *c, int phase, int predict, int step, h
   } else if (phase == 2) {
     // outside a run: after the densities changed, and in a capture, whose replays
     // may follow another change (a run forms the means when it starts)
-    if (step < 0 && (!c->rho_avg_valid || is_capturing(s))) {
+    if (step < 0 && reads_means(c) && (!c->rho_avg_valid || is_capturing(s))) {
       hipError_t e = launch_run_sums<T>(c, false, s);
       if (e != hipSuccess) return e;
     }
