@@ -574,6 +574,18 @@ void passes_by_option() {
       expect_passes("a node of no element", c, SEPARATE);
       CALL(wfx_destroy, c);
     }
+  // above 256 clusters, FP32-mixed: only what fits two work-groups on a CU
+  for (const bool tets : {false, true}) {
+    wfx_ctx *c = domain(tets ? Box(24, 24, 24, true) : Box(44, 44, 44), WFX_FP32_MIXED);
+    CALL(wfx_init, c, nullptr);
+    expect_passes("more than 256 clusters, plain", c, PAIRED);
+    CALL(wfx_set_cfl, c, 0.3);
+    expect_passes("more than 256 clusters, per-step time step", c, tets ? PAIRED : SEPARATE);
+    CALL(wfx_set_cfl, c, 0.0);
+    CALL(wfx_set_thermal, c, 1, 50.0, 460.0, 0.9);
+    expect_passes("more than 256 clusters, thermal", c, tets ? PAIRED : SEPARATE);
+    CALL(wfx_destroy, c);
+  }
   // 34 elements around an axis: more than the paired tables hold of a node
   Box fan(0);
   const int m = 34;

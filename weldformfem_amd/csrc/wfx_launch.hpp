@@ -78,7 +78,21 @@ int ensure_react_ring(wfx_ctx *c);
 
 // Whether a run takes the paired passes.  Thermal expansion does not: its
 // flat array divides by the masses the paired element pass is still forming.
-inline bool run_paired(const wfx_ctx *c) { return c->pair && !(c->thermal.on && c->thermal.exp_T != 0.0); }
+// Nor do FP32-mixed hexahedra in more than 256 clusters with thermal coupling or
+// the per-step CFL time step.  Above 256, two of the 512-thread work-groups have to
+// share a CU: the coupled element pass holds 136 registers a thread, more than
+// the 128 that leave room for two; the time step's reduction is repeated by every
+// work-group.  us per step in graph replay, paired / separate, 333 and 474
+// clusters: coupling 26.4 / 23.3 and 28.2 / 25.2, time step 24.9 / 22.5 and 26.4 /
+// 24.0, both with Johnson-Cook's law 36.1 / 27.6 and 38.2 / 29.2; neither 19.3 / 20.5
+// and 20.6 / 22.0.  (Tetrahedra, 366 and 504 clusters: coupling 16.3 / 16.4 and 17.6 /
+// 17.1, time step 18.0 / 17.3 and 19.3 / 18.0, but launched one by one 17.3 / 18.9,
+// 17.7 / 18.0, 19.3 / 18.7 and 19.7 / 22.6.)
+constexpr int kPairAlways = 256;
+inline bool run_paired(const wfx_ctx *c) {
+  if (!c->pair || (c->thermal.on && c->thermal.exp_T != 0.0)) return false;
+  return c->precision == 0 || c->n == 4 || c->ms.ncl <= kPairAlways || !(c->thermal.on || c->prm.cfl > 0.0);
+}
 // Whether a run takes the solo pass for all its steps but the last: a paired one
 // (whose tables it reads; every node then has a slot, so that as many slots as
 // nodes means no node of two clusters: meshes of up to 256 connected elements, or
