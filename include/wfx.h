@@ -15,6 +15,10 @@
  *
  * Threading: one context is used by one host thread at a time; kernels are
  * asynchronous on the stream passed in (NULL = default stream).
+ *
+ * Devices: a context's buffers are on the device that is current when its mesh
+ * is set.  Calls without a stream work on that device whichever is current;
+ * calls with one need a stream of it.
  */
 #ifndef WFX_H
 #define WFX_H
@@ -262,8 +266,10 @@ int wfx_step_api(wfx_ctx *ctx, wfx_stream s);
  * (see "check_status" under wfx_set_param); the same for wfx_step_fused and
  * wfx_graph_launch. */
 int wfx_run(wfx_ctx *ctx, int nsteps, double *reaction_hist, wfx_stream s);
-/* nsteps loop bodies of the same sequence regrouped into four fused kernels
- * per step (two element passes, two node passes).  Same state on return as
+/* nsteps loop bodies of the same sequence regrouped into fused kernels: four
+ * per step (two element passes, two node passes), two on small meshes (an
+ * element pass, a node pass), and in FP64 on the smallest up to 512 steps in
+ * one.  Same state on return as
  * wfx_run, except that the per-step intermediates detJ, dH*, str_rate,
  * rot_rate, strain_pl_incr, f_elem and f_hg are not kept (reading them fails
  * with WFX_ERR_STATE until a per-step API step has run). */
@@ -284,14 +290,17 @@ int wfx_reaction_force(wfx_ctx *ctx, int dim, double *out, wfx_stream s);
  * fused steps (max(reps, 10) steps per candidate, best of five rounds, two
  * sweeps), fastest kept (chosen[4], may be NULL; phases 1 and 3 run one
  * 256-thread work-group per element cluster and report 256); the state is
- * saved and restored around the measurement. */
+ * saved and restored around the measurement.  It times the four separate
+ * passes: on the small meshes whose runs take other ones (wfx_step_fused) only
+ * a run's last step, and the first of an even number, use the choice. */
 int wfx_autotune(wfx_ctx *ctx, int reps, int *chosen, wfx_stream s);
 /* Block sizes of the four fused phases (64/128/256/512 each; the element
  * passes' entries are accepted and not used). */
 int wfx_set_block_sizes(wfx_ctx *ctx, const int *block_sizes4);
 /* nsteps fused steps as wfx_step_fused runs them, with HIP events recorded on
  * stream s between the four passes: us4[k] = average duration of pass k+1 in
- * microseconds, in the order the passes run.  A measurement call with no
+ * microseconds, in the order the passes run (the four separate passes on
+ * every mesh).  A measurement call with no
  * reference counterpart; synchronous. */
 int wfx_time_fused_phases(wfx_ctx *ctx, int nsteps, double *us4, wfx_stream s);
 /* Capture nsteps fused steps (what wfx_step_fused(nsteps) enqueues) into a

@@ -303,13 +303,16 @@ constexpr double kCachedStepBytes[2] = {45e6, 240e6};
 // The line: in FP64 256 clusters, one work-group on each of the 256 CUs, in
 // FP32-mixed 512, two.  Below it the launches and dependent loads count and the
 // repeated node updates (1.7 times, hexahedra) are free; above it they are not.
-// us per step in graph replay, paired / separate: FP64 hexahedra 1 element 10.2 /
-// 11.2 (now the solo pass), 20^3 12.9 / 15.2, 40^3 (250 clusters) 17.4 / 20.9,
-// 42^3 (297) 26.2 / 24.1; tetrahedra 24 cells (255) 14.1 / 16.2, 32 cells 23.5 /
-// 21.6.  FP32-mixed hexahedra 40^3 14.6 / 18.4, 44^3 19.2 / 20.2, 48^3 (432) 19.2 /
-// 21.2, 50^3 (about 512) 27.1 / 24.5; tetrahedra 27 cells (363) 15.2 / 15.7, 30
-// cells (498) 15.9 / 16.5, 32 cells 18.5 / 17.9.  Launched one by one the separate
-// passes never take less than the 17 us their four launches cost.
+// us per step in graph replay, paired / separate, by clusters: FP64 hexahedra 20^3
+// (35) 12.9 / 15.1, 40^3 (250) 17.2 / 20.2, 42^3 (308) 25.6 / 23.6, 44^3 (333) 26.9 /
+// 24.6; tetrahedra, cells 24 (252) 13.4 / 15.3, 27 (366) 17.4 / 17.4, 32 (609) 23.3 /
+// 21.6.  FP32-mixed hexahedra 40^3 (250) 14.6 / 17.4, 44^3 (333) 19.1 / 20.6, 48^3
+// (432) 18.9 / 21.3, 48 x 51 x 50 (480) 19.2 / 21.4, 49^3 (574) 26.7 / 23.7, 50^3
+// (587) 26.5 / 24.3; tetrahedra 27 (366) 14.4 / 14.9, 30 (504) 15.6 / 15.8, 32 (609)
+// 18.4 / 17.5.  With Johnson-Cook's law, thermal coupling and the per-step time
+// step, FP64: 250 clusters 28.4 / 28.0, 432 50.1 / 35.4, 474 52.4 / 36.3; FP32-mixed has
+// a line of its own there (run_paired).  Launched one by one the separate passes
+// never take less than the 17 us their four launches cost.
 constexpr int kPairMaxClusters[2] = {256, 512};  // FP64, FP32-mixed
 constexpr int kPairMaxElems = 32;  // elements of a node
 // Entries per slot of the paired passes' table, or 0

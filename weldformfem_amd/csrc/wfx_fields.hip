@@ -6,8 +6,8 @@
 // transposition, the element permutation and the float conversion happen on
 // the device, in the same pass that crosses the host link.  Before, the host
 // did them in one thread over a pageable copy: the stress of the 4M-element
-// block (192 MB) took 92 ms to read, now 12; a nodal vector of one element 27
-// us, now 19.  What bounds it: the host link (57 GB/s pinned) and, for the
+// block (192 MB) took 92 ms to read, now 12; a nodal vector of one element 22
+// us, now 14 (where that way is still the shorter one it is taken: kCopyFrom).  What bounds it: the host link (57 GB/s pinned) and, for the
 // fresh pages of a new array, the host's page faults, which is why several
 // threads copy from the pinned ring to the caller's memory.
 #include <algorithm>
@@ -194,7 +194,7 @@ hipError_t launch_chunk(const FieldMove &f, long k0, long n, double *pinned) {
 class Copiers {
  public:
   Copiers(long chunks, int threads, void (*copy)(void *, long), void *arg)
-      : done_(chunks, 0), chunks_(chunks), copy_(copy), arg_(arg) {
+      : done_(chunks, 0), copy_(copy), arg_(arg) {
     try {
       for (int t = 0; t < threads; ++t) th_.emplace_back([this] { work(); });
     } catch (const std::exception &) {  // fewer threads (or none: the caller copies)
@@ -246,7 +246,7 @@ class Copiers {
     }
   }
   std::vector<char> done_;
-  long chunks_, ready_ = 0, next_ = 0;
+  long ready_ = 0, next_ = 0;
   void (*copy_)(void *, long);
   void *arg_;
   bool stop_ = false;
