@@ -27,7 +27,7 @@ SRC = os.path.join(HERE, "native", "host_calls_check.cpp")
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def program(tmp_path_factory):
     gxx = shutil.which("g++")
     if not gxx:
         pytest.skip("g++ not available")
@@ -42,6 +42,6 @@ CHECKS = ["adjoint_stray", "densities_captured", "densities_uniform", "other_dev
 
 
 @pytest.mark.parametrize("check", CHECKS)
-def test_host_calls(checker, check):
-    r = subprocess.run([checker, _lib.LIB_PATH, check], capture_output=True, text=True, timeout=100)
+def test_host_calls(program, check):
+    r = subprocess.run([program, _lib.LIB_PATH, check], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr
